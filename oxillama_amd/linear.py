@@ -13,7 +13,7 @@ import ctypes as C
 import numpy as np
 
 from . import capi
-from .quant import DimensionMismatch, HipKernel, QuantTensor, _check, _ptr, _u8
+from .quant import DimensionMismatch, HipKernel, QuantTensor, _check, _ptr, _u8, raw_stream as _stream
 
 
 class LoraAdapter:
@@ -80,10 +80,6 @@ class LoraStruct(C.Structure):
                 ("scale", C.c_float)]
 
 
-def _stream():
-    return HipKernel._stream()
-
-
 def _opt(t):
     return t.data_ptr() if t is not None else None
 
@@ -106,9 +102,10 @@ def linear_forward_dev(tensor_type, d_weights, d_out, out_features, in_features,
 
 def linear_forward_multi_dev(tensor_type, d_weights, d_acts, d_outs, out_features, in_features, d_biases=None):
     n = len(d_weights)
-    wp = (C.c_void_p * n)(*[w.data_ptr() for w in d_weights])
-    op = (C.c_void_p * n)(*[o.data_ptr() for o in d_outs])
-    bp = (C.c_void_p * n)(*[_opt(b) for b in d_biases]) if d_biases is not None else None
+    pointers = C.c_void_p * n
+    wp = pointers(*[w.data_ptr() for w in d_weights])
+    op = pointers(*[o.data_ptr() for o in d_outs])
+    bp = pointers(*[_opt(b) for b in d_biases]) if d_biases is not None else None
     of = (C.c_size_t * n)(*out_features)
     _check(capi.load().oxq_linear_forward_multi_dev(int(tensor_type), n, wp, d_acts.data_ptr(), bp, op, of,
                                                     in_features, _stream()))
@@ -136,7 +133,7 @@ def gate_up_swiglu_dev(tensor_type, d_gate, d_up, d_acts_q8, d_h, d_out_q8, inte
     """ffn_gate + ffn_up + SwiGLU + Q8_0 quantizer of h in one launch (d_h optional)."""
     _check(capi.load().oxq_ffn_gate_up_swiglu_q8_dev(int(tensor_type), d_gate.data_ptr(), d_up.data_ptr(),
                                                      d_acts_q8.data_ptr(), d_h.data_ptr() if d_h is not None else None,
-                                                     d_out_q8.data_ptr(), intermediate, hidden, HipKernel._stream()))
+                                                     d_out_q8.data_ptr(), intermediate, hidden, _stream()))
 
 
 def ffn_workspace_bytes(hidden, intermediate):

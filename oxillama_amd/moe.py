@@ -5,7 +5,12 @@ Routing follows MoeFfn::forward, crates/oxillama-arch/src/common/moe.rs:197-248:
 numerically stable softmax over the router logits, the top-k experts by descending
 softmax weight, weights renormalised over the selected experts.  All arithmetic is fp32.
 """
+import ctypes as C
+
 import numpy as np
+
+from . import capi
+from .quant import _check, raw_stream
 
 
 def route_top_k(logits, top_k):
@@ -50,29 +55,22 @@ def token_rows(offsets, token, slot, n_tokens, k):
 def route_dev(d_router, d_x, n_tokens, n_experts, hidden, top_k, d_experts, d_weights, d_offsets, d_pair_token,
               d_token_rows):
     """Steps 1-4 of MoeFfn::forward (moe.rs:189-250) and the grouping, on torch CUDA tensors."""
-    from . import capi
-    from .quant import HipKernel, _check
     _check(capi.load().oxq_moe_route_dev(d_router.data_ptr(), d_x.data_ptr(), n_tokens, n_experts, hidden, top_k,
                                          d_experts.data_ptr(), d_weights.data_ptr(), d_offsets.data_ptr(),
-                                         d_pair_token.data_ptr(), d_token_rows.data_ptr(), HipKernel._stream()))
+                                         d_pair_token.data_ptr(), d_token_rows.data_ptr(), raw_stream()))
 
 
 def gather_quantize_dev(d_x, d_pair_token, n_pairs, hidden, d_out_q8):
-    from . import capi
-    from .quant import HipKernel, _check
     _check(capi.load().oxq_moe_gather_quantize_q8_0_dev(d_x.data_ptr(), d_pair_token.data_ptr(), n_pairs, hidden,
-                                                        d_out_q8.data_ptr(), HipKernel._stream()))
+                                                        d_out_q8.data_ptr(), raw_stream()))
 
 
 def combine_dev(d_y_pairs, d_token_rows, d_weights, n_tokens, top_k, hidden, d_out):
-    from . import capi
-    from .quant import HipKernel, _check
     _check(capi.load().oxq_moe_combine_dev(d_y_pairs.data_ptr(), d_token_rows.data_ptr(), d_weights.data_ptr(),
-                                           n_tokens, top_k, hidden, d_out.data_ptr(), HipKernel._stream()))
+                                           n_tokens, top_k, hidden, d_out.data_ptr(), raw_stream()))
 
 
 def moe_ffn_workspace_bytes(types, n_pairs, hidden, intermediate):
-    from . import capi
     tg, tu, td = (int(t) for t in types)
     return capi.load().oxq_moe_ffn_workspace_bytes(tg, tu, td, n_pairs, hidden, intermediate)
 
@@ -81,19 +79,16 @@ def moe_ffn_dev(gate, up, down, n_experts, d_x, n_tokens, top_k, d_offsets, d_pa
                 max_rows, d_out, hidden, intermediate, workspace):
     """MoeFfn::forward (moe.rs:184-258) after routing, for n_tokens tokens on torch CUDA tensors, current
     stream.  gate / up / down: (tensor_type, device tensor of all experts, bytes per expert)."""
-    from . import capi
-    from .quant import HipKernel, _check
     args = []
     for t, d_w, stride in (gate, up, down):
         args += [int(t), d_w.data_ptr(), stride]
     _check(capi.load().oxq_moe_ffn_dev(*args, n_experts, d_x.data_ptr(), n_tokens, top_k, d_offsets.data_ptr(),
                                        d_pair_token.data_ptr(), d_token_rows.data_ptr(), d_weights.data_ptr(),
                                        max_rows, d_out.data_ptr(), hidden, intermediate, workspace.data_ptr(),
-                                       workspace.numel(), HipKernel._stream()))
+                                       workspace.numel(), raw_stream()))
 
 
 def moe_forward_workspace_bytes(types, n_tokens, top_k, n_experts, hidden, intermediate):
-    from . import capi
     tg, tu, td = (int(t) for t in types)
     return capi.load().oxq_moe_forward_workspace_bytes(tg, tu, td, n_tokens, top_k, n_experts, hidden, intermediate)
 
@@ -101,14 +96,12 @@ def moe_forward_workspace_bytes(types, n_tokens, top_k, n_experts, hidden, inter
 def moe_forward_dev(gate, up, down, n_experts, d_router, d_x, n_tokens, top_k, d_out, hidden, intermediate, workspace):
     """MoeFfn::forward (moe.rs:184-258) for n_tokens tokens on torch CUDA tensors, current stream: routing and
     the experts in one call, tables in the workspace.  gate / up / down as in moe_ffn_dev."""
-    from . import capi
-    from .quant import HipKernel, _check
     args = []
     for t, d_w, stride in (gate, up, down):
         args += [int(t), d_w.data_ptr(), stride]
     _check(capi.load().oxq_moe_forward_dev(*args, n_experts, d_router.data_ptr(), d_x.data_ptr(), n_tokens, top_k,
                                            d_out.data_ptr(), hidden, intermediate, workspace.data_ptr(),
-                                           workspace.numel(), HipKernel._stream()))
+                                           workspace.numel(), raw_stream()))
 
 
 class MoeFfn:
@@ -130,9 +123,6 @@ class MoeFfn:
         return self.forward_batch(x, 1, out)
 
     def forward_batch(self, x, n_tokens, out=None):
-        import ctypes as C
-        from . import capi
-        from .quant import _check
         x = np.ascontiguousarray(x, dtype=np.float32).ravel()
         if out is None:
             out = np.zeros(n_tokens * self.hidden_size, dtype=np.float32)

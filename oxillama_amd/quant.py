@@ -171,6 +171,20 @@ def _ptr(arr):
     return arr.ctypes.data_as(C.c_void_p)
 
 
+_torch_c = None
+
+
+def raw_stream():
+    """torch's current stream as an integer handle.  torch.cuda.current_stream() builds a Stream object, 2.7 us a call
+    and as long as the launch itself; the two calls below take 0.2 us."""
+    global _torch_c
+    if _torch_c is None:
+        import torch
+        torch.cuda.init()
+        _torch_c = torch._C
+    return _torch_c._cuda_getCurrentRawStream(_torch_c._cuda_getDevice())
+
+
 def quantize_f32_to_q8_0(data):
     """Q/quantize.rs:58: f32[n] -> n/32 Q8_0 blocks (34 bytes each), on the GPU."""
     lib = capi.load()
@@ -235,13 +249,12 @@ class HipKernel:
     # -- device-pointer route (torch CUDA tensors, current stream) ----------
     @staticmethod
     def _stream():
-        import torch
-        return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+        return C.c_void_p(raw_stream())
 
     def matvec_q8_fused_dev(self, d_weights, d_acts, d_out, n_rows, n_cols, accumulate=True):
         _check(self._lib.oxq_matvec_q8_fused_dev(self.tensor_type, d_weights.data_ptr(), d_acts.data_ptr(),
                                                  d_out.data_ptr(), n_rows, n_cols, int(accumulate),
-                                                 self._stream()))
+                                                 raw_stream()))
 
     def matvec_q8_fused_multi_dev(self, d_weights, d_acts, d_outs, n_rows, n_cols, accumulate=True):
         """Up to 4 matrices of one shape sharing d_acts, one launch (wq/wk/wv, ffn_gate/ffn_up)."""
@@ -250,19 +263,19 @@ class HipKernel:
         wp = (C.c_void_p * n)(*[w.data_ptr() for w in d_weights])
         op = (C.c_void_p * n)(*[o.data_ptr() for o in d_outs])
         _check(self._lib.oxq_matvec_q8_fused_multi_dev(self.tensor_type, n, wp, d_acts.data_ptr(), op, n_rows, n_cols,
-                                                       int(accumulate), self._stream()))
+                                                       int(accumulate), raw_stream()))
 
     def gemv_dev(self, d_weights, d_x, d_out, n_rows, n_cols, accumulate=False):
         """fp32 activations in, quantized to Q8_0 inside the kernel (one launch)."""
         _check(self._lib.oxq_gemv_dev(self.tensor_type, d_weights.data_ptr(), d_x.data_ptr(), d_out.data_ptr(),
-                                      n_rows, n_cols, int(accumulate), self._stream()))
+                                      n_rows, n_cols, int(accumulate), raw_stream()))
 
     def gemv_f32_dev(self, d_weights, d_x, d_out, n_rows, n_cols, accumulate=False, d_bias=None):
         """QuantKernel::gemv with the reference's numerics: fp32 activations against weights dequantized in
         registers (oxq_gemv_f32_dev)."""
         _check(self._lib.oxq_gemv_f32_dev(self.tensor_type, d_weights.data_ptr(), d_x.data_ptr(),
                                           d_bias.data_ptr() if d_bias is not None else None, d_out.data_ptr(),
-                                          n_rows, n_cols, int(accumulate), self._stream()))
+                                          n_rows, n_cols, int(accumulate), raw_stream()))
 
     def gemv_multi_dev(self, d_weights, d_x, d_outs, n_rows, n_cols, accumulate=False):
         import ctypes as C
@@ -270,7 +283,7 @@ class HipKernel:
         wp = (C.c_void_p * n)(*[w.data_ptr() for w in d_weights])
         op = (C.c_void_p * n)(*[o.data_ptr() for o in d_outs])
         _check(self._lib.oxq_gemv_multi_dev(self.tensor_type, n, wp, d_x.data_ptr(), op, n_rows, n_cols,
-                                            int(accumulate), self._stream()))
+                                            int(accumulate), raw_stream()))
 
     def gemm_workspace_bytes(self, m, n, k):
         return self._lib.oxq_gemm_q8_workspace_bytes(self.tensor_type, m, n, k)
@@ -280,25 +293,25 @@ class HipKernel:
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_len = workspace.numel() if workspace is not None else 0
         _check(self._lib.oxq_gemm_q8_dev(self.tensor_type, d_weights.data_ptr(), d_acts.data_ptr(),
-                                         d_out.data_ptr(), m, n, k, int(accumulate), ws_ptr, ws_len, self._stream()))
+                                         d_out.data_ptr(), m, n, k, int(accumulate), ws_ptr, ws_len, raw_stream()))
 
     def gemm_q8_static_dev(self, d_weights, d_acts, d_out, m, n, k, accumulate=False):
         """gemm_q8_dev on the library's static device scratch: allocates nothing (shapes up to the scratch size)."""
         _check(self._lib.oxq_gemm_q8_static_dev(self.tensor_type, d_weights.data_ptr(), d_acts.data_ptr(),
-                                                d_out.data_ptr(), m, n, k, int(accumulate), self._stream()))
+                                                d_out.data_ptr(), m, n, k, int(accumulate), raw_stream()))
 
     def gemm_block_sums_dev(self, d_weights, d_acts, d_out, d_sums, m, n, k, workspace=None):
         ws_ptr = workspace.data_ptr() if workspace is not None else None
         ws_len = workspace.numel() if workspace is not None else 0
         _check(self._lib.oxq_gemm_block_sums_dev(self.tensor_type, d_weights.data_ptr(), d_acts.data_ptr(),
                                                  d_out.data_ptr(), d_sums.data_ptr(), m, n, k, ws_ptr, ws_len,
-                                                 self._stream()))
+                                                 raw_stream()))
 
     def gemm_scaled_sums_dev(self, d_weights, d_acts, d_out, d_sums, m, n, k, workspace):
         """The prefill kernel's debug dump: sub-block scale times integer group sum per (token, row, sub-block)."""
         _check(self._lib.oxq_gemm_scaled_sums_dev(self.tensor_type, d_weights.data_ptr(), d_acts.data_ptr(),
                                                   d_out.data_ptr(), d_sums.data_ptr(), m, n, k, workspace.data_ptr(),
-                                                  workspace.numel(), self._stream()))
+                                                  workspace.numel(), raw_stream()))
 
     def moe_gemm_workspace_bytes(self, total_rows, n, k):
         return self._lib.oxq_moe_gemm_q8_workspace_bytes(self.tensor_type, total_rows, n, k)
@@ -311,16 +324,16 @@ class HipKernel:
                                              d_acts.data_ptr(), d_offsets.data_ptr(), total_rows, max_rows,
                                              d_out.data_ptr(), d_sums.data_ptr() if d_sums is not None else None,
                                              n, k, int(accumulate), workspace.data_ptr(), workspace.numel(),
-                                             self._stream()))
+                                             raw_stream()))
 
     def block_sums_dev(self, d_weights, d_acts, d_sums, n_rows, n_cols):
         _check(self._lib.oxq_block_sums_dev(self.tensor_type, d_weights.data_ptr(), d_acts.data_ptr(),
-                                            d_sums.data_ptr(), n_rows, n_cols, self._stream()))
+                                            d_sums.data_ptr(), n_rows, n_cols, raw_stream()))
 
 
 def quantize_q8_0_dev(d_x, d_out):
     lib = capi.load()
-    _check(lib.oxq_quantize_q8_0_dev(d_x.data_ptr(), d_x.numel(), d_out.data_ptr(), HipKernel._stream()))
+    _check(lib.oxq_quantize_q8_0_dev(d_x.data_ptr(), d_x.numel(), d_out.data_ptr(), raw_stream()))
 
 
 class KernelDispatcher:
