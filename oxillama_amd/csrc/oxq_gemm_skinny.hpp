@@ -655,18 +655,35 @@ __attribute__((amdgpu_waves_per_eu(skinny_waves_per_simd<F, NT, WAVES, TT, PER>(
 void gemm_skinny_kernel(
     const uint8_t *__restrict__ W, const uint8_t *__restrict__ A, float *__restrict__ out, int32_t *__restrict__ sums,
     uint32_t m, uint32_t n, uint32_t k, int accumulate, const float *__restrict__ bias, const int32_t *__restrict__ offsets, size_t w_stride,
-    float *__restrict__ partial, uint32_t sb_per_split, uint32_t grouped_splits) {
-    // row group; expert (grouped form); split of k: blockIdx.y is the expert, or the split (one matrix), or, in the
-    // grouped form with k split, expert * grouped_splits + split
+    float *__restrict__ partial, uint32_t sb_per_split, uint32_t grouped_splits, uint32_t n_experts) {
+    // row group; in the grouped form blockIdx.y = place * grouped_splits + split of k, with one place per expert (its
+    // first 16 * TT rows) and one for every further 16 * TT rows that the groups together can come to (each its own
+    // pass over the expert's weights); one matrix: blockIdx.y is the split, blockIdx.z the pass.
+    // The launch is shaped for the usual group.  One token tile: the further passes are dispatched first, so that the
+    // few work groups of the groups that overflow run beside the first pass instead of after it.  Two tiles: overflow
+    // is rare and comes last.  Places that no group needs exit.  (Walking the passes in a loop inside the work group
+    // was measured 7-9 % slower on every shape: the compiler allocates the looped body worse.)
     const uint32_t rg = blockIdx.x;
-    uint32_t gy = !offsets ? 0 : partial ? blockIdx.y / grouped_splits : blockIdx.y;
-    const uint32_t ks = !partial ? 0 : offsets ? blockIdx.y % grouped_splits : blockIdx.y;
+    uint32_t gy = 0, ks = 0, pass = blockIdx.z;
+    bool first = true;
+    if (!offsets) {
+        if (partial) ks = blockIdx.y;
+        if (TT == 1 && gridDim.z > 1 && blockIdx.z < 2) pass = 1 - blockIdx.z;
+    } else {
+        const uint32_t splits = partial ? grouped_splits : 1u;
+        const uint32_t place = blockIdx.y / splits, further = gridDim.y / splits - n_experts;
+        ks = blockIdx.y % splits;
+        first = TT == 1 ? place >= further : place < n_experts;
+        gy = TT == 1 && first ? place - further : place;
+        pass = 0;
+        if (!first && !find_group_tile<1>(offsets, n_experts, 16 * TT, TT == 1 ? place : place - n_experts, gy, pass)) return;
+    }
     if constexpr (TT == 2) {
         // Groups of two token tiles take longer than groups of one: hand the experts out largest group first
         // (ties by index), so that the long work groups start in the first round and the short ones fill the end.
         // Lane e ranks expert e; the work group takes the expert whose rank is its place in the grid.
-        const uint32_t n_e = offsets ? gridDim.y / (partial ? grouped_splits : 1u) : 0u;
-        if (n_e > 1 && n_e <= 64) {
+        const uint32_t n_e = offsets ? n_experts : 0u;
+        if (first && n_e > 1 && n_e <= 64) {
             const uint32_t lane = threadIdx.x & 63, e = min(lane, n_e - 1);
             const int size_e = offsets[e + 1] - offsets[e];
             uint32_t rank = 0;
@@ -683,14 +700,6 @@ void gemm_skinny_kernel(
         tok0 = (uint32_t)offsets[gy];
         tok_end = (uint32_t)offsets[gy + 1];
     }
-    // blockIdx.z = which 16 * TT token rows of the group: the launch is shaped for the usual group, a larger one
-    // takes further work groups per row group (each its own pass over the weights); the rest exit here.
-    // (One token tile: the second pass is dispatched before the first, so that the few work groups of the groups
-    // that overflow run beside the first pass instead of after it; further passes, nearly always empty, come last.
-    // Two tiles: overflow is rare, and a layer of work groups that only exit would delay the start.  Walking the
-    // passes in a loop inside the work group instead of by layers of the grid was measured 7-9 % slower on every
-    // shape: the compiler allocates the looped body worse.)
-    const uint32_t pass = (TT == 1 && gridDim.z > 1 && blockIdx.z < 2) ? 1 - blockIdx.z : blockIdx.z;
     const uint32_t tokb = tok0 + pass * (16 * TT);
     if (tokb >= tok_end) return;  // the whole work group
     if constexpr (TT == 2) {
@@ -771,11 +780,8 @@ static hipError_t launch_skinny_shape(const GemmArgs &a, const TilePlan &p, hipS
     const size_t strips = (size_t)WAVES * skinny_wave_lds<F, NT>();
     auto kern = &gemm_skinny_kernel<F, NT, WAVES, TT, PER, DUMP>;
     const size_t lds = (size_t)PER * 8 * TT * skinny_act_bytes<F>() + strips;
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       (int)lds);
+    hipError_t e = allow_lds(reinterpret_cast<const void *>(kern), lds);
     if (e != hipSuccess) return e;
-    // token passes: as many as the largest group can need (max_rows is the caller's bound, all rows if unknown)
-    const uint32_t group_rows = a.offsets ? a.max_rows : a.m;
     const uint32_t splits = !split_k ? 1 : a.offsets ? SKINNY_GROUPED_SPLITS : skinny_splits(a.n, a.k);
     float *const partial = splits > 1 ? p.partial : nullptr;
     if (splits > 1 && !partial) return hipErrorNotSupported;
@@ -783,11 +789,13 @@ static hipError_t launch_skinny_shape(const GemmArgs &a, const TilePlan &p, hipS
     const uint32_t sb_per_split = a.offsets ? a.k / 256 / SKINNY_GROUPED_SPLITS : skinny_sb_per_split(a.n, a.k);
     if (splits > 1 && a.offsets && a.k % (512 * SKINNY_GROUPED_SPLITS) != 0) return hipErrorNotSupported;
     const uint32_t row_groups = (a.n + 16 * NT * WAVES - 1) / (16 * NT * WAVES);
-    const dim3 grid(row_groups, a.offsets ? a.n_experts * splits : splits, (group_rows + 16 * TT - 1) / (16 * TT));
+    // grouped: a place per expert and one per further token tile that the groups together can come to
+    const uint32_t further = a.offsets ? group_tiles_bound(a.m, a.max_rows, a.n_experts, 16 * TT) - a.n_experts : 0;
+    const dim3 grid(row_groups, (a.offsets ? a.n_experts + further : 1) * splits, a.offsets ? 1 : (a.m + 16 * TT - 1) / (16 * TT));
     if (grid.z > 65535 || grid.y > 65535) return hipErrorNotSupported;
     note_launch("gemm_skinny_kernel", F::TYPE, NT, WAVES, TT, PER, grid.x, grid.y * grid.z, 64 * WAVES);
     hipLaunchKernelGGL(kern, grid, dim3(64 * WAVES), lds, stream, a.W, a.A, a.out, a.sums, a.m, a.n, a.k,
-                       a.accumulate, a.bias, a.offsets, a.w_stride, partial, sb_per_split, splits);
+                       a.accumulate, a.bias, a.offsets, a.w_stride, partial, sb_per_split, splits, a.offsets ? a.n_experts : 0u);
     e = hipGetLastError();
     if (e != hipSuccess || !partial) return e;
     if (a.defer_reduce && !a.accumulate && !a.bias) {  // the caller adds the splits' sums (in index order, as below)

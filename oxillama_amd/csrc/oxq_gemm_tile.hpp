@@ -394,6 +394,46 @@ __host__ __device__ __forceinline__ uint32_t tile_padded_sub_blocks(uint32_t k) 
 // activation bytes, P, the f16 scales, then the half planes: 32 + 4 + 2 bytes per token block before them).
 __host__ __device__ __forceinline__ size_t tile_p16_offset(size_t nsb, size_t mpad) { return nsb * mpad * 6; }
 
+// Token tiles that expert groups of `total` rows in all, none larger than max_rows, can come to: every expert rounds
+// up once, so at most total / tile_rows + n_experts, and never more than every expert at its largest.  (A grid of
+// n_experts times the largest group's tiles, as it was before, is far too large where the rows spread over many
+// experts: 4096 rows on 128 experts came to 128 x 128 tiles x 16 row groups = 262144 work groups, all but 2300 of them
+// empty, and starting those alone took most of the launch.)
+inline uint32_t group_tiles_bound(uint32_t total, uint32_t max_rows, uint32_t n_experts, uint32_t tile_rows) {
+    const uint64_t spread = (uint64_t)total / tile_rows + n_experts, each = (uint64_t)n_experts * ((max_rows + tile_rows - 1) / tile_rows);
+    return (uint32_t)(spread < each ? spread : each);
+}
+// The expert of token tile `ti` when every expert's rows are cut into tiles of tile_rows, and which of the expert's
+// tiles it is; false: there are fewer tiles.  FROM = 1: the experts' first tiles are left out of the count.  The 64
+// lanes count 64 experts' tiles at a time and scan them; the answers are wave-uniform.
+template <uint32_t FROM = 0>
+__device__ __forceinline__ bool find_group_tile(const int32_t *__restrict__ offsets, uint32_t n_experts, uint32_t tile_rows,
+                                                uint32_t ti, uint32_t &expert, uint32_t &tile) {
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t base = 0;
+    for (uint32_t e0 = 0; e0 < n_experts; e0 += 64) {
+        const uint32_t e = e0 + lane;
+        uint32_t incl = 0;
+        if (e < n_experts) incl = ((uint32_t)(offsets[e + 1] - offsets[e]) + tile_rows - 1) / tile_rows;
+        if (FROM) incl -= min(incl, FROM);
+        const uint32_t mine = incl;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t up = (uint32_t)__shfl_up((int)incl, d, 64);
+            if (lane >= (uint32_t)d) incl += up;
+        }
+        const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+        if (ti < base + all) {
+            const int at = __ffsll((unsigned long long)__ballot(ti < base + incl)) - 1;
+            expert = e0 + (uint32_t)at;
+            tile = FROM + ti - base - (uint32_t)__builtin_amdgcn_readlane((int)(incl - mine), at);
+            return true;
+        }
+        base += all;
+    }
+    return false;
+}
+
 // Work group = 4 waves as WM (tokens) x WN (weight rows); each wave owns MT x NT MFMA tiles
 // of 32 x 32: a (32*MT*WM)-token x (32*NT*WN)-row tile per work group.  Lane l: c = l % 32
 // is the token (A operand) / weight row (B operand) / output column it feeds, h = l / 32
@@ -412,14 +452,15 @@ __host__ __device__ __forceinline__ size_t tile_p16_offset(size_t nsb, size_t mp
 // same XCD at the same time (ids are dealt round-robin to the 8 XCDs), which turns their
 // weight reads into L2 hits.
 //
-// Grouped form (mixture-of-experts): blockIdx.y = expert; expert e multiplies the token
-// rows offsets[e] .. offsets[e+1]-1 by the weights at W + e * w_stride.
+// Grouped form (mixture-of-experts, n_experts != 0): expert e multiplies the token rows offsets[e] .. offsets[e+1]-1
+// by the weights at W + e * w_stride.  Only the device knows how many token tiles each expert needs: the grid holds as
+// many as all experts together can (group_tiles_bound), and a work group finds the expert of its tile by itself.
 template <class F, int MT, int NT, int WM, int DIST, bool DUMP, int ADIST>
 __device__ __forceinline__ void gemm_tile_body(
     const uint8_t *__restrict__ W, const uint8_t *__restrict__ q8t, const float *__restrict__ P,
     const uint16_t *__restrict__ da16, float *__restrict__ out, int32_t *__restrict__ sums, uint32_t m, uint32_t mpad,
     uint32_t n, uint32_t k, int accumulate, const float *__restrict__ bias, uint32_t m_tiles, uint32_t n_tiles,
-    const int32_t *__restrict__ offsets,
+    const int32_t *__restrict__ offsets, uint32_t n_experts,
     size_t w_stride) {
     constexpr bool SPLITK = WM == 0;  // the four waves share one tile and each walk a quarter of k
     constexpr int WMX = SPLITK ? 1 : WM, WN = SPLITK ? 1 : 4 / WMX;
@@ -458,15 +499,15 @@ __device__ __forceinline__ void gemm_tile_body(
     const uint32_t xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
     uint32_t n_tile = (loc / m_tiles) * 8 + xcd, m_tile = loc % m_tiles;
     uint32_t row0 = 0, row_end = m;
-    if (offsets) {
-        // expert groups: token tiles outermost, so that the tiles past an expert's rows (the grid is
-        // sized for the largest group) form one run at the end instead of sitting between live ones
+    if (n_experts) {
+        // expert groups: token tiles outermost, so that the tiles the experts do not need form one run at the end
         const uint32_t n_groups = (n_tiles + 7) / 8;
-        m_tile = loc / n_groups;
         n_tile = (loc % n_groups) * 8 + xcd;
-        row0 = (uint32_t)offsets[blockIdx.y];
-        row_end = (uint32_t)offsets[blockIdx.y + 1];
-        W += (size_t)blockIdx.y * w_stride;
+        uint32_t expert = 0;
+        if (!find_group_tile(offsets, n_experts, WG_TOK, loc / n_groups, expert, m_tile)) return;  // whole work group
+        row0 = (uint32_t)offsets[expert];
+        row_end = (uint32_t)offsets[expert + 1];
+        W += (size_t)expert * w_stride;
     }
     if (n_tile >= n_tiles || row0 + m_tile * WG_TOK >= row_end) return;  // whole work group
     const uint32_t m_wg = row0 + m_tile * WG_TOK, n_wg = n_tile * WG_ROWS;
@@ -756,9 +797,9 @@ __device__ __forceinline__ void gemm_tile_body(
         const uint8_t *__restrict__ W, const uint8_t *__restrict__ q8t, const float *__restrict__ P,                \
         const uint16_t *__restrict__ da16, float *__restrict__ out, int32_t *__restrict__ sums, uint32_t m,         \
         uint32_t mpad, uint32_t n, uint32_t k, int accumulate, const float *__restrict__ bias, uint32_t m_tiles,   \
-        uint32_t n_tiles, const int32_t *__restrict__ offsets, size_t w_stride) {                                   \
+        uint32_t n_tiles, const int32_t *__restrict__ offsets, uint32_t n_experts, size_t w_stride) {               \
         gemm_tile_body<F, MT, NT, WM, DIST, DUMP, ADIST>(W, q8t, P, da16, out, sums, m, mpad, n, k, accumulate,     \
-                                                         bias, m_tiles, n_tiles, offsets, w_stride);                \
+                                                         bias, m_tiles, n_tiles, offsets, n_experts, w_stride);     \
     }
 OXQ_TILE_KERNEL(gemm_tile_kernel, 2)
 OXQ_TILE_KERNEL(gemm_tile_kernel_occ3, 3)
@@ -781,20 +822,19 @@ bool tile_needs_p16_more(uint32_t type);
 template <class F, int MT, int NT, int WM, int DIST, bool DUMP, int OCC = 2, int ADIST = 1>
 static hipError_t launch_tile(const GemmArgs &a, const TilePlan &p, hipStream_t stream) {
     constexpr uint32_t WG_TOK = 32 * MT * (WM ? WM : 1), WG_ROWS = 32 * NT * (WM ? 4 / WM : 1);
-    const uint32_t rows = a.offsets ? a.max_rows : a.m;
-    const uint32_t m_tiles = (rows + WG_TOK - 1) / WG_TOK, n_tiles = (a.n + WG_ROWS - 1) / WG_ROWS;
-    const dim3 grid(8 * ((n_tiles + 7) / 8) * m_tiles, a.offsets ? a.n_experts : 1);
+    const uint32_t m_tiles = a.offsets ? group_tiles_bound(a.m, a.max_rows, a.n_experts, WG_TOK) : (a.m + WG_TOK - 1) / WG_TOK;
+    const uint32_t n_tiles = (a.n + WG_ROWS - 1) / WG_ROWS;
+    const dim3 grid(8 * ((n_tiles + 7) / 8) * m_tiles);
     const size_t lds = (size_t)tile_padded_sub_blocks(a.k) * WG_TOK * 2;
     auto kern = &gemm_tile_kernel<F, MT, NT, WM, DIST, DUMP, ADIST>;
     if constexpr (OCC == 3) kern = &gemm_tile_kernel_occ3<F, MT, NT, WM, DIST, DUMP, ADIST>;
     if (lds > 32 * 1024) {  // beyond the default dynamic LDS limit: opt in (up to the 160 KB of a CU)
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        hipError_t e = allow_lds(reinterpret_cast<const void *>(kern), lds);
         if (e != hipSuccess) return e;
     }
     note_launch(OCC == 3 ? "gemm_tile_kernel_occ3" : "gemm_tile_kernel", F::TYPE, MT, NT, WM, DIST, grid.x, grid.y, 256);
     hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, a.W, p.q8t, p.P, p.da16, a.out, a.sums, a.m, p.mpad, a.n,
-                       a.k, a.accumulate, a.bias, m_tiles, n_tiles, a.offsets, a.w_stride);
+                       a.k, a.accumulate, a.bias, m_tiles, n_tiles, a.offsets, a.offsets ? a.n_experts : 0u, a.w_stride);
     return hipGetLastError();
 }
 

@@ -74,6 +74,10 @@ extern std::atomic<size_t> g_phase_cap;
 // Number of compute units of the current device (cached per device).
 uint32_t device_cus();
 
+// Opt kernel `kern` in to `lds` bytes of dynamic LDS on the current device: a runtime call the first time a thread
+// asks, a table lookup afterwards (the runtime call costs about as much as a launch).
+hipError_t allow_lds(const void *kern, size_t lds);
+
 hipError_t launch_gemv_q8(uint32_t type, const GemvArgs &a, hipStream_t stream);
 // QuantKernel::gemv as the reference computes it (fp32 activations, weights dequantized in registers):
 // out[r] = (old ? old[r] : 0) + W[r, :] . x.  hipErrorNotSupported: no such kernel for this format.

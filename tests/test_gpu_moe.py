@@ -503,3 +503,27 @@ def test_moe_forward_on_device_pointers_degenerate(hip):
     with pytest.raises(KernelError):
         moe.moe_forward_dev((O.Q4_K, empty, 0), (O.Q4_K, empty, 0), (O.Q4_K, empty, 0), 4, empty, d_x, 2, 0, out, hidden,
                             256, empty)
+
+
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q6_K, O.Q4_0, O.Q8_0], ids=lambda t: O.NAMES[t])
+@pytest.mark.parametrize("n_exp,rows", [(65, (0, 1, 33, 2)), (130, (32, 0, 0, 65, 31)), (3, (16, 17, 129)), (70, (3,))], ids=str)
+def test_grouped_matmul_finds_every_tile_of_uneven_groups(hip, ref, t, n_exp, rows):
+    """The work groups look the expert of their token tile up in the offsets: more experts than a wave has lanes, empty
+    groups, groups one row past a tile, the last expert's last tile."""
+    n, k = 96, 512
+    sizes = [rows[e % len(rows)] for e in range(n_exp)]
+    offsets = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    total = int(offsets[-1])
+    say("grouped tiles", O.NAMES[t], n_exp, rows, total)
+    w = expert_weights(t, 700, n_exp, n, k)
+    x = synth.normal_f32(701, total * k).reshape(total, k)
+    stride = w.size // n_exp
+    acts = np.concatenate([ref.quantize_q8_0(r) for r in x])
+    kern = hip.HipKernel(t)
+    ws = torch.empty(kern.moe_gemm_workspace_bytes(total, n, k), dtype=torch.uint8, device=DEV)
+    for max_rows in (0, max(sizes)):
+        y = torch.full((total, n), float("nan"), dtype=torch.float32, device=DEV)
+        kern.moe_gemm_q8_dev(dev(w), stride, n_exp, dev(acts), dev(offsets), total, max_rows, y, n, k, ws)
+        want = np.concatenate([O.gemm_q8(t, w[e * stride:(e + 1) * stride], x[offsets[e]:offsets[e + 1]].copy(), sizes[e], n, k)
+                               for e in range(n_exp) if sizes[e]])
+        assert_close(host(y).reshape(total, n), want.reshape(total, n), f"max_rows {max_rows}")
