@@ -76,6 +76,29 @@ struct Scratch {
     }
 };
 
+// A growable host buffer that the GPU reads and writes in place.
+struct Pinned {
+    void *ptr = nullptr;
+    size_t cap = 0;
+    int reserve(size_t n) {
+        if (n <= cap) return OXQ_OK;
+        release();
+        const size_t want = n + n / 4 + 256;
+        hipError_t e = hipHostMalloc(&ptr, want, hipHostMallocPortable);
+        if (e != hipSuccess) {
+            ptr = nullptr;
+            return fail_hip(e, "hipHostMalloc(staging)");
+        }
+        cap = want;
+        return OXQ_OK;
+    }
+    void release() {
+        if (ptr) (void)hipHostFree(ptr);
+        ptr = nullptr;
+        cap = 0;
+    }
+};
+
 struct CacheKey {
     const void *ptr;
     size_t len;
@@ -110,6 +133,10 @@ struct State {
     uint64_t cache_pin = UINT64_MAX;  // entries used after this tick belong to the call in progress: not evicted
     Scratch s_weights, s_acts, s_x, s_out, s_sums, s_work, s_bias, s_lora_a, s_lora_b, s_lora_r;
     Scratch s_moe_up, s_moe_down, s_moe_tables;
+    // host-slice calls of a few vectors: input and output staged in memory the GPU reaches over the bus, and the word the
+    // last kernel of a call sets to the call's number
+    Pinned h_in, h_out, h_flag;
+    uint32_t h_seq = 0;
     std::atomic<bool> fuse_swiglu{true};  // oxq_ffn_swiglu_dev: gate, up, SwiGLU and the quantizer of h in one launch where possible
 };
 State g;
@@ -120,30 +147,27 @@ State g;
 uint64_t fingerprint(const uint8_t *p, size_t len, bool whole) {
     uint64_t h = 1469598103934665603ull ^ len;
     const size_t chunk = 64, samples = 64;
-    if (whole) {
-        uint64_t lanes[4] = {h, h ^ 0x9E3779B97F4A7C15ull, h ^ 0xC2B2AE3D27D4EB4Full, h ^ 0x165667B19E3779F9ull};
+    // eight bytes at a time on four chains: one chain of byte steps over the 4 KB of samples takes 5 us a call
+    uint64_t lanes[4] = {h, h ^ 0x9E3779B97F4A7C15ull, h ^ 0xC2B2AE3D27D4EB4Full, h ^ 0x165667B19E3779F9ull};
+    auto take = [&](const uint8_t *q, size_t n) {
         size_t i = 0;
-        for (; i + 32 <= len; i += 32) {
+        for (; i + 32 <= n; i += 32) {
             uint64_t w[4];
-            std::memcpy(w, p + i, 32);
+            std::memcpy(w, q + i, 32);
             for (int l = 0; l < 4; l++) {
                 lanes[l] = (lanes[l] ^ w[l]) * 0x100000001B3ull;
                 lanes[l] ^= lanes[l] >> 29;
             }
         }
-        for (; i < len; i++) lanes[i & 3] = (lanes[i & 3] ^ p[i]) * 0x100000001B3ull;
-        for (int l = 0; l < 4; l++) h = (h ^ lanes[l]) * 1099511628211ull;
-        return h;
+        for (; i < n; i++) lanes[i & 3] = (lanes[i & 3] ^ q[i]) * 0x100000001B3ull;
+    };
+    if (whole || len <= chunk * samples) {
+        take(p, len);
+    } else {
+        const size_t stride = (len - chunk) / (samples - 1);
+        for (size_t s = 0; s < samples; s++) take(p + s * stride, chunk);
     }
-    if (len <= chunk * samples) {
-        for (size_t i = 0; i < len; i++) h = (h ^ p[i]) * 1099511628211ull;
-        return h;
-    }
-    const size_t stride = (len - chunk) / (samples - 1);
-    for (size_t s = 0; s < samples; s++) {
-        const uint8_t *q = p + s * stride;
-        for (size_t i = 0; i < chunk; i++) h = (h ^ q[i]) * 1099511628211ull;
-    }
+    for (int l = 0; l < 4; l++) h = (h ^ lanes[l]) * 1099511628211ull;
     return h;
 }
 
@@ -199,6 +223,33 @@ int stage_weights(uint32_t type, const uint8_t *host, size_t len, const uint8_t 
     if (st != OXQ_OK) return st;
     OXQ_HIP(hipMemcpy(g.s_weights.ptr, host, len, hipMemcpyHostToDevice));
     *dev = (const uint8_t *)g.s_weights.ptr;
+    return OXQ_OK;
+}
+
+// Host-slice calls of a few vectors: the copies of a few KB that hipMemcpy makes one at a time, each waiting for the GPU
+// (about 15 us a piece), are replaced by staging in pinned memory.  The first kernel reads the input from there, the last
+// one writes the output there and then the flag, and the host watches the flag: one wait in a call instead of three.
+// Up to this many bytes; beyond it the copy engine's rate matters more than the waits.
+constexpr size_t PINNED_MAX = (size_t)1 << 20;
+
+// A device vector of `n` floats to the caller's memory, by way of the pinned output buffer.  Caller holds g.mu.
+int fetch_pinned(const float *d_src, float *output, size_t n) {
+    int st;
+    if ((st = g.h_out.reserve(n * sizeof(float))) != OXQ_OK) return st;
+    if ((st = g.h_flag.reserve(64)) != OXQ_OK) return st;
+    volatile uint32_t *flag = (volatile uint32_t *)g.h_flag.ptr;
+    const uint32_t seq = ++g.h_seq;
+    *flag = seq - 1;
+    OXQ_HIP(oxq::launch_copy_to_host(d_src, (float *)g.h_out.ptr, n, (uint32_t *)g.h_flag.ptr, seq, nullptr));
+    // the stream itself ends the wait if the flag does not: a long queue ahead of the call, or an error
+    for (uint32_t spins = 0; __atomic_load_n((uint32_t *)g.h_flag.ptr, __ATOMIC_ACQUIRE) != seq; spins++) {
+        if (spins > 200000) {
+            OXQ_HIP(hipStreamSynchronize(nullptr));
+            break;
+        }
+        __builtin_ia32_pause();
+    }
+    std::memcpy(output, g.h_out.ptr, n * sizeof(float));
     return OXQ_OK;
 }
 
@@ -343,6 +394,9 @@ int oxq_shutdown(void) {
     g.s_moe_up.release();
     g.s_moe_down.release();
     g.s_moe_tables.release();
+    g.h_in.release();
+    g.h_out.release();
+    g.h_flag.release();
     oxq::gguf_release_staging();
     g.initialised = false;
     g.device = -1;
@@ -658,12 +712,26 @@ static int gemm_host(uint32_t type, const uint8_t *data, size_t data_len, const 
     if ((st = g.s_x.reserve(m * k_pad * sizeof(float))) != OXQ_OK) return st;
     if ((st = g.s_acts.reserve(m * act_row_bytes)) != OXQ_OK) return st;
     if ((st = g.s_out.reserve(m * n_rows * sizeof(float))) != OXQ_OK) return st;
+    const bool f32_route = g.act_route.load(std::memory_order_relaxed) == OXQ_ROUTE_F32;
+    const bool pinned_in = !f32_route && m * k_pad * sizeof(float) <= PINNED_MAX;
+    const bool pinned_out = n == n_rows && m * n_rows * sizeof(float) <= PINNED_MAX;
+    const float *d_x = (const float *)g.s_x.ptr;
     // Gather the first n_cols floats of each input row (k may exceed n_cols).
-    if (k_pad != n_cols) OXQ_HIP(hipMemset(g.s_x.ptr, 0, m * k_pad * sizeof(float)));
-    OXQ_HIP(hipMemcpy2D(g.s_x.ptr, k_pad * sizeof(float), input, k * sizeof(float), n_cols * sizeof(float), m,
-                        hipMemcpyHostToDevice));
+    if (pinned_in) {
+        if ((st = g.h_in.reserve(m * k_pad * sizeof(float))) != OXQ_OK) return st;
+        float *h = (float *)g.h_in.ptr;
+        for (size_t r = 0; r < m; r++) {
+            std::memcpy(h + r * k_pad, input + r * k, n_cols * sizeof(float));
+            std::memset(h + r * k_pad + n_cols, 0, (k_pad - n_cols) * sizeof(float));
+        }
+        d_x = h;
+    } else {
+        if (k_pad != n_cols) OXQ_HIP(hipMemset(g.s_x.ptr, 0, m * k_pad * sizeof(float)));
+        OXQ_HIP(hipMemcpy2D(g.s_x.ptr, k_pad * sizeof(float), input, k * sizeof(float), n_cols * sizeof(float), m,
+                            hipMemcpyHostToDevice));
+    }
     const float *d_bias_f32 = nullptr;
-    if (g.act_route.load(std::memory_order_relaxed) == OXQ_ROUTE_F32) {
+    if (f32_route) {
         // the reference's own gemm: m gemvs on the fp32 rows (reference/q4_k.rs:186-201), bias per row (linear.rs:123-128)
         if (!oxq::gemv_f32_supported(type))
             return fail(OXQ_ERR_UNSUPPORTED_TYPE, type, 0, "no fp32-activation kernel for this type (OXQ_ROUTE_F32)");
@@ -681,7 +749,7 @@ static int gemm_host(uint32_t type, const uint8_t *data, size_t data_len, const 
                             hipMemcpyDeviceToHost));
         return OXQ_OK;
     }
-    OXQ_HIP(oxq::launch_quantize_q8_0((const float *)g.s_x.ptr, m * k_pad, (uint8_t *)g.s_acts.ptr, nullptr));
+    OXQ_HIP(oxq::launch_quantize_q8_0(d_x, m * k_pad, (uint8_t *)g.s_acts.ptr, nullptr));
     oxq::GemmArgs ga;
     ga.W = dW;
     ga.A = (const uint8_t *)g.s_acts.ptr;
@@ -708,6 +776,7 @@ static int gemm_host(uint32_t type, const uint8_t *data, size_t data_len, const 
         ga.bias = (const float *)g.s_bias.ptr;
     }
     OXQ_HIP(oxq::launch_gemm_q8(type, ga, nullptr));
+    if (pinned_out) return fetch_pinned((const float *)g.s_out.ptr, output, m * n_rows);
     OXQ_HIP(hipMemcpy2D(output, n * sizeof(float), g.s_out.ptr, n_rows * sizeof(float), n_rows * sizeof(float), m,
                         hipMemcpyDeviceToHost));
     return OXQ_OK;
@@ -1714,9 +1783,18 @@ int oxq_linear_forward(uint32_t type, const uint8_t *data, size_t data_len, cons
     if ((st = g.s_x.reserve(k_pad * sizeof(float))) != OXQ_OK) return st;
     if ((st = g.s_acts.reserve(k_pad / 32 * 34)) != OXQ_OK) return st;
     if ((st = g.s_out.reserve(n_rows * sizeof(float))) != OXQ_OK) return st;
-    if (k_pad != n_cols) OXQ_HIP(hipMemset(g.s_x.ptr, 0, k_pad * sizeof(float)));
-    OXQ_HIP(hipMemcpy(g.s_x.ptr, input, n_cols * sizeof(float), hipMemcpyHostToDevice));
-    OXQ_HIP(oxq::launch_quantize_q8_0((const float *)g.s_x.ptr, k_pad, (uint8_t *)g.s_acts.ptr, nullptr));
+    const bool f32_route = g.act_route.load(std::memory_order_relaxed) == OXQ_ROUTE_F32;
+    const bool pinned = k_pad * sizeof(float) <= PINNED_MAX && n_rows * sizeof(float) <= PINNED_MAX;
+    if (pinned && !has_lora && !f32_route) {  // the quantizer is the only reader of the fp32 input: over the bus, once
+        if ((st = g.h_in.reserve(k_pad * sizeof(float))) != OXQ_OK) return st;
+        std::memcpy(g.h_in.ptr, input, n_cols * sizeof(float));
+        std::memset((float *)g.h_in.ptr + n_cols, 0, (k_pad - n_cols) * sizeof(float));
+        OXQ_HIP(oxq::launch_quantize_q8_0((const float *)g.h_in.ptr, k_pad, (uint8_t *)g.s_acts.ptr, nullptr));
+    } else {
+        if (k_pad != n_cols) OXQ_HIP(hipMemset(g.s_x.ptr, 0, k_pad * sizeof(float)));
+        OXQ_HIP(hipMemcpy(g.s_x.ptr, input, n_cols * sizeof(float), hipMemcpyHostToDevice));
+        OXQ_HIP(oxq::launch_quantize_q8_0((const float *)g.s_x.ptr, k_pad, (uint8_t *)g.s_acts.ptr, nullptr));
+    }
     const float *d_bias = nullptr;
     if (bias && bias_len) {
         // the reference zips output with bias (linear.rs:87-89): a short bias covers its own length only
@@ -1726,7 +1804,7 @@ int oxq_linear_forward(uint32_t type, const uint8_t *data, size_t data_len, cons
         OXQ_HIP(hipMemcpy(g.s_bias.ptr, bias, nb * sizeof(float), hipMemcpyHostToDevice));
         d_bias = (const float *)g.s_bias.ptr;
     }
-    if (g.act_route.load(std::memory_order_relaxed) == OXQ_ROUTE_F32) {
+    if (f32_route) {
         if (!oxq::gemv_f32_supported(type))
             return fail(OXQ_ERR_UNSUPPORTED_TYPE, type, 0, "no fp32-activation kernel for this type (OXQ_ROUTE_F32)");
         OXQ_HIP(oxq::launch_gemv_f32(type, dW, (const float *)g.s_x.ptr, (float *)g.s_out.ptr, d_bias, (uint32_t)n_rows,
@@ -1746,6 +1824,7 @@ int oxq_linear_forward(uint32_t type, const uint8_t *data, size_t data_len, cons
                                        (float *)g.s_lora_r.ptr, (uint32_t)rank, scale, (const float *)g.s_x.ptr,
                                        (float *)g.s_out.ptr, (uint32_t)n_rows, (uint32_t)n_cols, nullptr));
     }
+    if (pinned) return fetch_pinned((const float *)g.s_out.ptr, output, n_rows);
     OXQ_HIP(hipMemcpy(output, g.s_out.ptr, n_rows * sizeof(float), hipMemcpyDeviceToHost));
     return OXQ_OK;
 }

@@ -128,6 +128,9 @@ hipError_t launch_gemv_vecs_more(uint32_t type, const GemvVecsArgs &a, hipStream
 // x: n floats (n % 32 == 0) -> n/32 Q8_0 blocks of 34 bytes.
 hipError_t launch_quantize_q8_0(const float *x, size_t n, uint8_t *out, hipStream_t stream);
 
+// n floats to pinned host memory, then `seq` to the word `flag` there, visible to the host in that order.
+hipError_t launch_copy_to_host(const float *src, float *dst, size_t n, uint32_t *flag, uint32_t seq, hipStream_t stream);
+
 // h = silu(gate) * up over n floats (n % 32 == 0); h (fp32) and/or out (Q8_0 blocks) may be null.
 hipError_t launch_swiglu_quantize(const float *gate, const float *up, size_t n, float *h, uint8_t *out,
                                   hipStream_t stream);

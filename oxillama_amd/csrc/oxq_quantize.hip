@@ -34,6 +34,26 @@ hipError_t launch_quantize_q8_0(const float *x, size_t n, uint8_t *out, hipStrea
     return hipGetLastError();
 }
 
+// The output of a host-slice call to pinned host memory.  One work group: each of its waves makes its own writes
+// visible to the host before the barrier, one thread then sets the flag.  Bound by the bus (57 KB in about 3 us); more
+// work groups would need a counter between them for no gain at these sizes.
+__global__ __launch_bounds__(1024) void copy_to_host_kernel(const float *__restrict__ src, float *__restrict__ dst, size_t n,
+                                                            uint32_t *__restrict__ flag, uint32_t seq) {
+    const size_t n4 = n / 4;
+    for (size_t i = threadIdx.x; i < n4; i += 1024)
+        reinterpret_cast<u32x4 *>(dst)[i] = reinterpret_cast<const u32x4 *>(src)[i];
+    const size_t tail = 4 * n4 + threadIdx.x;
+    if (tail < n) dst[tail] = src[tail];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+hipError_t launch_copy_to_host(const float *src, float *dst, size_t n, uint32_t *flag, uint32_t seq, hipStream_t stream) {
+    hipLaunchKernelGGL(copy_to_host_kernel, dim3(1), dim3(1024), 0, stream, src, dst, n, flag, seq);
+    return hipGetLastError();
+}
+
 // ---- dequantize ---------------------------------------------------------
 
 __device__ __forceinline__ float dq_q4_0(const uint8_t *b, uint32_t i) {

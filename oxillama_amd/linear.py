@@ -39,6 +39,19 @@ class QuantLinear:
         self.out_features = weight.shape[0] if len(weight.shape) > 0 else 0  # linear.rs:38-48
         self.in_features = weight.shape[1] if len(weight.shape) > 1 else 0
         self.lora = None
+        self._args = None
+
+    def _weight_args(self):
+        """(address, bytes, shape, dimensions, owner of the address) of the weight for the C ABI.  Kept from call to call
+        while the tensor holds the same array and shape: forming them takes as long as the library's part of a call."""
+        data, shape = self.weight.data, tuple(self.weight.shape)
+        if self._args is None or self._args[4] is not data or self._args[2][:] != list(shape):
+            w = _u8(data)
+            args = (_ptr(w), w.size, (C.c_size_t * len(shape))(*shape), len(shape), data if isinstance(data, np.ndarray) else w)
+            if not (isinstance(data, np.ndarray) and data.flags.c_contiguous):
+                return args[:4] + (w,)  # a copy of the bytes: made again on every call, as they may change
+            self._args = args
+        return self._args
 
     def set_lora(self, lora):
         self.lora = lora
@@ -49,8 +62,6 @@ class QuantLinear:
     def forward(self, kernel: HipKernel, input, output):
         """output = weight @ input + bias [+ lora delta] (linear.rs:77-98); output is filled in place."""
         lib = capi.load()
-        w = _u8(self.weight.data)
-        shape = (C.c_size_t * len(self.weight.shape))(*self.weight.shape)
         x = np.ascontiguousarray(input, dtype=np.float32).ravel()
         bias_p, bias_n = (_ptr(self.bias), self.bias.size) if self.bias is not None else (None, 0)
         if self.lora is not None:
@@ -58,18 +69,18 @@ class QuantLinear:
             lora_args = (_ptr(la), la.size, _ptr(lb), lb.size, self.lora.rank, self.lora.scale)
         else:
             lora_args = (None, 0, None, 0, 0, 0.0)
-        _check(lib.oxq_linear_forward(kernel.tensor_type, _ptr(w), w.size, shape, len(self.weight.shape), bias_p,
-                                      bias_n, *lora_args, _ptr(x), x.size, _ptr(output), output.size))
+        w_p, w_n, shape, n_dims, _owner = self._weight_args()
+        _check(lib.oxq_linear_forward(kernel.tensor_type, w_p, w_n, shape, n_dims, bias_p, bias_n, *lora_args, _ptr(x), x.size,
+                                      _ptr(output), output.size))
 
     def forward_batch(self, kernel: HipKernel, input, output, batch_size):
         """output[batch x out] = gemm + bias broadcast (linear.rs:105-132; no LoRA in batch mode)."""
         lib = capi.load()
-        w = _u8(self.weight.data)
-        shape = (C.c_size_t * len(self.weight.shape))(*self.weight.shape)
         x = np.ascontiguousarray(input, dtype=np.float32).ravel()
         bias_p, bias_n = (_ptr(self.bias), self.bias.size) if self.bias is not None else (None, 0)
-        _check(lib.oxq_linear_forward_batch(kernel.tensor_type, _ptr(w), w.size, shape, len(self.weight.shape),
-                                            bias_p, bias_n, _ptr(x), x.size, _ptr(output), output.size, batch_size))
+        w_p, w_n, shape, n_dims, _owner = self._weight_args()
+        _check(lib.oxq_linear_forward_batch(kernel.tensor_type, w_p, w_n, shape, n_dims, bias_p, bias_n, _ptr(x), x.size,
+                                            _ptr(output), output.size, batch_size))
 
 
 # ---- device route -------------------------------------------------------------------------
