@@ -204,6 +204,14 @@ hipError_t launch_gemm_q8(uint32_t type, const GemmArgs &a, hipStream_t stream) 
         }
     }
     if (a.scaled_sums) return hipErrorNotSupported;
+    if (!a.offsets && !a.sums) {
+        const int shape = variant == 0 ? gemm_f16_shape(type, a.m, a.n, a.k)
+                          : (variant == 301 || variant == 302) && gemm_f16_supported(type, a.m, a.n, a.k) ? variant - 300 : 0;
+        if (shape) {
+            const hipError_t e = launch_gemm_f16(type, a, shape, stream);
+            if (e != hipErrorNotSupported) return e;
+        }
+    }
     const uint32_t mpad = (a.m + 127) / 128 * 128 + 128, nsb = tile_padded_sub_blocks(a.k), nsb_row = a.k / 32;
     uint8_t *q8t = a.workspace;
     float *P = reinterpret_cast<float *>(q8t + (size_t)nsb * mpad * 32);

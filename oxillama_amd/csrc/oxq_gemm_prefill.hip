@@ -36,34 +36,9 @@
 // maximum: matrix and vector work do not overlap here beyond the first eight fmas.  The int8 form's step (one int8
 // MFMA 16.4 ns + 32 fmas 45.4 ns) is 61.8 ns by the same count, so this form's advantage is the unpacking and
 // scale handling it saves, not a factor of two.
-#include <utility>
-#include "oxq_gemm_tile.hpp"
+#include "oxq_gemm_f16_util.hpp"
 
 namespace oxq {
-
-template <class F, int... Q>
-__device__ __forceinline__ void static_for(std::integer_sequence<int, Q...>, F &&f) {
-    (f(std::integral_constant<int, Q>{}), ...);
-}
-
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-typedef __bf16 b8 __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-
-#define OXQ_LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
-
-// LDS is carved out of byte arrays here and written with one vector type and read with another (and filled by
-// direct-to-LDS loads): every such access goes through a may_alias type, or type-based alias analysis treats a
-// load as unrelated to the store that feeds it.
-typedef u32x4 __attribute__((may_alias)) lds_u32x4;
-typedef u32x2 __attribute__((may_alias)) lds_u32x2;
-typedef uint32_t __attribute__((may_alias)) lds_u32;
-typedef uint16_t __attribute__((may_alias)) lds_u16;
-typedef float __attribute__((may_alias)) lds_f32;
-typedef v4f __attribute__((may_alias)) lds_v4f;
-__device__ __forceinline__ h8 lds_h8(const uint8_t *p) { return __builtin_bit_cast(h8, *reinterpret_cast<const lds_u32x4 *>(p)); }
-__device__ __forceinline__ b8 lds_b8(const uint8_t *p) { return __builtin_bit_cast(b8, *reinterpret_cast<const lds_u32x4 *>(p)); }
 
 constexpr uint32_t PF_TOK = 128, PF_ROWS = 256, PF_WAVES = 8;   // tokens, weight rows and waves of a work group
 constexpr uint32_t PF_STAGE = 16384;              // f16 token operands of one stage: 2 sub-blocks x 128 tokens x 32 x 2 B
@@ -77,10 +52,6 @@ constexpr uint32_t PF_STAGE_DA = 512;             // + the tokens' two block sca
 __host__ __device__ inline size_t pf_tokf_bytes(size_t nsb, size_t mpad) { return nsb * mpad * 64; }
 __host__ __device__ inline size_t pf_dag_bytes(size_t nsb, size_t mpad) { return nsb / 2 * mpad * 4; }
 __host__ __device__ inline size_t pf_pbf_bytes(size_t nsb, size_t mpad) { return nsb / 8 * 4 * mpad * 16; }
-
-// Order of the eight k-slots of one operand register set: byte positions of the lane's 8 raw weight bytes.  The
-// unpack takes bytes 0 and 2 of a dword together (they sit in the two 16-bit halves), then bytes 1 and 3.
-__device__ __forceinline__ constexpr int pf_slot_byte(int j) { return (j & 4) | ((j & 1) << 1) | ((j >> 1) & 1); }
 
 // One thread per (sub-block j, token t).  Eight consecutive threads take the eight sub-blocks of one super-block of one
 // token (272 contiguous bytes of its row; their eight bf16 pieces of P make one 16-byte run), the next eight the next
@@ -138,11 +109,6 @@ __global__ __launch_bounds__(256) void prefill_prep_acts(const uint8_t *__restri
 //   mnb  [row][8 bf16]  the eight 6-bit mins
 //   drow [row] d,  ndm [row] -dmin   (fp32)
 constexpr uint32_t PF_TAB_SCK = 0, PF_TAB_MNB = 2048, PF_TAB_D = 2560, PF_TAB_NDM = 2688, PF_TAB_BYTES = 2816;
-
-__device__ __forceinline__ uint32_t f16x2_of(float v) {
-    const uint32_t b = f2h(v);
-    return b | (b << 16);
-}
 
 template <bool DUMP>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_prefill_q4k(

@@ -231,6 +231,12 @@ size_t gemm_grouped_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t
 bool gemm_prefill_supported(uint32_t type, uint32_t m, uint32_t n, uint32_t k);
 size_t gemm_prefill_workspace_bytes(uint32_t m, uint32_t k);
 hipError_t launch_gemm_prefill(uint32_t type, const GemmArgs &a, hipStream_t stream);
+// The f16 matrix-core kernel that takes the caller's Q8_0 rows as they are (oxq_gemm_f16.hip; Q4_K, Q5_K, Q6_K, plain
+// matmuls): no workspace.  shape 1: 128 tokens x 256 rows to a work group, 2: 64 x 128 with k in two halves;
+// gemm_f16_shape: the one that a call should take, or 0.
+bool gemm_f16_supported(uint32_t type, uint32_t m, uint32_t n, uint32_t k);
+int gemm_f16_shape(uint32_t type, uint32_t m, uint32_t n, uint32_t k);
+hipError_t launch_gemm_f16(uint32_t type, const GemmArgs &a, int shape, hipStream_t stream);
 // Tuning knobs (oxq_tuning.h), read once per call.
 extern std::atomic<int> g_gemm_variant;              // 0 = default tile shape
 extern std::atomic<uint32_t> g_gemm_tile_min_rows;   // 0 = default threshold

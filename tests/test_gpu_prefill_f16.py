@@ -114,6 +114,41 @@ def test_prefill_f16_kernel_is_the_default_where_it_fills_the_chip(hip, ref):
         assert np.abs(dy.cpu().numpy()[rows] - y_ref).max() <= FP32_REL_TOL * np.abs(y_ref).max()
 
 
+@pytest.mark.parametrize("shape", [(1, 32, 512), (33, 100, 1024), (65, 127, 768), (128, 257, 512), (129, 130, 2304), (200, 300, 4096)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q5_K, O.Q6_K], ids=lambda t: O.NAMES[t])
+@pytest.mark.parametrize("variant", [301, 302])
+def test_f16_kernel_on_raw_rows(hip, ref, tuning, variant, t, shape):
+    """The f16 kernel that takes the Q8_0 rows as they are, both shapes: tiles' edges in tokens and rows, an odd number of
+    super-blocks (the halves of k differ by one), two of them.  Weights with every scale and quant value the format has
+    (random block bytes); fp32 within the bar of the batch-1 matvec per token row."""
+    m, n, k = shape
+    say("f16 raw rows", variant, O.NAMES[t], shape)
+    tuning("gemm_variant", variant)
+    tuning("gemm_tile_min_rows", 1)
+    w = O.random_blocks(t, 40 + m, n, k)
+    x = synth.normal_f32(41 + n, m * k)
+    x[:k] *= 300.0
+    acts = ref.quantize_q8_0(x)
+    kern = hip.HipKernel(t)
+    ws = torch.empty(kern.gemm_workspace_bytes(m, n, k), dtype=torch.uint8, device="cuda")
+    dw, da = torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda()
+    dy = torch.full((m + 1, n), 7.0, dtype=torch.float32, device="cuda")
+    kern.gemm_q8_dev(dw, da, dy, m, n, k, accumulate=False, workspace=ws)
+    torch.cuda.synchronize()
+    assert last_launch().startswith("gemm_f16_kernel"), last_launch()
+    y = dy.cpu().numpy()
+    assert np.all(y[m] == 7.0)
+    y_ref = oracle_rows(ref, t, w, acts, n, k, range(m))
+    for r in range(m):
+        err, scale = np.abs(y[r] - y_ref[r]).max(), np.abs(y_ref[r]).max()
+        assert err <= FP32_REL_TOL * scale, f"token {r}: max err {err:.3e} vs |y|inf {scale:.3e}"
+    dy2 = dy.clone()
+    kern.gemm_q8_dev(dw, da, dy2, m, n, k, accumulate=True, workspace=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(dy2[:m], dy[:m] + dy[:m])
+
+
 def test_scaled_sums_errors(hip):
     kern = hip.HipKernel(O.Q6_K)
     z = torch.zeros(1 << 16, dtype=torch.uint8, device="cuda")
