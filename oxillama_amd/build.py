@@ -2,6 +2,7 @@
 
 `python -m oxillama_amd.build` compiles
   * oxillama_amd/liboxq_hip.so   -- HIP kernels + C ABI (include/oxq.h), gfx950 only
+  * oxillama_amd/_bind.so        -- CPython extension: the device entry points' calls into liboxq_hip.so
   * oxillama_amd/liboxq_synth.so -- host-side synthetic weight generator
   * oxillama_amd/liboxq_benchkit.so -- copy / streaming-read kernels for measurement calibration
   * tests/cpp/test_quant_kernel.bin -- C++ mirror of the reference interface + its replayed unit tests
@@ -10,11 +11,13 @@ hipcc cross-compiles gfx950 code objects without a GPU present.
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 HIP_SOURCES = ["oxq_api.hip", "oxq_gemv.hip", "oxq_gemv_more.hip", "oxq_gemv_f32.hip", "oxq_gemm.hip", "oxq_gemm_more.hip", "oxq_gemm_prefill.hip", "oxq_gemm_f16.hip", "oxq_quantize.hip", "oxq_linear.hip", "oxq_gguf.hip", "oxq_topk.hip", "oxq_lm_head.hip", "oxq_moe.hip"]
 HIP_LIB = os.path.join(HERE, "liboxq_hip.so")
+BIND_LIB = os.path.join(HERE, "_bind.so")
 SYNTH_LIB = os.path.join(HERE, "liboxq_synth.so")
 BENCHKIT_LIB = os.path.join(HERE, "liboxq_benchkit.so")
 CPP_TEST_BIN = os.path.join(os.path.dirname(HERE), "tests", "cpp", "test_quant_kernel.bin")
@@ -50,6 +53,12 @@ def build_synth():
     return SYNTH_LIB
 
 
+def build_bind():
+    run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-I", sysconfig.get_paths()["include"],
+         "-o", BIND_LIB, os.path.join(CSRC, "bind.cpp")])
+    return BIND_LIB
+
+
 def build_benchkit():
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
     run([hipcc, *HIPCC_FLAGS, "-shared", "-o", BENCHKIT_LIB, os.path.join(CSRC, "benchkit.hip")])
@@ -69,6 +78,7 @@ def build_cpp_tests():
 
 def build_all():
     build_hip()
+    build_bind()
     build_synth()
     build_benchkit()
     build_cpp_tests()

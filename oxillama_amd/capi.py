@@ -207,6 +207,7 @@ TUNING_SIGNATURES = {
 }
 
 _lib = None
+_attached = None
 
 
 def load():
@@ -223,8 +224,23 @@ def load():
         fn = getattr(lib, name)  # AttributeError if the ABI lost a symbol
         fn.restype = restype
         fn.argtypes = argtypes
+    try:
+        from . import _bind
+    except ImportError as e:
+        raise RuntimeError("oxillama_amd/_bind.so is missing or of another Python: build it with `python -m oxillama_amd.build`") from e
+    _bind.attach({name: C.cast(getattr(lib, name), C.c_void_p).value for name in SIGNATURES})
     _lib = lib
     return lib
+
+
+def bind():
+    """The extension module behind the device entry points, attached to the library."""
+    global _attached
+    if _attached is None:
+        load()
+        from . import _bind
+        _attached = _bind
+    return _attached
 
 
 def last_error():

@@ -91,10 +91,6 @@ class LoraStruct(C.Structure):
                 ("scale", C.c_float)]
 
 
-def _opt(t):
-    return t.data_ptr() if t is not None else None
-
-
 def lora_struct(d_a, d_b, d_r, rank, scale):
     return LoraStruct(d_a.data_ptr(), d_b.data_ptr(), d_r.data_ptr(), rank, scale)
 
@@ -106,38 +102,25 @@ def lora_apply_dev(lora, d_x, d_out, out_features, in_features):
 
 def linear_forward_dev(tensor_type, d_weights, d_out, out_features, in_features, d_x=None, d_acts=None, d_bias=None,
                        lora=None):
-    _check(capi.load().oxq_linear_forward_dev(int(tensor_type), d_weights.data_ptr(), _opt(d_x), _opt(d_acts),
-                                              _opt(d_bias), C.byref(lora) if lora is not None else None,
-                                              d_out.data_ptr(), out_features, in_features, _stream()))
+    _check(capi.bind().linear_forward(tensor_type, d_weights, d_x, d_acts, d_bias, C.addressof(lora) if lora is not None else None,
+                                      d_out, out_features, in_features))
 
 
 def linear_forward_multi_dev(tensor_type, d_weights, d_acts, d_outs, out_features, in_features, d_biases=None):
-    n = len(d_weights)
-    pointers = C.c_void_p * n
-    wp = pointers(*[w.data_ptr() for w in d_weights])
-    op = pointers(*[o.data_ptr() for o in d_outs])
-    bp = pointers(*[_opt(b) for b in d_biases]) if d_biases is not None else None
-    of = (C.c_size_t * n)(*out_features)
-    _check(capi.load().oxq_linear_forward_multi_dev(int(tensor_type), n, wp, d_acts.data_ptr(), bp, op, of,
-                                                    in_features, _stream()))
+    _check(capi.bind().linear_forward_multi(tensor_type, d_weights, d_acts, d_biases, d_outs, out_features, in_features))
 
 
 def linear_forward_batch_dev(tensor_type, d_weights, d_acts, d_out, batch, out_features, in_features, d_bias=None,
                              workspace=None):
-    _check(capi.load().oxq_linear_forward_batch_dev(int(tensor_type), d_weights.data_ptr(), d_acts.data_ptr(),
-                                                    _opt(d_bias), d_out.data_ptr(), batch, out_features, in_features,
-                                                    _opt(workspace), workspace.numel() if workspace is not None else 0,
-                                                    _stream()))
+    _check(capi.bind().linear_forward_batch(tensor_type, d_weights, d_acts, d_bias, d_out, batch, out_features, in_features, workspace))
 
 
 def swiglu_quantize_dev(d_gate, d_up, d_h=None, d_out_q8=None):
-    _check(capi.load().oxq_swiglu_quantize_q8_0_dev(d_gate.data_ptr(), d_up.data_ptr(), d_gate.numel(), _opt(d_h),
-                                                    _opt(d_out_q8), _stream()))
+    _check(capi.bind().swiglu_quantize(d_gate, d_up, d_h, d_out_q8))
 
 
 def rmsnorm_quantize_dev(d_x, d_weight, eps, rows, n, d_y=None, d_out_q8=None):
-    _check(capi.load().oxq_rmsnorm_quantize_q8_0_dev(d_x.data_ptr(), d_weight.data_ptr(), float(eps), rows, n,
-                                                     _opt(d_y), _opt(d_out_q8), _stream()))
+    _check(capi.bind().rmsnorm_quantize(d_x, d_weight, eps, rows, n, d_y, d_out_q8))
 
 
 def gate_up_swiglu_dev(tensor_type, d_gate, d_up, d_acts_q8, d_h, d_out_q8, intermediate, hidden):
@@ -153,16 +136,12 @@ def ffn_workspace_bytes(hidden, intermediate):
 
 def ffn_swiglu_dev(gate, up, down, d_acts, d_out, hidden, intermediate, workspace):
     """gate/up/down: (tensor_type, device weights).  d_out = down(silu(gate x) * up x)."""
-    _check(capi.load().oxq_ffn_swiglu_dev(int(gate[0]), gate[1].data_ptr(), int(up[0]), up[1].data_ptr(),
-                                          int(down[0]), down[1].data_ptr(), d_acts.data_ptr(), d_out.data_ptr(),
-                                          hidden, intermediate, workspace.data_ptr(), workspace.numel(), _stream()))
+    _check(capi.bind().ffn_swiglu(gate[0], gate[1], up[0], up[1], down[0], down[1], d_acts, d_out, hidden, intermediate, workspace))
 
 
 def topk_dev(d_values, k, d_out_values, d_out_indices, workspace):
     """The k largest of a float32 CUDA tensor, largest first, with their indices (uint32 viewed as int32)."""
-    lib = capi.load()
-    _check(lib.oxq_topk_dev(d_values.data_ptr(), d_values.numel(), k, d_out_values.data_ptr(), d_out_indices.data_ptr(),
-                            workspace.data_ptr(), workspace.numel() * workspace.element_size(), _stream()))
+    _check(capi.bind().topk(d_values, k, d_out_values, d_out_indices, workspace))
 
 
 def lm_head_topk_workspace_bytes(quant_type, n_rows, n_cols, k):
@@ -172,32 +151,21 @@ def lm_head_topk_workspace_bytes(quant_type, n_rows, n_cols, k):
 def lm_head_topk_dev(quant_type, d_weights, d_acts_q8, d_logits, n_rows, n_cols, k, d_out_values, d_out_indices, workspace):
     """The vocabulary projection (logits to d_logits) and the k largest logits with their row indices, in one launch
     where the shape allows it (oxq_lm_head_topk_dev)."""
-    _check(capi.load().oxq_lm_head_topk_dev(quant_type, d_weights.data_ptr(), d_acts_q8.data_ptr(), d_logits.data_ptr(),
-                                            n_rows, n_cols, k, d_out_values.data_ptr(), d_out_indices.data_ptr(),
-                                            workspace.data_ptr(), workspace.numel() * workspace.element_size(), _stream()))
+    _check(capi.bind().lm_head_topk(quant_type, d_weights, d_acts_q8, d_logits, n_rows, n_cols, k, d_out_values, d_out_indices,
+                                    workspace))
 
 
 def logits_edit_dev(d_logits, d_banned=None, d_bias_tokens=None, d_bias_values=None, d_recent=None, window=0,
                     repetition_penalty=1.0):
     """The sampler's edits of the logits before the candidate list (sampling/mod.rs:573-613), in place: banned tokens,
     logit bias, repetition penalty over the last `window` of d_recent.  Token lists: int32 / uint32 CUDA tensors."""
-    def ptr(t):
-        return t.data_ptr() if t is not None and t.numel() else None
-
-    def cnt(t):
-        return t.numel() if t is not None else 0
-    _check(capi.load().oxq_logits_edit_dev(d_logits.data_ptr(), d_logits.numel(), ptr(d_banned), cnt(d_banned),
-                                           ptr(d_bias_tokens), ptr(d_bias_values), cnt(d_bias_tokens), ptr(d_recent),
-                                           cnt(d_recent), window, repetition_penalty, _stream()))
+    _check(capi.bind().logits_edit(d_logits, d_banned, d_bias_tokens, d_bias_values, d_recent, window, repetition_penalty))
 
 
 def sample_candidates_dev(d_values, d_indices, k, temperature, min_p, top_p, d_rng_state, d_token, d_probs=None):
     """The sampler after its candidate list (sampling/mod.rs:487-564): temperature, softmax, min-p, top-p, the draw.
     d_rng_state: one uint64 (the reference's Xorshift64 state), d_token: one uint32, d_probs: optional k floats."""
-    lib = capi.load()
-    _check(lib.oxq_sample_candidates_dev(d_values.data_ptr(), d_indices.data_ptr(), k, temperature, min_p, top_p,
-                                         d_rng_state.data_ptr(), d_token.data_ptr(),
-                                         d_probs.data_ptr() if d_probs is not None else None, _stream()))
+    _check(capi.bind().sample_candidates(d_values, d_indices, k, temperature, min_p, top_p, d_rng_state, d_token, d_probs))
 
 
 def topk_workspace_bytes(n, k):

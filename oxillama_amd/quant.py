@@ -256,9 +256,7 @@ class HipKernel:
         return C.c_void_p(raw_stream())
 
     def matvec_q8_fused_dev(self, d_weights, d_acts, d_out, n_rows, n_cols, accumulate=True):
-        _check(self._lib.oxq_matvec_q8_fused_dev(self.tensor_type, d_weights.data_ptr(), d_acts.data_ptr(),
-                                                 d_out.data_ptr(), n_rows, n_cols, int(accumulate),
-                                                 raw_stream()))
+        _check(capi.bind().matvec_q8_fused(self.tensor_type, d_weights, d_acts, d_out, n_rows, n_cols, int(accumulate)))
 
     def matvec_q8_fused_multi_dev(self, d_weights, d_acts, d_outs, n_rows, n_cols, accumulate=True):
         """Up to 4 matrices of one shape sharing d_acts, one launch (wq/wk/wv, ffn_gate/ffn_up)."""
@@ -294,10 +292,7 @@ class HipKernel:
 
     def gemm_q8_dev(self, d_weights, d_acts, d_out, m, n, k, accumulate=False, workspace=None):
         """workspace: uint8 CUDA tensor of gemm_workspace_bytes(m, n, k) bytes (256-byte aligned), or None."""
-        ws_ptr = workspace.data_ptr() if workspace is not None else None
-        ws_len = workspace.numel() if workspace is not None else 0
-        _check(self._lib.oxq_gemm_q8_dev(self.tensor_type, d_weights.data_ptr(), d_acts.data_ptr(),
-                                         d_out.data_ptr(), m, n, k, int(accumulate), ws_ptr, ws_len, raw_stream()))
+        _check(capi.bind().gemm_q8(self.tensor_type, d_weights, d_acts, d_out, m, n, k, int(accumulate), workspace))
 
     def gemm_q8_static_dev(self, d_weights, d_acts, d_out, m, n, k, accumulate=False):
         """gemm_q8_dev on the library's static device scratch: allocates nothing (shapes up to the scratch size)."""
@@ -336,8 +331,7 @@ class HipKernel:
 
 
 def quantize_q8_0_dev(d_x, d_out):
-    lib = capi.load()
-    _check(lib.oxq_quantize_q8_0_dev(d_x.data_ptr(), d_x.numel(), d_out.data_ptr(), raw_stream()))
+    _check(capi.bind().quantize_q8_0(d_x, d_out))
 
 
 class KernelDispatcher:
