@@ -831,25 +831,38 @@ static hipError_t launch_skinny_shape(const GemmArgs &a, const TilePlan &p, hipS
 //    groups on no split is needed (57344 x 4096, 16 rows: 44 us against 56).
 enum SkinnyShape { SK_NONE = 0, SK_1_4, SK_1_8, SK_2_2, SK_1_4_SPLIT, SK_1_16, SK_2_8, SK_W4_1_8, SK_W4_2_4, SK_2_4, SK_2_2_SPLIT };
 
-// Expert groups of up to this many rows in the mean stay with the kernel's two-tile shapes (larger groups take further
-// passes over their expert's weights).  20 where the tile kernel is the alternative at its best (Q4_K, IQ4_XS: 8
-// experts of 14336 x 4096 with 13..28 rows 92-101 us against 105 + 5); the formats of 32-weight blocks, whose tile
-// kernel is bound by its many small loads, keep the few-token kernel up to 48 (the Mixtral-shaped layer at 96 / 128 /
-// 192 tokens, us: Q4_1 348 / 436 / 625 against 527 / 671 / 712 on the tile kernel, Q4_0 348 / 440 / 630 against 486 /
-// 619 / 663, IQ4_NL 331 / 438 / 627 against 490 / 628 / 648; at 256 tokens, a mean of 64, the tile kernel is level).
+// Expert groups of up to this many rows in the mean stay with this kernel (groups beyond its tiles take further passes
+// over their expert's weights).  Against the tile kernel, us per matmul, groups of random sizes about the mean:
+//   128 experts of 768 x 2048, mean 24 / 32: Q4_K 67 / 70 against 89 / 106, IQ4_XS 63 / 74 against 88 / 105, Q5_K 78 / 88
+//   against 114 / 133, Q6_K 98 / 120 against 140 / 168; of 1536 x 3072: Q4_K 146 / 183 against 171 / 210, Q5_K 213 / 245
+//   against 221 / 268, Q6_K 280 / 316 against 285 / 345; 8 of 14336 x 4096: Q4_K 117 / 136 against 122 / 151, Q6_K 226 /
+//   244 against 232 / 266 (Q5_K 169 / 187 against 160 / 199).  At 40 and 48 the 64-token tiles are level or ahead (64
+//   experts of 1536 x 3072 at 48: Q4_K 139 against 136, Q6_K 218 against 186).
+//   Q6_K and Q8_0, one token tile of 16 at a time, on rows of up to 1536 columns, where the 64 x 128 tiles of the tile
+// kernel have no split sums to add: up to 24 and 20 (128 experts of 2048 x 768 / 3072 x 1536 at 24: Q6_K 129 / 283 against
+// 130 / 300, at 32 145 / 335 against 131 / 307; Q8_0 at 24 130 / 309 against 125 / 297).  Q2_K, the tile kernel's cheapest,
+// up to 17 (128 of 1536 x 3072 at 18 / 24 183 / 214 against 188 / 199).
+// The 4-bit formats of 32-weight blocks, whose tile kernel is bound by its many small loads, keep it up to 48 (the
+// Mixtral-shaped layer at 96 / 128 / 192 tokens, us: Q4_1 348 / 436 / 625 against 527 / 671 / 712 on the tile kernel, Q4_0
+// 348 / 440 / 630 against 486 / 619 / 663, IQ4_NL 331 / 438 / 627 against 490 / 628 / 648; at 256 tokens, a mean of 64, the
+// tile kernel is level).
 template <class F>
-constexpr uint32_t skinny_grouped_mean_limit() {
-    return tile_ragged_k<F>::value ? 48 : 20;
+static uint32_t skinny_grouped_mean_limit(uint32_t k) {
+    if (F::TYPE == OXQ_TYPE_Q2_K) return 17;
+    if (F::TYPE == OXQ_TYPE_Q6_K) return k <= 1536 ? 24 : 32;
+    if (F::TYPE == OXQ_TYPE_Q8_0) return k <= 1536 ? 20 : 32;
+    if (Skinny<F>::ONE_TILE) return 32;
+    return tile_ragged_k<F>::value ? 48 : k >= 768 ? 32 : 20;  // (one step of k: not measured beyond 20)
 }
 
 template <class F>
 static int skinny_shape(const GemmArgs &a, bool has_partial, uint32_t rows, int variant) {
     if constexpr (Skinny<F>::OK) {
-        constexpr size_t MEAN_LIMIT = skinny_grouped_mean_limit<F>();
+        const size_t mean_limit = skinny_grouped_mean_limit<F>(a.k);
         // whole steps of two super-blocks
-        // (expert groups of a mean of up to 20 rows: the launch may be shaped for more than 32 -- twice the mean --
+        // (expert groups: the launch may be shaped for more than 32 -- twice the mean --
         // and the groups beyond 32 rows take further passes)
-        if (a.k % 256 != 0 || a.k < 512 || (rows > 32 && !(a.offsets && (size_t)a.m <= MEAN_LIMIT * (size_t)a.n_experts))) return SK_NONE;
+        if (a.k % 256 != 0 || a.k < 512 || (rows > 32 && !(a.offsets && (size_t)a.m <= mean_limit * (size_t)a.n_experts))) return SK_NONE;
         const bool two = rows > 16;
         // the formats with the long strips: the one-tile shapes only (see launch_skinny)
         if (Skinny<F>::ONE_TILE && variant != 0 && variant != 200) return SK_NONE;
@@ -871,14 +884,11 @@ static int skinny_shape(const GemmArgs &a, bool has_partial, uint32_t rows, int 
                 return (has_partial && skinny_splits(a.n, a.k) >= 2) ? SK_1_4_SPLIT : SK_NONE;
             }
             const bool many = (size_t)((a.n + 127) / 128) * a.n_experts >= 2 * (size_t)device_cus();
-            // two token tiles: only with many row groups and a mean of at most 20 rows per expert
+            // two token tiles
             if (two) {
-                // one tile per work group: a group of 17..32 rows takes a second pass over its expert's weights (the
-                // launch's second layer of work groups; those of the smaller groups exit at once).  8 experts of
-                // 14336 x 4096, 11..23 rows: Q6_K 152 us, Q8_0 155 against 195 / 227 on the tile kernel; a pass costs
-                // 117 / 8 us per expert, so up to a mean of 17 rows (two passes for about half the experts).
+                // one tile per work group: a group of 17..32 rows takes a second pass over its expert's weights
                 if (Skinny<F>::ONE_TILE) {
-                    if ((size_t)a.m > 17 * (size_t)a.n_experts) return SK_NONE;
+                    if ((size_t)a.m > mean_limit * (size_t)a.n_experts) return SK_NONE;
                     if (many) return SK_1_4;
                     // few row groups per expert (one work group per compute unit in the first pass): the second
                     // pass's work groups would double up on some compute units and set the time; with each expert's
@@ -887,9 +897,7 @@ static int skinny_shape(const GemmArgs &a, bool has_partial, uint32_t rows, int 
                                            (size_t)((a.n + 127) / 128) * a.n_experts * SKINNY_GROUPED_SPLITS >= device_cus();
                     return can_split ? SK_1_4_SPLIT : SK_1_8;
                 }
-                // (a mean of up to 20 rows: 8 experts of 14336 x 4096 with 13..28 rows 92-101 us against 105 + 5 on
-                // the tile kernel and its token re-layout)
-                if ((size_t)a.m > MEAN_LIMIT * (size_t)a.n_experts) return SK_NONE;
+                if ((size_t)a.m > mean_limit * (size_t)a.n_experts) return SK_NONE;
                 if (many) return SK_2_2;
                 // few row groups per expert: each expert's k in two halves, where that gives every compute unit a
                 // work group and the workspace has room for the halves' sums

@@ -875,12 +875,21 @@ static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t
     // against the second): 4096 x 14336, 128 / 256 / 384 tokens, Q4_K 131 / 136 / 143 against 47 / 87 / 127, Q6_K
     // 196 / 198 / 206 against 66 / 125 / 183; 4096 x 4096 Q4_K 44 / 45 / 48 against 19 / 27 / 37, Q8_0 51 / 51 / 54
     // against 21 / 33 / 46; 14336 x 4096 Q4_K 128 / 192 tokens 49 / 70 against 45 / 63, 256 a tie, 384 108 against 113.
-    const bool mid_split_k = mid && (narrow || (size_t)((rows + 63) / 64) * ((a.n + 127) / 128) * (a.offsets ? a.n_experts : 1) * 4 <
-                                                   7 * (size_t)device_cus());
+    const bool wide_grid = (size_t)((rows + 63) / 64) * ((a.n + 127) / 128) * (a.offsets ? a.n_experts : 1) * 4 >= 7 * (size_t)device_cus();
+    // Expert groups, whose 64-row tiles are part empty: the split-k tiles also on a full chip where k feeds four waves
+    // (64 / 96 rows in the mean on 1536 x 3072: Q4_K 200 / 130 us against 174 / 117, Q6_K 290 / 187 against 244 / 163,
+    // 768 x 2048, 64 rows, Q6_K 113 against 100); on 14336 x 4096 a tie.  With rows of up to 1536 columns it is the other
+    // way round, from 33 rows on: 64 experts of 2048 x 768 at 48 rows Q4_K 77 against 61, Q6_K 95 against 75, of 3072 x 1536
+    // 159 against 138 and 197 against 175.
+    const bool mid_split_k = mid && (narrow || !wide_grid || (a.offsets && a.k >= 2048 && a.n < 8192));
+    // (groups of unknown sizes from a mean of 25 on: 128 of 2048 x 768 / 3072 x 1536 at 32 rows, Q6_K, 173 / 357 on 32-token
+    // tiles against 131 / 307; at 20 rows of 3072 x 1536 270 against 299)
+    const bool short_groups = a.offsets && rows > (a.shape_rows < a.max_rows ? 24u : 32u) && rows <= 64 && fits64 && a.k <= 1536 && wide_grid;
     if (a.sums)  // debug dump: the same tile layout (and fp32 summation order) as the production choice below
         return big   ? launch_tile<F, 2, 1, 2, 1, true>(a, p, stream)
                : mid ? (mid_split_k ? launch_tile<F, 2, 1, 0, 2, true, 2, 2>(a, p, stream)
                                     : launch_tile<F, 2, 1, 1, 2, true>(a, p, stream))
+               : short_groups ? launch_tile<F, 2, 1, 1, 2, true>(a, p, stream)
                : (rows > 32 && fits64) ? launch_tile<F, 2, 1, 0, 2, true, 2, 2>(a, p, stream)
                                        : launch_tile<F, 1, 2, 0, 2, true, 2, 2>(a, p, stream);
 #ifndef OXQ_TILE_DEFAULT_SHAPES_ONLY
@@ -933,6 +942,7 @@ static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t
         }
         if (mid)
             return mid_split_k ? launch_tile<F, 2, 1, 0, 2, false, 2, 2>(a, p, stream) : launch_tile<F, 2, 1, 1, 2, false>(a, p, stream);
+        if (short_groups) return launch_tile<F, 2, 1, 1, 2, false>(a, p, stream);
         // split k; 64 weight rows (or 64 tokens) per work group only where that still leaves every
         // compute unit at least one work group, else 32 x 32
         const size_t groups = a.offsets ? a.n_experts : 1;

@@ -379,3 +379,25 @@ def test_grouped_matmul_of_a_handful_of_rows_is_one_gemv_launch(hip, ref, t, cou
     # accumulate
     dy2, _ = _run(hip, t, w, acts, offsets, n, k_, max(counts), accumulate=True, out=dy.clone())
     assert torch.equal(dy2[:rows], dy[:rows] + dy[:rows]) and torch.equal(dy2[rows:], dy[rows:])
+
+
+@pytest.mark.parametrize("t,mean,n,k_,kernel", [
+    (O.Q4_K, 32, 2052, 768, "gemm_skinny_kernel"), (O.Q4_K, 33, 2048, 768, "gemm_tile_kernel<Q4_K,2,1,1"),
+    (O.Q6_K, 24, 260, 768, "gemm_skinny_kernel"), (O.Q6_K, 25, 2048, 768, "gemm_tile_kernel<Q6_K,2,1,1"),
+    (O.Q6_K, 32, 260, 1792, "gemm_skinny_kernel"), (O.Q8_0, 21, 260, 1536, "gemm_tile_kernel"),
+    (O.IQ4_XS, 65, 2052, 2048, "gemm_tile_kernel<IQ4_XS,2,1,0")],
+    ids=["Q4_K_32", "Q4_K_33", "Q6_K_24", "Q6_K_25", "Q6_K_32", "Q8_0_21", "IQ4_XS_65"])
+def test_grouped_kernel_by_mean_and_row_length(hip, ref, t, mean, n, k_, kernel):
+    """Groups of sizes the host does not know, on both sides of each bound between this kernel and the tile kernel's shapes;
+    sizes about the mean, one group empty, one twice the mean."""
+    counts = [mean + e % 5 - 2 for e in range(32)]
+    counts[3], counts[7] = 0, counts[7] + counts[3]
+    offsets, acts, w = _case(ref, t, counts, n, k_, 8100 + mean)
+    rows = int(offsets[-1])
+    dy, _ = _run(hip, t, w, acts, offsets, n, k_, 0)
+    assert last_launch().startswith(kernel), last_launch()
+    y = dy.cpu().numpy()
+    assert np.all(y[rows:] == 7.0)
+    for e in (0, 7, 17, 31):
+        for r in {int(offsets[e]), int(offsets[e + 1]) - 1}:
+            assert_close(y[r], canonical_ref(ref, t, w[e], acts[r], n, k_), f"expert {e} row {r}")
