@@ -25,64 +25,73 @@ namespace oxq {
 // grouped rows (offsets[e] = how many chosen experts lie below e), every row belongs to token 0,
 // and each row's activations are the token's Q8_0 blocks, written k times while the logits are
 // formed.  Same tables and bytes as the separate launches.
-// The logits of experts e0 .. e0 + 7 for one token, by the 256 threads of a work group: per-thread sums over the
-// columns (16-byte loads), lane sums, one partial per wave into part[4 * q + wave].
+// The logits of experts e0 .. e0 + 7 for TB tokens from t0 on (past the last: the last once more), by the 256 threads of a
+// work group: per-thread sums over the columns (16-byte loads), lane sums, one partial per wave into part[4 * (EP * token +
+// q) + wave].
 constexpr int ROUTE_EP = 8;  // experts per pass: their loads are in flight together
-template <bool ONE>
-__device__ __forceinline__ void route_logits_pass(const float *__restrict__ router, const float *__restrict__ xr, uint32_t e0,
-                                                  uint32_t n_exp, uint32_t hidden, uint32_t k, uint8_t *__restrict__ acts,
-                                                  float *part) {
+template <bool ONE, int TB>
+__device__ __forceinline__ void route_logits_pass(const float *__restrict__ router, const float *__restrict__ x, uint32_t t0,
+                                                  uint32_t n_tokens, uint32_t e0, uint32_t n_exp, uint32_t hidden, uint32_t k,
+                                                  uint8_t *__restrict__ acts, float *part) {
     constexpr int EP = ROUTE_EP;
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const uint32_t n4 = (hidden & 3) == 0 ? hidden / 4 : 0;
-    const float *rr[EP];
-    float acc[EP];
-    for (int q = 0; q < EP; q++) {
-        rr[q] = router + (size_t)min(e0 + q, n_exp - 1) * hidden;
-        acc[q] = 0.0f;
-    }
+    const float *rr[EP], *xr[TB];
+    float acc[TB][EP];
+    for (int q = 0; q < EP; q++) rr[q] = router + (size_t)min(e0 + q, n_exp - 1) * hidden;
+    for (int t = 0; t < TB; t++) xr[t] = x + (size_t)min(t0 + t, n_tokens - 1) * hidden;
+    for (int t = 0; t < TB; t++)
+        for (int q = 0; q < EP; q++) acc[t][q] = 0.0f;
     if (n4) {
         for (uint32_t c = threadIdx.x; c < n4; c += 256) {
-            float xv[4], rv[EP][4];
-            load4(xv, xr + 4 * c);
+            float xv[TB][4], rv[EP][4];
+#pragma unroll
+            for (int t = 0; t < TB; t++) load4(xv[t], xr[t] + 4 * c);
 #pragma unroll
             for (int q = 0; q < EP; q++) load4(rv[q], rr[q] + 4 * c);
 #pragma unroll
-            for (int q = 0; q < EP; q++)
-                for (int i = 0; i < 4; i++) acc[q] += rv[q][i] * xv[i];
+            for (int t = 0; t < TB; t++)
+#pragma unroll
+                for (int q = 0; q < EP; q++)
+                    for (int i = 0; i < 4; i++) acc[t][q] += rv[q][i] * xv[t][i];
             if (ONE && e0 == 0) {
                 // the activation rows are k copies of the token's Q8_0 blocks whichever experts get chosen:
                 // written from the values in hand (eight consecutive lanes hold one block, as in the quantizer;
                 // hidden is a multiple of 32 here, so a block's lanes are in the loop together)
                 for (uint32_t r = 0; r < k; r++)
-                    encode_q8_0_lanes(xv, true, acts + ((size_t)r * (hidden / 32) + c / 8) * 34, c & 7);
+                    encode_q8_0_lanes(xv[0], true, acts + ((size_t)r * (hidden / 32) + c / 8) * 34, c & 7);
             }
         }
     } else {
         for (uint32_t c = threadIdx.x; c < hidden; c += 256)
-            for (int q = 0; q < EP; q++) acc[q] += rr[q][c] * xr[c];
+            for (int t = 0; t < TB; t++)
+                for (int q = 0; q < EP; q++) acc[t][q] += rr[q][c] * xr[t][c];
     }
 #pragma unroll
-    for (int q = 0; q < EP; q++) {
-        const float v = wave_sum(acc[q]);
-        if (lane == 0 && e0 + q < n_exp) part[4 * q + wave] = v;
-    }
+    for (int t = 0; t < TB; t++)
+#pragma unroll
+        for (int q = 0; q < EP; q++) {
+            const float v = wave_sum(acc[t][q]);
+            if (lane == 0 && e0 + q < n_exp) part[4 * (EP * t + q) + wave] = v;
+        }
 }
 
-// Many experts: the logits by a launch of their own, a work group per (token, eight experts) -- the same sums in the
+// Many experts: the logits by a launch of their own, a work group per (TB tokens, eight experts) -- the same sums in the
 // same order as inside moe_route_kernel, which then starts from them.  (One work group per token walks 128 experts of
-// 2048 columns in 35 us.)
-template <bool ONE>
+// 2048 columns in 35 us.)  What bounds it is the L2's delivery of the router's rows, once per work group: four tokens
+// at a time where that leaves two work groups per compute unit (512 tokens, 128 experts of 2048 columns: 26 to 17 us).
+template <bool ONE, int TB>
 __global__ __launch_bounds__(256) void moe_logits_kernel(const float *__restrict__ router, const float *__restrict__ x,
-                                                        float *__restrict__ logits, uint32_t n_exp, uint32_t hidden,
-                                                        uint32_t k, uint8_t *__restrict__ acts) {
-    __shared__ float part[4 * ROUTE_EP];
-    const uint32_t t = blockIdx.x, e0 = blockIdx.y * ROUTE_EP;
-    route_logits_pass<ONE>(router, x + (size_t)t * hidden, e0, n_exp, hidden, k, acts, part);
+                                                        float *__restrict__ logits, uint32_t n_tokens, uint32_t n_exp,
+                                                        uint32_t hidden, uint32_t k, uint8_t *__restrict__ acts) {
+    __shared__ float part[4 * ROUTE_EP * TB];
+    const uint32_t t0 = blockIdx.x * TB, e0 = blockIdx.y * ROUTE_EP;
+    route_logits_pass<ONE, TB>(router, x, t0, n_tokens, e0, n_exp, hidden, k, acts, part);
     __syncthreads();
-    if (threadIdx.x < ROUTE_EP && e0 + threadIdx.x < n_exp) {
-        const uint32_t q = threadIdx.x;
-        logits[(size_t)t * n_exp + e0 + q] = (part[4 * q] + part[4 * q + 1]) + (part[4 * q + 2] + part[4 * q + 3]);
+    const uint32_t t = t0 + threadIdx.x / ROUTE_EP, e = e0 + threadIdx.x % ROUTE_EP;
+    if (threadIdx.x < ROUTE_EP * TB && t < n_tokens && e < n_exp) {
+        const float *p = part + 4 * threadIdx.x;
+        logits[(size_t)t * n_exp + e] = (p[0] + p[1]) + (p[2] + p[3]);
     }
 }
 
@@ -99,8 +108,8 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float *__restrict_
     if (logits) {  // formed by moe_logits_kernel
         for (uint32_t e = threadIdx.x; e < n_exp; e += 256) probs[e] = logits[(size_t)t * n_exp + e];
     } else {
-        const float *xr = x + (size_t)t * hidden;
-        for (uint32_t e0 = 0; e0 < n_exp; e0 += ROUTE_EP) route_logits_pass<ONE>(router, xr, e0, n_exp, hidden, k, acts, part + 4 * e0);
+        for (uint32_t e0 = 0; e0 < n_exp; e0 += ROUTE_EP)
+            route_logits_pass<ONE, 1>(router, x, t, t + 1, e0, n_exp, hidden, k, acts, part + 4 * e0);
         __syncthreads();
         for (uint32_t e = threadIdx.x; e < n_exp; e += 256)
             probs[e] = (part[4 * e] + part[4 * e + 1]) + (part[4 * e + 2] + part[4 * e + 3]);
@@ -173,40 +182,55 @@ __global__ __launch_bounds__(256) void moe_route_kernel(const float *__restrict_
 // grouped row of e); pass 2 walks the pairs in ascending p = token * k + choice and gives the
 // matching ones consecutive rows.  Writes offsets[e + 1] (and offsets[0]), pair_token[row] and
 // token_rows[p]; no work group reads what another writes.
+// A chain of loads and barriers: a thread takes four consecutive pairs, and a trip of pass 2 has one barrier (the waves'
+// counts in two buffers in turn).  4096 pairs, 128 experts: 11.6 to 6.4 us.
 __global__ __launch_bounds__(256) void moe_group_kernel(const int32_t *__restrict__ experts, uint32_t n_pairs,
                                                        uint32_t k, int32_t *__restrict__ offsets,
                                                        int32_t *__restrict__ pair_token,
                                                        int32_t *__restrict__ token_rows) {
-    __shared__ uint32_t wave_cnt[4];
+    constexpr uint32_t PP = 4;
+    __shared__ uint32_t wave_cnt[2][4];
     const int32_t e = (int32_t)blockIdx.x;
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    auto load_pairs = [&](uint32_t p, int32_t (&v)[PP]) {  // pairs past the end: no expert's
+        for (uint32_t i = 0; i < PP; i++) {
+            const int32_t x = experts[min(p + i, n_pairs - 1)];
+            v[i] = p + i < n_pairs ? x : 0x7FFFFFFF;
+        }
+    };
     uint32_t below = 0;  // per wave, the same in every lane
-    for (uint32_t p0 = 0; p0 < n_pairs; p0 += 256) {
-        const uint32_t p = p0 + threadIdx.x;
-        below += (uint32_t)__popcll(__ballot(p < n_pairs && experts[p] < e));
+    for (uint32_t p0 = 0; p0 < n_pairs; p0 += 256 * PP) {
+        int32_t v[PP];
+        load_pairs(p0 + PP * threadIdx.x, v);
+        for (uint32_t i = 0; i < PP; i++) below += (uint32_t)__popcll(__ballot(v[i] < e));
     }
-    if (lane == 0) wave_cnt[wave] = below;
+    if (lane == 0) wave_cnt[1][wave] = below;
     __syncthreads();
-    uint32_t run = wave_cnt[0] + wave_cnt[1] + wave_cnt[2] + wave_cnt[3];
-    __syncthreads();
-    for (uint32_t p0 = 0; p0 < n_pairs; p0 += 256) {
-        const uint32_t p = p0 + threadIdx.x;
-        const bool match = p < n_pairs && experts[p] == e;
-        const unsigned long long ballot = __ballot(match);
-        if (lane == 0) wave_cnt[wave] = (uint32_t)__popcll(ballot);
+    uint32_t run = wave_cnt[1][0] + wave_cnt[1][1] + wave_cnt[1][2] + wave_cnt[1][3], trip = 0;
+    for (uint32_t p0 = 0; p0 < n_pairs; p0 += 256 * PP, trip ^= 1) {
+        const uint32_t p = p0 + PP * threadIdx.x;
+        int32_t v[PP];
+        load_pairs(p, v);
+        uint32_t in_wave = 0, before = 0;  // matches of the wave; of its lanes before this one
+        for (uint32_t i = 0; i < PP; i++) {
+            const unsigned long long ballot = __ballot(v[i] == e);
+            in_wave += (uint32_t)__popcll(ballot);
+            before += (uint32_t)__popcll(ballot & ((1ull << lane) - 1ull));
+        }
+        if (lane == 0) wave_cnt[trip][wave] = in_wave;
         __syncthreads();
-        uint32_t before = 0, total = 0;
+        uint32_t total = 0;
         for (uint32_t w = 0; w < 4; w++) {
-            before += w < wave ? wave_cnt[w] : 0u;
-            total += wave_cnt[w];
+            before += w < wave ? wave_cnt[trip][w] : 0u;
+            total += wave_cnt[trip][w];
         }
-        if (match) {
-            const uint32_t row = run + before + (uint32_t)__popcll(ballot & ((1ull << lane) - 1ull));
-            pair_token[row] = (int32_t)(p / k);
-            token_rows[p] = (int32_t)row;
-        }
+        uint32_t row = run + before;
+        for (uint32_t i = 0; i < PP; i++)
+            if (v[i] == e) {
+                pair_token[row] = (int32_t)((p + i) / k);
+                token_rows[p + i] = (int32_t)row++;
+            }
         run += total;
-        __syncthreads();
     }
     if (threadIdx.x == 0) {
         offsets[e + 1] = (int32_t)run;
@@ -236,23 +260,34 @@ __global__ __launch_bounds__(256) void moe_gather_quantize_kernel(const float *_
 // (moe.rs:236-254: output zeroed, then `*o += weight * e` per expert; multiply and add rounded separately).
 // splits > 1: an expert output is the sum, in index order, of `splits` partial results split_stride floats apart
 // (the down matmul left its halves of k unadded).
+// V = 4: four columns a thread (hidden a multiple of 4, buffers 16-byte aligned).  A grid row is a token; the
+// loads of four choices are in flight together (512 tokens, top 8 of 2048 columns: 14 to 7 us).
+template <int V>
 __global__ __launch_bounds__(256) void moe_combine_kernel(const float *__restrict__ y_pairs,
                                                          const int32_t *__restrict__ token_rows,
                                                          const float *__restrict__ weights, float *__restrict__ out,
-                                                         uint32_t n_tokens, uint32_t top_k, uint32_t hidden,
-                                                         uint32_t splits, size_t split_stride) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)n_tokens * hidden) return;
-    const uint32_t t = (uint32_t)(i / hidden), c = (uint32_t)(i % hidden);
-    float o = 0.0f;
-    for (uint32_t j = 0; j < top_k; j++) {
-        const size_t at = (size_t)token_rows[t * top_k + j] * hidden + c;
-        float e = y_pairs[at];
-        for (uint32_t s = 1; s < splits; s++) e += y_pairs[at + s * split_stride];
-        const float p = weights[t * top_k + j] * e;
-        o += p;
+                                                         uint32_t top_k, uint32_t hidden, uint32_t splits, size_t split_stride) {
+    typedef float vec __attribute__((ext_vector_type(V)));
+    const uint32_t t = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * V;
+    if (c >= hidden) return;
+    vec o = 0.0f;
+    for (uint32_t j0 = 0; j0 < top_k; j0 += 4) {
+        vec e[4];
+        const uint32_t nj = min(4u, top_k - j0);
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++) {  // (choices past the last: the last one's loads, not used)
+            const size_t at = (size_t)token_rows[t * top_k + j0 + min(j, nj - 1)] * hidden + c;
+            e[j] = *reinterpret_cast<const vec *>(y_pairs + at);
+            for (uint32_t s = 1; s < splits; s++) e[j] = e[j] + *reinterpret_cast<const vec *>(y_pairs + at + s * split_stride);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++)
+            if (j < nj) {
+                const vec p = weights[t * top_k + j0 + j] * e[j];
+                o = o + p;
+            }
     }
-    out[i] = o;
+    *reinterpret_cast<vec *>(out + (size_t)t * hidden + c) = o;
 }
 
 __global__ __launch_bounds__(256) void fill_zero_kernel(float *__restrict__ out, size_t n) {
@@ -280,11 +315,24 @@ hipError_t launch_moe_gather_quantize(const float *x, const int32_t *pair_token,
 hipError_t launch_moe_combine(const float *y_pairs, const int32_t *token_rows, const float *weights, float *out,
                               uint32_t n_tokens, uint32_t top_k, uint32_t hidden, hipStream_t stream, uint32_t splits,
                               size_t split_stride) {
-    const size_t n = (size_t)n_tokens * hidden;
-    if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(moe_combine_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, y_pairs, token_rows,
-                       weights, out, n_tokens, top_k, hidden, splits, split_stride);
-    return hipGetLastError();
+    if (n_tokens == 0 || hidden == 0) return hipSuccess;
+    const bool vec4 = hidden % 4 == 0 && split_stride % 4 == 0 &&
+                      ((reinterpret_cast<uintptr_t>(y_pairs) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+    for (uint32_t t = 0; t < n_tokens; t += 65535) {  // (a grid's y dimension)
+        const uint32_t nt = n_tokens - t < 65535u ? n_tokens - t : 65535u;
+        const int32_t *rows = token_rows + (size_t)t * top_k;
+        const float *w = weights + (size_t)t * top_k;
+        float *o = out + (size_t)t * hidden;
+        if (vec4)
+            hipLaunchKernelGGL(moe_combine_kernel<4>, dim3((hidden / 4 + 255) / 256, nt), dim3(256), 0, stream, y_pairs, rows, w,
+                               o, top_k, hidden, splits, split_stride);
+        else
+            hipLaunchKernelGGL(moe_combine_kernel<1>, dim3((hidden + 255) / 256, nt), dim3(256), 0, stream, y_pairs, rows, w, o,
+                               top_k, hidden, splits, split_stride);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_moe_route(const float *router, const float *x, int32_t *experts, float *weights, uint32_t n_tokens,
@@ -296,13 +344,16 @@ hipError_t launch_moe_route(const float *router, const float *x, int32_t *expert
     // floats: the logits by a launch of their own.
     const float *logits = nullptr;
     if (logits_scratch && n_exp >= 32 && n_tokens <= 65535) {
-        const dim3 grid(n_tokens, (n_exp + ROUTE_EP - 1) / ROUTE_EP);
+        const uint32_t passes = (n_exp + ROUTE_EP - 1) / ROUTE_EP;
         if (acts_one)
-            hipLaunchKernelGGL(moe_logits_kernel<true>, grid, dim3(256), 0, stream, router, x, logits_scratch, n_exp, hidden, k,
-                               acts_one);
+            hipLaunchKernelGGL((moe_logits_kernel<true, 1>), dim3(n_tokens, passes), dim3(256), 0, stream, router, x,
+                               logits_scratch, n_tokens, n_exp, hidden, k, acts_one);
+        else if ((uint64_t)(n_tokens / 4) * passes >= 2 * device_cus())
+            hipLaunchKernelGGL((moe_logits_kernel<false, 4>), dim3((n_tokens + 3) / 4, passes), dim3(256), 0, stream, router, x,
+                               logits_scratch, n_tokens, n_exp, hidden, k, acts_one);
         else
-            hipLaunchKernelGGL(moe_logits_kernel<false>, grid, dim3(256), 0, stream, router, x, logits_scratch, n_exp, hidden, k,
-                               acts_one);
+            hipLaunchKernelGGL((moe_logits_kernel<false, 1>), dim3(n_tokens, passes), dim3(256), 0, stream, router, x,
+                               logits_scratch, n_tokens, n_exp, hidden, k, acts_one);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         logits = logits_scratch;
