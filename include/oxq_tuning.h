@@ -33,7 +33,8 @@ int oxq_set_gemm_tile_min_rows(unsigned rows);
  * choice, never the few-token kernel nor the prefill kernel; 300: the prefill kernel (f16 matrix cores, Q4_K) for any
  * number of token rows; 301, 302: the f16 matrix-core kernel without a preparation launch (Q4_K, Q5_K, Q6_K) in its large
  * and its small shape; 200..205: the
- * few-token kernel (16 x 16 x 32 MFMA, groups of at most 32 token rows) in a fixed shape.  A value a format or
+ * few-token kernel (16 x 16 x 32 MFMA, groups of at most 32 token rows) in a fixed shape; 206: its form that holds the
+ * whole k of up to 16 token rows in LDS.  A value a format or
  * shape cannot take falls back to the default tile choice. */
 int oxq_set_gemm_variant(int variant);
 /* Launch-phase probe of the decode GEMV (Q4_0, Q8_0, Q4_K, Q6_K rows of at most two 64-unit steps, and the

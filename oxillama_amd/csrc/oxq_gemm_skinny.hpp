@@ -273,6 +273,213 @@ constexpr uint32_t skinny_wave_lds() {
 
 typedef float v4f32 __attribute__((ext_vector_type(4)));
 struct __attribute__((packed, aligned(4))) StripA4 { u32x4 v; };
+struct __attribute__((may_alias)) lds_word { float f; };
+
+// Where a work group's tokens lie in LDS, for `units` (sub-block, token tile) pairs: int8 operands, fp32 scales, P (one
+// factor per sub-block) or the MFMA's addends of the two halves, and with those P of each half; `end`: behind them.
+struct SkinnyLds {
+    uint8_t *A;
+    float *D, *P;
+    int *C;  // [unit][half][16 tokens]
+    float *P2;
+    uint8_t *end;
+};
+template <class F>
+__device__ __forceinline__ SkinnyLds skinny_lds(uint8_t *lds, uint32_t units) {
+    constexpr int KS = Skinny<F>::KSPLIT;
+    SkinnyLds L;
+    L.A = lds;
+    L.D = reinterpret_cast<float *>(L.A + (size_t)units * 512);
+    L.P = L.D + (size_t)units * 16;
+    L.C = reinterpret_cast<int *>(L.P);
+    L.P2 = L.P + (size_t)units * 16 * KS;
+    L.end = reinterpret_cast<uint8_t *>(L.P2 + (KS == 2 && Skinny<F>::HAS_MIN ? (size_t)units * 32 : 0));
+    return L;
+}
+
+// Thread (cc, qq) of a unit's 64: bytes 8 qq .. 8 qq + 7 of token cc's block, with the block's scale, to LDS.
+template <class F>
+__device__ __forceinline__ void skinny_put_token(u32x2 v, const float d, const uint32_t unit, const uint32_t cc, const uint32_t qq,
+                                                 const SkinnyLds &L) {
+    using S = Skinny<F>;
+    constexpr int KS = S::KSPLIT;
+    if constexpr (S::HAS_MIN && KS == 1) {
+        int sum = sdot4(v[0], 0x01010101u, sdot4(v[1], 0x01010101u, 0));
+        sum += xor1_i(sum);  // the four threads of a block
+        sum += xor2_i(sum);
+        if (qq == 0) L.P[unit * 16 + cc] = d * (float)sum;
+    }
+    if constexpr (S::HAS_MIN && KS == 2) {  // a zero-point factor per 16 weights: P of each half
+        int sum = sdot4(v[0], 0x01010101u, sdot4(v[1], 0x01010101u, 0));
+        sum += xor1_i(sum);
+        if ((qq & 1) == 0) L.P2[(unit * 2 + (qq >> 1)) * 16 + cc] = d * (float)sum;
+    }
+    if constexpr (KS == 2) {
+        // per half of the block (threads 0, 1 and 2, 3): the addend that turns sum(q a) into sum((q - OFFSET) a),
+        // on top of the 1.5 * 2^23 every result carries
+        int sum = sdot4(v[0], 0x01010101u, sdot4(v[1], 0x01010101u, 0));
+        sum += xor1_i(sum);
+        if ((qq & 1) == 0) L.C[(unit * 2 + (qq >> 1)) * 16 + cc] = 0x4B400000 - S::OFFSET * sum;
+    }
+    if (S::ACT_PERM == 1) {  // even bytes, then odd bytes
+        const uint32_t x0 = v[0], x1 = v[1];
+        v[0] = __builtin_amdgcn_perm(x1, x0, 0x06040200u);
+        v[1] = __builtin_amdgcn_perm(x1, x0, 0x07050301u);
+    }
+    if constexpr (S::ACT_PERM == 2) {
+        // weights j and j + 16 share a byte: k-slot q holds token bytes 4q .. 4q + 3, then 16 + 4q .. 16 + 4q + 3
+#pragma unroll
+        for (uint32_t i = 0; i < 2; i++)
+            *reinterpret_cast<uint32_t *>(L.A + ((size_t)unit * 64 + (2 * (qq & 1) + i) * 16 + cc) * 8 + 4 * (qq >> 1)) = v[i];
+    } else {
+        *reinterpret_cast<u32x2 *>(L.A + ((size_t)unit * 64 + qq * 16 + cc) * 8) = v;
+    }
+    if (qq == 0) L.D[unit * 16 + cc] = d;
+}
+
+// One step (two super-blocks of the wave's rows, their bytes in the strip) against the tokens whose blocks start at
+// super-block `first` of the staged ones.  sink(t, j, v, u, s, is, sum): every integer sum, as the MFMA left it.
+template <class F, int NT, int TT, int SPREAD_LOG, class Sink>
+__device__ __forceinline__ void skinny_step(uint8_t *const strip, float *const dscT, float *const minT, const SkinnyLds &L,
+                                            const uint32_t first, const uint32_t lane, const uint32_t tiles_here,
+                                            const v4i32 magic, v4f32 (&acc)[TT][NT], const Sink &sink) {
+    using S = Skinny<F>;
+    constexpr float MAGIC = 12582912.0f;  // 1.5 * 2^23: as_float(0x4B400000 + i) == MAGIC + i for |i| < 2^22
+    constexpr int KS = S::KSPLIT;  // MFMAs (and scale factors) per sub-block
+    constexpr uint32_t RS = S::ROW_STRIDE, FS = SKINNY_FAC_STRIDE;
+    constexpr uint32_t DEAD_SLOTS = (1u << SPREAD_LOG) - 1;
+    const uint32_t c = lane & 15, q = lane >> 4;
+    const uint64_t half_mask = q < 2 ? ~0ull : 0ull;
+    // scale factors of the step, decoded once: lane (c, q) takes row c, super-block q / 2, sub-blocks
+    // 4 (q % 2) .. + 3, for each tile (two factors per sub-block: per block, below)
+    if constexpr (KS == 1 && S::TABLE)
+#pragma unroll
+    for (int j = 0; j < NT; j++) {
+        typename S::Raw hd;
+        S::read_hdr(hd, strip + (16 * j + c) * RS + (q >> 1) * S::BLOCK, q & 1);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float dsc, qneg;
+            S::factors(hd, q & 1, i, dsc, qneg);
+            dscT[(16 * j + c) * FS + 4 * q + i] = dsc;
+            if (S::HAS_MIN) minT[(16 * j + c) * FS + 4 * q + i] = qneg;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        typename S::Raw raw[NT];
+#pragma unroll
+        for (int j = 0; j < NT; j++) {  // (u is a constant once the loop is unrolled)
+            const uint8_t *blk = strip + (16 * j + c) * RS + u * S::BLOCK;
+            if (u == 0) S::template read<0>(raw[j], blk, q);
+            else S::template read<1>(raw[j], blk, q);
+        }
+        const uint32_t b0 = (first + u) * 8;
+        if constexpr (KS == 2) {
+            // the block's factors (the table holds one block's: the last block's readers are done)
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                float f[4];
+                const uint8_t *blk = strip + (16 * j + c) * RS + u * S::BLOCK;
+                if constexpr (S::HAS_MIN) {
+                    float mn[4];
+                    if (u == 0) S::template block_factors<0>(blk, q, f, mn);
+                    else S::template block_factors<1>(blk, q, f, mn);
+#pragma unroll
+                    for (int b = 0; b < 4; b++) minT[(16 * j + c) * FS + 4 * q + b] = mn[b];
+                } else {
+                    if (u == 0) S::template block_factors<0>(blk, q, f);
+                    else S::template block_factors<1>(blk, q, f);
+                }
+#pragma unroll
+                for (int b = 0; b < 4; b++) dscT[(16 * j + c) * FS + 4 * q + b] = f[b];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+        if constexpr (S::HAS_MIN && KS == 2) {
+            // zero-point term, a factor per 16 weights: per four halves (slot = 2 * sub-block + half) one
+            // 16 x 16 x 4 fp32 product of P (tokens x halves) and the rows' factors of the block
+#pragma unroll
+            for (int g = 0; g < 4; g++)
+#pragma unroll
+                for (int t = 0; t < TT; t++)
+                    if (TT == 1 || t < (int)tiles_here) {
+                        const float pa = L.P2[(((b0 + 2 * g + (q >> 1)) * TT + t) * 2 + (q & 1)) * 16 + c];
+#pragma unroll
+                        for (int j = 0; j < NT; j++) {
+                            const float zb = minT[(16 * j + c) * FS + 4 * g + q];
+                            acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, zb, acc[t][j], 0, 0, 0);
+                        }
+                    }
+        }
+        if constexpr (S::HAS_MIN && KS == 1) {
+            // zero-point term: per four sub-blocks one 16 x 16 x 4 fp32 product of P (tokens x sub-blocks) and the
+            // rows' factors, straight into the accumulators
+#pragma unroll
+            for (int hf = 0; hf < 2; hf++)
+#pragma unroll
+                for (int t = 0; t < TT; t++)
+                    if (TT == 1 || t < (int)tiles_here) {
+                        const float pa = L.P[((b0 + 4 * hf + q) * TT + t) * 16 + c];
+#pragma unroll
+                        for (int j = 0; j < NT; j++) {
+                            const float zb = minT[(16 * j + c) * FS + u * 8 + 4 * hf + q];
+                            acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, zb, acc[t][j], 0, 0, 0);
+                        }
+                    }
+        }
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            float dsc[NT][KS], corr[NT][KS];
+            long bop[NT][KS];
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const long op = S::operand(raw[j], s);
+#pragma unroll
+                for (int is = 0; is < KS; is++) {
+                    if constexpr (S::TABLE) dsc[j][is] = dscT[(16 * j + c) * FS + (KS == 2 ? 2 * s + is : u * 8 + s)];
+                    else dsc[j][is] = S::scale(raw[j], s);
+                    corr[j][is] = -(MAGIC * dsc[j][is]);
+                    // two factors: k-values 0..15 come from the lanes q = 0, 1, the others supply zeros; and so on
+                    bop[j][is] = KS == 2 ? (long)((uint64_t)op & (is == 0 ? half_mask : ~half_mask)) : op;
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < TT; t++) {
+                if (TT == 1 || t < (int)tiles_here) {
+                    const uint32_t e = (b0 + s) * TT + t;
+                    const u32x2 av = *reinterpret_cast<const u32x2 *>(L.A + ((size_t)e * 64 + lane) * 8);
+                    const long a = (long)(((uint64_t)av[1] << 32) | av[0]);
+                    const v4f32 da = *reinterpret_cast<const v4f32 *>(L.D + (size_t)e * 16 + 4 * q);
+#pragma unroll
+                    for (int is = 0; is < KS; is++) {
+                        v4i32 addend = magic;
+                        if constexpr (KS == 2) addend = *reinterpret_cast<const v4i32 *>(L.C + ((size_t)e * 2 + is) * 16 + 4 * q);
+#pragma unroll
+                        for (int j = 0; j < NT; j++) {
+                            const v4i32 r = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bop[j][is], addend, 0, 0, 0);
+#pragma unroll
+                            for (int v = 0; v < 4; v++) {
+                                if (SPREAD_LOG != 0 && t == 1 && (v & DEAD_SLOTS)) continue;  // a slot without a token
+                                const int ri = r[v];
+                                const float tt = fmaf(__builtin_bit_cast(float, ri), dsc[j][is], corr[j][is]);  // fl(dsc * isum)
+                                acc[t][j][v] = fmaf(tt, da[v], acc[t][j][v]);
+                                sink(t, j, v, u, s, is, ri);
+                            }
+                        }
+                    }
+                }
+            }
+        }
+    }
+}
 
 // Work group = WAVES waves, each with its own NT x 16 weight rows; all of them the same token tiles (at most TT of
 // 16 tokens).  k is walked in chunks of `per` super-blocks (even): the work group stages the chunk's token bytes,
@@ -300,8 +507,7 @@ __device__ __forceinline__ void gemm_skinny_body(
     float *__restrict__ partial, uint32_t sb_per_split, const uint32_t tokb, const uint32_t tok_end, const uint32_t rg,
     const uint32_t gy, const uint32_t ks) {
     using S = Skinny<F>;
-    constexpr float MAGIC = 12582912.0f;  // 1.5 * 2^23: as_float(0x4B400000 + i) == MAGIC + i for |i| < 2^22
-    constexpr int KS = S::KSPLIT;  // MFMAs (and scale factors) per sub-block
+    constexpr int KS = S::KSPLIT;
     // a row's bytes of a step as 16-byte pieces: FULL whole ones from the start, and where the step's length is not
     // a multiple of 16 one more that ends with the step (overlapping the last whole one).  Four lanes share a row:
     // a load instruction takes 64 consecutive bytes of each of 16 rows, the next one the next 64, so that a lane's
@@ -319,12 +525,8 @@ __device__ __forceinline__ void gemm_skinny_body(
     const uint32_t n_super = partial ? min(k / 256, sb_lo + sb_per_split) : k / 256;
     const bool odd_super = (n_super & 1) != 0;  // (sb_lo is even: only the end of k can leave half a step)
     constexpr uint32_t per = PER, nblk_max = PER * 8;  // sub-blocks (Q8_0 blocks per token) of a full chunk
-    uint8_t *const ldsA = lds;
-    float *const ldsD = reinterpret_cast<float *>(ldsA + (size_t)nblk_max * TT * 512);
-    float *const ldsP = ldsD + (size_t)nblk_max * TT * 16;       // one factor per sub-block: P
-    int *const ldsC = reinterpret_cast<int *>(ldsP);             // two: the MFMA addends, [block][tile][half][16 tokens]
-    float *const ldsP2 = ldsP + (size_t)nblk_max * TT * 16 * KS;  // two factors and a zero-point term: P per half
-    uint8_t *const strip = reinterpret_cast<uint8_t *>(ldsP2 + (KS == 2 && S::HAS_MIN ? (size_t)nblk_max * TT * 32 : 0)) + wave * WAVE_LDS;
+    const SkinnyLds L = skinny_lds<F>(lds, nblk_max * TT);
+    uint8_t *const strip = L.end + wave * WAVE_LDS;
     float *const dscT = reinterpret_cast<float *>(strip + NT * 16 * RS);
     float *const minT = dscT + NT * 16 * FS;
 
@@ -372,40 +574,7 @@ __device__ __forceinline__ void gemm_skinny_body(
             const uint32_t idx = threadIdx.x + i * THREADS;
             if (idx >= total) continue;  // whole waves: total and THREADS are multiples of 64
             const uint32_t l = idx & 63, cc = l >> 2, qq = l & 3;
-            u32x2 v = tokA[i];
-            const float d = h2f(tokD[i]);
-            if constexpr (S::HAS_MIN && KS == 1) {
-                int sum = sdot4(v[0], 0x01010101u, sdot4(v[1], 0x01010101u, 0));
-                sum += xor1_i(sum);  // the four threads of a block
-                sum += xor2_i(sum);
-                if (qq == 0) ldsP[(idx >> 6) * 16 + cc] = d * (float)sum;
-            }
-            if constexpr (S::HAS_MIN && KS == 2) {  // a zero-point factor per 16 weights: P of each half
-                int sum = sdot4(v[0], 0x01010101u, sdot4(v[1], 0x01010101u, 0));
-                sum += xor1_i(sum);
-                if ((qq & 1) == 0) ldsP2[((idx >> 6) * 2 + (qq >> 1)) * 16 + cc] = d * (float)sum;
-            }
-            if constexpr (KS == 2) {
-                // per half of the block (threads 0, 1 and 2, 3): the addend that turns sum(q a) into sum((q - OFFSET) a),
-                // on top of the 1.5 * 2^23 every result carries
-                int sum = sdot4(v[0], 0x01010101u, sdot4(v[1], 0x01010101u, 0));
-                sum += xor1_i(sum);
-                if ((qq & 1) == 0) ldsC[((idx >> 6) * 2 + (qq >> 1)) * 16 + cc] = 0x4B400000 - S::OFFSET * sum;
-            }
-            if (S::ACT_PERM == 1) {  // even bytes, then odd bytes
-                const uint32_t x0 = v[0], x1 = v[1];
-                v[0] = __builtin_amdgcn_perm(x1, x0, 0x06040200u);
-                v[1] = __builtin_amdgcn_perm(x1, x0, 0x07050301u);
-            }
-            if constexpr (S::ACT_PERM == 2) {
-                // weights j and j + 16 share a byte: k-slot q holds token bytes 4q .. 4q + 3, then 16 + 4q .. 16 + 4q + 3
-#pragma unroll
-                for (uint32_t i = 0; i < 2; i++)
-                    *reinterpret_cast<uint32_t *>(ldsA + ((size_t)(idx >> 6) * 64 + (2 * (qq & 1) + i) * 16 + cc) * 8 + 4 * (qq >> 1)) = v[i];
-            } else {
-                *reinterpret_cast<u32x2 *>(ldsA + ((size_t)(idx >> 6) * 64 + qq * 16 + cc) * 8) = v;
-            }
-            if (qq == 0) ldsD[(idx >> 6) * 16 + cc] = d;
+            skinny_put_token<F>(tokA[i], h2f(tokD[i]), idx >> 6, cc, qq, L);
         }
     };
 
@@ -447,7 +616,6 @@ __device__ __forceinline__ void gemm_skinny_body(
     v4i32 magic;
     asm volatile("v_mov_b32 %0, 0x4b400000\n\tv_mov_b32 %1, 0x4b400000\n\tv_mov_b32 %2, 0x4b400000\n\tv_mov_b32 %3, 0x4b400000"
                  : "=v"(magic[0]), "=v"(magic[1]), "=v"(magic[2]), "=v"(magic[3]));
-    const uint64_t half_mask = q < 2 ? ~0ull : 0ull;
     u32x4 stage[NL];
     load_step(stage, sb_lo / 2);
     // (token blocks are staged by whole steps: an odd last super-block brings a dead one along)
@@ -463,8 +631,6 @@ __device__ __forceinline__ void gemm_skinny_body(
     // different sub-blocks interleave.  Two: each tile's work sits behind a branch on the group's tile count --
     // measured faster than the branch-free form, which needs more registers than two work groups per
     // compute unit leave (14336 x 4096, 8 experts, mean 12 rows: 88 us against 101).
-    {
-    constexpr int TN = TT;
     if (active)
     for (uint32_t st = sb0 / 2; st < (sb0 + nsbc) / 2; st++) {
         // the step's bytes to the strip (pieces past the end, on the last load: the last piece again, same value)
@@ -483,146 +649,19 @@ __device__ __forceinline__ void gemm_skinny_body(
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        // scale factors of the step, decoded once: lane (c, q) takes row c, super-block q / 2, sub-blocks
-        // 4 (q % 2) .. + 3, for each tile (two factors per sub-block: per block, below)
-        if constexpr (KS == 1 && S::TABLE)
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-            typename S::Raw hd;
-            S::read_hdr(hd, strip + (16 * j + c) * RS + (q >> 1) * S::BLOCK, q & 1);
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                float dsc, qneg;
-                S::factors(hd, q & 1, i, dsc, qneg);
-                dscT[(16 * j + c) * FS + 4 * q + i] = dsc;
-                if (S::HAS_MIN) minT[(16 * j + c) * FS + 4 * q + i] = qneg;
+        auto sink = [&](int t, int j, int v, int u, int s, int is, int ri) __attribute__((always_inline)) {
+            if (DUMP) {  // the integer sum of (token, weight row, sub-block or half of one)
+                const uint32_t tok = token_of(t, 4 * q + v), row = rbase + 16 * j + c;
+                // (the odd last step: its first half is the dead one, its second the last super-block)
+                const bool last_odd = odd_super && st == steps - 1;
+                const uint32_t sbi = last_odd ? n_super - 1 : st * 2 + u;
+                if (tok < tok_end && row < n && !(last_odd && u == 0))
+                    sums[((size_t)tok * n + row) * (k / 32 * KS) + (sbi * 8 + s) * KS + is] = ri - 0x4B400000;
             }
-        }
+        };
+        skinny_step<F, NT, TT, SPREAD_LOG>(strip, dscT, minT, L, st * 2 - sb0, lane, tiles_here, magic, acc, sink);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
-            typename S::Raw raw[NT];
-#pragma unroll
-            for (int j = 0; j < NT; j++) {  // (u is a constant once the loop is unrolled)
-                const uint8_t *blk = strip + (16 * j + c) * RS + u * S::BLOCK;
-                if (u == 0) S::template read<0>(raw[j], blk, q);
-                else S::template read<1>(raw[j], blk, q);
-            }
-            const uint32_t b0 = (st * 2 + u - sb0) * 8;
-            if constexpr (KS == 2) {
-                // the block's factors (the table holds one block's: the last block's readers are done)
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-#pragma unroll
-                for (int j = 0; j < NT; j++) {
-                    float f[4];
-                    const uint8_t *blk = strip + (16 * j + c) * RS + u * S::BLOCK;
-                    if constexpr (S::HAS_MIN) {
-                        float mn[4];
-                        if (u == 0) S::template block_factors<0>(blk, q, f, mn);
-                        else S::template block_factors<1>(blk, q, f, mn);
-#pragma unroll
-                        for (int b = 0; b < 4; b++) minT[(16 * j + c) * FS + 4 * q + b] = mn[b];
-                    } else {
-                        if (u == 0) S::template block_factors<0>(blk, q, f);
-                        else S::template block_factors<1>(blk, q, f);
-                    }
-#pragma unroll
-                    for (int b = 0; b < 4; b++) dscT[(16 * j + c) * FS + 4 * q + b] = f[b];
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            }
-            if constexpr (S::HAS_MIN && KS == 2) {
-                // zero-point term, a factor per 16 weights: per four halves (slot = 2 * sub-block + half) one
-                // 16 x 16 x 4 fp32 product of P (tokens x halves) and the rows' factors of the block
-#pragma unroll
-                for (int g = 0; g < 4; g++)
-#pragma unroll
-                    for (int t = 0; t < TN; t++)
-                        if (TT == 1 || t < (int)tiles_here) {
-                            const float pa = ldsP2[(((b0 + 2 * g + (q >> 1)) * TT + t) * 2 + (q & 1)) * 16 + c];
-#pragma unroll
-                            for (int j = 0; j < NT; j++) {
-                                const float zb = minT[(16 * j + c) * FS + 4 * g + q];
-                                acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, zb, acc[t][j], 0, 0, 0);
-                            }
-                        }
-            }
-            if constexpr (S::HAS_MIN && KS == 1) {
-                // zero-point term: per four sub-blocks one 16 x 16 x 4 fp32 product of P (tokens x sub-blocks) and the
-                // rows' factors, straight into the accumulators
-#pragma unroll
-                for (int hf = 0; hf < 2; hf++)
-#pragma unroll
-                    for (int t = 0; t < TN; t++)
-                        if (TT == 1 || t < (int)tiles_here) {
-                            const float pa = ldsP[((b0 + 4 * hf + q) * TT + t) * 16 + c];
-#pragma unroll
-                            for (int j = 0; j < NT; j++) {
-                                const float zb = minT[(16 * j + c) * FS + u * 8 + 4 * hf + q];
-                                acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, zb, acc[t][j], 0, 0, 0);
-                            }
-                        }
-            }
-#pragma unroll
-            for (int s = 0; s < 8; s++) {
-                float dsc[NT][KS], corr[NT][KS];
-                long bop[NT][KS];
-#pragma unroll
-                for (int j = 0; j < NT; j++) {
-                    const long op = S::operand(raw[j], s);
-#pragma unroll
-                    for (int is = 0; is < KS; is++) {
-                        if constexpr (S::TABLE) dsc[j][is] = dscT[(16 * j + c) * FS + (KS == 2 ? 2 * s + is : u * 8 + s)];
-                        else dsc[j][is] = S::scale(raw[j], s);
-                        corr[j][is] = -(MAGIC * dsc[j][is]);
-                        // two factors: k-values 0..15 come from the lanes q = 0, 1, the others supply zeros; and so on
-                        bop[j][is] = KS == 2 ? (long)((uint64_t)op & (is == 0 ? half_mask : ~half_mask)) : op;
-                    }
-                }
-#pragma unroll
-                for (int t = 0; t < TN; t++) {
-                    if (TT == 1 || t < (int)tiles_here) {
-                        const uint32_t e = (b0 + s) * TT + t;
-                        const u32x2 av = *reinterpret_cast<const u32x2 *>(ldsA + ((size_t)e * 64 + lane) * 8);
-                        const long a = (long)(((uint64_t)av[1] << 32) | av[0]);
-                        const v4f32 da = *reinterpret_cast<const v4f32 *>(ldsD + (size_t)e * 16 + 4 * q);
-#pragma unroll
-                        for (int is = 0; is < KS; is++) {
-                            v4i32 addend = magic;
-                            if constexpr (KS == 2) addend = *reinterpret_cast<const v4i32 *>(ldsC + ((size_t)e * 2 + is) * 16 + 4 * q);
-#pragma unroll
-                            for (int j = 0; j < NT; j++) {
-                                const v4i32 r = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bop[j][is], addend, 0, 0, 0);
-#pragma unroll
-                                for (int v = 0; v < 4; v++) {
-                                    if (SPREAD_LOG != 0 && t == 1 && (v & DEAD_SLOTS)) continue;  // a slot without a token
-                                    const int ri = r[v];
-                                    const float tt = fmaf(__builtin_bit_cast(float, ri), dsc[j][is], corr[j][is]);  // fl(dsc * isum)
-                                    acc[t][j][v] = fmaf(tt, da[v], acc[t][j][v]);
-                                    if (DUMP) {  // the integer sum of (token, weight row, sub-block or half of one)
-                                        const uint32_t tok = token_of(t, 4 * q + v), row = rbase + 16 * j + c;
-                                        // (the odd last step: its first half is the dead one, its second the last super-block)
-                                        const bool last_odd = odd_super && st == steps - 1;
-                                        const uint32_t sbi = last_odd ? n_super - 1 : st * 2 + u;
-                                        if (tok < tok_end && row < n && !(last_odd && u == 0))
-                                            sums[((size_t)tok * n + row) * (k / 32 * KS) + (sbi * 8 + s) * KS + is] =
-                                                ri - 0x4B400000;
-                                    }
-                                }
-                            }
-                        }
-                    }
-                }
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
     }
     }
 #pragma unroll
@@ -644,6 +683,157 @@ __device__ __forceinline__ void gemm_skinny_body(
                 }
             }
         }
+}
+
+// One matrix, at most 16 token rows of at most 4096 columns: the tokens of the whole k fit into LDS.  A work group stages them
+// once and goes through row tiles of 16; its eight waves are PARTS parts of k -- one step each -- of 8 / PARTS row tiles,
+// the parts' sums meet in LDS (in the order of k), so there is neither a reduction launch nor a chunk loop, and the next
+// two tiles' weights are in flight meanwhile.
+// What bounds it: one step's chain of LDS accesses per wave and tile, at two waves per SIMD; for a matrix of one tile per
+// work group, the latency of the first loads.  Against the other kernels: skinny_whole_pays.
+template <class F, int PARTS>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_skinny_whole_kernel(
+    const uint8_t *__restrict__ W, const uint8_t *__restrict__ A, float *__restrict__ out, uint32_t m, uint32_t n, uint32_t k,
+    int accumulate, const float *__restrict__ bias) {
+    using S = Skinny<F>;
+    constexpr uint32_t RW = 8 / PARTS;  // row tiles at a time
+    constexpr uint32_t RS = S::ROW_STRIDE, SEG = 2 * S::BLOCK, FULL = SEG / 16, TAIL = SEG % 16 ? 1 : 0;
+    constexpr uint32_t PPR = FULL + TAIL, ITR = (PPR + 3) / 4;  // a step's pieces, as in gemm_skinny_body
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const uint32_t lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), part = wave % PARTS, rw = wave / PARTS;
+    const uint32_t n_super = k / 256, steps = (n_super + 1) / 2, tiles = (n + 15) / 16;
+    const bool odd_super = (n_super & 1) != 0, live = part < steps;
+    const SkinnyLds L = skinny_lds<F>(lds, 16 * steps);
+    auto strip_of = [&](uint32_t w) { return L.end + w * skinny_wave_lds<F, 1>(); };
+    uint8_t *const strip = strip_of(wave);
+    float *const dscT = reinterpret_cast<float *>(strip + 16 * RS), *const minT = dscT + 16 * SKINNY_FAC_STRIDE;
+    const size_t row_bytes = (size_t)n_super * S::BLOCK;
+
+    const uint32_t lrow = lane >> 2, sub = lane & 3, last_piece = min(sub + 4 * (ITR - 1), PPR - 1);
+    const uint32_t last_at = ((TAIL && last_piece == PPR - 1) ? SEG - 16 : 16 * last_piece) - 16 * sub;
+    const uint32_t dst = lrow * RS + 16 * sub;
+    // (an odd last super-block: the strip holds the last two, the first of them against zeros)
+    const size_t k_off = odd_super && part == steps - 1 ? (size_t)(n_super - 2) * S::BLOCK : (size_t)part * SEG;
+    auto load_step = [&](u32x4 (&stage)[ITR], uint32_t tile) __attribute__((always_inline)) {
+        if (!live || tile >= tiles) return;
+        const uint8_t *sp = W + (size_t)min(16 * tile + lrow, n - 1) * row_bytes + k_off + 16 * sub;
+#pragma unroll
+        for (uint32_t i = 0; i < ITR; i++) stage[i] = ld16(sp + (i + 1 < ITR ? 64 * i : last_at));
+    };
+    const uint32_t stride = gridDim.x * RW;
+    u32x4 stage0[ITR], stage1[ITR];
+    load_step(stage0, blockIdx.x * RW + rw);
+    load_step(stage1, blockIdx.x * RW + stride + rw);
+
+    // (a loop, not unrolled: a short launch spends much of its time fetching instructions for the first time; with all of a
+    // thread's blocks in one batch 1024 x 4096 takes 13.9 us against 11)
+    const size_t arow = (size_t)(k / 32) * Q8_BLOCK_BYTES;
+    const uint32_t total = steps * 16 * 64, tok = (threadIdx.x & 63) >> 2, qq = threadIdx.x & 3;
+    constexpr uint32_t TB = 8;  // blocks of a thread in flight
+#pragma unroll 1
+    for (uint32_t base = threadIdx.x >> 6; base < total / 64; base += 8 * TB) {
+        u32x2 qv[TB];
+        uint32_t dv[TB];
+#pragma unroll
+        for (uint32_t i = 0; i < TB; i++) {
+            const uint32_t b = base + 8 * i;
+            uint32_t sbi = b >> 3;
+            const bool dead = odd_super && sbi == n_super - 1;
+            if (odd_super && sbi == n_super) sbi = n_super - 1;
+            qv[i] = u32x2{0, 0};
+            dv[i] = 0;
+            if (b < total / 64 && tok < m && !dead) {
+                const uint8_t *blk = A + (size_t)tok * arow + (size_t)(sbi * 8 + (b & 7)) * Q8_BLOCK_BYTES;
+                qv[i] = ld8(blk + 2 + 8 * qq);
+                dv[i] = ld2(blk);
+            }
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < TB; i++)
+            if (base + 8 * i < total / 64) skinny_put_token<F>(qv[i], h2f(dv[i]), base + 8 * i, tok, qq, L);
+    }
+    __syncthreads();
+
+    v4i32 magic;
+    asm volatile("v_mov_b32 %0, 0x4b400000\n\tv_mov_b32 %1, 0x4b400000\n\tv_mov_b32 %2, 0x4b400000\n\tv_mov_b32 %3, 0x4b400000"
+                 : "=v"(magic[0]), "=v"(magic[1]), "=v"(magic[2]), "=v"(magic[3]));
+    auto one_tile = [&](u32x4 (&stage)[ITR], uint32_t base) __attribute__((always_inline)) {
+        const uint32_t tile = base + rw;
+        const bool active = live && tile < tiles;
+        if (active) {
+#pragma unroll
+            for (uint32_t i = 0; i < ITR; i++) {
+                if (i + 1 < ITR)
+                    *reinterpret_cast<u32x4 *>(strip + dst + 64 * i) = stage[i];
+                else if (TAIL)
+                    reinterpret_cast<StripA4 *>(strip + dst + last_at)->v = stage[i];
+                else
+                    *reinterpret_cast<u32x4 *>(strip + dst + last_at) = stage[i];
+            }
+            load_step(stage, tile + 2 * stride);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            v4f32 acc[1][1] = {{v4f32{0.0f, 0.0f, 0.0f, 0.0f}}};
+            skinny_step<F, 1, 1, 0>(strip, dscT, minT, L, 2 * part, lane, 1, magic, acc, [](int, int, int, int, int, int, int) {});
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            // the sums over the strip's first KB: [result of the lane][lane]
+#pragma unroll
+            for (int v = 0; v < 4; v++) reinterpret_cast<lds_word *>(strip)[v * 64 + lane].f = acc[0][0][v];
+        }
+        __syncthreads();
+        const uint32_t row = 16 * tile + c;
+        if (row < n) {
+#pragma unroll
+            for (uint32_t v = part; v < 4; v += PARTS) {
+                float y = reinterpret_cast<const lds_word *>(strip_of(rw * PARTS))[v * 64 + lane].f;
+                for (uint32_t p = 1; p < steps; p++) y += reinterpret_cast<const lds_word *>(strip_of(rw * PARTS + p))[v * 64 + lane].f;
+                if (4 * q + v < m) {
+                    float *o = out + (size_t)(4 * q + v) * n + row;
+                    *o = accumulate ? *o + y : bias ? y + bias[row] : y;
+                }
+            }
+        }
+        __syncthreads();
+    };
+    for (uint32_t base = blockIdx.x * RW; base < tiles; base += 2 * stride) {
+        one_tile(stage0, base);
+        if (base + stride < tiles) one_tile(stage1, base + stride);  // (the same for the whole work group)
+    }
+}
+
+constexpr uint32_t SKINNY_WHOLE_MAX_K = 4096;
+// Where it is the better kernel: matrices of fewer than 2^25 weights.  Up to 16 rows, us, against the tile kernel with its
+// token re-layout or, from 4096 columns on, k split over work groups with a reduction launch: 2560 x 2560 Q4_K 16.2 to 10.4,
+// IQ4_XS 14.5 to 9.4, Q6_K 19.0 to 14.0, Q8_0 17.1 to 10.0; 8960 x 1536 Q4_K 17.0 to 12.5; 6144 x 3072 Q5_K 19.2 to 17.4; 1024 x
+// 4096 Q4_K 12.9 to 11.3, 4096 x 4096 Q4_K 14.2 to 13.2, IQ4_XS 14.8 to 13.1, Q8_0 17.7 to 16.2.  14336 x 4096 is a tie for
+// Q4_K (20.5 / 20.9) and a loss for Q6_K (29.4 / 35.2); at 4096 columns the formats whose high bits lie apart are too (4096 x
+// 4096 Q5_K 15.6 / 17.0, Q5_0 16.2 / 17.4), Q6_K but for (18.1 / 18.3, 1024 x 4096 16.8 / 15.8).
+static inline bool skinny_whole_pays(uint32_t type, uint32_t n, uint32_t k) {
+    if (k % 256 != 0 || k < 512 || k > SKINNY_WHOLE_MAX_K || (uint64_t)n * k >= (1ull << 25)) return false;
+    return k < 4096 || !(type == OXQ_TYPE_Q5_K || type == OXQ_TYPE_Q5_0 || type == OXQ_TYPE_Q5_1 || type == OXQ_TYPE_Q3_K ||
+                         type == OXQ_TYPE_Q2_K);
+}
+
+template <class F>
+static hipError_t launch_skinny_whole(const GemmArgs &a, hipStream_t stream) {
+    const uint32_t steps = (a.k / 256 + 1) / 2;
+    if (a.offsets || a.sums || a.m == 0 || a.m > 16 || a.n == 0 || a.k % 256 != 0 || a.k < 512 || steps > 8) return hipErrorNotSupported;
+    const uint32_t parts = steps > 4 ? 8 : steps > 2 ? 4 : 2;
+    auto kern = parts == 8 ? &gemm_skinny_whole_kernel<F, 8> : parts == 4 ? &gemm_skinny_whole_kernel<F, 4> : &gemm_skinny_whole_kernel<F, 2>;
+    const size_t lds = (size_t)16 * steps * skinny_act_bytes<F>() + 8 * skinny_wave_lds<F, 1>();
+    if (lds > 160 * 1024) return hipErrorNotSupported;
+    const hipError_t e = allow_lds(reinterpret_cast<const void *>(kern), lds);
+    if (e != hipSuccess) return e;
+    // one work group per compute unit at most, all with the same number of row tiles but the last
+    const uint32_t sets = ((a.n + 15) / 16 + 8 / parts - 1) / (8 / parts), each = (sets + device_cus() - 1) / device_cus();
+    const dim3 grid((sets + each - 1) / each);
+    note_launch("gemm_skinny_whole_kernel", F::TYPE, (int)parts, 0, 0, 0, grid.x, 1, 512);
+    hipLaunchKernelGGL(kern, grid, dim3(512), lds, stream, a.W, a.A, a.out, a.m, a.n, a.k, a.accumulate, a.bias);
+    return hipGetLastError();
 }
 
 // The kernel: finds the work group's token rows and runs the body.  A launch shaped for two token tiles runs the
@@ -829,7 +1019,7 @@ static hipError_t launch_skinny_shape(const GemmArgs &a, const TilePlan &p, hipS
 //    14336 x 4096 18.0 us against 19.6, 4096 x 14336 21.4 against 29.5, 28672 x 8192 40 against 49; 4096 x 4096
 //    14.4 against 12.3 (not taken below 2^25 weights); 17..32 rows 24.6 against 19.7 (not taken).  From 512 row
 //    groups on no split is needed (57344 x 4096, 16 rows: 44 us against 56).
-enum SkinnyShape { SK_NONE = 0, SK_1_4, SK_1_8, SK_2_2, SK_1_4_SPLIT, SK_1_16, SK_2_8, SK_W4_1_8, SK_W4_2_4, SK_2_4, SK_2_2_SPLIT };
+enum SkinnyShape { SK_NONE = 0, SK_1_4, SK_1_8, SK_2_2, SK_1_4_SPLIT, SK_1_16, SK_2_8, SK_W4_1_8, SK_W4_2_4, SK_2_4, SK_2_2_SPLIT, SK_WHOLE };
 
 // Expert groups of up to this many rows in the mean stay with this kernel (groups beyond its tiles take further passes
 // over their expert's weights).  Against the tile kernel, us per matmul, groups of random sizes about the mean:
@@ -865,11 +1055,12 @@ static int skinny_shape(const GemmArgs &a, bool has_partial, uint32_t rows, int 
         if (a.k % 256 != 0 || a.k < 512 || (rows > 32 && !(a.offsets && (size_t)a.m <= mean_limit * (size_t)a.n_experts))) return SK_NONE;
         const bool two = rows > 16;
         // the formats with the long strips: the one-tile shapes only (see launch_skinny)
-        if (Skinny<F>::ONE_TILE && variant != 0 && variant != 200) return SK_NONE;
+        if (Skinny<F>::ONE_TILE && variant != 0 && variant != 200 && variant != 206) return SK_NONE;
         if (a.sums && variant != 0 && variant != 200) return SK_NONE;  // the dump exists for the default shapes
         switch (variant) {
         case 0: {
             if (!a.offsets) {
+                if (!a.sums && !two && skinny_whole_pays(F::TYPE, a.n, a.k)) return SK_WHOLE;
                 // one matrix, up to 16 token rows: enough row groups by themselves (a vocabulary projection), or k
                 // split over work groups (the workspace has room for the sums)
                 if (two) {
@@ -916,6 +1107,7 @@ static int skinny_shape(const GemmArgs &a, bool has_partial, uint32_t rows, int 
         case 203: return two ? SK_W4_2_4 : SK_W4_1_8;
         case 204: return two ? SK_2_2 : SK_1_4;
         case 205: return two ? SK_2_4 : SK_1_8;
+        case 206: return !two && !a.offsets && a.k <= SKINNY_WHOLE_MAX_K ? SK_WHOLE : SK_NONE;
         default: return SK_NONE;
         }
     }
@@ -925,6 +1117,8 @@ static int skinny_shape(const GemmArgs &a, bool has_partial, uint32_t rows, int 
 // <NT, WAVES, TT, PER>; LDS = PER * 8 * TT * 640 + WAVES * NT * 7 KB
 template <class F>
 static hipError_t launch_skinny(const GemmArgs &a, const TilePlan &p, hipStream_t stream, int shape) {
+    if constexpr (Skinny<F>::OK)
+        if (shape == SK_WHOLE) return launch_skinny_whole<F>(a, stream);
     if constexpr (Skinny<F>::OK && Skinny<F>::ONE_TILE) {
         // Q6_K, Q8_0: 8 KB of LDS and more per wave; with chunks of two super-blocks of one token tile two work
         // groups still share a compute unit (75 and 78 KB each)

@@ -401,3 +401,53 @@ def test_grouped_kernel_by_mean_and_row_length(hip, ref, t, mean, n, k_, kernel)
     for e in (0, 7, 17, 31):
         for r in {int(offsets[e]), int(offsets[e + 1]) - 1}:
             assert_close(y[r], canonical_ref(ref, t, w[e], acts[r], n, k_), f"expert {e} row {r}")
+
+
+@pytest.mark.parametrize("t", FORMATS_1TILE, ids=lambda t: O.NAMES[t])
+@pytest.mark.parametrize("shape", [(16, 33, 512), (1, 16, 768), (7, 20, 1280), (16, 4112, 1536), (13, 100, 2304), (5, 8300, 2048),
+                                   (9, 4099, 3840), (16, 40, 4096)], ids=lambda s: "x".join(map(str, s)))
+def test_whole_k_in_lds(hip, ref, tuning, t, shape):
+    """Up to 16 token rows of up to 4096 columns, the whole k at once: 2, 4 and 8 parts of k, the last of them half a step
+    where the super-blocks are odd (3, 5, 9, 15), parts without work, row tiles with rows to spare and more tiles than
+    work groups; overwrite, accumulate and bias."""
+    import torch
+    from oxillama_amd import linear
+    m, n, k_ = shape
+    w = weights(t, 91, n, k_)
+    acts = ref.quantize_q8_0(synth.normal_f32(92 + m, m * k_)).reshape(m, k_ // 32 * 34)
+    bias = synth.normal_f32(93, n)
+    kern = hip.HipKernel(t)
+    dw, da, db = torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda(), torch.from_numpy(bias).cuda()
+    tuning("gemm_tile_min_rows", 1)
+    tuning("gemm_variant", 206)
+    ws = torch.empty(kern.gemm_workspace_bytes(m, n, k_), dtype=torch.uint8, device="cuda")
+    dy = torch.full((m + 1, n), 7.0, dtype=torch.float32, device="cuda")
+    kern.gemm_q8_dev(dw, da, dy, m, n, k_, workspace=ws)
+    torch.cuda.synchronize()
+    assert last_launch().startswith("gemm_skinny_whole_kernel"), last_launch()
+    y = dy.cpu().numpy()
+    assert np.all(y[m:] == 7.0)
+    for r in range(m):
+        assert_close(y[r], canonical_ref(ref, t, w, acts[r], n, k_), f"{shape} row {r}")
+    dy2 = dy[:m].clone()
+    kern.gemm_q8_dev(dw, da, dy2, m, n, k_, accumulate=True, workspace=ws)
+    dy3 = torch.zeros((m, n), dtype=torch.float32, device="cuda")
+    linear.linear_forward_batch_dev(t, dw, da, dy3, m, n, k_, d_bias=db, workspace=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(dy2, dy[:m] + dy[:m]) and torch.equal(dy3, dy[:m] + db[None, :])
+
+
+def test_whole_k_in_lds_by_default(hip, ref):
+    """The default choice for matrices below 2^25 weights: from the rows on at which the GEMV launches end, up to 16."""
+    import torch
+    t, n, k_ = O.Q4_K, 2560, 2560
+    w, kern = weights(t, 95, n, k_), hip.HipKernel(O.Q4_K)
+    dw = torch.from_numpy(w).cuda()
+    for m, whole in ((8, False), (9, True), (16, True), (17, False)):
+        acts = ref.quantize_q8_0(synth.normal_f32(96, m * k_)).reshape(m, k_ // 32 * 34)
+        da, dy = torch.from_numpy(acts).cuda(), torch.zeros((m, n), dtype=torch.float32, device="cuda")
+        ws = torch.empty(kern.gemm_workspace_bytes(m, n, k_), dtype=torch.uint8, device="cuda")
+        kern.gemm_q8_dev(dw, da, dy, m, n, k_, workspace=ws)
+        torch.cuda.synchronize()
+        assert last_launch().startswith("gemm_skinny_whole_kernel") == whole, (m, last_launch())
+        assert_close(dy[m - 1].cpu().numpy(), canonical_ref(ref, t, w, acts[m - 1], n, k_), f"m={m}")
