@@ -51,11 +51,15 @@ struct Args {
         Py_DECREF(r);
         return n;
     }
-    template <class T> T *ptr_of(PyObject *o) {
-        if (!ok || o == Py_None) return nullptr;
-        return (T *)(uintptr_t)(PyLong_Check(o) ? number(o) : method(o, s_data_ptr));
-    }
-    template <class T> T *ptr(int i) { return ptr_of<T>(v[i]); }
+    // A tensor that the call cannot do without: what has no data_ptr() -- None and integers among it -- is an
+    // AttributeError here, as the C ABI launches with the addresses that it gets.
+    template <class T> T *tensor_of(PyObject *o) { return (T *)(uintptr_t)method(o, s_data_ptr); }
+    template <class T> T *tensor(int i) { return tensor_of<T>(v[i]); }
+    // One that it can do without: None is a null pointer.
+    template <class T> T *maybe_of(PyObject *o) { return o == Py_None ? nullptr : tensor_of<T>(o); }
+    template <class T> T *maybe(int i) { return maybe_of<T>(v[i]); }
+    // The address of a host structure, or None.
+    template <class T> T *address(int i) { return v[i] == Py_None ? nullptr : (T *)(uintptr_t)number(v[i]); }
     size_t size(int i) { return (size_t)number(v[i]); }
     uint32_t u32(int i) { return (uint32_t)number(v[i]); }
     float f32(int i) {
@@ -103,79 +107,79 @@ struct Args {
 
 OXQ_ENTRY(rmsnorm_quantize, 7,
           p_oxq_rmsnorm_quantize_q8_0_dev(x, w, eps, rows, cols, y, q8, stream),
-          auto x = a.ptr<float>(0); auto w = a.ptr<float>(1); float eps = a.f32(2); size_t rows = a.size(3), cols = a.size(4);
-          auto y = a.ptr<float>(5); auto q8 = a.ptr<uint8_t>(6);)
+          auto x = a.tensor<float>(0); auto w = a.tensor<float>(1); float eps = a.f32(2); size_t rows = a.size(3), cols = a.size(4);
+          auto y = a.maybe<float>(5); auto q8 = a.maybe<uint8_t>(6);)
 
 OXQ_ENTRY(linear_forward, 9,
           p_oxq_linear_forward_dev(t, w, x, acts, bias, lora, out, of, in, stream),
-          uint32_t t = a.u32(0); auto w = a.ptr<uint8_t>(1); auto x = a.ptr<float>(2); auto acts = a.ptr<uint8_t>(3);
-          auto bias = a.ptr<float>(4); auto lora = a.ptr<oxq_lora>(5); auto out = a.ptr<float>(6);
+          uint32_t t = a.u32(0); auto w = a.tensor<uint8_t>(1); auto x = a.maybe<float>(2); auto acts = a.maybe<uint8_t>(3);
+          auto bias = a.maybe<float>(4); auto lora = a.address<oxq_lora>(5); auto out = a.tensor<float>(6);
           size_t of = a.size(7), in = a.size(8);)
 
 OXQ_ENTRY(linear_forward_batch, 9,
           p_oxq_linear_forward_batch_dev(t, w, acts, bias, out, batch, of, in, ws, ws_n, stream),
-          uint32_t t = a.u32(0); auto w = a.ptr<uint8_t>(1); auto acts = a.ptr<uint8_t>(2); auto bias = a.ptr<float>(3);
-          auto out = a.ptr<float>(4); size_t batch = a.size(5), of = a.size(6), in = a.size(7);
-          auto ws = a.ptr<void>(8); size_t ws_n = a.numel(8);)
+          uint32_t t = a.u32(0); auto w = a.tensor<uint8_t>(1); auto acts = a.tensor<uint8_t>(2); auto bias = a.maybe<float>(3);
+          auto out = a.tensor<float>(4); size_t batch = a.size(5), of = a.size(6), in = a.size(7);
+          auto ws = a.maybe<void>(8); size_t ws_n = a.numel(8);)
 
 OXQ_ENTRY(gemm_q8, 9,
           p_oxq_gemm_q8_dev(t, w, acts, out, m, rows, k, acc, ws, ws_n, stream),
-          uint32_t t = a.u32(0); auto w = a.ptr<uint8_t>(1); auto acts = a.ptr<uint8_t>(2); auto out = a.ptr<float>(3);
-          size_t m = a.size(4), rows = a.size(5), k = a.size(6); int acc = (int)a.size(7); auto ws = a.ptr<void>(8);
+          uint32_t t = a.u32(0); auto w = a.tensor<uint8_t>(1); auto acts = a.tensor<uint8_t>(2); auto out = a.tensor<float>(3);
+          size_t m = a.size(4), rows = a.size(5), k = a.size(6); int acc = (int)a.size(7); auto ws = a.maybe<void>(8);
           size_t ws_n = a.numel(8);)
 
 OXQ_ENTRY(matvec_q8_fused, 7,
           p_oxq_matvec_q8_fused_dev(t, w, acts, out, rows, cols, acc, stream),
-          uint32_t t = a.u32(0); auto w = a.ptr<uint8_t>(1); auto acts = a.ptr<uint8_t>(2); auto out = a.ptr<float>(3);
+          uint32_t t = a.u32(0); auto w = a.tensor<uint8_t>(1); auto acts = a.tensor<uint8_t>(2); auto out = a.tensor<float>(3);
           size_t rows = a.size(4), cols = a.size(5); int acc = (int)a.size(6);)
 
 OXQ_ENTRY(swiglu_quantize, 4,
           p_oxq_swiglu_quantize_q8_0_dev(g, u, total, h, q8, stream),
-          auto g = a.ptr<float>(0); auto u = a.ptr<float>(1); size_t total = a.numel(0); auto h = a.ptr<float>(2);
-          auto q8 = a.ptr<uint8_t>(3);)
+          auto g = a.tensor<float>(0); auto u = a.tensor<float>(1); size_t total = a.numel(0); auto h = a.maybe<float>(2);
+          auto q8 = a.maybe<uint8_t>(3);)
 
 OXQ_ENTRY(quantize_q8_0, 2,
           p_oxq_quantize_q8_0_dev(x, total, out, stream),
-          auto x = a.ptr<float>(0); size_t total = a.numel(0); auto out = a.ptr<uint8_t>(1);)
+          auto x = a.tensor<float>(0); size_t total = a.numel(0); auto out = a.tensor<uint8_t>(1);)
 
 OXQ_ENTRY(ffn_swiglu, 11,
           p_oxq_ffn_swiglu_dev(tg, g, tu, u, td, d, acts, out, hidden, inter, ws, ws_n, stream),
-          uint32_t tg = a.u32(0); auto g = a.ptr<uint8_t>(1); uint32_t tu = a.u32(2); auto u = a.ptr<uint8_t>(3);
-          uint32_t td = a.u32(4); auto d = a.ptr<uint8_t>(5); auto acts = a.ptr<uint8_t>(6); auto out = a.ptr<float>(7);
-          size_t hidden = a.size(8), inter = a.size(9); auto ws = a.ptr<void>(10); size_t ws_n = a.numel(10);)
+          uint32_t tg = a.u32(0); auto g = a.tensor<uint8_t>(1); uint32_t tu = a.u32(2); auto u = a.tensor<uint8_t>(3);
+          uint32_t td = a.u32(4); auto d = a.tensor<uint8_t>(5); auto acts = a.tensor<uint8_t>(6); auto out = a.tensor<float>(7);
+          size_t hidden = a.size(8), inter = a.size(9); auto ws = a.tensor<void>(10); size_t ws_n = a.numel(10);)
 
 OXQ_ENTRY(topk, 5,
           p_oxq_topk_dev(x, total, k, ov, oi, ws, ws_n, stream),
-          auto x = a.ptr<float>(0); size_t total = a.numel(0), k = a.size(1); auto ov = a.ptr<float>(2);
-          auto oi = a.ptr<uint32_t>(3); auto ws = a.ptr<void>(4); size_t ws_n = a.bytes(4);)
+          auto x = a.tensor<float>(0); size_t total = a.numel(0), k = a.size(1); auto ov = a.tensor<float>(2);
+          auto oi = a.tensor<uint32_t>(3); auto ws = a.tensor<void>(4); size_t ws_n = a.bytes(4);)
 
 OXQ_ENTRY(lm_head_topk, 10,
           p_oxq_lm_head_topk_dev(t, w, acts, logits, rows, cols, k, ov, oi, ws, ws_n, stream),
-          uint32_t t = a.u32(0); auto w = a.ptr<uint8_t>(1); auto acts = a.ptr<uint8_t>(2); auto logits = a.ptr<float>(3);
-          size_t rows = a.size(4), cols = a.size(5), k = a.size(6); auto ov = a.ptr<float>(7); auto oi = a.ptr<uint32_t>(8);
-          auto ws = a.ptr<void>(9); size_t ws_n = a.bytes(9);)
+          uint32_t t = a.u32(0); auto w = a.tensor<uint8_t>(1); auto acts = a.tensor<uint8_t>(2); auto logits = a.tensor<float>(3);
+          size_t rows = a.size(4), cols = a.size(5), k = a.size(6); auto ov = a.tensor<float>(7); auto oi = a.tensor<uint32_t>(8);
+          auto ws = a.tensor<void>(9); size_t ws_n = a.bytes(9);)
 
 OXQ_ENTRY(logits_edit, 7,
           p_oxq_logits_edit_dev(x, total, ban, n_ban, bt, bv, n_bias, rec, n_rec, window, pen, stream),
-          auto x = a.ptr<float>(0); size_t total = a.numel(0), n_ban = a.numel(1), n_bias = a.numel(2), n_rec = a.numel(4);
-          auto ban = n_ban ? a.ptr<uint32_t>(1) : nullptr; auto bt = n_bias ? a.ptr<uint32_t>(2) : nullptr;
-          auto bv = v[3] != Py_None && a.numel(3) ? a.ptr<float>(3) : nullptr; auto rec = n_rec ? a.ptr<uint32_t>(4) : nullptr;
+          auto x = a.tensor<float>(0); size_t total = a.numel(0), n_ban = a.numel(1), n_bias = a.numel(2), n_rec = a.numel(4);
+          auto ban = n_ban ? a.maybe<uint32_t>(1) : nullptr; auto bt = n_bias ? a.maybe<uint32_t>(2) : nullptr;
+          auto bv = v[3] != Py_None && a.numel(3) ? a.maybe<float>(3) : nullptr; auto rec = n_rec ? a.maybe<uint32_t>(4) : nullptr;
           size_t window = a.size(5); float pen = a.f32(6);)
 
 OXQ_ENTRY(sample_candidates, 9,
           p_oxq_sample_candidates_dev(x, idx, k, temp, min_p, top_p, rng, tok, probs, stream),
-          auto x = a.ptr<float>(0); auto idx = a.ptr<uint32_t>(1); size_t k = a.size(2);
-          float temp = a.f32(3), min_p = a.f32(4), top_p = a.f32(5); auto rng = a.ptr<uint64_t>(6);
-          auto tok = a.ptr<uint32_t>(7); auto probs = a.ptr<float>(8);)
+          auto x = a.tensor<float>(0); auto idx = a.tensor<uint32_t>(1); size_t k = a.size(2);
+          float temp = a.f32(3), min_p = a.f32(4), top_p = a.f32(5); auto rng = a.tensor<uint64_t>(6);
+          auto tok = a.tensor<uint32_t>(7); auto probs = a.maybe<float>(8);)
 
 OXQ_ENTRY(moe_forward, 18,
           p_oxq_moe_forward_dev(tg, g, sg, tu, u, su, td, d, sd, n_exp, router, x, tokens, top_k, out, hidden, inter, ws, ws_n,
                                 stream),
-          uint32_t tg = a.u32(0); auto g = a.ptr<uint8_t>(1); size_t sg = a.size(2); uint32_t tu = a.u32(3);
-          auto u = a.ptr<uint8_t>(4); size_t su = a.size(5); uint32_t td = a.u32(6); auto d = a.ptr<uint8_t>(7);
-          size_t sd = a.size(8), n_exp = a.size(9); auto router = a.ptr<float>(10); auto x = a.ptr<float>(11);
-          size_t tokens = a.size(12), top_k = a.size(13); auto out = a.ptr<float>(14); size_t hidden = a.size(15);
-          size_t inter = a.size(16); auto ws = a.ptr<void>(17); size_t ws_n = a.numel(17);)
+          uint32_t tg = a.u32(0); auto g = a.tensor<uint8_t>(1); size_t sg = a.size(2); uint32_t tu = a.u32(3);
+          auto u = a.tensor<uint8_t>(4); size_t su = a.size(5); uint32_t td = a.u32(6); auto d = a.tensor<uint8_t>(7);
+          size_t sd = a.size(8), n_exp = a.size(9); auto router = a.tensor<float>(10); auto x = a.tensor<float>(11);
+          size_t tokens = a.size(12), top_k = a.size(13); auto out = a.tensor<float>(14); size_t hidden = a.size(15);
+          size_t inter = a.size(16); auto ws = a.tensor<void>(17); size_t ws_n = a.numel(17);)
 
 // (type, weights, acts, biases or None, outs, rows of each, columns): sequences of the same length, at most MAX_MATS
 constexpr Py_ssize_t MAX_MATS = 64;
@@ -199,13 +203,13 @@ PyObject *linear_forward_multi(PyObject *, PyObject *const *v, Py_ssize_t n) {
         }
     }
     for (Py_ssize_t j = 0; j < mats && a.ok; j++) {
-        w[j] = a.ptr_of<uint8_t>(PySequence_Fast_GET_ITEM(seq[0], j));
-        bias[j] = seq[1] ? a.ptr_of<float>(PySequence_Fast_GET_ITEM(seq[1], j)) : nullptr;
-        out[j] = a.ptr_of<float>(PySequence_Fast_GET_ITEM(seq[2], j));
+        w[j] = a.tensor_of<uint8_t>(PySequence_Fast_GET_ITEM(seq[0], j));
+        bias[j] = seq[1] ? a.maybe_of<float>(PySequence_Fast_GET_ITEM(seq[1], j)) : nullptr;
+        out[j] = a.tensor_of<float>(PySequence_Fast_GET_ITEM(seq[2], j));
         rows[j] = (size_t)a.number(PySequence_Fast_GET_ITEM(seq[3], j));
     }
     const uint32_t t = a.u32(0);
-    auto acts = a.ptr<uint8_t>(2);
+    auto acts = a.tensor<uint8_t>(2);
     const size_t cols = a.size(6);
     void *const stream = a.stream();
     const bool has_bias = seq[1] != nullptr;
