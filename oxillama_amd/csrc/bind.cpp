@@ -181,7 +181,9 @@ OXQ_ENTRY(moe_forward, 18,
           size_t tokens = a.size(12), top_k = a.size(13); auto out = a.tensor<float>(14); size_t hidden = a.size(15);
           size_t inter = a.size(16); auto ws = a.tensor<void>(17); size_t ws_n = a.numel(17);)
 
-// (type, weights, acts, biases or None, outs, rows of each, columns): sequences of the same length, at most MAX_MATS
+// (type, weights, acts, biases or None, outs, rows of each, columns).  An output for every weight; a matrix past the end
+// of the biases has none, one past the end of the row counts has no rows, which the C ABI refuses, as it does more than
+// four matrices (the first MAX_MATS are looked at).
 constexpr Py_ssize_t MAX_MATS = 64;
 PyObject *linear_forward_multi(PyObject *, PyObject *const *v, Py_ssize_t n) {
     if (n != 7) return PyErr_Format(PyExc_TypeError, "linear_forward_multi takes 7 arguments");
@@ -197,27 +199,31 @@ PyObject *linear_forward_multi(PyObject *, PyObject *const *v, Py_ssize_t n) {
         if (i == 1 && v[3] == Py_None) continue;
         if (!(seq[i] = PySequence_Fast(v[at[i]], "a sequence with an entry per matrix"))) a.ok = false;
         else if (i == 0) mats = PySequence_Fast_GET_SIZE(seq[0]);
-        if (a.ok && (PySequence_Fast_GET_SIZE(seq[i]) != mats || mats > MAX_MATS)) {
+        const Py_ssize_t have = a.ok ? PySequence_Fast_GET_SIZE(seq[i]) : 0;
+        if (a.ok && (have > mats || (i == 2 && have < mats))) {
             PyErr_SetString(PyExc_ValueError, "linear_forward_multi: one weight, output, row count (and bias) per matrix");
             a.ok = false;
         }
     }
-    for (Py_ssize_t j = 0; j < mats && a.ok; j++) {
-        w[j] = a.tensor_of<uint8_t>(PySequence_Fast_GET_ITEM(seq[0], j));
-        bias[j] = seq[1] ? a.maybe_of<float>(PySequence_Fast_GET_ITEM(seq[1], j)) : nullptr;
-        out[j] = a.tensor_of<float>(PySequence_Fast_GET_ITEM(seq[2], j));
-        rows[j] = (size_t)a.number(PySequence_Fast_GET_ITEM(seq[3], j));
+    auto item = [&](int i, Py_ssize_t j) { return j < PySequence_Fast_GET_SIZE(seq[i]) ? PySequence_Fast_GET_ITEM(seq[i], j) : nullptr; };
+    for (Py_ssize_t j = 0; j < mats && j < MAX_MATS && a.ok; j++) {
+        w[j] = a.tensor_of<uint8_t>(item(0, j));
+        PyObject *const b = seq[1] ? item(1, j) : nullptr, *const r = item(3, j);
+        bias[j] = b ? a.maybe_of<float>(b) : nullptr;
+        out[j] = a.tensor_of<float>(item(2, j));
+        rows[j] = r ? (size_t)a.number(r) : 0;
     }
     const uint32_t t = a.u32(0);
     auto acts = a.tensor<uint8_t>(2);
     const size_t cols = a.size(6);
     void *const stream = a.stream();
-    const bool has_bias = seq[1] != nullptr;
+    int st = 0;
+    if (a.ok) {
+        Py_BEGIN_ALLOW_THREADS st = p_oxq_linear_forward_multi_dev(t, (size_t)mats, w, acts, seq[1] ? bias : nullptr, out, rows, cols, stream);
+        Py_END_ALLOW_THREADS
+    }
     for (PyObject *s : seq) Py_XDECREF(s);
-    if (!a.ok) return nullptr;
-    int st;
-    Py_BEGIN_ALLOW_THREADS st = p_oxq_linear_forward_multi_dev(t, (size_t)mats, w, acts, has_bias ? bias : nullptr, out, rows, cols, stream);
-    Py_END_ALLOW_THREADS return PyLong_FromLong(st);
+    return a.ok ? PyLong_FromLong(st) : nullptr;
 }
 
 // attach({name: address}): the functions of the library that capi.py loaded

@@ -93,3 +93,35 @@ refused(AttributeError, linear.swiglu_quantize_dev, None, T)
 refused(AttributeError, linear.rmsnorm_quantize_dev, T, None, 1e-5, 1, 64)
 refused(AttributeError, linear.linear_forward_dev, 8, T, None, 1, 32, d_acts=T)
 """)
+
+
+def test_linear_forward_multi_with_fewer_biases_than_matrices():
+    """A bias list that ends early leaves the matrices past it without one; the row count of a matrix past the end of the
+    row counts is 0 and the number of matrices is not cut short (both refused by the C ABI); an output is needed for
+    every weight."""
+    run(r"""
+V, P = C.c_void_p, C.POINTER(C.c_void_p)
+seen = []
+def record(t, n, w, acts, b, o, rows, cols):
+    k = min(n, 64)
+    seen.append((n, [b[i] for i in range(k)] if b else None, [rows[i] for i in range(k)]))
+    return 0
+f = C.CFUNCTYPE(C.c_int, C.c_uint32, C.c_size_t, P, V, P, P, C.POINTER(C.c_size_t), C.c_size_t)(record)
+address["oxq_linear_forward_multi_dev"] = C.cast(f, V).value
+_bind.attach(address)
+multi = linear.linear_forward_multi_dev
+b = torch.zeros(8)
+multi(8, [T, T, T], T, [T, T, T], [4, 5, 6], 32, [b])
+assert seen.pop() == (3, [b.data_ptr(), None, None], [4, 5, 6])
+multi(8, [T, T], T, [T, T], [4, 5], 32, [])
+assert seen.pop() == (2, [None, None], [4, 5])
+multi(8, (T, T), T, (t for t in (T, T)), (4,), 32)
+assert seen.pop() == (2, None, [4, 0])
+multi(8, [T] * 70, T, [T] * 70, [1] * 70, 32)
+assert seen.pop() == (70, None, [1] * 64)
+multi(8, [], T, [], [], 32)
+assert seen.pop()[0] == 0
+for args in (([T, T], T, [T], [1, 1], 32), ([T], T, [T, T], [1], 32), ([T], T, [T], [1, 1], 32), ([T], T, [T], [1], 32, [b, b])):
+    refused(ValueError, multi, 8, *args)
+assert not seen
+""")
