@@ -62,11 +62,29 @@ struct Args {
     template <class T> T *address(int i) { return v[i] == Py_None ? nullptr : (T *)(uintptr_t)number(v[i]); }
     size_t size(int i) { return (size_t)number(v[i]); }
     uint32_t u32(int i) { return (uint32_t)number(v[i]); }
-    float f32(int i) {
+    float real(PyObject *o) {
         if (!ok) return 0.0f;
-        const double d = PyFloat_AsDouble(v[i]);
+        const double d = PyFloat_AsDouble(o);
         if (d == -1.0 && PyErr_Occurred()) ok = false;
         return (float)d;
+    }
+    float f32(int i) { return real(v[i]); }
+    // Tensor types and eps are taken as int() and float() take them (a type as a number of any kind or as text).
+    uint32_t type(int i) {
+        if (!ok || PyLong_Check(v[i])) return u32(i);
+        PyObject *o = PyNumber_Long(v[i]);
+        if (!o) return ok = false, 0;
+        const uint64_t r = number(o);
+        Py_DECREF(o);
+        return (uint32_t)r;
+    }
+    float eps(int i) {
+        if (!ok || PyFloat_Check(v[i])) return f32(i);
+        PyObject *o = PyNumber_Float(v[i]);
+        if (!o) return ok = false, 0.0f;
+        const float r = real(o);
+        Py_DECREF(o);
+        return r;
     }
     size_t numel(int i) { return v[i] == Py_None ? 0 : (size_t)method(v[i], s_numel); }
     size_t bytes(int i) { return v[i] == Py_None ? 0 : numel(i) * (size_t)method(v[i], s_element_size); }
@@ -107,18 +125,18 @@ struct Args {
 
 OXQ_ENTRY(rmsnorm_quantize, 7,
           p_oxq_rmsnorm_quantize_q8_0_dev(x, w, eps, rows, cols, y, q8, stream),
-          auto x = a.tensor<float>(0); auto w = a.tensor<float>(1); float eps = a.f32(2); size_t rows = a.size(3), cols = a.size(4);
+          auto x = a.tensor<float>(0); auto w = a.tensor<float>(1); float eps = a.eps(2); size_t rows = a.size(3), cols = a.size(4);
           auto y = a.maybe<float>(5); auto q8 = a.maybe<uint8_t>(6);)
 
 OXQ_ENTRY(linear_forward, 9,
           p_oxq_linear_forward_dev(t, w, x, acts, bias, lora, out, of, in, stream),
-          uint32_t t = a.u32(0); auto w = a.tensor<uint8_t>(1); auto x = a.maybe<float>(2); auto acts = a.maybe<uint8_t>(3);
+          uint32_t t = a.type(0); auto w = a.tensor<uint8_t>(1); auto x = a.maybe<float>(2); auto acts = a.maybe<uint8_t>(3);
           auto bias = a.maybe<float>(4); auto lora = a.address<oxq_lora>(5); auto out = a.tensor<float>(6);
           size_t of = a.size(7), in = a.size(8);)
 
 OXQ_ENTRY(linear_forward_batch, 9,
           p_oxq_linear_forward_batch_dev(t, w, acts, bias, out, batch, of, in, ws, ws_n, stream),
-          uint32_t t = a.u32(0); auto w = a.tensor<uint8_t>(1); auto acts = a.tensor<uint8_t>(2); auto bias = a.maybe<float>(3);
+          uint32_t t = a.type(0); auto w = a.tensor<uint8_t>(1); auto acts = a.tensor<uint8_t>(2); auto bias = a.maybe<float>(3);
           auto out = a.tensor<float>(4); size_t batch = a.size(5), of = a.size(6), in = a.size(7);
           auto ws = a.maybe<void>(8); size_t ws_n = a.numel(8);)
 
@@ -144,8 +162,8 @@ OXQ_ENTRY(quantize_q8_0, 2,
 
 OXQ_ENTRY(ffn_swiglu, 11,
           p_oxq_ffn_swiglu_dev(tg, g, tu, u, td, d, acts, out, hidden, inter, ws, ws_n, stream),
-          uint32_t tg = a.u32(0); auto g = a.tensor<uint8_t>(1); uint32_t tu = a.u32(2); auto u = a.tensor<uint8_t>(3);
-          uint32_t td = a.u32(4); auto d = a.tensor<uint8_t>(5); auto acts = a.tensor<uint8_t>(6); auto out = a.tensor<float>(7);
+          uint32_t tg = a.type(0); auto g = a.tensor<uint8_t>(1); uint32_t tu = a.type(2); auto u = a.tensor<uint8_t>(3);
+          uint32_t td = a.type(4); auto d = a.tensor<uint8_t>(5); auto acts = a.tensor<uint8_t>(6); auto out = a.tensor<float>(7);
           size_t hidden = a.size(8), inter = a.size(9); auto ws = a.tensor<void>(10); size_t ws_n = a.numel(10);)
 
 OXQ_ENTRY(topk, 5,
@@ -175,8 +193,8 @@ OXQ_ENTRY(sample_candidates, 9,
 OXQ_ENTRY(moe_forward, 18,
           p_oxq_moe_forward_dev(tg, g, sg, tu, u, su, td, d, sd, n_exp, router, x, tokens, top_k, out, hidden, inter, ws, ws_n,
                                 stream),
-          uint32_t tg = a.u32(0); auto g = a.tensor<uint8_t>(1); size_t sg = a.size(2); uint32_t tu = a.u32(3);
-          auto u = a.tensor<uint8_t>(4); size_t su = a.size(5); uint32_t td = a.u32(6); auto d = a.tensor<uint8_t>(7);
+          uint32_t tg = a.type(0); auto g = a.tensor<uint8_t>(1); size_t sg = a.size(2); uint32_t tu = a.type(3);
+          auto u = a.tensor<uint8_t>(4); size_t su = a.size(5); uint32_t td = a.type(6); auto d = a.tensor<uint8_t>(7);
           size_t sd = a.size(8), n_exp = a.size(9); auto router = a.tensor<float>(10); auto x = a.tensor<float>(11);
           size_t tokens = a.size(12), top_k = a.size(13); auto out = a.tensor<float>(14); size_t hidden = a.size(15);
           size_t inter = a.size(16); auto ws = a.tensor<void>(17); size_t ws_n = a.numel(17);)
@@ -213,7 +231,7 @@ PyObject *linear_forward_multi(PyObject *, PyObject *const *v, Py_ssize_t n) {
         out[j] = a.tensor_of<float>(item(2, j));
         rows[j] = r ? (size_t)a.number(r) : 0;
     }
-    const uint32_t t = a.u32(0);
+    const uint32_t t = a.type(0);
     auto acts = a.tensor<uint8_t>(2);
     const size_t cols = a.size(6);
     void *const stream = a.stream();

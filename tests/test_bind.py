@@ -125,3 +125,31 @@ for args in (([T, T], T, [T], [1, 1], 32), ([T], T, [T, T], [1], 32), ([T], T, [
     refused(ValueError, multi, 8, *args)
 assert not seen
 """)
+
+
+def test_types_and_eps_convert_as_int_and_float_do():
+    run(r"""
+import numpy as np
+stub("oxq_linear_forward_dev", C.c_uint32)
+stub("oxq_linear_forward_batch_dev", C.c_uint32)
+stub("oxq_linear_forward_multi_dev", C.c_uint32)
+stub("oxq_ffn_swiglu_dev", C.c_uint32, C.c_void_p, C.c_uint32, C.c_void_p, C.c_uint32)
+f = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_void_p, C.c_float)(lambda x, w, e: calls.append(e) or 0)
+address["oxq_rmsnorm_quantize_q8_0_dev"] = C.cast(f, C.c_void_p).value
+_bind.attach(address)
+for t in (12, 12.0, "12", np.float32(12), np.int64(12), torch.tensor(12), quant.GgufTensorType.Q4K):
+    linear.linear_forward_dev(t, T, T, 1, 32, d_acts=T)
+    linear.linear_forward_batch_dev(t, T, T, T, 1, 1, 32)
+    linear.linear_forward_multi_dev(t, [T], T, [T], [1], 32)
+    assert [calls.pop() for _ in range(3)] == [(12,)] * 3, t
+    linear.ffn_swiglu_dev((t, T), (t, T), (t, T), T, T, 32, 32, T)
+    a = calls.pop()
+    assert (a[0], a[2], a[4]) == (12, 12, 12)
+for e in (0.5, 1, "0.5", np.float32(0.5), torch.tensor(0.5)):
+    linear.rmsnorm_quantize_dev(T, T, e, 1, 64, T)
+    assert calls.pop() == float(e), e
+for bad in (None, "q4", [1]):
+    refused((TypeError, ValueError), linear.linear_forward_dev, bad, T, T, 1, 32, d_acts=T)
+    refused((TypeError, ValueError), linear.rmsnorm_quantize_dev, T, T, bad, 1, 64, T)
+refused(TypeError, linear.linear_forward_dev, 8, T, T, 1.0, 32, d_acts=T)
+""")
