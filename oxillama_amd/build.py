@@ -6,6 +6,7 @@
   * oxillama_amd/liboxq_synth.so -- host-side synthetic weight generator
   * oxillama_amd/liboxq_benchkit.so -- copy / streaming-read kernels for measurement calibration
   * tests/cpp/test_quant_kernel.bin -- C++ mirror of the reference interface + its replayed unit tests
+  * tests/cpp/test_lds_opt_in.bin -- host test of the kernels' LDS limits
 hipcc cross-compiles gfx950 code objects without a GPU present.
 """
 import os
@@ -21,6 +22,7 @@ BIND_LIB = os.path.join(HERE, "_bind.so")
 SYNTH_LIB = os.path.join(HERE, "liboxq_synth.so")
 BENCHKIT_LIB = os.path.join(HERE, "liboxq_benchkit.so")
 CPP_TEST_BIN = os.path.join(os.path.dirname(HERE), "tests", "cpp", "test_quant_kernel.bin")
+LDS_TEST_BIN = os.path.join(os.path.dirname(HERE), "tests", "cpp", "test_lds_opt_in.bin")
 
 # -ffp-contract=off: the fp32 epilogues follow the reference's operation order (Rust
 # never fuses a*b+c).  Packed fp32 instructions are switched off.
@@ -67,12 +69,14 @@ def build_benchkit():
 
 def build_cpp_tests():
     """The C++ mirror of the reference interface (include/oxq/quant_kernel.hpp) and the
-    program that replays the reference's unit tests through it."""
+    program that replays the reference's unit tests through it; the host test of the LDS limits."""
     root = os.path.dirname(HERE)
     run(["g++", "-O1", "-std=c++17", "-Wall", "-I", os.path.join(root, "include"),
          os.path.join(root, "tests", "cpp", "test_quant_kernel.cpp"), "-o", CPP_TEST_BIN,
          "-L", HERE, "-loxq_hip", "-Wl,-rpath,$ORIGIN/../../oxillama_amd",
          "-Wl,-rpath-link,/opt/rocm/lib", "-Wl,--allow-shlib-undefined"])
+    run(["g++", "-O1", "-std=c++17", "-Wall", "-pthread", os.path.join(root, "tests", "cpp", "test_lds_opt_in.cpp"),
+         "-o", LDS_TEST_BIN])
     return CPP_TEST_BIN
 
 

@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "oxq_internal.hpp"
+#include "oxq_lds_opt_in.hpp"
 
 namespace oxq {
 hipError_t launch_dequant(uint32_t type, const uint8_t *blocks, size_t n_blocks, float *out, hipStream_t stream);
@@ -325,22 +326,16 @@ uint32_t device_cus() { return g.cus ? g.cus : 256; }
 int set_error(int status, size_t a, size_t b, const char *msg) { return fail(status, a, b, msg); }
 int ensure_device() { return ensure_init(); }
 
+static LdsOptIn g_lds;
+
 hipError_t allow_lds(const void *kern, size_t lds) {
     int device = 0;
     hipError_t e = hipGetDevice(&device);
     if (e != hipSuccess) return e;
-    // what this thread has opted in to, by (kernel, device); a slot that another pair took is simply asked for again
-    struct Entry {
-        const void *kern = nullptr;
-        int device = -1;
-        size_t lds = 0;
-    };
-    thread_local Entry table[256];
-    Entry &t = table[((reinterpret_cast<uintptr_t>(kern) >> 4) ^ (uintptr_t)device * 31) & 255];
-    if (t.kern == kern && t.device == device && t.lds >= lds) return hipSuccess;
-    e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    if (e == hipSuccess) t = Entry{kern, device, lds};
-    return e;
+    const int st = g_lds.raise(kern, device, lds, (int)hipErrorOutOfMemory, [&](size_t bytes) {
+        return (int)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    });
+    return (hipError_t)st;
 }
 }  // namespace oxq
 

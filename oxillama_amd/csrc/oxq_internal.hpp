@@ -74,8 +74,8 @@ extern std::atomic<size_t> g_phase_cap;
 // Number of compute units of the current device (cached per device).
 uint32_t device_cus();
 
-// Opt kernel `kern` in to `lds` bytes of dynamic LDS on the current device: a runtime call the first time a thread
-// asks, a table lookup afterwards (the runtime call costs about as much as a launch).
+// Opt kernel `kern` in to at least `lds` bytes of dynamic LDS on the current device: a runtime call when no thread of the
+// process has asked for as much yet, a table lookup otherwise (the runtime call costs about as much as a launch).
 hipError_t allow_lds(const void *kern, size_t lds);
 
 hipError_t launch_gemv_q8(uint32_t type, const GemvArgs &a, hipStream_t stream);

@@ -1,21 +1,27 @@
 """Runs tests/cpp/test_quant_kernel.bin: the reference crate's own unit tests replayed
-through the C++ mirror of its interface (include/oxq/quant_kernel.hpp -> C ABI)."""
+through the C++ mirror of its interface (include/oxq/quant_kernel.hpp -> C ABI), and
+tests/cpp/test_lds_opt_in.bin: the kernels' LDS limits asked for by several threads."""
 import os
 import subprocess
 
 import pytest
 
-BIN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp", "test_quant_kernel.bin")
+CPP = os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpp")
+BIN = os.path.join(CPP, "test_quant_kernel.bin")
 
 
-def _run(mode):
-    if not os.path.exists(BIN):
-        pytest.fail(f"{BIN} is not built: run `python -m oxillama_amd.build`")
-    p = subprocess.run([BIN, mode], capture_output=True, text=True, timeout=120)
+def _run(*args, binary=BIN):
+    if not os.path.exists(binary):
+        pytest.fail(f"{binary} is not built: run `python -m oxillama_amd.build`")
+    p = subprocess.run([binary, *args], capture_output=True, text=True, timeout=120)
     print(p.stdout)
     print(p.stderr)
     assert p.returncode == 0, p.stdout[-4000:]
-    assert " 0 failed" in p.stdout
+    assert "0 failed" in p.stdout.split("\n")[-2]
+
+
+def test_lds_limits_are_only_raised():
+    _run(binary=os.path.join(CPP, "test_lds_opt_in.bin"))
 
 
 def test_cpp_mirror_host_cases():
