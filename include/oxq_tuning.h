@@ -47,6 +47,9 @@ int oxq_set_gemv_phase_probe(void *d_buffer, size_t bytes);
  * launch used, as "name<type,p0,p1,p2,p3> grid XxY block B" (template parameters in the kernel's own order):
  * lets a measurement name what it timed and notice when a launch policy has changed under it. */
 int oxq_last_launch(char *out, size_t out_len);
+/* The allocation flags of the host-slice calls' staging memory as the runtime reports them: input, output, completion
+ * word (0: not allocated yet). */
+int oxq_host_staging_flags(unsigned *flags, size_t n);
 /* oxq_ffn_swiglu_dev: 1 (default) = gate, up, SwiGLU and the quantizer of h in one launch where a kernel
  * exists for the type and row length; 0 = the separate launches (same bits). */
 int oxq_set_ffn_fusion(int enabled);

@@ -77,15 +77,18 @@ struct Scratch {
     }
 };
 
-// A growable host buffer that the GPU reads and writes in place.
+// A growable host buffer that the GPU reads and writes in place.  Coherent by request: host and GPU hand it to and fro
+// without a runtime call between them (the host watches a word that a running kernel writes, and rewrites the input of
+// the last call), which the default allocation allows only as HIP_HOST_COHERENT is set.
 struct Pinned {
+    static constexpr unsigned FLAGS = hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent;
     void *ptr = nullptr;
     size_t cap = 0;
     int reserve(size_t n) {
         if (n <= cap) return OXQ_OK;
         release();
         const size_t want = n + n / 4 + 256;
-        hipError_t e = hipHostMalloc(&ptr, want, hipHostMallocPortable);
+        hipError_t e = hipHostMalloc(&ptr, want, FLAGS);
         if (e != hipSuccess) {
             ptr = nullptr;
             return fail_hip(e, "hipHostMalloc(staging)");
@@ -521,6 +524,17 @@ int oxq_set_gemv_rows_per_batch(unsigned rows) {
 
 int oxq_set_gemv_waves_per_row(unsigned waves) {
     g.waves_per_row = waves >= 4 ? 4 : (waves ? 1 : 0);
+    return OXQ_OK;
+}
+
+int oxq_host_staging_flags(unsigned *flags, size_t n) {
+    if (!flags) return fail(OXQ_ERR_INTERNAL, 0, 0, "null output");
+    std::lock_guard<std::mutex> lock(g.mu);
+    const Pinned *const buf[] = {&g.h_in, &g.h_out, &g.h_flag};
+    for (size_t i = 0; i < n; i++) {
+        flags[i] = 0;
+        if (i < 3 && buf[i]->ptr) OXQ_HIP(hipHostGetFlags(&flags[i], buf[i]->ptr));
+    }
     return OXQ_OK;
 }
 
