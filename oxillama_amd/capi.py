@@ -225,21 +225,21 @@ def load():
         fn = getattr(lib, name)  # AttributeError if the ABI lost a symbol
         fn.restype = restype
         fn.argtypes = argtypes
-    try:
-        from . import _bind
-    except ImportError as e:
-        raise RuntimeError("oxillama_amd/_bind.so is missing or of another Python: build it with `python -m oxillama_amd.build`") from e
-    _bind.attach({name: C.cast(getattr(lib, name), C.c_void_p).value for name in SIGNATURES})
     _lib = lib
     return lib
 
 
 def bind():
-    """The extension module behind the device entry points, attached to the library."""
+    """The extension module behind the device entry points, attached to the library.  Raises if it is not built; the
+    host-slice calls do without it."""
     global _attached
     if _attached is None:
-        load()
-        from . import _bind
+        lib = load()
+        try:
+            from . import _bind
+        except ImportError as e:
+            raise RuntimeError("oxillama_amd/_bind.so is missing or of another Python: build it with `python -m oxillama_amd.build`") from e
+        _bind.attach({name: C.cast(getattr(lib, name), C.c_void_p).value for name in SIGNATURES})
         _attached = _bind
     return _attached
 

@@ -153,3 +153,18 @@ for bad in (None, "q4", [1]):
     refused((TypeError, ValueError), linear.rmsnorm_quantize_dev, T, T, bad, 1, 64, T)
 refused(TypeError, linear.linear_forward_dev, 8, T, T, 1.0, 32, d_acts=T)
 """)
+
+
+def test_the_library_loads_without_the_extension():
+    """Host-slice calls and the ABI need ctypes alone; the device entry points say what is missing."""
+    run(r"""
+import sys
+capi._attached = None
+sys.modules["oxillama_amd._bind"] = None  # importing it raises ImportError
+import oxillama_amd
+del oxillama_amd._bind
+assert capi.load().oxq_block_size(8) == 32
+assert quant.KernelDispatcher().get_kernel(8).block_bytes() == 34
+refused(RuntimeError, quant.quantize_q8_0_dev, T, T)
+refused(RuntimeError, capi.bind)
+""")
