@@ -15,6 +15,17 @@ import numpy as np
 from . import capi
 from .quant import DimensionMismatch, HipKernel, QuantTensor, _check, _ptr, _u8, raw_stream as _stream
 
+_U8, _F32 = np.dtype(np.uint8), np.dtype(np.float32)
+
+
+def _plain(a, dtype):
+    """An array whose memory can be handed over as it is."""
+    return type(a) is np.ndarray and a.dtype == dtype and a.ndim == 1 and a.flags.c_contiguous
+
+
+def _f32(a):
+    return a if _plain(a, _F32) else np.ascontiguousarray(a, dtype=np.float32).ravel()
+
 
 class LoraAdapter:
     """delta = B @ (A @ input) * scale; A is [rank x in_features], B is [out_features x rank]."""
@@ -39,19 +50,22 @@ class QuantLinear:
         self.out_features = weight.shape[0] if len(weight.shape) > 0 else 0  # linear.rs:38-48
         self.in_features = weight.shape[1] if len(weight.shape) > 1 else 0
         self.lora = None
-        self._args = None
+        self._shape = self._view = None
 
     def _weight_args(self):
-        """(address, bytes, shape, dimensions, owner of the address) of the weight for the C ABI.  Kept from call to call
-        while the tensor holds the same array and shape: forming them takes as long as the library's part of a call."""
-        data, shape = self.weight.data, tuple(self.weight.shape)
-        if self._args is None or self._args[4] is not data or self._args[2][:] != list(shape):
-            w = _u8(data)
-            args = (_ptr(w), w.size, (C.c_size_t * len(shape))(*shape), len(shape), data if isinstance(data, np.ndarray) else w)
-            if not (isinstance(data, np.ndarray) and data.flags.c_contiguous):
-                return args[:4] + (w,)  # a copy of the bytes: made again on every call, as they may change
-            self._args = args
-        return self._args
+        """(address, bytes, shape, dimensions, array behind the address) of the weight for the C ABI, from the tensor as it
+        is now.  Kept from call to call: the ctypes form of a shape, by its values, and the address of an array that is a
+        view (QuantTensor makes one), which stays where it is; an array with memory of its own may move on resize()."""
+        w, shape = self.weight.data, tuple(self.weight.shape)
+        if not _plain(w, _U8):
+            w = _u8(w)
+        if self._shape is None or self._shape[0] != shape:
+            self._shape = (shape, (C.c_size_t * len(shape))(*shape))
+        view = self._view
+        if view is None or view[0] is not w:
+            view = (w, _ptr(w))
+            self._view = None if w.flags.owndata or w is not self.weight.data else view
+        return view[1], w.size, self._shape[1], len(shape), w
 
     def set_lora(self, lora):
         self.lora = lora
@@ -62,23 +76,23 @@ class QuantLinear:
     def forward(self, kernel: HipKernel, input, output):
         """output = weight @ input + bias [+ lora delta] (linear.rs:77-98); output is filled in place."""
         lib = capi.load()
-        x = np.ascontiguousarray(input, dtype=np.float32).ravel()
+        x = _f32(input)
         bias_p, bias_n = (_ptr(self.bias), self.bias.size) if self.bias is not None else (None, 0)
         if self.lora is not None:
             la, lb = self.lora.a, self.lora.b
             lora_args = (_ptr(la), la.size, _ptr(lb), lb.size, self.lora.rank, self.lora.scale)
         else:
             lora_args = (None, 0, None, 0, 0, 0.0)
-        w_p, w_n, shape, n_dims, _owner = self._weight_args()
+        w_p, w_n, shape, n_dims, _array = self._weight_args()
         _check(lib.oxq_linear_forward(kernel.tensor_type, w_p, w_n, shape, n_dims, bias_p, bias_n, *lora_args, _ptr(x), x.size,
                                       _ptr(output), output.size))
 
     def forward_batch(self, kernel: HipKernel, input, output, batch_size):
         """output[batch x out] = gemm + bias broadcast (linear.rs:105-132; no LoRA in batch mode)."""
         lib = capi.load()
-        x = np.ascontiguousarray(input, dtype=np.float32).ravel()
+        x = _f32(input)
         bias_p, bias_n = (_ptr(self.bias), self.bias.size) if self.bias is not None else (None, 0)
-        w_p, w_n, shape, n_dims, _owner = self._weight_args()
+        w_p, w_n, shape, n_dims, _array = self._weight_args()
         _check(lib.oxq_linear_forward_batch(kernel.tensor_type, w_p, w_n, shape, n_dims, bias_p, bias_n, _ptr(x), x.size,
                                             _ptr(output), output.size, batch_size))
 

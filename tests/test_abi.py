@@ -206,3 +206,53 @@ def test_gemm_workspace_size_is_a_function_of_the_shape():
     assert w(q8_0, 64, 4864, 224) == 0                                                 # fewer than eight blocks
     assert w(q8_0, 64, 4864, 300) == 0                                                 # ends inside a block
     assert w(q6k, 64, 4864, 288) == 0
+
+
+def test_quant_linear_hands_over_the_weight_as_it_is_at_the_call(monkeypatch):
+    """The address, length and shape that a call passes are the weight's of that moment: its array resized or replaced,
+    its bytes in another array type, its shape changed."""
+    from oxillama_amd import linear
+    seen = []
+
+    class Lib:
+        @staticmethod
+        def oxq_linear_forward(t, w, w_n, shape, n_dims, *rest):
+            seen.append((w, w_n, list(shape), n_dims))
+            return capi.OK
+
+        @staticmethod
+        def oxq_linear_forward_batch(*a):
+            return Lib.oxq_linear_forward(*a)
+
+    kern = quant.HipKernel(8)
+    lin = linear.QuantLinear(quant.QuantTensor(np.zeros(2 * 34, np.uint8), [2, 32], 8))
+    monkeypatch.setattr(linear.capi, "load", lambda: Lib)
+    x, y = np.zeros(32, np.float32), np.zeros(2, np.float32)
+
+    def call():
+        lin.forward(kern, x, y)
+        lin.forward_batch(kern, x, y, 1)
+        assert seen[-1] == seen[-2]
+        return seen.pop()
+
+    assert call() == (lin.weight.data.ctypes.data, 68, [2, 32], 2)
+    lin.weight.data = np.zeros(68, np.uint8)
+    assert call() == (lin.weight.data.ctypes.data, 68, [2, 32], 2)
+    lin.weight.data.resize(1 << 24, refcheck=False)  # in place: the same array at another address
+    assert call() == (lin.weight.data.ctypes.data, 1 << 24, [2, 32], 2)
+    lin.weight.data.resize(34, refcheck=False)
+    lin.weight.shape[0] = 1
+    assert call() == (lin.weight.data.ctypes.data, 34, [1, 32], 2)
+    lin.weight.data = np.frombuffer(bytes(3 * 34), dtype=np.uint8)  # read-only
+    lin.weight.shape = (3, 32)
+    assert call() == (lin.weight.data.ctypes.data, 102, [3, 32], 2)
+    whole = np.zeros(204, np.uint8)
+    lin.weight.data = whole[:102]  # a view ...
+    for _ in range(3):
+        assert call() == (whole.ctypes.data, 102, [3, 32], 2)
+    lin.weight.data = whole[102:]  # ... and another
+    assert call() == (whole.ctypes.data + 102, 102, [3, 32], 2)
+    lin.weight.data = np.zeros((3, 17), np.uint16)
+    assert call() == (lin.weight.data.ctypes.data, 102, [3, 32], 2)
+    lin.weight.data = bytes(102)  # a copy of the bytes
+    assert call()[1:] == (102, [3, 32], 2)
