@@ -308,14 +308,12 @@ __global__ __launch_bounds__(64 * RW * KS) __attribute__((amdgpu_waves_per_eu(2,
             sum += xor1_i(sum);
             // P = d * sum: at most 23 significant bits; three truncated bf16 pieces hold it exactly
             const float P = d * (float)sum;
-            const uint32_t p1 = __builtin_bit_cast(uint32_t, P) & 0xFFFF0000u;
-            const float r1 = P - __builtin_bit_cast(float, p1);
-            const uint32_t p2 = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
-            const float r2 = r1 - __builtin_bit_cast(float, p2);
+            uint16_t piece[3];
+            bf16_pieces(P, piece);
             uint8_t *at = pl[par] + tl * 16 + 2 * (2 * (g & 3) + pe);
-            *reinterpret_cast<lds_u16 *>(at) = (uint16_t)(p1 >> 16);
-            *reinterpret_cast<lds_u16 *>(at + TOK * 16) = (uint16_t)(p2 >> 16);
-            *reinterpret_cast<lds_u16 *>(at + 2 * TOK * 16) = (uint16_t)(__builtin_bit_cast(uint32_t, r2) >> 16);
+            *reinterpret_cast<lds_u16 *>(at) = piece[0];
+            *reinterpret_cast<lds_u16 *>(at + TOK * 16) = piece[1];
+            *reinterpret_cast<lds_u16 *>(at + 2 * TOK * 16) = piece[2];
         }
     };
     // End of a stage: this wave's LDS traffic is done, then everybody's; loads to registers stay in flight.  It makes the

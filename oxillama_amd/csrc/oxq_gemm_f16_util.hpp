@@ -33,6 +33,19 @@ __device__ __forceinline__ b8 lds_b8(const uint8_t *p) { return __builtin_bit_ca
 // unpack takes bytes 0 and 2 of a dword together (they sit in the two 16-bit halves), then bytes 1 and 3.
 __device__ __forceinline__ constexpr int pf_slot_byte(int j) { return (j & 4) | ((j & 1) << 1) | ((j >> 1) & 1); }
 
+// The bits of three truncated bf16 pieces whose sum is x, exact for up to 23 significant bits.  A piece that is x itself
+// leaves no rest: of an infinity, x - x would be a NaN.
+__device__ __forceinline__ void bf16_pieces(float x, uint16_t (&piece)[3]) {
+    const uint32_t p1 = __builtin_bit_cast(uint32_t, x) & 0xFFFF0000u;
+    const float f1 = __builtin_bit_cast(float, p1);
+    const float r1 = x == f1 ? 0.0f : x - f1;  // exact
+    const uint32_t p2 = __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u;
+    const float r2 = r1 - __builtin_bit_cast(float, p2);  // exact, at most 8 significant bits
+    piece[0] = (uint16_t)(p1 >> 16);
+    piece[1] = (uint16_t)(p2 >> 16);
+    piece[2] = (uint16_t)(__builtin_bit_cast(uint32_t, r2) >> 16);
+}
+
 __device__ __forceinline__ uint32_t f16x2_of(float v) {
     const uint32_t b = f2h(v);
     return b | (b << 16);

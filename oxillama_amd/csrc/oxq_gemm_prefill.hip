@@ -91,15 +91,12 @@ __global__ __launch_bounds__(256) void prefill_prep_acts(const uint8_t *__restri
     dag[((size_t)(j >> 1) * mpad + t) * 2 + (j & 1)] = (uint16_t)dbits;
     // P = da * sum(q): at most 23 significant bits; three truncated bf16 pieces hold it exactly
     const float P = h2f(dbits) * (float)s;
-    const uint32_t pb = __builtin_bit_cast(uint32_t, P);
-    const float p1 = __builtin_bit_cast(float, pb & 0xFFFF0000u);
-    const float r1 = P - p1;  // exact
-    const float p2 = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, r1) & 0xFFFF0000u);
-    const float r2 = r1 - p2;  // exact, at most 8 significant bits
+    uint16_t piece[3];
+    bf16_pieces(P, piece);
     const size_t pbase = (size_t)(j >> 3) * 4 * mpad;
-    pbf[((pbase + 0 * (size_t)mpad + t) * 8) + (j & 7)] = (uint16_t)(pb >> 16);
-    pbf[((pbase + 1 * (size_t)mpad + t) * 8) + (j & 7)] = (uint16_t)(__builtin_bit_cast(uint32_t, p2) >> 16);
-    pbf[((pbase + 2 * (size_t)mpad + t) * 8) + (j & 7)] = (uint16_t)(__builtin_bit_cast(uint32_t, r2) >> 16);
+    pbf[((pbase + 0 * (size_t)mpad + t) * 8) + (j & 7)] = piece[0];
+    pbf[((pbase + 1 * (size_t)mpad + t) * 8) + (j & 7)] = piece[1];
+    pbf[((pbase + 2 * (size_t)mpad + t) * 8) + (j & 7)] = piece[2];
     pbf[((pbase + 3 * (size_t)mpad + t) * 8) + (j & 7)] = 0;
 }
 

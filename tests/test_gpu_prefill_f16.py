@@ -149,6 +149,43 @@ def test_f16_kernel_on_raw_rows(hip, ref, tuning, variant, t, shape):
     assert torch.equal(dy2[:m], dy[:m] + dy[:m])
 
 
+@pytest.mark.parametrize("t,variant", [(O.Q4_K, 300), (O.Q4_K, 301), (O.Q4_K, 302), (O.Q5_K, 301), (O.Q5_K, 302),
+                                       (O.Q6_K, 301), (O.Q6_K, 302)])
+def test_f16_kernels_on_infinite_block_scales(hip, ref, tuning, t, variant):
+    """Activations beyond the range of a block's f16 scale (the quantizer's scale is an infinity there): infinities of the
+    same sign and NaNs where the int8 tile kernel has them, and every other token as without them.  (Q6_K: no number; the
+    tile kernel adds the two halves of a sub-block as infinities, this one before the scale, the oracle has NaNs.)"""
+    m, n, k = 70, 160, 768
+    w = O.random_blocks(t, 71, n, k)
+    acts = ref.quantize_q8_0(synth.normal_f32(72, m * k)).reshape(m, k // 32, 34)
+    clean = acts.copy()
+    acts[3, 5, :2] = [0x00, 0x7C]   # +inf in one block of token 3
+    acts[66, :, :2] = [0x00, 0x7C]  # in all of token 66
+    acts[40, 23, :2] = [0x00, 0x7E]  # a NaN
+    kern = hip.HipKernel(t)
+    ws = torch.empty(kern.gemm_workspace_bytes(m, n, k), dtype=torch.uint8, device="cuda")
+    dw = torch.from_numpy(w).cuda()
+    tuning("gemm_tile_min_rows", 1)
+
+    def product(a, v):
+        tuning("gemm_variant", v)
+        dy = torch.empty((m, n), dtype=torch.float32, device="cuda")
+        kern.gemm_q8_dev(dw, torch.from_numpy(a.reshape(-1)).cuda(), dy, m, n, k, accumulate=False, workspace=ws)
+        torch.cuda.synchronize()
+        return dy.cpu().numpy()
+
+    y, y_tile, y_clean = product(acts, variant), product(acts, 99), product(clean, variant)
+    assert np.isinf(y_tile[3]).any() and np.isnan(y_tile[40]).all()
+    for r in (3, 66, 40):
+        if t == O.Q6_K:
+            assert not np.isfinite(y[r]).any()
+            continue
+        assert np.array_equal(np.isnan(y[r]), np.isnan(y_tile[r])), r
+        assert np.array_equal(np.sign(y[r][np.isinf(y[r])]), np.sign(y_tile[r][np.isinf(y_tile[r])])), r
+    rest = [r for r in range(m) if r not in (3, 66, 40)]
+    assert np.array_equal(y[rest], y_clean[rest])
+
+
 def test_scaled_sums_errors(hip):
     kern = hip.HipKernel(O.Q6_K)
     z = torch.zeros(1 << 16, dtype=torch.uint8, device="cuda")
