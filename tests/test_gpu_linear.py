@@ -114,6 +114,32 @@ def test_rmsnorm_quantize(hip, ref):
         assert np.array_equal(host(d_q2), q)
 
 
+@pytest.mark.parametrize("n", [1024, 1056, 2080, 4128, 8224, 16384, 16416])
+@pytest.mark.parametrize("many", [False, True], ids=["few rows", "many rows"])
+def test_rmsnorm_quantize_every_row_length_class(hip, ref, many, n):
+    """Every arm of the launch's choice: 1, 2, 4, 8, 16 chunks a thread of 256 or 1024 threads (more rows than two per
+    compute unit: 256), the two-pass kernel behind them, lengths that leave the last chunk part empty, in place too.
+    Against float64: a sum of squares is a chain of at most 64 fp32 additions a thread and 8 levels above it, halved by
+    the root, with four roundings behind it: (72 / 2 + 4) 2^-24 = 2.4e-6 of the value."""
+    rows = 2 * hip.device_info()["compute_units"] + 8 if many else 3
+    say("rmsnorm", rows, "x", n)
+    x = synth.normal_f32(n, rows * n, 2.0).reshape(rows, n)
+    w = (1.0 + 0.1 * synth.normal_f32(n + 1, n, 1.0)).astype(np.float32)
+    d_x, d_w = dev(x), dev(w)
+    d_y = torch.full((rows + 1, n), 7.0, dtype=torch.float32, device=DEV)
+    d_q = torch.full((rows * n // 32 * 34 + 34,), 9, dtype=torch.uint8, device=DEV)
+    L.rmsnorm_quantize_dev(d_x, d_w, 1e-5, rows, n, d_y, d_q)
+    y, q = host(d_y), host(d_q)
+    assert np.all(y[rows] == 7.0) and np.all(q[-34:] == 9)
+    x64 = x.astype(np.float64)
+    want = x64 / np.sqrt((x64 * x64).mean(1, keepdims=True) + np.float64(np.float32(1e-5))) * w
+    assert np.all(np.abs(y[:rows] - want) <= 2.4e-6 * np.abs(want) + 1e-30)
+    pick = sorted({0, 1, rows // 2, rows - 2, rows - 1})
+    assert np.array_equal(q[:-34].reshape(rows, -1)[pick].ravel(), ref.quantize_q8_0(y[pick].ravel()))
+    L.rmsnorm_quantize_dev(d_x, d_w, 1e-5, rows, n, d_x, None)  # in place
+    assert np.array_equal(host(d_x), y[:rows])
+
+
 def test_rmsnorm_reference_values(hip):
     # crates/oxillama-arch/src/common/rms_norm.rs:72-88, padded with zeros to 32 (same sum of squares,
     # mean over 32 instead of 4)

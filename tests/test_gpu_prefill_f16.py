@@ -13,7 +13,7 @@ import pytest
 import torch
 
 import oracle as O
-from oxillama_amd import capi, synth
+from oxillama_amd import capi, linear, synth
 
 pytestmark = pytest.mark.gpu
 FP32_REL_TOL = 1e-5
@@ -147,6 +147,116 @@ def test_f16_kernel_on_raw_rows(hip, ref, tuning, variant, t, shape):
     kern.gemm_q8_dev(dw, da, dy2, m, n, k, accumulate=True, workspace=ws)
     torch.cuda.synchronize()
     assert torch.equal(dy2[:m], dy[:m] + dy[:m])
+
+
+@pytest.mark.parametrize("k", [256, 512, 768])
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q5_K, O.Q6_K], ids=lambda t: O.NAMES[t])
+@pytest.mark.parametrize("variant", [301, 302])
+def test_f16_kernel_is_exact_in_whole_numbers(hip, ref, tuning, variant, t, k):
+    """Weights that are whole numbers (d = dmin = 1, every scale and quant value of the format, the largest among them)
+    against tokens with one sub-block of whole numbers over 8: a result is at most 2^24 eighths, so that every step of the
+    kernel is exact if its operands are (Q6_K's two pieces, P's three), and == is the bar.  k = 256: the small shape's
+    second half of k has nothing to do."""
+    m, n = 37, 96
+    say("f16 exact", variant, O.NAMES[t], k)
+    tuning("gemm_variant", variant)
+    tuning("gemm_tile_min_rows", 1)
+    bb = O.BLOCK[t][1]
+    w = O.random_blocks(t, 81, n, k).reshape(n, k // 256, bb)
+    for off in O.F16_FIELDS[t]:
+        w[:, :, off:off + 2] = [0x00, 0x3C]  # 1.0
+    if t == O.Q6_K:  # rows of scale -128 and -127 against the lowest and the highest quant value
+        w[0, :, :192], w[0, :, 192:208] = 0, 0x80
+        w[1, :, :192], w[1, :, 192:208] = 0, 0x81
+        w[2, :, :192], w[2, :, 192:208] = 0xFF, 0x80
+    else:  # the largest of everything
+        w[0, :, 4:] = 0xFF
+    rng = np.random.default_rng(82)
+    a = np.zeros((m, k // 32, 32), np.int64)
+    for r in range(m):
+        v = rng.integers(-127, 128, 32)
+        if r < 6:
+            v[:] = (-128, 127)[r % 2]
+        a[r, (5 * r) % (k // 32)] = v
+    acts = np.zeros((m, k // 32, 34), np.uint8)
+    acts[:, :, :2] = [0x00, 0x30]  # 1 / 8
+    acts[:, :, 2:] = a.astype(np.int8).view(np.uint8)
+    want = a.reshape(m, k) @ ref.dequant_rows(t, w.reshape(-1), n, k).reshape(n, k).astype(np.int64).T
+    assert np.abs(want).max() <= 1 << 24
+    kern = hip.HipKernel(t)
+    ws = torch.empty(kern.gemm_workspace_bytes(m, n, k), dtype=torch.uint8, device="cuda")
+    dy = torch.empty((m, n), dtype=torch.float32, device="cuda")
+    kern.gemm_q8_dev(torch.from_numpy(w.reshape(-1)).cuda(), torch.from_numpy(acts.reshape(-1)).cuda(), dy, m, n, k,
+                     accumulate=False, workspace=ws)
+    torch.cuda.synchronize()
+    assert last_launch().startswith("gemm_f16_kernel"), last_launch()
+    assert np.array_equal(dy.cpu().numpy().astype(np.float64) * 8, want)
+
+
+@pytest.mark.parametrize("n", [160, 161])
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q6_K], ids=lambda t: O.NAMES[t])
+@pytest.mark.parametrize("variant", [301, 302])
+def test_f16_kernel_adds_the_bias(hip, ref, tuning, variant, t, n):
+    """The bias is one fp32 addition behind the sum: bit for bit result + bias, in the stores of four rows and of one (rows
+    not a multiple of four, an output or a bias off the 16-byte grid)."""
+    m, k = 70, 512
+    say("f16 bias", variant, O.NAMES[t], n)
+    tuning("gemm_variant", variant)
+    tuning("gemm_tile_min_rows", 1)
+    kern = hip.HipKernel(t)
+    dw = torch.from_numpy(O.random_blocks(t, 91, n, k)).cuda()
+    da = torch.from_numpy(ref.quantize_q8_0(synth.normal_f32(92, m * k))).cuda()
+    bias = torch.from_numpy(synth.normal_f32(93, n + 1)).cuda()
+    ws = torch.empty(kern.gemm_workspace_bytes(m, n, k), dtype=torch.uint8, device="cuda")
+    y = torch.empty((m, n), dtype=torch.float32, device="cuda")
+    linear.linear_forward_batch_dev(t, dw, da, y, m, n, k, workspace=ws)
+    assert last_launch().startswith("gemm_f16_kernel"), last_launch()
+    for o_off, b_off in ((0, 0), (1, 0), (0, 1)):
+        buf = torch.full((m * n + 2,), 7.0, dtype=torch.float32, device="cuda")
+        out, b = buf[o_off:o_off + m * n], bias[b_off:b_off + n]
+        linear.linear_forward_batch_dev(t, dw, da, out, m, n, k, d_bias=b, workspace=ws)
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(m, n), y + b)
+        assert (buf[:o_off] == 7.0).all() and (buf[o_off + m * n:] == 7.0).all()
+
+
+LARGE, SMALL = "4,8,1", "2,4,2"
+
+
+@pytest.mark.parametrize("t,m,n,k,shape", [
+    (O.Q6_K, 128, 256 * 164, 1024, LARGE),  # 164 of 256 large tiles in one round
+    (O.Q6_K, 128, 256 * 163, 1024, None),
+    (O.Q6_K, 128, 256 * 164, 768, None),    # (short rows)
+    (O.Q6_K, 128, 128 * 103, 1024, SMALL),  # 206 small tiles
+    (O.Q6_K, 128, 128 * 102, 1024, None),
+    (O.Q6_K, 80, 128 * 103, 1024, None),    # (token tiles a quarter empty and more)
+    (O.Q5_K, 128, 256 * 246, 1024, LARGE),
+    (O.Q5_K, 128, 256 * 245, 1024, None),
+    (O.Q5_K, 448, 128 * 36, 1024, SMALL),
+    (O.Q5_K, 448, 128 * 35, 1024, None),
+    (O.Q4_K, 448, 128 * 36, 1024, SMALL),
+    (O.Q4_K, 384, 128 * 42, 1024, None),
+])
+def test_f16_kernel_by_default(hip, ref, t, m, n, k, shape):
+    """Which calls take the f16 kernel on raw rows, and in which shape, on both sides of the lines; results of a few tokens
+    against the oracle."""
+    if hip.device_info()["compute_units"] != 256:
+        pytest.skip("the tile counts are of 256 compute units")
+    say("f16 default", O.NAMES[t], m, n, k)
+    w = O.random_blocks(t, 95, n, k)
+    acts = ref.quantize_q8_0(synth.normal_f32(96, m * k))
+    kern = hip.HipKernel(t)
+    ws = torch.empty(kern.gemm_workspace_bytes(m, n, k), dtype=torch.uint8, device="cuda")
+    dy = torch.empty((m, n), dtype=torch.float32, device="cuda")
+    kern.gemm_q8_dev(torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda(), dy, m, n, k, accumulate=False, workspace=ws)
+    torch.cuda.synchronize()
+    if shape:
+        assert last_launch().startswith(f"gemm_f16_kernel<{O.NAMES[t]},{shape}"), last_launch()
+    else:
+        assert not last_launch().startswith("gemm_f16_kernel"), last_launch()
+    rows = [0, 63, 64, m - 1]
+    y_ref = oracle_rows(ref, t, w, acts, n, k, rows)
+    assert np.abs(dy.cpu().numpy()[rows] - y_ref).max() <= FP32_REL_TOL * np.abs(y_ref).max()
 
 
 @pytest.mark.parametrize("t,variant", [(O.Q4_K, 300), (O.Q4_K, 301), (O.Q4_K, 302), (O.Q5_K, 301), (O.Q5_K, 302),
