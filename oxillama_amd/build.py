@@ -6,7 +6,7 @@
   * oxillama_amd/liboxq_synth.so -- host-side synthetic weight generator
   * oxillama_amd/liboxq_benchkit.so -- copy / streaming-read kernels for measurement calibration
   * tests/cpp/test_quant_kernel.bin -- C++ mirror of the reference interface + its replayed unit tests
-  * tests/cpp/test_lds_opt_in.bin -- host test of the kernels' LDS limits
+  * tests/cpp/test_lds_opt_in.bin, test_tile_order.bin -- host tests of the kernels' LDS limits and of their tile order
 hipcc cross-compiles gfx950 code objects without a GPU present.
 """
 import os
@@ -22,7 +22,7 @@ BIND_LIB = os.path.join(HERE, "_bind.so")
 SYNTH_LIB = os.path.join(HERE, "liboxq_synth.so")
 BENCHKIT_LIB = os.path.join(HERE, "liboxq_benchkit.so")
 CPP_TEST_BIN = os.path.join(os.path.dirname(HERE), "tests", "cpp", "test_quant_kernel.bin")
-LDS_TEST_BIN = os.path.join(os.path.dirname(HERE), "tests", "cpp", "test_lds_opt_in.bin")
+HOST_TESTS = [os.path.join(os.path.dirname(HERE), "tests", "cpp", name) for name in ("test_lds_opt_in", "test_tile_order")]
 
 # -ffp-contract=off: the fp32 epilogues follow the reference's operation order (Rust
 # never fuses a*b+c).  Packed fp32 instructions are switched off.
@@ -69,14 +69,14 @@ def build_benchkit():
 
 def build_cpp_tests():
     """The C++ mirror of the reference interface (include/oxq/quant_kernel.hpp) and the
-    program that replays the reference's unit tests through it; the host test of the LDS limits."""
+    program that replays the reference's unit tests through it; the host tests."""
     root = os.path.dirname(HERE)
     run(["g++", "-O1", "-std=c++17", "-Wall", "-I", os.path.join(root, "include"),
          os.path.join(root, "tests", "cpp", "test_quant_kernel.cpp"), "-o", CPP_TEST_BIN,
          "-L", HERE, "-loxq_hip", "-Wl,-rpath,$ORIGIN/../../oxillama_amd",
          "-Wl,-rpath-link,/opt/rocm/lib", "-Wl,--allow-shlib-undefined"])
-    run(["g++", "-O1", "-std=c++17", "-Wall", "-pthread", os.path.join(root, "tests", "cpp", "test_lds_opt_in.cpp"),
-         "-o", LDS_TEST_BIN])
+    for test in HOST_TESTS:
+        run(["g++", "-O1", "-std=c++17", "-Wall", "-pthread", test + ".cpp", "-o", test + ".bin"])
     return CPP_TEST_BIN
 
 

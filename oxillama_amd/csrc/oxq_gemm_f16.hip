@@ -28,6 +28,7 @@
 // 8192 542 / 656, 512 x 14336 x 4096 130 / 166, 512 x 4096 x 14336 175 / 207; Q4_K 512 x 4096 x 4096 42 / 48.5, 2048 x 1024 x 4096
 // 42 / 51; Q5_K 2048 x 4096 x 14336 388 / 454, 512 x 4096 x 4096 48 / 54.
 #include "oxq_gemm_f16_util.hpp"
+#include "oxq_tile_order.hpp"
 
 namespace oxq {
 namespace {
@@ -251,11 +252,8 @@ __global__ __launch_bounds__(64 * RW * KS) __attribute__((amdgpu_waves_per_eu(2,
     const uint32_t per_part = (n_super + KS - 1) / KS, blk0 = part * per_part, nblk = min(blk0 + per_part, n_super);
     const uint32_t c = lane & 31, h = lane >> 5;
 
-    // work groups of one set of weight rows (all token tiles) get consecutive ids on one XCD (ids are dealt round-robin
-    // to the 8 XCDs), so that their weight reads meet in that XCD's L2
-    const uint32_t xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
-    const uint32_t n_tile = (loc / m_tiles) * 8 + xcd, m_tile = loc % m_tiles;
-    if (n_tile >= n_tiles) return;
+    uint32_t m_tile, n_tile;
+    if (!tile_order_at(blockIdx.x, gridDim.x, m_tiles, n_tiles, m_tile, n_tile)) return;  // the whole work group
     const uint32_t m_wg = m_tile * TOK, n_wg = n_tile * ROWS, n_wave = n_wg + 32 * wave;
 
     const uint32_t row_bytes = n_super * F::BLOCK;
@@ -521,7 +519,7 @@ __global__ __launch_bounds__(64 * RW * KS) __attribute__((amdgpu_waves_per_eu(2,
 template <class F, int MT, int RW, int KS>
 hipError_t launch_f16_shape(const GemmArgs &a, hipStream_t stream) {
     const uint32_t m_tiles = (a.m + 32 * MT - 1) / (32 * MT), n_tiles = (a.n + 32 * RW - 1) / (32 * RW);
-    const dim3 grid(8 * ((n_tiles + 7) / 8) * m_tiles);
+    const dim3 grid(tile_order_grid(m_tiles, n_tiles));
     note_launch("gemm_f16_kernel", F::TYPE, MT, RW, KS, 0, grid.x, 1, 64 * RW * KS);
     hipLaunchKernelGGL((gemm_f16_kernel<F, MT, RW, KS>), grid, dim3(64 * RW * KS), 0, stream, a.W, a.A, a.out, a.m, a.n, a.k,
                        a.accumulate, a.bias, m_tiles, n_tiles);

@@ -1,0 +1,29 @@
+// Which tile of m_tiles x n_tiles a work group takes, by its number: ids are dealt round-robin to the 8 XCDs, and an XCD
+// takes a run of tiles with the token tiles of one set of weight rows next to each other, so that their weight reads meet
+// in its L2.  The runs differ by at most 7 tiles and none is longer than an eighth of all, rounded up: a grid of as many
+// tiles as there are compute units is one round of the chip whatever its sides (dealing whole sets of weight rows to the
+// XCDs instead, 36 sets of 7 token tiles gave four of them 35 work groups for 32 compute units: 448 x 4608 x 4096, Q4_K,
+// 74 us against 40).
+// (No HIP header here: a host test walks the grids.)
+#pragma once
+#include <cstdint>
+
+#ifdef __HIPCC__
+#define OXQ_HOST_DEVICE __host__ __device__ __forceinline__
+#else
+#define OXQ_HOST_DEVICE inline
+#endif
+
+namespace oxq {
+
+OXQ_HOST_DEVICE uint32_t tile_order_grid(uint32_t m_tiles, uint32_t n_tiles) { return (m_tiles * n_tiles + 7) / 8 * 8; }
+
+// false: no tile left for this work group
+OXQ_HOST_DEVICE bool tile_order_at(uint32_t block, uint32_t grid, uint32_t m_tiles, uint32_t n_tiles, uint32_t &m_tile, uint32_t &n_tile) {
+    const uint32_t t = (block & 7) * (grid >> 3) + (block >> 3);
+    n_tile = t / m_tiles;
+    m_tile = t - n_tile * m_tiles;
+    return n_tile < n_tiles;
+}
+
+}  // namespace oxq

@@ -1,6 +1,7 @@
 """Runs tests/cpp/test_quant_kernel.bin: the reference crate's own unit tests replayed
-through the C++ mirror of its interface (include/oxq/quant_kernel.hpp -> C ABI), and
-tests/cpp/test_lds_opt_in.bin: the kernels' LDS limits asked for by several threads."""
+through the C++ mirror of its interface (include/oxq/quant_kernel.hpp -> C ABI), and the
+host tests beside it: the kernels' LDS limits asked for by several threads, and the order
+in which work groups take tiles."""
 import os
 import subprocess
 
@@ -22,6 +23,10 @@ def _run(*args, binary=BIN):
 
 def test_lds_limits_are_only_raised():
     _run(binary=os.path.join(CPP, "test_lds_opt_in.bin"))
+
+
+def test_tiles_are_dealt_evenly_to_the_xcds():
+    _run(binary=os.path.join(CPP, "test_tile_order.bin"))
 
 
 def test_cpp_mirror_host_cases():
