@@ -812,7 +812,12 @@ constexpr uint32_t SKINNY_WHOLE_MAX_K = 4096;
 // 4096 Q4_K 12.9 to 11.3, 4096 x 4096 Q4_K 14.2 to 13.2, IQ4_XS 14.8 to 13.1, Q8_0 17.7 to 16.2.  14336 x 4096 is a tie for
 // Q4_K (20.5 / 20.9) and a loss for Q6_K (29.4 / 35.2); at 4096 columns the formats whose high bits lie apart are too (4096 x
 // 4096 Q5_K 15.6 / 17.0, Q5_0 16.2 / 17.4), Q6_K but for (18.1 / 18.3, 1024 x 4096 16.8 / 15.8).
-static inline bool skinny_whole_pays(uint32_t type, uint32_t n, uint32_t k) {
+// With more row tiles than compute units some work groups walk two, which the split of k (`can_split`: rows of 4096 columns,
+// and room for its sums) does not: 4096 / 4352 / 7168 x 4096, 16 rows, us, weights of the call before still in the
+// cache, whole k against split: Q4_K 8.9 / 10.9 / 11.5 against 9.9 / 10.2 / 11.1, Q8_0 9.6 / 13.3 / 14.7 against 12.3 / 12.5 /
+// 13.6, Q6_K 11.0 / 14.6 / 17.7 against 12.9 / 13.2 / 14.5, IQ4_XS 8.1 / 10.5 / 11.2 against 10.0 / 10.4 / 11.3.
+static inline bool skinny_whole_pays(uint32_t type, uint32_t n, uint32_t k, bool can_split) {
+    if (can_split && n > 16 * device_cus()) return false;
     if (k % 256 != 0 || k < 512 || k > SKINNY_WHOLE_MAX_K || (uint64_t)n * k >= (1ull << 25)) return false;
     return k < 4096 || !(type == OXQ_TYPE_Q5_K || type == OXQ_TYPE_Q5_0 || type == OXQ_TYPE_Q5_1 || type == OXQ_TYPE_Q3_K ||
                          type == OXQ_TYPE_Q2_K);
@@ -1060,7 +1065,7 @@ static int skinny_shape(const GemmArgs &a, bool has_partial, uint32_t rows, int 
         switch (variant) {
         case 0: {
             if (!a.offsets) {
-                if (!a.sums && !two && skinny_whole_pays(F::TYPE, a.n, a.k)) return SK_WHOLE;
+                if (!a.sums && !two && skinny_whole_pays(F::TYPE, a.n, a.k, has_partial && skinny_splits(a.n, a.k) >= 2)) return SK_WHOLE;
                 // one matrix, up to 16 token rows: enough row groups by themselves (a vocabulary projection), or k
                 // split over work groups (the workspace has room for the sums)
                 if (two) {

@@ -451,3 +451,25 @@ def test_whole_k_in_lds_by_default(hip, ref):
         torch.cuda.synchronize()
         assert last_launch().startswith("gemm_skinny_whole_kernel") == whole, (m, last_launch())
         assert_close(dy[m - 1].cpu().numpy(), canonical_ref(ref, t, w, acts[m - 1], n, k_), f"m={m}")
+
+
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q6_K], ids=lambda t: O.NAMES[t])
+def test_whole_k_in_lds_up_to_a_row_tile_per_compute_unit(hip, ref, t):
+    """Rows of 4096 columns, whose k can be split over work groups instead: the whole k at once as long as no work group
+    walks a second row tile."""
+    import torch
+    m, k_ = 16, 4096
+    one_each = 16 * hip.device_info()["compute_units"]
+    kern = hip.HipKernel(t)
+    acts = ref.quantize_q8_0(synth.normal_f32(97, m * k_)).reshape(m, k_ // 32 * 34)
+    da = torch.from_numpy(acts).cuda()
+    for n, whole in ((one_each, True), (one_each + 1, False)):
+        say("whole k, a tile each", O.NAMES[t], n)
+        w = weights(t, 98, n, k_)
+        ws = torch.empty(kern.gemm_workspace_bytes(m, n, k_), dtype=torch.uint8, device="cuda")
+        dw, dy = torch.from_numpy(w).cuda(), torch.zeros((m, n), dtype=torch.float32, device="cuda")
+        kern.gemm_q8_dev(dw, da, dy, m, n, k_, workspace=ws)
+        torch.cuda.synchronize()
+        assert last_launch().startswith("gemm_skinny_whole_kernel") == whole, (n, last_launch())
+        for r in (0, m - 1):
+            assert_close(dy[r].cpu().numpy(), canonical_ref(ref, t, w, acts[r], n, k_), f"{n} row {r}")
