@@ -545,12 +545,17 @@ bool gemm_f16_supported(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
 // 110-130 us (large shape) and 47-54 (small), Q5_K 100-108 and 41-48, Q4_K 92-100 and 36-42; a round with rows and columns to
 // spare costs as much as a full one.
 // Q6_K, whose tile kernel takes four vector instructions per result where this one takes one: either shape once its
-// grid is three quarters full (768 x 4096 x 4096 96 us against 105; the small one in a single round a tie there: 333 x 4096
-// x 4096; two thirds are not enough: 192 x 14336 x 4096 94 against 86), the large one from 64 % on in a single round (333 x
-// 14336 x 4096 116 against 147).
+// grid is three quarters full (768 x 4096 x 4096 95 us against 103; in one round of the small shape 192 tiles are a tie, 51
+// against 50, and 206 win, 52 against 62), the large one from 64 % on in a single round (333 x 14336 x 4096 115 against 145).
+// Two rounds of the small shape up to 384 rows, where the tile kernel splits k inside work groups of 64 x 32 and keeps
+// the chip full: from 82 % on (384 tiles: 256 x 12288 x 4096 93 against 82, 384 x 8192 x 8192 176 against 153, x 3072 72 against
+// 66; 420 tiles, 333 x 8960 x 1536, 42 against 47; 432, 256 x 13824 x 5120, a tie).
 // Q4_K and Q5_K, whose tile kernel is about as fast per result: only full rounds, the large shape of Q5_K (Q4_K has the
-// prefill kernel there) and the small one where the tile kernel's larger tiles do not fill the chip (at most one round
-// of 64 x 128: 512 x 4096 x 4096 42 us against 48.5; 1024 x 4096 x 4096, two rounds, 78 against 69).
+// prefill kernel there) and the small one in a single round (512 x 4096 x 4096, 256 tiles, Q4_K 40 against 45, Q5_K 44 against
+// 50; with 208 to 240 tiles 39-40 against 40-41 and 43-44 against 45, with 192 it loses, 37 against 34; 264 tiles, two rounds,
+// 72 against 62 and 80 against 73) of more than 384 rows: up to there the tile kernel's own tiles fill the chip as well (256
+// tiles at k = 4096 / 8192, 128 rows Q4_K 41 / 77 against 41 / 75, Q5_K 45 / 89 against 46 / 89, 256 rows Q4_K 40 / 76 against 40 /
+// 73, Q5_K 44 / 83 against 45 / 83; only on rows of 1024 columns this one wins, 16 against 19).
 int gemm_f16_shape(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
     if (!gemm_f16_supported(type, m, n, k) || k < 1024) return 0;
     const uint64_t cus = device_cus();
@@ -560,7 +565,7 @@ int gemm_f16_shape(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
     const bool large_ok = 100 * (uint64_t)m >= 70 * 128 * ((m + 127) / 128), small_ok = m > 64 && 100 * (uint64_t)m >= 80 * 64 * ((m + 63) / 64);
     if (type == OXQ_TYPE_Q6_K) {
         if (large_ok && rl * 130 <= rs * 54) return 100 * large >= (rl == 1 ? 64u : 72u) * rl * cus ? 1 : 0;
-        return small_ok && 100 * small >= (rs == 1 ? 80u : 74u) * rs * cus ? 2 : 0;
+        return small_ok && 100 * small >= (rs == 1 ? 80u : rs == 2 && m <= 384 ? 82u : 74u) * rs * cus ? 2 : 0;
     }
     if (type == OXQ_TYPE_Q5_K && large_ok && 100 * large >= 96 * rl * cus && (rl == 1 || k >= 8192)) return 1;
     return small_ok && rs == 1 && 100 * small >= 96 * cus && m > 384 ? 2 : 0;

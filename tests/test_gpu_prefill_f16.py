@@ -230,6 +230,10 @@ LARGE, SMALL = "4,8,1", "2,4,2"
     (O.Q6_K, 128, 128 * 103, 1024, SMALL),  # 206 small tiles
     (O.Q6_K, 128, 128 * 102, 1024, None),
     (O.Q6_K, 80, 128 * 103, 1024, None),    # (token tiles a quarter empty and more)
+    (O.Q6_K, 384, 128 * 69, 1024, None),    # two rounds of small tiles, 414 and 420 of 512
+    (O.Q6_K, 384, 128 * 70, 1024, SMALL),
+    (O.Q6_K, 448, 128 * 55, 1024, SMALL),   # 385 of 512 behind 384 rows
+    (O.Q6_K, 448, 128 * 54, 1024, None),
     (O.Q5_K, 128, 256 * 246, 1024, LARGE),
     (O.Q5_K, 128, 256 * 245, 1024, None),
     (O.Q5_K, 448, 128 * 36, 1024, SMALL),
