@@ -500,11 +500,14 @@ __device__ __forceinline__ void gemm_tile_body(
     uint32_t n_tile = (loc / m_tiles) * 8 + xcd, m_tile = loc % m_tiles;
     uint32_t row0 = 0, row_end = m;
     if (n_experts) {
-        // expert groups: token tiles outermost, so that the tiles the experts do not need form one run at the end
-        const uint32_t n_groups = (n_tiles + 7) / 8;
-        n_tile = (loc % n_groups) * 8 + xcd;
+        // expert groups: token tiles outermost, so that the tiles the experts do not need form one run at the end; a
+        // token tile's work groups are consecutive, which deals them evenly to the XCDs whatever their number (six or
+        // twelve 128-row tiles, every one on the XCD of its number modulo 8, left XCDs idle: Q4_K, 64 rows in the mean, 128
+        // experts of 768 x 2048 117 us against 100, 64 of 1536 x 2048 109 against 94)
         uint32_t expert = 0;
-        if (!find_group_tile(offsets, n_experts, WG_TOK, loc / n_groups, expert, m_tile)) return;  // whole work group
+        const uint32_t place = blockIdx.x / n_tiles;
+        n_tile = blockIdx.x - place * n_tiles;
+        if (!find_group_tile(offsets, n_experts, WG_TOK, place, expert, m_tile)) return;  // whole work group
         row0 = (uint32_t)offsets[expert];
         row_end = (uint32_t)offsets[expert + 1];
         W += (size_t)expert * w_stride;
@@ -824,7 +827,7 @@ static hipError_t launch_tile(const GemmArgs &a, const TilePlan &p, hipStream_t 
     constexpr uint32_t WG_TOK = 32 * MT * (WM ? WM : 1), WG_ROWS = 32 * NT * (WM ? 4 / WM : 1);
     const uint32_t m_tiles = a.offsets ? group_tiles_bound(a.m, a.max_rows, a.n_experts, WG_TOK) : (a.m + WG_TOK - 1) / WG_TOK;
     const uint32_t n_tiles = (a.n + WG_ROWS - 1) / WG_ROWS;
-    const dim3 grid(8 * ((n_tiles + 7) / 8) * m_tiles);
+    const dim3 grid((a.offsets ? n_tiles : 8 * ((n_tiles + 7) / 8)) * m_tiles);
     const size_t lds = (size_t)tile_padded_sub_blocks(a.k) * WG_TOK * 2;
     auto kern = &gemm_tile_kernel<F, MT, NT, WM, DIST, DUMP, ADIST>;
     if constexpr (OCC == 3) kern = &gemm_tile_kernel_occ3<F, MT, NT, WM, DIST, DUMP, ADIST>;
@@ -844,6 +847,7 @@ static hipError_t launch_tile(const GemmArgs &a, const TilePlan &p, hipStream_t 
 template <class F>
 static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t stream) {
     uint32_t rows = a.offsets ? (a.shape_rows ? a.shape_rows : a.max_rows) : a.m;
+    uint32_t tiles64 = 0;  // 64-row tiles of a group, in 32nds, where the mean says more than `rows`
     // Expert groups whose sizes only the device knows (the launch is shaped for twice the mean, the grid covers the
     // worst case): the tile follows the mean -- a larger group takes more tiles, while a tile twice the usual group
     // is half empty everywhere.  8 experts of 14336 x 4096 / 4096 x 14336, IQ4_XS, 12..25 rows each: 108 / 108 us on
@@ -854,6 +858,7 @@ static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t
     if (a.offsets && a.n_experts && a.shape_rows && a.shape_rows < a.max_rows) {
         const uint32_t mean = (a.m + a.n_experts - 1) / a.n_experts;
         rows = mean > 48 && mean < 65 ? 65 : mean;
+        if (rows == 65) tiles64 = (mean - 16) * 5 / 8;  // (a group comes to 1 tile at 48 rows, 1.25 at 56, 1.5 at 64)
     }
     const int variant = g_gemm_variant.load(std::memory_order_relaxed);
     (void)variant;  // (read by the fixed-shape knobs, which the second translation unit leaves out)
@@ -875,14 +880,18 @@ static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t
     // against the second): 4096 x 14336, 128 / 256 / 384 tokens, Q4_K 131 / 136 / 143 against 47 / 87 / 127, Q6_K
     // 196 / 198 / 206 against 66 / 125 / 183; 4096 x 4096 Q4_K 44 / 45 / 48 against 19 / 27 / 37, Q8_0 51 / 51 / 54
     // against 21 / 33 / 46; 14336 x 4096 Q4_K 128 / 192 tokens 49 / 70 against 45 / 63, 256 a tie, 384 108 against 113.
-    const bool wide_grid = (size_t)((rows + 63) / 64) * ((a.n + 127) / 128) * (a.offsets ? a.n_experts : 1) * 4 >= 7 * (size_t)device_cus();
-    // Expert groups, whose 64-row tiles are part empty: the split-k tiles also on a full chip where k feeds four waves
-    // (64 / 96 rows in the mean on 1536 x 3072: Q4_K 200 / 130 us against 174 / 117, Q6_K 290 / 187 against 244 / 163,
-    // 768 x 2048, 64 rows, Q6_K 113 against 100); on 14336 x 4096 a tie.  With rows of up to 1536 columns it is the other
-    // way round, from 33 rows on: 64 experts of 2048 x 768 at 48 rows Q4_K 77 against 61, Q6_K 95 against 75, of 3072 x 1536
-    // 159 against 138 and 197 against 175.
-    const bool mid_split_k = mid && (narrow || !wide_grid || (a.offsets && a.k >= 2048 && a.n < 8192));
-    // (groups of unknown sizes from a mean of 25 on: 128 of 2048 x 768 / 3072 x 1536 at 32 rows, Q6_K, 173 / 357 on 32-token
+    if (!tiles64) tiles64 = 32 * ((rows + 63) / 64);
+    const bool wide_grid = (size_t)tiles64 * ((a.n + 127) / 128) * (a.offsets ? a.n_experts : 1) * 4 >= 32 * 7 * (size_t)device_cus();
+    // Expert groups, whose tiles are part empty, follow the same line (a full chip, 64 x 128 against 64 x 32 split, Q4_K: 8 of
+    // 4096 x 14336 at a mean of 80 / 96 rows 235 against 296 / 237 against 302, of 6144 x 2048 54 against 64, 128 of 1536 x 3072
+    // at 96 346 against 409; Q6_K 8 of 4096 x 14336 at 96 379 against 428).  A mean of 49..64 rows comes to between one and
+    // one and a half 64-row tiles a group, some with few rows: 64 x 128 from 2.8 expected ones per compute unit on (640
+    // tiles, 32 of 2048 x 2048 at 56, 64 x 128 against split Q4_K 97 / 95, Q6_K 116 / 106, Q8_0 127 / 122; 768, the same at 64,
+    // 98 / 104, 121 / 119, 135 / 146; 320, 8 of 4096 x 14336 at 56, Q4_K 240 / 192, Q6_K 394 / 280).
+    const bool mid_split_k = mid && (narrow || !wide_grid);
+    // Short rows on a full chip take 64 x 128 tiles from 33 rows on, groups of unknown sizes from a mean of 25 on: 64 experts of
+    // 2048 x 768 at 48 rows Q4_K 77 (64 x 32 split) against 61, Q6_K 95 against 75, of 3072 x 1536 159 against 138 and 197
+    // against 175 (128 of 2048 x 768 / 3072 x 1536 at 32 rows, Q6_K, 173 / 357 on 32-token
     // tiles against 131 / 307; at 20 rows of 3072 x 1536 270 against 299)
     const bool short_groups = a.offsets && rows > (a.shape_rows < a.max_rows ? 24u : 32u) && rows <= 64 && fits64 && a.k <= 1536 && wide_grid;
     if (a.sums)  // debug dump: the same tile layout (and fp32 summation order) as the production choice below
