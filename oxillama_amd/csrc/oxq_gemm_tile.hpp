@@ -858,7 +858,7 @@ static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t
     if (a.offsets && a.n_experts && a.shape_rows && a.shape_rows < a.max_rows) {
         const uint32_t mean = (a.m + a.n_experts - 1) / a.n_experts;
         rows = mean > 48 && mean < 65 ? 65 : mean;
-        if (rows == 65) tiles64 = (mean - 16) * 5 / 8;  // (a group comes to 1 tile at 48 rows, 1.25 at 56, 1.5 at 64)
+        if (mean > 48 && mean < 65 && a.k >= 2048) tiles64 = mean - 16;  // (1 tile at 48 rows, 1.25 at 56, 1.5 at 64)
     }
     const int variant = g_gemm_variant.load(std::memory_order_relaxed);
     (void)variant;  // (read by the fixed-shape knobs, which the second translation unit leaves out)
@@ -880,14 +880,27 @@ static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t
     // against the second): 4096 x 14336, 128 / 256 / 384 tokens, Q4_K 131 / 136 / 143 against 47 / 87 / 127, Q6_K
     // 196 / 198 / 206 against 66 / 125 / 183; 4096 x 4096 Q4_K 44 / 45 / 48 against 19 / 27 / 37, Q8_0 51 / 51 / 54
     // against 21 / 33 / 46; 14336 x 4096 Q4_K 128 / 192 tokens 49 / 70 against 45 / 63, 256 a tie, 384 108 against 113.
-    if (!tiles64) tiles64 = 32 * ((rows + 63) / 64);
-    const bool wide_grid = (size_t)tiles64 * ((a.n + 127) / 128) * (a.offsets ? a.n_experts : 1) * 4 >= 32 * 7 * (size_t)device_cus();
+    const size_t row_tiles = (a.n + 127) / 128, group_32 = tiles64 ? tiles64 : 32 * ((rows + 63) / 64);
+    const uint32_t line_32 = !tiles64 ? 56 : F::BLOCK_BYTES >= 210 ? 112 : 90;  // 32nds of a tile, per compute unit
+    bool wide_grid = group_32 * row_tiles * (a.offsets ? a.n_experts : 1) >= line_32 * (size_t)device_cus();
     // Expert groups, whose tiles are part empty, follow the same line (a full chip, 64 x 128 against 64 x 32 split, Q4_K: 8 of
-    // 4096 x 14336 at a mean of 80 / 96 rows 235 against 296 / 237 against 302, of 6144 x 2048 54 against 64, 128 of 1536 x 3072
-    // at 96 346 against 409; Q6_K 8 of 4096 x 14336 at 96 379 against 428).  A mean of 49..64 rows comes to between one and
-    // one and a half 64-row tiles a group, some with few rows: 64 x 128 from 2.8 expected ones per compute unit on (640
-    // tiles, 32 of 2048 x 2048 at 56, 64 x 128 against split Q4_K 97 / 95, Q6_K 116 / 106, Q8_0 127 / 122; 768, the same at 64,
-    // 98 / 104, 121 / 119, 135 / 146; 320, 8 of 4096 x 14336 at 56, Q4_K 240 / 192, Q6_K 394 / 280).
+    // 4096 x 14336 at a mean of 80 / 96 rows 230 against 295 / 228 against 299, of 6144 x 2048 59 against 69, 128 of 1536 x 3072
+    // at 96 349 against 379; Q6_K 8 of 4096 x 14336 at 96 366 against 428).  But:
+    //   - A mean of 49..64 rows comes to between one and one and a half 64-row tiles a group, some with few rows: 64 x 128
+    //     from 2.8 expected ones per compute unit on (2.5, 32 of 2048 x 2048 at 56, Q4_K 97 / 95, Q6_K 116 / 106, Q8_0 127 / 122;
+    //     2.9, of 2052 x 2048 at 60, Q4_K 67 / 73; 1.3, 8 of 4096 x 14336 at 56, Q4_K 240 / 192, Q6_K 394 / 280), from 3.5 on
+    //     for the formats of 0.8 bytes and more per weight (3.2, 64 of 1536 x 2048 at 50, Q6_K 123 / 114, Q8_0 106 / 103; 4.1,
+    //     at 60, 125 / 136 and 111 / 120).  Rows of fewer than 2048 columns, four waves to a short k, keep the line at two
+    //     tiles a group (16 of 4096 x 1024 at 50 Q4_K 28 / 37, Q6_K 40 / 47, Q8_0 38 / 44; 32 of 2048 x 1024 at 60 37 / 46).
+    //   - At 65..71 rows the second tile holds a few rows in many groups and the gain (0-14 %) is less than what row tiles with
+    //     more than a twentieth to spare cost: 32 of 2052 x 2048, 17 row tiles, IQ4_XS 78 / 78, Q6_K 117 / 109, Q8_0 117 / 111.
+    //   - Formats of a byte and more per weight: not where the row tiles are no multiple of the eight XCDs, as the second
+    //     token tile of an expert then reads its weights into another XCD's L2 (Q8_0, 128 of 1536 x 3072 at 68 / 96 rows
+    //     459 / 427 and 527 / 498; of 768 x 2048, 64 of 1536 x 2048: +-7 %; 64 of 3072 x 3072 at 68 383 / 411).
+    if (a.offsets && wide_grid && a.k >= 2048) {
+        if (rows >= 65 && rows < 72 && !tiles64 && 100 * (size_t)a.n < 95 * 128 * row_tiles) wide_grid = false;
+        if (F::BLOCK_BYTES >= 256 && row_tiles % 8 != 0 && a.n < 8192) wide_grid = false;
+    }
     const bool mid_split_k = mid && (narrow || !wide_grid);
     // Short rows on a full chip take 64 x 128 tiles from 33 rows on, groups of unknown sizes from a mean of 25 on: 64 experts of
     // 2048 x 768 at 48 rows Q4_K 77 (64 x 32 split) against 61, Q6_K 95 against 75, of 3072 x 1536 159 against 138 and 197

@@ -381,12 +381,18 @@ def test_grouped_matmul_of_a_handful_of_rows_is_one_gemv_launch(hip, ref, t, cou
     assert torch.equal(dy2[:rows], dy[:rows] + dy[:rows]) and torch.equal(dy2[rows:], dy[rows:])
 
 
+# (tile kernel shapes: 2,1,1 is 64 tokens x 128 rows, 2,1,0 is 64 x 32 with k split over the waves)
 @pytest.mark.parametrize("t,mean,n,k_,kernel", [
     (O.Q4_K, 32, 2052, 768, "gemm_skinny_kernel"), (O.Q4_K, 33, 2048, 768, "gemm_tile_kernel<Q4_K,2,1,1"),
     (O.Q6_K, 24, 260, 768, "gemm_skinny_kernel"), (O.Q6_K, 25, 2048, 768, "gemm_tile_kernel<Q6_K,2,1,1"),
     (O.Q6_K, 32, 260, 1792, "gemm_skinny_kernel"), (O.Q8_0, 21, 260, 1536, "gemm_tile_kernel"),
-    (O.IQ4_XS, 65, 2052, 2048, "gemm_tile_kernel<IQ4_XS,2,1,0")],
-    ids=["Q4_K_32", "Q4_K_33", "Q6_K_24", "Q6_K_25", "Q6_K_32", "Q8_0_21", "IQ4_XS_65"])
+    (O.IQ4_XS, 65, 2052, 2048, "gemm_tile_kernel<IQ4_XS,2,1,0"), (O.IQ4_XS, 72, 2052, 2048, "gemm_tile_kernel<IQ4_XS,2,1,1"),
+    (O.Q4_K, 65, 2048, 2048, "gemm_tile_kernel<Q4_K,2,1,1"), (O.Q4_K, 50, 2048, 2048, "gemm_tile_kernel<Q4_K,2,1,0"),
+    (O.Q4_K, 50, 2048, 1024, "gemm_tile_kernel<Q4_K,2,1,1"), (O.Q4_K, 50, 3072, 2048, "gemm_tile_kernel<Q4_K,2,1,1"),
+    (O.Q6_K, 50, 3072, 2048, "gemm_tile_kernel<Q6_K,2,1,0"), (O.Q8_0, 72, 1536, 2048, "gemm_tile_kernel<Q8_0,2,1,0"),
+    (O.Q8_0, 72, 2048, 2048, "gemm_tile_kernel<Q8_0,2,1,1")],
+    ids=["Q4_K_32", "Q4_K_33", "Q6_K_24", "Q6_K_25", "Q6_K_32", "Q8_0_21", "IQ4_XS_65", "IQ4_XS_72", "Q4_K_65", "Q4_K_50",
+         "Q4_K_50_short", "Q4_K_50_wide", "Q6_K_50_wide", "Q8_0_72_narrow", "Q8_0_72"])
 def test_grouped_kernel_by_mean_and_row_length(hip, ref, t, mean, n, k_, kernel):
     """Groups of sizes the host does not know, on both sides of each bound between this kernel and the tile kernel's shapes;
     sizes about the mean, one group empty, one twice the mean."""
