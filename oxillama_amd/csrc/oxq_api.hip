@@ -1129,8 +1129,9 @@ static int moe_gemm_impl(uint32_t type, const uint8_t *d_weights, size_t expert_
                                                  : total_rows);
     ga.shape_rows = ga.max_rows;
     if (!max_rows_per_expert) {
-        // Row counts known only on the device: the grid covers the worst case (one expert takes every
-        // row; tiles past an expert's rows exit at once), the tile shape is chosen for twice the mean.
+        // Row counts known only on the device: one expert may take every row.  The tile shape is chosen for twice
+        // the mean; the grid holds the token tiles that the groups can come to together (group_tiles_bound), and a
+        // work group finds its expert and tile from the offsets, or exits.
         const size_t mean = (total_rows + n_experts - 1) / n_experts;
         ga.shape_rows = (uint32_t)(2 * mean < total_rows ? 2 * mean : total_rows);
     }

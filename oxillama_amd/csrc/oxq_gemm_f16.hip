@@ -526,6 +526,7 @@ hipError_t launch_f16_shape(const GemmArgs &a, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// (the large shape of Q4_K is for the fixed-shape knob alone: those calls go to the prefill kernel)
 template <class F>
 hipError_t launch_f16(const GemmArgs &a, int shape, hipStream_t stream) {
     return shape == 1 ? launch_f16_shape<F, 4, 8, 1>(a, stream) : launch_f16_shape<F, 2, 4, 2>(a, stream);

@@ -484,10 +484,11 @@ __device__ __forceinline__ void skinny_step(uint8_t *const strip, float *const d
 // Work group = WAVES waves, each with its own NT x 16 weight rows; all of them the same token tiles (at most TT of
 // 16 tokens).  k is walked in chunks of `per` super-blocks (even): the work group stages the chunk's token bytes,
 // every wave runs its rows over the chunk, accumulators staying in registers; the weight prefetch runs on across
-// the chunk boundary.  blockIdx.x = row group, blockIdx.y = expert (grouped form), blockIdx.z = token pass.
-// One matrix (no experts) with too few row groups to fill the chip: blockIdx.y = which sb_per_split super-blocks of
-// k the work group walks; it stores its sums to partial[blockIdx.y][token][row] and gemm_skinny_reduce adds the
-// splits in index order.
+// the chunk boundary.  rg = row group, gy = expert (grouped form), tokb .. tok_end = the token rows; how
+// a work group's number comes to them is gemm_skinny_kernel's.
+// Too few row groups to fill the chip: ks = which sb_per_split super-blocks of k the work group walks; it stores its sums
+// to partial[ks][token][row] and gemm_skinny_reduce (expert groups: the layer's combine, where it can) adds the splits
+// in index order.
 // LDS: [A operands | fp32 token scales | P] of a chunk, then per wave [weight strip | dsc table | zero-point table].
 // Waves per SIMD the shape is meant to run at: two work groups on a compute unit where their LDS allows it.
 template <class F, int NT, int WAVES, int TT, int PER>
@@ -1021,9 +1022,10 @@ static hipError_t launch_skinny_shape(const GemmArgs &a, const TilePlan &p, hipS
 //    layer 293-303 us;
 //  * one matrix, no experts, up to 16 token rows: too few row groups as it is (14336 x 4096: 24 us against 19);
 //    with k split over work groups and the splits added by a second launch (call totals, with the token re-layout):
-//    14336 x 4096 18.0 us against 19.6, 4096 x 14336 21.4 against 29.5, 28672 x 8192 40 against 49; 4096 x 4096
-//    14.4 against 12.3 (not taken below 2^25 weights); 17..32 rows 24.6 against 19.7 (not taken).  From 512 row
-//    groups on no split is needed (57344 x 4096, 16 rows: 44 us against 56).
+//    14336 x 4096 18.0 us against 19.6, 4096 x 14336 21.4 against 29.5, 28672 x 8192 40 against 49; 17..32 rows of
+//    14336 x 4096 24.6 against 19.7 (taken below 8192 rows of weights only).  Smaller matrices: skinny_whole_pays, and
+//    for what is left skinny_sb_per_split.  From 512 row groups on no split is needed (57344 x 4096, 16 rows: 44 us
+//    against 56).
 enum SkinnyShape { SK_NONE = 0, SK_1_4, SK_1_8, SK_2_2, SK_1_4_SPLIT, SK_1_16, SK_2_8, SK_W4_1_8, SK_W4_2_4, SK_2_4, SK_2_2_SPLIT, SK_WHOLE };
 
 // Expert groups of up to this many rows in the mean stay with this kernel (groups beyond its tiles take further passes

@@ -848,8 +848,8 @@ template <class F>
 static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t stream) {
     uint32_t rows = a.offsets ? (a.shape_rows ? a.shape_rows : a.max_rows) : a.m;
     uint32_t tiles64 = 0;  // 64-row tiles of a group, in 32nds, where the mean says more than `rows`
-    // Expert groups whose sizes only the device knows (the launch is shaped for twice the mean, the grid covers the
-    // worst case): the tile follows the mean -- a larger group takes more tiles, while a tile twice the usual group
+    // Expert groups whose sizes only the device knows (the launch is shaped for twice the mean, the grid for the tiles
+    // the groups can come to): the tile follows the mean -- a larger group takes more tiles, while a tile twice the usual group
     // is half empty everywhere.  8 experts of 14336 x 4096 / 4096 x 14336, IQ4_XS, 12..25 rows each: 108 / 108 us on
     // 32-token tiles against 152 / 164 on 64-token ones; 24..42 rows 136 / 140 against 155 / 167; 38..63 rows on
     // 64 x 32 split-k tiles 163 / 172 against 159 / 258 on 64 x 128.
@@ -907,7 +907,10 @@ static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t
     // against 175 (128 of 2048 x 768 / 3072 x 1536 at 32 rows, Q6_K, 173 / 357 on 32-token
     // tiles against 131 / 307; at 20 rows of 3072 x 1536 270 against 299)
     const bool short_groups = a.offsets && rows > (a.shape_rows < a.max_rows ? 24u : 32u) && rows <= 64 && fits64 && a.k <= 1536 && wide_grid;
-    if (a.sums)  // debug dump: the same tile layout (and fp32 summation order) as the production choice below
+    // The debug dump of the integer sums: the tile layout (and fp32 summation order) that this kernel takes by default.
+    // Plain matmuls that go to the kernels without a dump (gemm_f16_kernel, gemm_skinny_whole_kernel) come here for it
+    // too: their integer sums are these, their fp32 sums are added in another order.
+    if (a.sums)
         return big   ? launch_tile<F, 2, 1, 2, 1, true>(a, p, stream)
                : mid ? (mid_split_k ? launch_tile<F, 2, 1, 0, 2, true, 2, 2>(a, p, stream)
                                     : launch_tile<F, 2, 1, 1, 2, true>(a, p, stream))
