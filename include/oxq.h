@@ -276,7 +276,9 @@ int oxq_activation_route(void);
  * workspace size.  Q4_K matmuls of many token rows whose 128-token x
  * 256-row work groups fill the chip (the prefill shapes) run on the f16 matrix cores instead,
  * with the 6-bit sub-block scale inside the weight operand (exact) and d / dmin applied per
- * super-block: the same integers, fp32 inside the same 1e-5 bar; the workspace size covers both. */
+ * super-block: the same integers, fp32 inside the same 1e-5 bar; the workspace size covers both.  Many token rows of
+ * Q6_K, and of Q5_K and Q4_K on other shapes that fill the chip, take the same arithmetic from the Q8_0 rows
+ * themselves, without workspace. */
 size_t oxq_gemm_q8_workspace_bytes(uint32_t type, size_t m, size_t n, size_t k);
 int oxq_gemm_q8_dev(uint32_t type, const uint8_t *d_weights, const uint8_t *d_acts_q8,
                     float *d_out, size_t m, size_t n, size_t k, int accumulate,

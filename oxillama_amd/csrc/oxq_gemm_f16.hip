@@ -23,7 +23,10 @@
 //              for matrices and prompts that do not fill the chip with the large tile
 // What bounds it: the issue of a SIMD's instructions.  Matrix and vector instructions of its two waves take turns (measured
 // with mixes of both: 64 cycles for two MFMAs, and 2.2 a v_fmac, 3 to 4.4 an integer or packed instruction on top of
-// them), and in this loop they come to about 150 cycles a step for Q4_K and 220 for Q6_K against 190 and 260 measured.
+// them).  By rocprofv3's counters a step of the large shape takes 254 to 266 cycles
+// for Q6_K: 128 of matrix work, 37 other vector instructions, 67 cycles of both at once.  The small shape, which unpacks
+// and stages twice as much per result, takes 415 (Q6_K, 56 vector instructions; k = 14336), 432 (Q4_K, 46) and 468 (Q5_K, 57;
+// k = 4096, the launch's ramp and the exchange of the halves included).
 // Measured, us, this kernel against the tile kernel: Q6_K 2048 x 8192 x 28672 1893 against 2946 (508 TOPS), 2048 x 8192 x
 // 8192 542 / 656, 512 x 14336 x 4096 130 / 166, 512 x 4096 x 14336 175 / 207; Q4_K 512 x 4096 x 4096 42 / 48.5, 2048 x 1024 x 4096
 // 42 / 51; Q5_K 2048 x 4096 x 14336 388 / 454, 512 x 4096 x 4096 48 / 54.
