@@ -257,11 +257,14 @@ struct Skinny<TileQ6K> {
     }
 };
 
+// A unit's int8 operands, [k-slot of 8][token], and a pad that puts the units of a token's eight blocks, which are written by
+// neighbouring threads, into different banks.
+constexpr uint32_t SKINNY_UNIT = 512 + 32;
 // LDS bytes per (sub-block, token tile): int8 operands, fp32 scales, and fp32 P (one factor per sub-block) or the
 // MFMA addends of the two halves (two factors; with a zero-point term, P of each half as well)
 template <class F>
 constexpr uint32_t skinny_act_bytes() {
-    return 512 + 64 + (Skinny<F>::KSPLIT == 2 ? 128 : 64) + (Skinny<F>::KSPLIT == 2 && Skinny<F>::HAS_MIN ? 128 : 0);
+    return SKINNY_UNIT + 64 + (Skinny<F>::KSPLIT == 2 ? 128 : 64) + (Skinny<F>::KSPLIT == 2 && Skinny<F>::HAS_MIN ? 128 : 0);
 }
 constexpr uint32_t SKINNY_FAC_STRIDE = 17;  // floats per weight row in a wave's factor tables (16 + pad)
 // LDS bytes of a wave: the strip of its rows' bytes of a step, and the factor tables (one factor per sub-block: of
@@ -289,7 +292,7 @@ __device__ __forceinline__ SkinnyLds skinny_lds(uint8_t *lds, uint32_t units) {
     constexpr int KS = Skinny<F>::KSPLIT;
     SkinnyLds L;
     L.A = lds;
-    L.D = reinterpret_cast<float *>(L.A + (size_t)units * 512);
+    L.D = reinterpret_cast<float *>(L.A + (size_t)units * SKINNY_UNIT);
     L.P = L.D + (size_t)units * 16;
     L.C = reinterpret_cast<int *>(L.P);
     L.P2 = L.P + (size_t)units * 16 * KS;
@@ -297,44 +300,62 @@ __device__ __forceinline__ SkinnyLds skinny_lds(uint8_t *lds, uint32_t units) {
     return L;
 }
 
-// Thread (cc, qq) of a unit's 64: bytes 8 qq .. 8 qq + 7 of token cc's block, with the block's scale, to LDS.
+// A pair of Q8_0 blocks (an even one and the next) is 17 dwords: scale and payload of the first, two bytes into a dword, then
+// the second's scale, its payload on a dword.  Four threads of a token's 64 take half a block each: one dword-aligned 16-byte
+// load and the dword behind it, which ends the first payload and holds the second scale.  (Loads of 8 bytes at the payloads'
+// own 2-byte alignment and the scales by themselves are twice the instructions, and those and the lines each touches, not bytes,
+// are what the texture unit counts -- 40 to 50 cycles a load whose lanes lie in sixteen or more lines.  16 rows, us, before and
+// after: Q4_K 4096 x 4096 9.5 / 8.0, 1024 x 4096 8.3 / 6.8, IQ4_XS 4096 x 4096 8.7 / 7.4, Q6_K 11.1 / 9.3 at 12 rows; the layer
+// of eight IQ4_XS experts of 14336 x 4096 at 64 tokens 269 / 256.)
+struct SkinnyToken {
+    u32x4 q;
+    uint32_t x;
+};
+// thread: bit 0 the half, bit 1 the second block; pair: the first block of the two
+__device__ __forceinline__ SkinnyToken skinny_get_token(const uint8_t *pair, const uint32_t thread) {
+    const uint8_t *p = pair + 16 * (thread & 1) + ((thread & 2) ? 36 : 0);
+    SkinnyToken r;
+    r.q = ld16(p);
+    r.x = ld4(p + ((thread & 2) ? 12 : 16));  // (the second block's threads do not need it: no byte past the pair)
+    return r;
+}
+// ... to LDS: token cc of the block's unit
 template <class F>
-__device__ __forceinline__ void skinny_put_token(u32x2 v, const float d, const uint32_t unit, const uint32_t cc, const uint32_t qq,
-                                                 const SkinnyLds &L) {
+__device__ __forceinline__ void skinny_put_token(const SkinnyToken tk, const uint32_t unit, const uint32_t cc, const uint32_t thread, const SkinnyLds &L) {
     using S = Skinny<F>;
     constexpr int KS = S::KSPLIT;
-    if constexpr (S::HAS_MIN && KS == 1) {
-        int sum = sdot4(v[0], 0x01010101u, sdot4(v[1], 0x01010101u, 0));
-        sum += xor1_i(sum);  // the four threads of a block
-        sum += xor2_i(sum);
-        if (qq == 0) L.P[unit * 16 + cc] = d * (float)sum;
-    }
-    if constexpr (S::HAS_MIN && KS == 2) {  // a zero-point factor per 16 weights: P of each half
-        int sum = sdot4(v[0], 0x01010101u, sdot4(v[1], 0x01010101u, 0));
-        sum += xor1_i(sum);
-        if ((qq & 1) == 0) L.P2[(unit * 2 + (qq >> 1)) * 16 + cc] = d * (float)sum;
-    }
-    if constexpr (KS == 2) {
-        // per half of the block (threads 0, 1 and 2, 3): the addend that turns sum(q a) into sum((q - OFFSET) a),
-        // on top of the 1.5 * 2^23 every result carries
-        int sum = sdot4(v[0], 0x01010101u, sdot4(v[1], 0x01010101u, 0));
-        sum += xor1_i(sum);
-        if ((qq & 1) == 0) L.C[(unit * 2 + (qq >> 1)) * 16 + cc] = 0x4B400000 - S::OFFSET * sum;
-    }
-    if (S::ACT_PERM == 1) {  // even bytes, then odd bytes
-        const uint32_t x0 = v[0], x1 = v[1];
-        v[0] = __builtin_amdgcn_perm(x1, x0, 0x06040200u);
-        v[1] = __builtin_amdgcn_perm(x1, x0, 0x07050301u);
-    }
-    if constexpr (S::ACT_PERM == 2) {
-        // weights j and j + 16 share a byte: k-slot q holds token bytes 4q .. 4q + 3, then 16 + 4q .. 16 + 4q + 3
+    const uint32_t half = thread & 1, shift = (thread & 2) ? 0u : 16u;
+    // the scales of both blocks, in the first block's threads; of the four: 0, 0, 1, 1
+    const float d = h2f((uint32_t)dpp_i<0x50>((int)(half ? tk.x >> 16 : tk.q[0])) & 0xFFFF);
+    uint32_t v[4];
 #pragma unroll
-        for (uint32_t i = 0; i < 2; i++)
-            *reinterpret_cast<uint32_t *>(L.A + ((size_t)unit * 64 + (2 * (qq & 1) + i) * 16 + cc) * 8 + 4 * (qq >> 1)) = v[i];
-    } else {
-        *reinterpret_cast<u32x2 *>(L.A + ((size_t)unit * 64 + qq * 16 + cc) * 8) = v;
+    for (int i = 0; i < 4; i++) v[i] = __builtin_amdgcn_alignbit(i < 3 ? tk.q[i + 1] : tk.x, tk.q[i], shift);
+    if constexpr (S::HAS_MIN || KS == 2) {
+        int sum = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) sum = sdot4(v[i], 0x01010101u, sum);
+        if constexpr (KS == 1) L.P[unit * 16 + cc] = d * (float)(sum + xor1_i(sum));  // (both halves: the same value)
+        // a zero-point factor per 16 weights: P of each half
+        if constexpr (KS == 2 && S::HAS_MIN) L.P2[(unit * 2 + half) * 16 + cc] = d * (float)sum;
+        // per half of the block: the addend that turns sum(q a) into sum((q - OFFSET) a), on top of the 1.5 * 2^23 every
+        // result carries
+        if constexpr (KS == 2) L.C[(unit * 2 + half) * 16 + cc] = 0x4B400000 - S::OFFSET * sum;
     }
-    if (qq == 0) L.D[unit * 16 + cc] = d;
+#pragma unroll
+    for (uint32_t j = 0; j < 2; j++) {
+        u32x2 w = {v[2 * j], v[2 * j + 1]};
+        if (S::ACT_PERM == 1)  // even bytes, then odd bytes
+            w = u32x2{__builtin_amdgcn_perm(v[2 * j + 1], v[2 * j], 0x06040200u), __builtin_amdgcn_perm(v[2 * j + 1], v[2 * j], 0x07050301u)};
+        if constexpr (S::ACT_PERM == 2) {
+            // weights j and j + 16 share a byte: k-slot q holds token bytes 4q .. 4q + 3, then 16 + 4q .. 16 + 4q + 3
+#pragma unroll
+            for (uint32_t i = 0; i < 2; i++)
+                *reinterpret_cast<uint32_t *>(L.A + (size_t)unit * SKINNY_UNIT + ((2 * j + i) * 16 + cc) * 8 + 4 * half) = w[i];
+        } else {
+            *reinterpret_cast<u32x2 *>(L.A + (size_t)unit * SKINNY_UNIT + ((2 * half + j) * 16 + cc) * 8) = w;
+        }
+    }
+    L.D[unit * 16 + cc] = d;  // (both halves: the same value)
 }
 
 // One step (two super-blocks of the wave's rows, their bytes in the strip) against the tokens whose blocks start at
@@ -455,7 +476,7 @@ __device__ __forceinline__ void skinny_step(uint8_t *const strip, float *const d
             for (int t = 0; t < TT; t++) {
                 if (TT == 1 || t < (int)tiles_here) {
                     const uint32_t e = (b0 + s) * TT + t;
-                    const u32x2 av = *reinterpret_cast<const u32x2 *>(L.A + ((size_t)e * 64 + lane) * 8);
+                    const u32x2 av = *reinterpret_cast<const u32x2 *>(L.A + (size_t)e * SKINNY_UNIT + lane * 8);
                     const long a = (long)(((uint64_t)av[1] << 32) | av[0]);
                     const v4f32 da = *reinterpret_cast<const v4f32 *>(L.D + (size_t)e * 16 + 4 * q);
 #pragma unroll
@@ -534,9 +555,9 @@ __device__ __forceinline__ void gemm_skinny_body(
     // ---- a chunk's tokens: their Q8_0 blocks (34 bytes: f16 scale, 32 int8) from the caller's rows into registers
     // (requested a chunk ahead, in flight while the last chunk is computed), from there into LDS in operand order,
     // with what gemm_prep_acts would have made of them: the bytes of each 8 in the format's order, the scale as
-    // fp32, P = d * sum(q) (exact integer sum, one rounding).  Thread (cc, qq) of a 64-thread unit takes bytes
-    // 8 qq .. 8 qq + 7 of token cc's block; token rows past the group's end read as zeros. ----
-    constexpr uint32_t KA = (nblk_max * TT * 64 + THREADS - 1) / THREADS;
+    // fp32, P = d * sum(q) (exact integer sum, one rounding).  64 threads take a pair of blocks of a tile's sixteen tokens, half
+    // a block each; token rows past the group's end read as zeros. ----
+    constexpr uint32_t KA = (nblk_max / 2 * TT * 64 + THREADS - 1) / THREADS;
     const size_t arow = (size_t)(k / 32) * Q8_BLOCK_BYTES;
     static_assert(SPREAD_LOG == 0 || TT == 2, "spread slots: the second token tile");
     constexpr uint32_t DEAD_SLOTS = (1u << SPREAD_LOG) - 1;  // the second tile's slot holds a token where slot & DEAD_SLOTS == 0
@@ -545,37 +566,33 @@ __device__ __forceinline__ void gemm_skinny_body(
         if (SPREAD_LOG != 0 && t == 1) return (slot & DEAD_SLOTS) ? tok_end : tokb + 16 + (slot >> SPREAD_LOG);
         return tokb + 16 * t + slot;
     };
-    u32x2 tokA[KA];
-    uint32_t tokD[KA];
+    SkinnyToken tokA[KA];
     auto load_tokens = [&](uint32_t sb0, uint32_t nblk) {
-        const uint32_t total = nblk * TT * 64;
+        const uint32_t total = nblk / 2 * TT * 64;
 #pragma unroll
         for (uint32_t i = 0; i < KA; i++) {
             const uint32_t idx = threadIdx.x + i * THREADS;
-            const uint32_t l = idx & 63, t = (idx >> 6) % TT, b = (idx >> 6) / TT;
-            const uint32_t cc = l >> 2, qq = l & 3, tok = token_of(t, cc);
-            tokA[i] = u32x2{0, 0};
-            tokD[i] = 0;
+            // a pair of blocks of the tile's sixteen tokens at a time, four threads each
+            const uint32_t l = idx & 63, t = (idx >> 6) % TT, b = (idx >> 6) / TT * 2;  // b: the pair's first block
+            const uint32_t tok = token_of(t, l >> 2);
+            tokA[i] = SkinnyToken{u32x4{0, 0, 0, 0}, 0};
             // an odd number of super-blocks: the last step's strip holds the last two super-blocks, the one before the
             // last (done by the step before) in its first half -- that half meets zeros, the second the last one's tokens
             uint32_t sbi = sb0 + (b >> 3);
             const bool dead = odd_super && sbi == n_super - 1;
             if (odd_super && sbi == n_super) sbi = n_super - 1;
-            if (idx < total && tok < tok_end && !dead) {
-                const uint8_t *blk = A + (size_t)tok * arow + (size_t)(sbi * 8 + (b & 7)) * Q8_BLOCK_BYTES;
-                tokA[i] = ld8(blk + 2 + 8 * qq);
-                tokD[i] = ld2(blk);
-            }
+            if (idx < total && tok < tok_end && !dead)
+                tokA[i] = skinny_get_token(A + (size_t)tok * arow + (size_t)(sbi * 8 + (b & 7)) * Q8_BLOCK_BYTES, l);
         }
     };
     auto store_tokens = [&](uint32_t nblk) {
-        const uint32_t total = nblk * TT * 64;
+        const uint32_t total = nblk / 2 * TT * 64;
 #pragma unroll
         for (uint32_t i = 0; i < KA; i++) {
             const uint32_t idx = threadIdx.x + i * THREADS;
             if (idx >= total) continue;  // whole waves: total and THREADS are multiples of 64
-            const uint32_t l = idx & 63, cc = l >> 2, qq = l & 3;
-            skinny_put_token<F>(tokA[i], h2f(tokD[i]), idx >> 6, cc, qq, L);
+            const uint32_t l = idx & 63, t = (idx >> 6) % TT, b = (idx >> 6) / TT * 2;
+            skinny_put_token<F>(tokA[i], (b + ((l >> 1) & 1)) * TT + t, l >> 2, l, L);
         }
     };
 
@@ -727,32 +744,30 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     load_step(stage0, blockIdx.x * RW + rw);
     load_step(stage1, blockIdx.x * RW + stride + rw);
 
-    // (a loop, not unrolled: a short launch spends much of its time fetching instructions for the first time; with all of a
-    // thread's blocks in one batch 1024 x 4096 takes 13.9 us against 11)
+    // (a loop, not unrolled: a short launch spends much of its time fetching instructions for the first time; with all eight half
+    // blocks of a thread in one batch 1024 x 4096 takes 0.3 us longer.  Sixteen threads read a token's super-block, 272 bytes that
+    // lie in three lines: 4096 x 4096 7.8 us against 8.6 with four threads to each of sixteen tokens)
     const size_t arow = (size_t)(k / 32) * Q8_BLOCK_BYTES;
-    const uint32_t total = steps * 16 * 64, tok = (threadIdx.x & 63) >> 2, qq = threadIdx.x & 3;
-    constexpr uint32_t TB = 8;  // blocks of a thread in flight
+    const uint32_t loads = steps * 8, lt = threadIdx.x & 63;  // four tokens of a super-block at a time, sixteen threads each
+    constexpr uint32_t TB = 4;  // half blocks of a thread in flight
 #pragma unroll 1
-    for (uint32_t base = threadIdx.x >> 6; base < total / 64; base += 8 * TB) {
-        u32x2 qv[TB];
-        uint32_t dv[TB];
+    for (uint32_t base = threadIdx.x >> 6; base < loads; base += 8 * TB) {
+        SkinnyToken tk[TB];
 #pragma unroll
         for (uint32_t i = 0; i < TB; i++) {
-            const uint32_t b = base + 8 * i;
-            uint32_t sbi = b >> 3;
+            const uint32_t at = base + 8 * i, tok = 4 * (at & 3) + (lt >> 4);
+            uint32_t sbi = at >> 2;
             const bool dead = odd_super && sbi == n_super - 1;
             if (odd_super && sbi == n_super) sbi = n_super - 1;
-            qv[i] = u32x2{0, 0};
-            dv[i] = 0;
-            if (b < total / 64 && tok < m && !dead) {
-                const uint8_t *blk = A + (size_t)tok * arow + (size_t)(sbi * 8 + (b & 7)) * Q8_BLOCK_BYTES;
-                qv[i] = ld8(blk + 2 + 8 * qq);
-                dv[i] = ld2(blk);
-            }
+            tk[i] = SkinnyToken{u32x4{0, 0, 0, 0}, 0};
+            if (at < loads && tok < m && !dead)
+                tk[i] = skinny_get_token(A + (size_t)tok * arow + (size_t)(sbi * 8 + 2 * ((lt >> 2) & 3)) * Q8_BLOCK_BYTES, lt);
         }
 #pragma unroll
-        for (uint32_t i = 0; i < TB; i++)
-            if (base + 8 * i < total / 64) skinny_put_token<F>(qv[i], h2f(dv[i]), base + 8 * i, tok, qq, L);
+        for (uint32_t i = 0; i < TB; i++) {
+            const uint32_t at = base + 8 * i;
+            if (at < loads) skinny_put_token<F>(tk[i], 8 * (at >> 2) + ((lt >> 1) & 7), 4 * (at & 3) + (lt >> 4), lt, L);
+        }
     }
     __syncthreads();
 
