@@ -21,7 +21,10 @@ hipError_t launch_dequant(uint32_t type, const uint8_t *blocks, size_t n_blocks,
 // its own copy at its own address until the process ends; host code reaches it only through the address that
 // hipGetSymbolAddress returned for that device (static_scratch_ptr), never through this name.
 constexpr size_t STATIC_SCRATCH_BYTES = (size_t)16 << 20;
-static __device__ __align__(256) uint8_t scratch[STATIC_SCRATCH_BYTES];
+// ... and room for the sums that the f16 kernel's even deal exchanges (128 KB twice for each of 256 compute units), which a
+// call's size for that limit leaves out: what ran with 16 MiB runs, and in the kernels of the workspace form
+constexpr size_t STATIC_DEAL_BYTES = (size_t)64 << 20;
+static __device__ __align__(256) uint8_t scratch[STATIC_DEAL_BYTES];
 
 namespace {
 
@@ -999,13 +1002,14 @@ static int gemm_dev(uint32_t type, const uint8_t *d_weights, const uint8_t *d_ac
     // a few rows fewer still pay on the few-token kernel, if the caller's workspace has the room (without one the
     // call would have to take the library's scratch and wait for the stream: the GEMV launches stay)
     if (!tiles && d_workspace && !d_sums && oxq::gemm_few_rows_pay(type, (uint32_t)m, (uint32_t)n, (uint32_t)k) &&
-        workspace_bytes >= oxq::gemm_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) &&
+        workspace_bytes >= oxq::gemm_workspace_least_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) &&
         (reinterpret_cast<uintptr_t>(d_workspace) & 255) == 0)
         tiles = true;
     ga.by_rows = !tiles;
     const size_t need = tiles ? oxq::gemm_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) : 0;
     if (need && d_workspace) {
-        if (workspace_bytes < need) return fail(OXQ_ERR_BUFFER_TOO_SMALL, need, workspace_bytes, "workspace too small");
+        if (workspace_bytes < oxq::gemm_workspace_least_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type))
+            return fail(OXQ_ERR_BUFFER_TOO_SMALL, need, workspace_bytes, "workspace too small");
         if (reinterpret_cast<uintptr_t>(d_workspace) & 255)
             return fail(OXQ_ERR_KERNEL, 256, reinterpret_cast<uintptr_t>(d_workspace) & 255, "workspace must be 256-byte aligned");
         ga.workspace = (uint8_t *)d_workspace;
@@ -1052,8 +1056,8 @@ int oxq_gemm_q8_static_dev(uint32_t type, const uint8_t *d_weights, const uint8_
     if (m == 0 || n == 0 || k == 0) return OXQ_OK;
     const bool tiles = oxq::gemm_uses_tiles(type, (uint32_t)m, (uint32_t)n, (uint32_t)k) ||
                        (oxq::gemm_few_rows_pay(type, (uint32_t)m, (uint32_t)n, (uint32_t)k) &&
-                        oxq::gemm_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) <= STATIC_SCRATCH_BYTES);
-    const size_t need = tiles ? oxq::gemm_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) : 0;
+                        oxq::gemm_workspace_least_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) <= STATIC_SCRATCH_BYTES);
+    const size_t need = tiles ? oxq::gemm_workspace_least_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) : 0;
     if (need > STATIC_SCRATCH_BYTES)
         return fail(OXQ_ERR_BUFFER_TOO_SMALL, need, STATIC_SCRATCH_BYTES,
                     "shape needs more workspace than the static scratch holds: use oxq_gemm_q8_dev with a workspace");
@@ -1062,7 +1066,7 @@ int oxq_gemm_q8_static_dev(uint32_t type, const uint8_t *d_weights, const uint8_
     ga.A = d_acts_q8;
     ga.out = d_out;
     ga.sums = nullptr;
-    ga.workspace_bytes = tiles ? STATIC_SCRATCH_BYTES : 0;
+    ga.workspace_bytes = tiles ? STATIC_DEAL_BYTES : 0;
     ga.workspace = tiles ? static_scratch_ptr[device] : nullptr;    // every byte the tile kernel reads is written
     ga.by_rows = !tiles;                                            // by the preparation kernel of this same call
     ga.m = (uint32_t)m;

@@ -85,6 +85,11 @@ size_t gemm_grouped_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t
     return planes + gemm_grouped_partial_bytes(type, m, n, k);
 }
 size_t gemm_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t type) {
+    const size_t least = gemm_workspace_least_bytes(m, k, n, type);
+    const size_t deal = gemm_f16_deal_pays(type, m, n, k) ? gemm_f16_deal_bytes() : 0;
+    return least > deal ? least : deal;
+}
+size_t gemm_workspace_least_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t type) {
     const size_t planes = (gemm_planes_bytes(m, k) + 255) & ~(size_t)255;
     const size_t tiles = planes + gemm_partial_bytes(type, m, n, k);
     // the prefill kernel lays its own planes (f16 token operands) over the head of the same workspace; the size is
@@ -99,7 +104,7 @@ size_t gemm_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t type) {
 // groups 194 against 172, 168 a tie, 128 and fewer far behind (the tile kernel's smaller tiles spread better).
 // And its token tiles must be mostly full: a work group costs the same with 32 of its 128 token rows in use (128256 x
 // 4096: 32 / 64 / 96 / 128 tokens 208 / 220 / 234 / 245 us against 115 / 185 / 275 / 285 on the tile kernel).
-static bool gemm_prefill_pays(uint32_t m, uint32_t n) {
+bool gemm_prefill_pays(uint32_t m, uint32_t n) {
     const uint64_t token_tiles = (m + 127) / 128;
     const uint64_t wgs = token_tiles * ((n + 255) / 256), cus = device_cus();
     const uint64_t rounds = (wgs + cus - 1) / cus;
@@ -194,6 +199,12 @@ hipError_t launch_gemm_q8(uint32_t type, const GemmArgs &a, hipStream_t stream) 
         return gemm_by_rows(type, a, stream);
     }
     const int variant = g_gemm_variant.load(std::memory_order_relaxed);
+    // prompts whose grids of whole tiles lie between the rounds of the chip: the f16 kernel on an even deal
+    if (!a.offsets && !a.sums && ((variant == 0 && gemm_f16_deal_pays(type, a.m, a.n, a.k)) || variant == 303) &&
+        a.workspace_bytes >= gemm_f16_deal_bytes()) {
+        const hipError_t e = launch_gemm_f16_deal(type, a, reinterpret_cast<float *>(a.workspace), stream);
+        if (e != hipErrorNotSupported) return e;
+    }
     // many token rows of a format whose scaled weights are exact in f16: the prefill kernel (oxq_gemm_prefill.hip).
     // The debug dump of the integer sums stays on the tile kernel; the dump of the scaled sums is this kernel's.
     if (!a.offsets && (variant == 0 || variant == 300) && (!a.sums || a.scaled_sums) &&
@@ -225,7 +236,7 @@ hipError_t launch_gemm_q8(uint32_t type, const GemmArgs &a, hipStream_t stream) 
     const int perm = act_perm(type);
     TilePlan plan = {q8t, P, da16, mpad};
     if (!a.offsets && gemm_partial_bytes(type, a.m, a.n, a.k) &&
-        a.workspace_bytes >= gemm_workspace_bytes(a.m, a.k, a.n, type))
+        a.workspace_bytes >= gemm_workspace_least_bytes(a.m, a.k, a.n, type))
         plan.partial = reinterpret_cast<float *>(a.workspace + ((gemm_planes_bytes(a.m, a.k) + 255) & ~(size_t)255));
     if (a.offsets && gemm_grouped_partial_bytes(type, a.m, a.n, a.k) &&
         a.workspace_bytes >= gemm_grouped_workspace_bytes(a.m, a.k, a.n, type))

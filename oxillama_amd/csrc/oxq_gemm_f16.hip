@@ -17,6 +17,14 @@
 // read; the block sums P of the zero-point term are formed on the way.  That is about 3.5 vector instructions per step of
 // 27 (the prefill kernel's preparation launch is 6 us at 512 x 4096 and reads and writes the tokens once more).
 //
+// The even deal (DEAL; the large shape): whole tiles cost a round of the chip what the fullest compute unit has, and most
+// prompts' grids lie between rounds (333 rows on 11008 weight rows: 129 tiles for 256 compute units).  Here a work group per
+// compute unit takes the same number of whole tiles and then a run of (tile, super-block) units of the rest; a tile that
+// several have runs of is added up by a second launch, in the order of k.  What it costs: a ramp of the pipeline per run and 128 KB
+// of sums, 32 to 64 MB written together at the end and read by the second launch (8 to 11 us): 128 x 4096 x 14336, Q4_K,
+// runs of four super-blocks, 36 us + 8, where whole tiles take 5.8 per super-block.  Storing the sums past the caches: no gain
+// (333 x 11008 x 4096 77 us against 75).
+//
 // Shapes: MT token tiles of 32 against RW waves of 32 rows, KS parts of k; eight waves, one work group per compute unit.
 //   (4, 8, 1)  128 tokens x 256 rows: the least unpacking and staging per result
 //   (2, 4, 2)  64 tokens x 128 rows, each half of k by four waves (their sums meet in LDS): four times the work groups,
@@ -228,11 +236,12 @@ struct F16Q6K {
     }
 };
 
-template <class F, int MT, int RW, int KS>
+template <class F, int MT, int RW, int KS, bool DEAL>
 __global__ __launch_bounds__(64 * RW * KS) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_f16_kernel(
     const uint8_t *__restrict__ W, const uint8_t *__restrict__ A, float *__restrict__ out, uint32_t m, uint32_t n, uint32_t k,
-    int accumulate, const float *__restrict__ bias, uint32_t m_tiles, uint32_t n_tiles) {
+    int accumulate, const float *__restrict__ bias, uint32_t m_tiles, uint32_t n_tiles, float *__restrict__ partial) {
     static_assert(MT * 2 == RW, "one 16-byte piece of a stage per thread");
+    static_assert(!DEAL || KS == 1, "the deal is over whole work groups");
     static_assert(MT % KS == 0, "the parts of k share the token tiles out at the end");
     constexpr uint32_t TOK = 32 * MT, ROWS = 32 * RW, STAGE = TOK * 128;
     constexpr int NS = 8 * MT;  // steps of a super-block
@@ -252,11 +261,37 @@ __global__ __launch_bounds__(64 * RW * KS) __attribute__((amdgpu_waves_per_eu(2,
     auto &pl = pl_all[part];
     auto &tab = tab_all[part];
     // this part's super-blocks, the first part's the longer run
-    const uint32_t per_part = (n_super + KS - 1) / KS, blk0 = part * per_part, nblk = min(blk0 + per_part, n_super);
+    const uint32_t per_part = (n_super + KS - 1) / KS;
+    uint32_t blk0 = part * per_part, nblk = min(blk0 + per_part, n_super);
     const uint32_t c = lane & 31, h = lane >> 5;
 
     uint32_t m_tile, n_tile;
-    if (!tile_order_at(blockIdx.x, gridDim.x, m_tiles, n_tiles, m_tile, n_tile)) return;  // the whole work group
+    // DEAL: whole tiles first, as many to every work group, the rest of them as runs of super-blocks
+    uint32_t tile = 0, whole = 0, unit = 0, unit_end = 0, slot = 0;
+    bool dealt = false;
+    if constexpr (DEAL) {
+        const uint32_t rank = deal_rank(blockIdx.x, gridDim.x), rounds = m_tiles * n_tiles / gridDim.x;
+        const DealRange r = deal_range(rank, gridDim.x, (m_tiles * n_tiles - rounds * gridDim.x) * n_super);
+        tile = rank * rounds, whole = rounds, unit = r.begin, unit_end = r.end, slot = 2 * rank;
+        if (whole == 0 && unit == unit_end) return;
+    } else {
+        if (!tile_order_at(blockIdx.x, gridDim.x, m_tiles, n_tiles, m_tile, n_tile)) return;  // the whole work group
+    }
+    do {  // (DEAL: the work group's run of a tile, then its run of the next one)
+    if constexpr (DEAL) {
+        uint32_t t = tile;
+        if (whole) {
+            blk0 = 0, nblk = n_super;
+            tile++, whole--;
+        } else {
+            t = unit / n_super;
+            blk0 = unit - t * n_super, nblk = min(n_super, blk0 + (unit_end - unit));
+            unit += nblk - blk0;
+            dealt = true;
+            t += m_tiles * n_tiles / gridDim.x * gridDim.x;
+        }
+        n_tile = t / m_tiles, m_tile = t - n_tile * m_tiles;
+    }
     const uint32_t m_wg = m_tile * TOK, n_wg = n_tile * ROWS, n_wave = n_wg + 32 * wave;
 
     const uint32_t row_bytes = n_super * F::BLOCK;
@@ -488,6 +523,19 @@ __global__ __launch_bounds__(64 * RW * KS) __attribute__((amdgpu_waves_per_eu(2,
             }
     }
 
+    if constexpr (DEAL) {
+        if (nblk - blk0 != n_super) {  // a tile that others have runs of: the sums as they lie in the registers
+            v4f *const to = reinterpret_cast<v4f *>(partial) + (size_t)slot * (TOK * ROWS / 4) + wave * (MT * 256) + lane;
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++)
+#pragma unroll
+                for (int a = 0; a < 4 && m_wg + 32 * mt < m; a++)
+                    to[(mt * 4 + a) * 64] = v4f{y[mt][4 * a], y[mt][4 * a + 1], y[mt][4 * a + 2], y[mt][4 * a + 3]};
+            slot |= 1;
+            continue;
+        }
+        if (dealt) slot |= 1;
+    }
     // ---- store: lane (token c, half h) holds rows 8a + 4h + 0..3 of its wave's 32, for MT token tiles -----------------
     const bool vec4 = (n & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 &&
                       (!bias || (reinterpret_cast<uintptr_t>(bias) & 15) == 0);
@@ -517,6 +565,67 @@ __global__ __launch_bounds__(64 * RW * KS) __attribute__((amdgpu_waves_per_eu(2,
             }
         }
     }
+    } while (DEAL && (whole || unit < unit_end));
+}
+
+// The sums of the tiles that several work groups had runs of, added in the order of k: a work group here takes the 32 rows
+// of one wave against one token tile, a thread four rows of a token, so that a token's 128 bytes are stored together.
+template <int MT, int RW>
+__global__ __launch_bounds__(256) void gemm_f16_deal_sum(const float *__restrict__ partial, float *__restrict__ out, uint32_t m,
+                                                         uint32_t n, uint32_t n_super, int accumulate,
+                                                         const float *__restrict__ bias, uint32_t m_tiles, uint32_t n_tiles,
+                                                         uint32_t groups) {
+    constexpr uint32_t TOK = 32 * MT, ROWS = 32 * RW;
+    const uint32_t tile = blockIdx.x / (RW * MT), at = blockIdx.x % (RW * MT), wave = at / MT, mt = at % MT;
+    const uint32_t tile0 = m_tiles * n_tiles / groups * groups;  // the whole rounds before the deal
+    const uint32_t units = (m_tiles * n_tiles - tile0) * n_super;
+    const uint32_t first = deal_owner(tile * n_super, groups, units), last = deal_owner(tile * n_super + n_super - 1, groups, units);
+    if (first == last) return;  // stored by the one work group that had all of it
+    const uint32_t c = threadIdx.x >> 3, piece = threadIdx.x & 7;  // token c, rows 4 piece ..: register group piece / 2, half piece % 2
+    const uint32_t n_tile = (tile0 + tile) / m_tiles, t = (tile0 + tile - n_tile * m_tiles) * TOK + mt * 32 + c, row = n_tile * ROWS + wave * 32 + piece * 4;
+    if (t >= m || row >= n) return;
+    const v4f *const p = reinterpret_cast<const v4f *>(partial) + (wave * MT + mt) * 256 + (piece >> 1) * 64 + (piece & 1) * 32 + c;
+    v4f y = p[(size_t)deal_slot(first, tile * n_super, groups, units) * (TOK * ROWS / 4)];
+    // (behind the first a work group's run began inside this tile: its first slot.  Four loads in flight, added in order)
+    for (uint32_t w = first + 1; w <= last; w += 4) {
+        v4f v[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) v[i] = p[(size_t)(2 * min(w + i, last)) * (TOK * ROWS / 4)];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++)
+            if (w + i <= last) y = y + v[i];
+    }
+    float *const o = out + (size_t)t * n + row;
+    if ((n & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 && (!bias || (reinterpret_cast<uintptr_t>(bias) & 15) == 0)) {
+        if (accumulate)
+            y = *reinterpret_cast<const v4f *>(o) + y;
+        else if (bias)
+            y = y + *reinterpret_cast<const v4f *>(bias + row);
+        *reinterpret_cast<v4f *>(o) = y;
+    } else {
+        for (int b = 0; b < 4; b++)
+            if (row + b < n) o[b] = accumulate ? o[b] + y[b] : bias ? y[b] + bias[row + b] : y[b];
+    }
+}
+
+// One work group per compute unit, the same number on each XCD.
+uint32_t f16_deal_groups() { return device_cus() < 16 ? 8 : device_cus() / 8 * 8; }
+
+template <class F>
+hipError_t launch_f16_deal(const GemmArgs &a, float *partial, hipStream_t stream) {
+    constexpr int MT = 4, RW = 8;
+    const uint32_t m_tiles = (a.m + 32 * MT - 1) / (32 * MT), n_tiles = (a.n + 32 * RW - 1) / (32 * RW), groups = f16_deal_groups();
+    // (every run has a unit, so that the work groups between a tile's first and last have all left sums)
+    const uint32_t rest = m_tiles * n_tiles % groups;
+    if (rest && (uint64_t)rest * (a.k / 256) < groups) return hipErrorNotSupported;
+    note_launch("gemm_f16_deal_kernel", F::TYPE, MT, RW, 1, 0, groups, 1, 64 * RW);
+    hipLaunchKernelGGL((gemm_f16_kernel<F, MT, RW, 1, true>), dim3(groups), dim3(64 * RW), 0, stream, a.W, a.A, a.out, a.m, a.n,
+                       a.k, a.accumulate, a.bias, m_tiles, n_tiles, partial);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || m_tiles * n_tiles % groups == 0) return e;
+    hipLaunchKernelGGL((gemm_f16_deal_sum<MT, RW>), dim3(m_tiles * n_tiles % groups * MT * RW), dim3(256), 0, stream, partial, a.out, a.m,
+                       a.n, a.k / 256, a.accumulate, a.bias, m_tiles, n_tiles, groups);
+    return hipGetLastError();
 }
 
 template <class F, int MT, int RW, int KS>
@@ -524,8 +633,8 @@ hipError_t launch_f16_shape(const GemmArgs &a, hipStream_t stream) {
     const uint32_t m_tiles = (a.m + 32 * MT - 1) / (32 * MT), n_tiles = (a.n + 32 * RW - 1) / (32 * RW);
     const dim3 grid(tile_order_grid(m_tiles, n_tiles));
     note_launch("gemm_f16_kernel", F::TYPE, MT, RW, KS, 0, grid.x, 1, 64 * RW * KS);
-    hipLaunchKernelGGL((gemm_f16_kernel<F, MT, RW, KS>), grid, dim3(64 * RW * KS), 0, stream, a.W, a.A, a.out, a.m, a.n, a.k,
-                       a.accumulate, a.bias, m_tiles, n_tiles);
+    hipLaunchKernelGGL((gemm_f16_kernel<F, MT, RW, KS, false>), grid, dim3(64 * RW * KS), 0, stream, a.W, a.A, a.out, a.m, a.n, a.k,
+                       a.accumulate, a.bias, m_tiles, n_tiles, nullptr);
     return hipGetLastError();
 }
 
@@ -573,6 +682,60 @@ int gemm_f16_shape(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
     }
     if (type == OXQ_TYPE_Q5_K && large_ok && 100 * large >= 96 * rl * cus && (rl == 1 || k >= 8192)) return 1;
     return small_ok && rs == 1 && 100 * small >= 96 * cus && m > 384 ? 2 : 0;
+}
+
+// Whether a call takes the even deal: where its time, estimated, is less than that of the kernel that the call would take
+// otherwise.  Both are lines through measured times (294 calls with 40 to 2048 rows, 768 to 28672 weight rows and columns):
+//   the deal     17 / 20 / 21 us (Q4_K / Q5_K / Q6_K) for the ramp, the exchange of up to 64 MB of sums and the second launch,
+//                6.9 / 7.4 / 9.5 per super-block of the longest run, 8 where whole tiles go before the runs; nine calls in ten within 10 %
+//   the others   a time per round of the chip and 4096 columns, the least that was measured for the shape (the calls with
+//                short rows and partly used tiles take up to a third more): the prefill kernel 90, this kernel's whole
+//                tiles 100 / 122 (Q5_K / Q6_K) and 38 / 43 / 45.6 (small), the tile kernel 57 / 57 / 88 (128 x 128 tiles), 30 / 33
+//                / 53 (128 x 64), 33 / 37.5 / 50 (64 x 128), 9.7 / 11.3 / 14.7 (64 x 32, k split)
+// so that the line errs towards the kernels with whole tiles.  On those 294 calls the mean is 8 % less, the best choice of
+// each 10 % less, and the worst of the calls that change loses 3 %.  us, before and now: Q4_K 333 x 11008 x 4096 93 and 75, 1100 x
+// 4096 x 14336 384 and 225, 512 x 4096 x 14336 126 and 104; Q5_K 333 x 11008 x 4096 105 and 82; Q6_K 333 x 4096 x 11008 135 and 97, 768
+// x 4096 x 14336 307 and 209, 1100 x 4096 x 4096 143 and 104.  Q4_K 333 x 4096 x 4096, where runs are three super-blocks, stays (33, 38).
+bool gemm_f16_deal_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
+    if (!gemm_f16_supported(type, m, n, k) || m <= 64) return false;  // (a token tile half empty, against 32-token tiles)
+    const int f = type == OXQ_TYPE_Q4_K ? 0 : type == OXQ_TYPE_Q5_K ? 1 : 2;
+    const uint64_t groups = f16_deal_groups(), cus = device_cus(), n_super = k / 256;
+    auto tiles_of = [&](uint32_t t, uint32_t r) { return (uint64_t)((m + t - 1) / t) * ((n + r - 1) / r); };
+    const uint64_t tiles = tiles_of(128, 256), whole = tiles / groups, rest = tiles % groups;
+    if (rest * n_super < groups) return false;
+    // tenths of a microsecond
+    static constexpr uint32_t RAMP[3] = {175, 203, 209}, RUN[3] = {69, 74, 95};
+    const uint64_t deal = RAMP[f] + RUN[f] * (whole * n_super + (rest * n_super + groups - 1) / groups) + (whole ? 80 : 0);
+    static constexpr uint32_t PREFILL = 900, LARGE[3] = {0, 1000, 1220}, SMALL[3] = {380, 430, 456}, T128X128[3] = {570, 570, 880},
+                              T128X64[3] = {300, 330, 530}, T64X128[3] = {330, 375, 500}, T64X32[3] = {97, 113, 147};
+    uint64_t per_round, wgs;
+    if (gemm_prefill_supported(type, m, n, k) && gemm_prefill_pays(m, n)) {
+        per_round = PREFILL, wgs = tiles;
+    } else if (const int shape = gemm_f16_shape(type, m, n, k)) {
+        per_round = shape == 1 ? LARGE[f] : SMALL[f], wgs = shape == 1 ? tiles : tiles_of(64, 128);
+    } else if (m > 384 && k <= 16384 && tiles_of(128, 64) >= cus) {  // (the tile kernel's shapes: launch_tiles)
+        wgs = tiles_of(128, 128);
+        const bool square = 2 * wgs >= 3 * cus || (2 * wgs > cus && wgs <= cus && (f != 0 || k >= 8192));
+        per_round = square ? T128X128[f] : T128X64[f];
+        if (!square) wgs = tiles_of(128, 64);
+    } else if (k <= 32768) {
+        const bool wide = !(m > 384 && k <= 16384) && 4 * tiles_of(64, 128) >= 7 * cus;
+        per_round = wide ? T64X128[f] : T64X32[f], wgs = wide ? tiles_of(64, 128) : tiles_of(64, 32);
+    } else {
+        return false;
+    }
+    return deal * 4096 < per_round * ((wgs + cus - 1) / cus) * k;
+}
+
+size_t gemm_f16_deal_bytes() { return (size_t)2 * f16_deal_groups() * (128 * 256 * sizeof(float)); }
+
+hipError_t launch_gemm_f16_deal(uint32_t type, const GemmArgs &a, float *partial, hipStream_t stream) {
+    if (!gemm_f16_supported(type, a.m, a.n, a.k) || a.offsets || a.sums) return hipErrorNotSupported;
+    switch (type) {
+    case OXQ_TYPE_Q4_K: return launch_f16_deal<F16Q4K>(a, partial, stream);
+    case OXQ_TYPE_Q5_K: return launch_f16_deal<F16Q5K>(a, partial, stream);
+    default: return launch_f16_deal<F16Q6K>(a, partial, stream);
+    }
 }
 
 hipError_t launch_gemm_f16(uint32_t type, const GemmArgs &a, int shape, hipStream_t stream) {

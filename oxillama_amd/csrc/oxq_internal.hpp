@@ -221,7 +221,10 @@ hipError_t launch_gemm_q8(uint32_t type, const GemmArgs &a, hipStream_t stream);
 // Device scratch the tile kernel needs for m tokens of k columns (activation re-layout).
 // With n and the format: plus, for a matmul of at most 32 token rows that the few-token kernel would split over k,
 // the room for its per-split sums (behind the re-tiled activations, 256-byte aligned).
+// And for the f16 kernel's even deal the sums of shared tiles, at the head.  The least size is the one without them: a
+// call with a workspace in between takes the kernels that need no more.
 size_t gemm_workspace_bytes(uint32_t m, uint32_t k, uint32_t n = 0, uint32_t type = 0);
+size_t gemm_workspace_least_bytes(uint32_t m, uint32_t k, uint32_t n = 0, uint32_t type = 0);
 // ... of the grouped form: the planes, plus room for two per-split sums of [m x n] where the few-token kernel may
 // split an expert's k in two (Q4_K / IQ4_XS, k a multiple of 1024, at most 8192 rows per expert).
 size_t gemm_grouped_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t type);
@@ -237,6 +240,12 @@ hipError_t launch_gemm_prefill(uint32_t type, const GemmArgs &a, hipStream_t str
 bool gemm_f16_supported(uint32_t type, uint32_t m, uint32_t n, uint32_t k);
 int gemm_f16_shape(uint32_t type, uint32_t m, uint32_t n, uint32_t k);
 hipError_t launch_gemm_f16(uint32_t type, const GemmArgs &a, int shape, hipStream_t stream);
+// ... in its large shape with the (tile, part of k) steps dealt evenly to the compute units: whether a call should take it,
+// the room for the sums of the tiles that several work groups share, the two launches.
+bool gemm_prefill_pays(uint32_t m, uint32_t n);  // where a plain Q4_K matmul takes the prefill kernel
+bool gemm_f16_deal_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k);
+size_t gemm_f16_deal_bytes();
+hipError_t launch_gemm_f16_deal(uint32_t type, const GemmArgs &a, float *partial, hipStream_t stream);
 // Tuning knobs (oxq_tuning.h), read once per call.
 extern std::atomic<int> g_gemm_variant;              // 0 = default tile shape
 extern std::atomic<uint32_t> g_gemm_tile_min_rows;   // 0 = default threshold

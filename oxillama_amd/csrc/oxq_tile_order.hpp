@@ -26,4 +26,23 @@ OXQ_HOST_DEVICE bool tile_order_at(uint32_t block, uint32_t grid, uint32_t m_til
     return n_tile < n_tiles;
 }
 
+// An even deal of units (a unit: one super-block of one tile, the tiles one after another) over as many work groups as there
+// are compute units: a work group takes a run of units, so that at most two of the tiles it meets are not all its own, the
+// first and the last of its run, and their sums go to its two slots.  Neighbouring runs sit on one XCD.
+struct DealRange {
+    uint32_t begin, end;
+};
+OXQ_HOST_DEVICE uint32_t deal_rank(uint32_t block, uint32_t groups) { return (block & 7) * (groups >> 3) + (block >> 3); }
+OXQ_HOST_DEVICE DealRange deal_range(uint32_t rank, uint32_t groups, uint32_t units) {
+    return DealRange{(uint32_t)((uint64_t)rank * units / groups), (uint32_t)((uint64_t)(rank + 1) * units / groups)};
+}
+// whose run holds this unit
+OXQ_HOST_DEVICE uint32_t deal_owner(uint32_t unit, uint32_t groups, uint32_t units) {
+    return (uint32_t)((((uint64_t)unit + 1) * groups - 1) / units);
+}
+// where work group `rank` leaves its sums of the tile whose first unit is tile_begin
+OXQ_HOST_DEVICE uint32_t deal_slot(uint32_t rank, uint32_t tile_begin, uint32_t groups, uint32_t units) {
+    return 2 * rank + (deal_range(rank, groups, units).begin < tile_begin ? 1 : 0);
+}
+
 }  // namespace oxq

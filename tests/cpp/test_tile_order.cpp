@@ -1,5 +1,6 @@
 // The order in which work groups take the tiles of a matmul: every tile once, and no XCD with more than an eighth of them
-// rounded up (ids are dealt round-robin to the 8 XCDs).
+// rounded up (ids are dealt round-robin to the 8 XCDs).  The even deal of (tile, part of k) units: every unit in one run, runs
+// that differ by one unit, and the sums of a shared tile where the kernel that adds them looks.
 #include <cstdio>
 #include <vector>
 
@@ -29,6 +30,44 @@ int main() {
                 failed++;
             }
         }
-    std::printf("%d grids, %d failed\n", grids, failed);
+    int deals = 0;
+    for (uint32_t groups : {8u, 240u, 256u})
+        for (uint32_t per_tile : {1u, 3u, 16u, 43u, 56u})
+            for (uint32_t tiles = 1; tiles <= 700; tiles += tiles < 20 ? 1 : 13) {
+                const uint32_t units = tiles * per_tile;
+                std::vector<uint32_t> rank_of(units, ~0u), slot_of(units, ~0u);  // slot: 2 * groups for a tile of one's own
+                std::vector<int> ranks(groups, 0);
+                bool ok = true;
+                for (uint32_t b = 0; b < groups; b++) {  // as the kernel walks them
+                    const uint32_t rank = oxq::deal_rank(b, groups);
+                    ok = ok && rank < groups && ranks[rank]++ == 0;
+                    const oxq::DealRange r = oxq::deal_range(rank, groups, units);
+                    ok = ok && r.end <= units && r.end - r.begin <= (units + groups - 1) / groups;
+                    uint32_t slot = 2 * rank;
+                    for (uint32_t u = r.begin; ok && u < r.end;) {
+                        const uint32_t lo = u % per_tile, left = r.end - u, hi = lo + left < per_tile ? lo + left : per_tile;
+                        for (uint32_t i = 0; i < hi - lo; i++) {
+                            ok = ok && rank_of[u + i] == ~0u;
+                            rank_of[u + i] = rank;
+                            slot_of[u + i] = hi - lo == per_tile ? 2 * groups : slot;
+                        }
+                        if (hi - lo != per_tile)  // no slot twice
+                            ok = ok && (slot == 2 * rank || u != r.begin) && (u == r.begin || u + (hi - lo) == r.end);
+                        slot |= 1;
+                        u += hi - lo;
+                    }
+                }
+                for (uint32_t u = 0; ok && u < units; u++) {
+                    const uint32_t begin = u / per_tile * per_tile, owner = oxq::deal_owner(u, groups, units);
+                    const bool shared = oxq::deal_owner(begin, groups, units) != oxq::deal_owner(begin + per_tile - 1, groups, units);
+                    ok = owner == rank_of[u] && slot_of[u] == (shared ? oxq::deal_slot(owner, begin, groups, units) : 2 * groups);
+                }
+                deals++;
+                if (!ok) {
+                    std::printf("%u tiles of %u units to %u work groups\n", tiles, per_tile, groups);
+                    failed++;
+                }
+            }
+    std::printf("%d grids, %d deals, %d failed\n", grids, deals, failed);
     return failed != 0;
 }

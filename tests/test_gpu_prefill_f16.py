@@ -308,3 +308,82 @@ def test_scaled_sums_errors(hip):
     kern = hip.HipKernel(O.Q4_K)
     with pytest.raises(hip.BufferTooSmall):
         kern.gemm_scaled_sums_dev(z, z, z, z, 4, 32, 256, z[:256])
+
+
+@pytest.mark.parametrize("shape", [(130, 300, 16384), (97, 1030, 14336), (257, 1283, 4608), (40, 256 * 288 - 3, 2048)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q5_K, O.Q6_K], ids=lambda t: O.NAMES[t])
+def test_f16_kernel_on_an_even_deal(hip, ref, tuning, t, shape):
+    """Runs of (tile, super-block) units: a unit each (4 tiles of 64 to 256 work groups), runs that cross tiles, a whole tile
+    before the run; tokens and rows past the edges.  The bars of the kernel's other shapes, the bias and accumulation bit for
+    bit, and too little room for the sums (or too few units) takes another kernel."""
+    if hip.device_info()["compute_units"] != 256:
+        pytest.skip("the runs are those of 256 compute units")
+    m, n, k = shape
+    say("f16 even deal", O.NAMES[t], shape)
+    tuning("gemm_variant", 303)
+    w = O.random_blocks(t, 40 + m, n, k)
+    x = synth.normal_f32(41 + n, m * k)
+    x[:k] *= 300.0
+    acts = ref.quantize_q8_0(x)
+    kern = hip.HipKernel(t)
+    ws = torch.full((64 << 20,), 255, dtype=torch.uint8, device="cuda")  # (NaNs wherever nothing is stored)
+    dw, da = torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda()
+    dy = torch.full((m + 1, n), 7.0, dtype=torch.float32, device="cuda")
+    kern.gemm_q8_dev(dw, da, dy, m, n, k, accumulate=False, workspace=ws)
+    torch.cuda.synchronize()
+    assert last_launch().startswith("gemm_f16_deal_kernel"), last_launch()
+    y = dy.cpu().numpy()
+    assert np.all(y[m] == 7.0)
+    rows = range(m) if n < 2000 else [0, 1, 31, 32, m - 1]
+    y_ref = oracle_rows(ref, t, w, acts, n, k, rows)
+    for r, want in zip(rows, y_ref):
+        err, scale = np.abs(y[r] - want).max(), np.abs(want).max()
+        assert err <= FP32_REL_TOL * scale, f"token {r}: max err {err:.3e} vs |y|inf {scale:.3e}"
+    dy2 = dy.clone()
+    kern.gemm_q8_dev(dw, da, dy2, m, n, k, accumulate=True, workspace=ws)
+    bias = torch.from_numpy(synth.normal_f32(93, n + 1)).cuda()
+    dy3 = torch.empty(m * n + 1, dtype=torch.float32, device="cuda")
+    for off in (0, 1):
+        linear.linear_forward_batch_dev(t, dw, da, dy3[off:off + m * n], m, n, k, d_bias=bias[off:off + n], workspace=ws)
+        torch.cuda.synchronize()
+        assert torch.equal(dy3[off:off + m * n].view(m, n), dy[:m] + bias[off:off + n])
+    assert torch.equal(dy2[:m], dy[:m] + dy[:m])
+    for small, width in ((ws[:-256], n), (ws, 100)):
+        kern.gemm_q8_dev(dw, da, dy2, m, width, k, accumulate=False, workspace=small)
+        assert not last_launch().startswith("gemm_f16_deal_kernel"), last_launch()
+    torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("t,m,n,k,deal", [
+    (O.Q4_K, 333, 4096, 14336, True), (O.Q4_K, 333, 4096, 4096, False), (O.Q5_K, 65, 28672, 4096, True),
+    (O.Q5_K, 64, 28672, 4096, False), (O.Q6_K, 200, 4096, 4096, False), (O.Q6_K, 200, 4096, 11008, True),
+    (O.Q6_K, 512, 14336, 4096, False)])
+def test_f16_even_deal_by_default(hip, ref, t, m, n, k, deal):
+    """Which calls take the even deal; with a workspace that has no room for it, of the size without it, another kernel
+    serves; the static scratch gives the workspace form's bits though its limit counts no such room."""
+    if hip.device_info()["compute_units"] != 256:
+        pytest.skip("the lines are of 256 compute units")
+    say("f16 even deal by default", O.NAMES[t], m, n, k)
+    kern = hip.HipKernel(t)
+    need = kern.gemm_workspace_bytes(m, n, k)
+    assert (need == 64 << 20) == deal
+    w = O.random_blocks(t, 95, n, k)
+    acts = ref.quantize_q8_0(synth.normal_f32(96, m * k))
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    dw, da = torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda()
+    dy, other = (torch.empty((m, n), dtype=torch.float32, device="cuda") for _ in range(2))
+    kern.gemm_q8_dev(dw, da, dy, m, n, k, accumulate=False, workspace=ws)
+    assert last_launch().startswith("gemm_f16_deal_kernel") == deal, last_launch()
+    kern.gemm_q8_static_dev(dw, da, other, m, n, k)
+    torch.cuda.synchronize()
+    assert torch.equal(other, dy)
+    if deal:
+        least = ((k // 32) * ((m + 127) // 128 * 128 + 128) * 74 + 255) // 256 * 256
+        kern.gemm_q8_dev(dw, da, other, m, n, k, accumulate=False, workspace=ws[:least])
+        assert not last_launch().startswith("gemm_f16_deal_kernel"), last_launch()
+    torch.cuda.synchronize()
+    rows = [0, 63, 64 % m, m - 1]
+    y_ref = oracle_rows(ref, t, w, acts, n, k, rows)
+    for got in (dy, other):
+        assert np.abs(got.cpu().numpy()[rows] - y_ref).max() <= FP32_REL_TOL * np.abs(y_ref).max()
