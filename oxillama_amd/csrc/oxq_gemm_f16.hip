@@ -697,7 +697,9 @@ int gemm_f16_shape(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
 // 4096 x 14336 384 and 225, 512 x 4096 x 14336 126 and 104; Q5_K 333 x 11008 x 4096 105 and 82; Q6_K 333 x 4096 x 11008 135 and 97, 768
 // x 4096 x 14336 307 and 209, 1100 x 4096 x 4096 143 and 104.  Q4_K 333 x 4096 x 4096, where runs are three super-blocks, stays (33, 38).
 bool gemm_f16_deal_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
-    if (!gemm_f16_supported(type, m, n, k) || m <= 64) return false;  // (a token tile half empty, against 32-token tiles)
+    // (a token tile half empty, against 32-token tiles; matrices narrower than a tile keep the kernel whose fp32 sums the
+    // dump of the integer sums repeats bit for bit)
+    if (!gemm_f16_supported(type, m, n, k) || m <= 64 || n < 256) return false;
     const int f = type == OXQ_TYPE_Q4_K ? 0 : type == OXQ_TYPE_Q5_K ? 1 : 2;
     const uint64_t groups = f16_deal_groups(), cus = device_cus(), n_super = k / 256;
     auto tiles_of = [&](uint32_t t, uint32_t r) { return (uint64_t)((m + t - 1) / t) * ((n + r - 1) / r); };
