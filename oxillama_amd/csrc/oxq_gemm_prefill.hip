@@ -126,11 +126,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t c = lane & 31, h = lane >> 5;
 
-    // work groups of one set of weight rows (all token tiles) get consecutive ids on one XCD (ids are dealt
-    // round-robin to the 8 XCDs), so that their weight reads meet in that XCD's L2
-    const uint32_t xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
-    const uint32_t n_tile = (loc / m_tiles) * 8 + xcd, m_tile = loc % m_tiles;
-    if (n_tile >= n_tiles) return;
+    // the token tiles of one set of weight rows sit on one XCD, so that their weight reads meet in its L2
+    uint32_t m_tile, n_tile;
+    if (!tile_order_at(blockIdx.x, gridDim.x, m_tiles, n_tiles, m_tile, n_tile)) return;
     const uint32_t m_wg = m_tile * PF_TOK, n_wg = n_tile * PF_ROWS, n_wave = n_wg + 32 * wave;
     const uint32_t tt0 = m_wg >> 5;
 
@@ -418,7 +416,7 @@ hipError_t launch_gemm_prefill(uint32_t type, const GemmArgs &a, hipStream_t str
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     const uint32_t m_tiles = mpad / PF_TOK, n_tiles = (a.n + PF_ROWS - 1) / PF_ROWS;
-    const dim3 grid(8 * ((n_tiles + 7) / 8) * m_tiles);
+    const dim3 grid(tile_order_grid(m_tiles, n_tiles));
     note_launch("gemm_prefill_q4k", type, a.sums ? 1 : 0, 0, 0, 0, grid.x, 1, 512);
     if (a.sums)
         hipLaunchKernelGGL(gemm_prefill_q4k<true>, grid, dim3(512), 0, stream, a.W, tokf, dag, pbf, a.out, a.sums, a.m,

@@ -30,6 +30,7 @@
 #include <type_traits>
 #include "oxq_gemv_kernel.hpp"
 #include "oxq_internal.hpp"
+#include "oxq_tile_order.hpp"
 
 namespace oxq {
 
@@ -449,8 +450,8 @@ __device__ __forceinline__ bool find_group_tile(const int32_t *__restrict__ offs
 // of sub-blocks.  Weight bytes are fetched DIST groups ahead (a ring of registers), token
 // bytes one group ahead.
 // Work groups are numbered so that the token tiles of one set of weight rows run on the
-// same XCD at the same time (ids are dealt round-robin to the 8 XCDs), which turns their
-// weight reads into L2 hits.
+// same XCD at the same time, which turns their weight reads into L2 hits, and every XCD has an eighth of them
+// (oxq_tile_order.hpp).
 //
 // Grouped form (mixture-of-experts, n_experts != 0): expert e multiplies the token rows offsets[e] .. offsets[e+1]-1
 // by the weights at W + e * w_stride.  Only the device knows how many token tiles each expert needs: the grid holds as
@@ -496,8 +497,7 @@ __device__ __forceinline__ void gemm_tile_body(
     // super-blocks of this wave: all of them, or its quarter
     const uint32_t blk_begin = SPLITK ? wave * nblk / 4 : 0, blk_end = SPLITK ? (wave + 1) * nblk / 4 : nblk;
 
-    const uint32_t xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
-    uint32_t n_tile = (loc / m_tiles) * 8 + xcd, m_tile = loc % m_tiles;
+    uint32_t n_tile, m_tile;
     uint32_t row0 = 0, row_end = m;
     if (n_experts) {
         // expert groups: token tiles outermost, so that the tiles the experts do not need form one run at the end; a
@@ -511,6 +511,8 @@ __device__ __forceinline__ void gemm_tile_body(
         row0 = (uint32_t)offsets[expert];
         row_end = (uint32_t)offsets[expert + 1];
         W += (size_t)expert * w_stride;
+    } else if (!tile_order_at3(blockIdx.x, blockIdx.y + blockIdx.z * gridDim.y, m_tiles, n_tiles, m_tile, n_tile)) {
+        return;  // whole work group
     }
     if (n_tile >= n_tiles || row0 + m_tile * WG_TOK >= row_end) return;  // whole work group
     const uint32_t m_wg = row0 + m_tile * WG_TOK, n_wg = n_tile * WG_ROWS;
@@ -827,7 +829,8 @@ static hipError_t launch_tile(const GemmArgs &a, const TilePlan &p, hipStream_t 
     constexpr uint32_t WG_TOK = 32 * MT * (WM ? WM : 1), WG_ROWS = 32 * NT * (WM ? 4 / WM : 1);
     const uint32_t m_tiles = a.offsets ? group_tiles_bound(a.m, a.max_rows, a.n_experts, WG_TOK) : (a.m + WG_TOK - 1) / WG_TOK;
     const uint32_t n_tiles = (a.n + WG_ROWS - 1) / WG_ROWS;
-    const dim3 grid((a.offsets ? n_tiles : 8 * ((n_tiles + 7) / 8)) * m_tiles);
+    const TileGrid tg = tile_order_grid3(m_tiles, n_tiles);
+    const dim3 grid = a.offsets ? dim3(n_tiles * m_tiles) : dim3(tg.x, tg.y, tg.z);
     const size_t lds = (size_t)tile_padded_sub_blocks(a.k) * WG_TOK * 2;
     auto kern = &gemm_tile_kernel<F, MT, NT, WM, DIST, DUMP, ADIST>;
     if constexpr (OCC == 3) kern = &gemm_tile_kernel_occ3<F, MT, NT, WM, DIST, DUMP, ADIST>;

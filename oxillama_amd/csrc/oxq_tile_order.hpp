@@ -1,9 +1,10 @@
-// Which tile of m_tiles x n_tiles a work group takes, by its number: ids are dealt round-robin to the 8 XCDs, and an XCD
-// takes a run of tiles with the token tiles of one set of weight rows next to each other, so that their weight reads meet
-// in its L2.  The runs differ by at most 7 tiles and none is longer than an eighth of all, rounded up: a grid of as many
-// tiles as there are compute units is one round of the chip whatever its sides (dealing whole sets of weight rows to the
-// XCDs instead, 36 sets of 7 token tiles gave four of them 35 work groups for 32 compute units: 448 x 4608 x 4096, Q4_K,
-// 74 us against 40).
+// Which tile of m_tiles x n_tiles a work group takes, by its number: ids are dealt round-robin to the 8 XCDs, and the
+// token tiles of one set of weight rows sit next to each other on one XCD, so that their weight reads meet in its L2.  Sets of
+// weight rows go to the XCDs in turn while there are eight left; the tiles of the last few sets are dealt out in eighths.
+// No XCD has more than an eighth of all tiles, rounded up: a grid of as many tiles as there are compute units is one round
+// of the chip whatever its sides (whole sets to the end instead, 36 sets of 7 token tiles gave four XCDs 35 work groups for
+// 32 compute units: 448 x 4608 x 4096, Q4_K, 74 us against 40; 1480 x 4608 x 4608 218 against 130 on the prefill kernel, 1073 x
+// 3328 x 8192, IQ4_XS, 192 against 137 on the tile kernel).
 // (No HIP header here: a host test walks the grids.)
 #pragma once
 #include <cstdint>
@@ -20,9 +21,38 @@ OXQ_HOST_DEVICE uint32_t tile_order_grid(uint32_t m_tiles, uint32_t n_tiles) { r
 
 // false: no tile left for this work group
 OXQ_HOST_DEVICE bool tile_order_at(uint32_t block, uint32_t grid, uint32_t m_tiles, uint32_t n_tiles, uint32_t &m_tile, uint32_t &n_tile) {
-    const uint32_t t = (block & 7) * (grid >> 3) + (block >> 3);
+    const uint32_t xcd = block & 7, at = block >> 3, set = at / m_tiles, sets = n_tiles / 8;
+    if (set < sets) {
+        n_tile = set * 8 + xcd;
+        m_tile = at - set * m_tiles;
+        return true;
+    }
+    const uint32_t t = xcd * ((grid >> 3) - sets * m_tiles) + (at - sets * m_tiles);
     n_tile = t / m_tiles;
     m_tile = t - n_tile * m_tiles;
+    n_tile += sets * 8;
+    return n_tile < n_tiles;
+}
+
+// The same order for a grid of (8 x m_tiles, sets of eight n_tiles and the tail, more of them) work groups, whose coordinates
+// spare the kernel the division: for short work groups.
+struct TileGrid {
+    uint32_t x, y, z;
+};
+OXQ_HOST_DEVICE TileGrid tile_order_grid3(uint32_t m_tiles, uint32_t n_tiles) {
+    const uint32_t sets = (n_tiles + 7) / 8, y = sets < 32768 ? sets : 32768;
+    return TileGrid{8 * m_tiles, y, (sets + y - 1) / y};
+}
+OXQ_HOST_DEVICE bool tile_order_at3(uint32_t x, uint32_t set, uint32_t m_tiles, uint32_t n_tiles, uint32_t &m_tile, uint32_t &n_tile) {
+    m_tile = x >> 3;
+    n_tile = set * 8 + (x & 7);
+    const uint32_t left = n_tiles - set * 8;  // sets of weight rows from here on
+    if (set * 8 < n_tiles && left < 8) {
+        const uint32_t per = (left * m_tiles + 7) / 8, t = (x & 7) * per + m_tile;
+        if (m_tile >= per) return false;
+        m_tile = t % m_tiles;
+        n_tile = set * 8 + t / m_tiles;
+    }
     return n_tile < n_tiles;
 }
 

@@ -24,6 +24,20 @@ int main() {
             }
             for (int t : taken) ok = ok && t == 1;
             for (uint32_t x : on_xcd) ok = ok && x <= most;
+            const oxq::TileGrid g = oxq::tile_order_grid3(m, n);  // (x fastest, a multiple of 8: the XCD is x % 8)
+            uint32_t on3[8] = {0};
+            ok = ok && g.x == 8 * m;
+            for (uint32_t s = 0; ok && s < g.y * g.z; s++)
+                for (uint32_t x = 0; x < g.x; x++) {
+                    uint32_t mt, nt;
+                    if (!oxq::tile_order_at3(x, s, m, n, mt, nt)) continue;
+                    ok = ok && mt < m && nt < n;
+                    if (!ok) break;
+                    taken[nt * m + mt]++;
+                    on3[x & 7]++;
+                }
+            for (int t : taken) ok = ok && t == 2;
+            for (uint32_t x : on3) ok = ok && x <= most;
             grids++;
             if (!ok) {
                 std::printf("%u x %u tiles\n", m, n);
