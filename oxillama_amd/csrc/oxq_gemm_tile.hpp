@@ -456,13 +456,50 @@ __device__ __forceinline__ bool find_group_tile(const int32_t *__restrict__ offs
 // Grouped form (mixture-of-experts, n_experts != 0): expert e multiplies the token rows offsets[e] .. offsets[e+1]-1
 // by the weights at W + e * w_stride.  Only the device knows how many token tiles each expert needs: the grid holds as
 // many as all experts together can (group_tiles_bound), and a work group finds the expert of its tile by itself.
+struct TilePlace {
+    uint32_t m_wg, n_tile, row_end;  // the tile's first token row, its set of weight rows, the end of its group's rows
+    size_t w_off;                    // the group's weights
+};
+template <uint32_t WG_TOK>
+__device__ __forceinline__ bool tile_place(uint32_t m, uint32_t m_tiles, uint32_t n_tiles, const int32_t *__restrict__ offsets,
+                                           uint32_t n_experts, size_t w_stride, TilePlace &at) {
+    uint32_t n_tile, m_tile;
+    uint32_t row0 = 0, row_end = m;
+    size_t w_off = 0;
+    if (n_experts) {
+        // expert groups: token tiles outermost, so that the tiles the experts do not need form one run at the end; a
+        // token tile's work groups are consecutive, which deals them evenly to the XCDs whatever their number (six or
+        // twelve 128-row tiles, every one on the XCD of its number modulo 8, left XCDs idle: Q4_K, 64 rows in the mean, 128
+        // experts of 768 x 2048 117 us against 100, 64 of 1536 x 2048 109 against 94)
+        uint32_t expert = 0;
+        const uint32_t place = blockIdx.x / n_tiles;
+        n_tile = blockIdx.x - place * n_tiles;
+        if (!find_group_tile(offsets, n_experts, WG_TOK, place, expert, m_tile)) return false;
+        row0 = (uint32_t)offsets[expert];
+        row_end = (uint32_t)offsets[expert + 1];
+        w_off = (size_t)expert * w_stride;
+    } else if (!tile_order_at3(blockIdx.x, blockIdx.y + blockIdx.z * gridDim.y, m_tiles, n_tiles, m_tile, n_tile)) {
+        return false;
+    }
+    if (n_tile >= n_tiles || row0 + m_tile * WG_TOK >= row_end) return false;
+    at = TilePlace{row0 + m_tile * WG_TOK, n_tile, row_end, w_off};
+    return true;
+}
+
+// LDS bytes of the factors of a work group's weight rows; the split-k reduction at the end reuses the same memory (after a
+// barrier), so that it does not cost occupancy.
+template <class F, int MT, int NT, int WM>
+constexpr size_t tile_lds_static_bytes() {
+    constexpr int NP = 2 * F::KSPLIT + (F::HAS_MIN ? tile_min_planes<F>::value : 0);
+    constexpr size_t SC_BYTES = sizeof(float) * 4 * 8 * NP * 32 * NT, RED_BYTES = WM == 0 ? sizeof(float) * 4 * MT * NT * 16 * 64 : 0;
+    return SC_BYTES > RED_BYTES ? SC_BYTES : RED_BYTES;
+}
+
 template <class F, int MT, int NT, int WM, int DIST, bool DUMP, int ADIST>
 __device__ __forceinline__ void gemm_tile_body(
     const uint8_t *__restrict__ W, const uint8_t *__restrict__ q8t, const float *__restrict__ P,
-    const uint16_t *__restrict__ da16, float *__restrict__ out, int32_t *__restrict__ sums, uint32_t m, uint32_t mpad,
-    uint32_t n, uint32_t k, int accumulate, const float *__restrict__ bias, uint32_t m_tiles, uint32_t n_tiles,
-    const int32_t *__restrict__ offsets, uint32_t n_experts,
-    size_t w_stride) {
+    const uint16_t *__restrict__ da16, float *__restrict__ out, int32_t *__restrict__ sums, uint32_t mpad,
+    uint32_t n, uint32_t k, int accumulate, const float *__restrict__ bias, const TilePlace &at, uint8_t *lds_static) {
     constexpr bool SPLITK = WM == 0;  // the four waves share one tile and each walk a quarter of k
     constexpr int WMX = SPLITK ? 1 : WM, WN = SPLITK ? 1 : 4 / WMX;
     constexpr int WG_TOK = 32 * MT * WMX, WG_ROWS = 32 * NT * WN, MTILES = MT * WMX;
@@ -473,11 +510,7 @@ __device__ __forceinline__ void gemm_tile_body(
     constexpr int LPR = 64 / W_ROWS, SPL = 8 / LPR;   // scale decode: lanes per row, sub-blocks per lane
     static_assert(NT <= 2 && DIST >= 1, "tile configuration");
     extern __shared__ uint16_t lds_da[];            // [nsb][MTILES][2 halves][16] f16 token scales
-    // [wave][sub-block][KS x dsc, KS x -MAGIC*dsc, zero-point factor][row of the wave]; the split-k
-    // reduction at the end reuses the same memory (after a barrier), so that it does not cost occupancy
-    constexpr size_t SC_BYTES = sizeof(float) * 4 * 8 * NP * W_ROWS;
-    constexpr size_t RED_BYTES = SPLITK ? sizeof(float) * 4 * MT * NT * 16 * 64 : 0;
-    __shared__ __align__(16) uint8_t lds_static[SC_BYTES > RED_BYTES ? SC_BYTES : RED_BYTES];
+    // [wave][sub-block][KS x dsc, KS x -MAGIC*dsc, zero-point factor][row of the wave] (tile_lds_static_bytes)
     float (*lds_sc)[8][NP][W_ROWS] = reinterpret_cast<float (*)[8][NP][W_ROWS]>(lds_static);
     // A row that ends inside its last group of eight blocks (formats of independent 32-weight blocks only): the
     // last group is read through the window of the row's last eight blocks, so that no load leaves the row, and
@@ -497,25 +530,8 @@ __device__ __forceinline__ void gemm_tile_body(
     // super-blocks of this wave: all of them, or its quarter
     const uint32_t blk_begin = SPLITK ? wave * nblk / 4 : 0, blk_end = SPLITK ? (wave + 1) * nblk / 4 : nblk;
 
-    uint32_t n_tile, m_tile;
-    uint32_t row0 = 0, row_end = m;
-    if (n_experts) {
-        // expert groups: token tiles outermost, so that the tiles the experts do not need form one run at the end; a
-        // token tile's work groups are consecutive, which deals them evenly to the XCDs whatever their number (six or
-        // twelve 128-row tiles, every one on the XCD of its number modulo 8, left XCDs idle: Q4_K, 64 rows in the mean, 128
-        // experts of 768 x 2048 117 us against 100, 64 of 1536 x 2048 109 against 94)
-        uint32_t expert = 0;
-        const uint32_t place = blockIdx.x / n_tiles;
-        n_tile = blockIdx.x - place * n_tiles;
-        if (!find_group_tile(offsets, n_experts, WG_TOK, place, expert, m_tile)) return;  // whole work group
-        row0 = (uint32_t)offsets[expert];
-        row_end = (uint32_t)offsets[expert + 1];
-        W += (size_t)expert * w_stride;
-    } else if (!tile_order_at3(blockIdx.x, blockIdx.y + blockIdx.z * gridDim.y, m_tiles, n_tiles, m_tile, n_tile)) {
-        return;  // whole work group
-    }
-    if (n_tile >= n_tiles || row0 + m_tile * WG_TOK >= row_end) return;  // whole work group
-    const uint32_t m_wg = row0 + m_tile * WG_TOK, n_wg = n_tile * WG_ROWS;
+    const uint32_t m_wg = at.m_wg, row_end = at.row_end, n_wg = at.n_tile * WG_ROWS;
+    W += at.w_off;
     const uint32_t m_wave = m_wg + wm * (32 * MT), n_wave = n_wg + wn * (32 * NT);
 
     // Token scales of this work group's tokens, permuted so that the 16 values a lane needs
@@ -793,6 +809,16 @@ __device__ __forceinline__ void gemm_tile_body(
         }
 }
 
+// A 64-token tile with at most 32 rows (the last of a prompt, half of the expert groups around a mean of 32) computes
+// one token tile, not a second one of padding: the time is the vector instructions per result, of full and short tiles alike.
+// Same bits, no more registers.  us, before and after: a layer of a small Q4_0 / Q8_0 model (1536 columns) at 77 tokens 133.6 and
+// 130.6, 512 tokens over 128 experts whose Q6_K down takes these tiles 283.4 and 280.8 (less than the padding: the weights and the
+// ramp are the same).  Not for the 128-token tiles: four bodies a kernel for one tile in a prompt of several hundred rows.
+template <int MT, int WM, bool DUMP>
+constexpr bool tile_short_body() {
+    return MT == 2 && WM <= 1 && !DUMP;
+}
+
 // The kernel proper, compiled for a fixed number of waves per SIMD (OCC = 2: up to 256 VGPRs,
 // OCC = 3: up to 168): the register budget decides how far the compiler lets loads and MFMAs
 // run ahead of their use.
@@ -803,8 +829,18 @@ __device__ __forceinline__ void gemm_tile_body(
         const uint16_t *__restrict__ da16, float *__restrict__ out, int32_t *__restrict__ sums, uint32_t m,         \
         uint32_t mpad, uint32_t n, uint32_t k, int accumulate, const float *__restrict__ bias, uint32_t m_tiles,   \
         uint32_t n_tiles, const int32_t *__restrict__ offsets, uint32_t n_experts, size_t w_stride) {               \
-        gemm_tile_body<F, MT, NT, WM, DIST, DUMP, ADIST>(W, q8t, P, da16, out, sums, m, mpad, n, k, accumulate,     \
-                                                         bias, m_tiles, n_tiles, offsets, n_experts, w_stride);     \
+        __shared__ __align__(16) uint8_t lds_static[tile_lds_static_bytes<F, MT, NT, WM>()];                          \
+        TilePlace at;                                                                                               \
+        if (!tile_place<32 * MT * (WM ? WM : 1)>(m, m_tiles, n_tiles, offsets, n_experts, w_stride, at)) return;      \
+        if constexpr (tile_short_body<MT, WM, DUMP>()) {                                                            \
+            if (at.row_end - at.m_wg <= 32) {                                                                       \
+                gemm_tile_body<F, 1, NT, WM, DIST, DUMP, ADIST>(W, q8t, P, da16, out, sums, mpad, n, k, accumulate,  \
+                                                                bias, at, lds_static);                              \
+                return;                                                                                             \
+            }                                                                                                       \
+        }                                                                                                           \
+        gemm_tile_body<F, MT, NT, WM, DIST, DUMP, ADIST>(W, q8t, P, da16, out, sums, mpad, n, k, accumulate, bias,   \
+                                                         at, lds_static);                                           \
     }
 OXQ_TILE_KERNEL(gemm_tile_kernel, 2)
 OXQ_TILE_KERNEL(gemm_tile_kernel_occ3, 3)

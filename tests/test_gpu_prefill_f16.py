@@ -387,3 +387,40 @@ def test_f16_even_deal_by_default(hip, ref, t, m, n, k, deal):
     y_ref = oracle_rows(ref, t, w, acts, n, k, rows)
     for got in (dy, other):
         assert np.abs(got.cpu().numpy()[rows] - y_ref).max() <= FP32_REL_TOL * np.abs(y_ref).max()
+
+
+@pytest.mark.parametrize("variant", [16, 23])
+@pytest.mark.parametrize("t,k", [(O.Q4_K, 1024), (O.Q6_K, 768), (O.Q4_0, 1056), (O.IQ4_XS, 1280)], ids=lambda v: str(v))
+def test_tiles_of_at_most_32_rows(hip, ref, tuning, t, k, variant):
+    """The 64-token tiles of the tile kernel compute one token tile of 32 where they hold no more rows: the bits of full
+    tiles (a token's sums do not depend on its neighbours), plain and in expert groups, nothing past the rows, 1e-5 of the oracle."""
+    n, groups = 193, [1, 32, 33, 0, 64, 65, 96, 97]
+    offsets = np.concatenate([[0], np.cumsum(groups)]).astype(np.int32)
+    m = int(offsets[-1])
+    say("short tiles", O.NAMES[t], k, variant)
+    tuning("gemm_variant", variant)
+    tuning("gemm_tile_min_rows", 1)
+    w = O.random_blocks(t, 70 + variant, n, k).reshape(-1)
+    acts = ref.quantize_q8_0(synth.normal_f32(71, m * k)).reshape(-1)
+    kern, row = hip.HipKernel(t), k // 32 * 34
+    dw, da = torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda()
+    full = torch.empty((448, n), dtype=torch.float32, device="cuda")  # (whole tiles: the rows past m are zeros)
+    da_full = torch.zeros(448 * row, dtype=torch.uint8, device="cuda")
+    da_full[:m * row] = da
+    ws = torch.empty(max(kern.gemm_workspace_bytes(448, n, k), kern.moe_gemm_workspace_bytes(m, n, k)), dtype=torch.uint8, device="cuda")
+    kern.gemm_q8_dev(dw, da_full, full, 448, n, k, accumulate=False, workspace=ws)
+    assert last_launch().startswith("gemm_tile_kernel"), last_launch()
+    for rows in (1, 31, 32, 33, 65, 95, 96, 97):
+        y = torch.full((rows + 1, n), 7.0, dtype=torch.float32, device="cuda")
+        kern.gemm_q8_dev(dw, da, y, rows, n, k, accumulate=False, workspace=ws)
+        assert last_launch().startswith("gemm_tile_kernel"), last_launch()
+        assert torch.equal(y[:rows], full[:rows]) and bool((y[rows] == 7.0).all()), rows
+    d_off = torch.from_numpy(offsets).cuda()
+    y = torch.full((m + 1, n), 7.0, dtype=torch.float32, device="cuda")
+    experts = dw.repeat(len(groups))
+    kern.moe_gemm_q8_dev(experts, w.nbytes, len(groups), da, d_off, m, max(groups), y, n, k, ws)
+    assert last_launch().startswith("gemm_tile_kernel"), last_launch()
+    assert torch.equal(y[:m], full[:m]) and bool((y[m] == 7.0).all())
+    rows = [0, 31, 32, m - 1]
+    want = oracle_rows(ref, t, w, acts, n, k, rows)
+    assert np.abs(full.cpu().numpy()[rows] - want).max() <= FP32_REL_TOL * np.abs(want).max()
