@@ -460,7 +460,7 @@ struct TilePlace {
     uint32_t m_wg, n_tile, row_end;  // the tile's first token row, its set of weight rows, the end of its group's rows
     size_t w_off;                    // the group's weights
 };
-template <uint32_t WG_TOK>
+template <uint32_t WG_TOK, bool SHORT>
 __device__ __forceinline__ bool tile_place(uint32_t m, uint32_t m_tiles, uint32_t n_tiles, const int32_t *__restrict__ offsets,
                                            uint32_t n_experts, size_t w_stride, TilePlace &at) {
     uint32_t n_tile, m_tile;
@@ -478,8 +478,11 @@ __device__ __forceinline__ bool tile_place(uint32_t m, uint32_t m_tiles, uint32_
         row0 = (uint32_t)offsets[expert];
         row_end = (uint32_t)offsets[expert + 1];
         w_off = (size_t)expert * w_stride;
-    } else if (!tile_order_at3(blockIdx.x, blockIdx.y + blockIdx.z * gridDim.y, m_tiles, n_tiles, m_tile, n_tile)) {
-        return false;
+    } else {
+        const uint32_t set = blockIdx.y + blockIdx.z * gridDim.y;
+        if (!(SHORT && gridDim.x != 8 * m_tiles ? tile_order_at3_short_last(blockIdx.x, set, m_tiles, n_tiles, m_tile, n_tile)
+                                                : tile_order_at3(blockIdx.x, set, m_tiles, n_tiles, m_tile, n_tile)))
+            return false;
     }
     if (n_tile >= n_tiles || row0 + m_tile * WG_TOK >= row_end) return false;
     at = TilePlace{row0 + m_tile * WG_TOK, n_tile, row_end, w_off};
@@ -831,7 +834,9 @@ constexpr bool tile_short_body() {
         uint32_t n_tiles, const int32_t *__restrict__ offsets, uint32_t n_experts, size_t w_stride) {               \
         __shared__ __align__(16) uint8_t lds_static[tile_lds_static_bytes<F, MT, NT, WM>()];                          \
         TilePlace at;                                                                                               \
-        if (!tile_place<32 * MT * (WM ? WM : 1)>(m, m_tiles, n_tiles, offsets, n_experts, w_stride, at)) return;      \
+        if (!tile_place<32 * MT * (WM ? WM : 1), tile_short_body<MT, WM, DUMP>()>(m, m_tiles, n_tiles, offsets,      \
+                                                                                  n_experts, w_stride, at))         \
+            return;                                                                                                 \
         if constexpr (tile_short_body<MT, WM, DUMP>()) {                                                            \
             if (at.row_end - at.m_wg <= 32) {                                                                       \
                 gemm_tile_body<F, 1, NT, WM, DIST, DUMP, ADIST>(W, q8t, P, da16, out, sums, mpad, n, k, accumulate,  \
@@ -865,7 +870,16 @@ static hipError_t launch_tile(const GemmArgs &a, const TilePlan &p, hipStream_t 
     constexpr uint32_t WG_TOK = 32 * MT * (WM ? WM : 1), WG_ROWS = 32 * NT * (WM ? 4 / WM : 1);
     const uint32_t m_tiles = a.offsets ? group_tiles_bound(a.m, a.max_rows, a.n_experts, WG_TOK) : (a.m + WG_TOK - 1) / WG_TOK;
     const uint32_t n_tiles = (a.n + WG_ROWS - 1) / WG_ROWS;
-    const TileGrid tg = tile_order_grid3(m_tiles, n_tiles);
+    // A last token tile of at most 32 rows behind all others where the grid is more than the chip holds at a time (two work
+    // groups per compute unit): among them, compute units that had a short one took a full one more than others at the end
+    // (333 x 4096 x 4096, 768 work groups for 512 places, us without short tiles / with them in their set's place / at the end: Q5_K
+    // 39.2 / 43.5 / 38.6, Q4_K 34.4 / 37.7 / 33.9; 145 x 8192 x 2048 Q4_0 26.0 / 29.4 / 24.3; ten matrices at 145 to 345 rows, twelve
+    // formats, in the mean 0.98 / 0.94 of the first, at worst 1.14 / 1.04).  Two token tiles stay in their sets, where they share the weights'
+    // reads: 77 x 11008 x 4096 Q4_0 41.4 / 38.8 / 43.6, 8960 x 1536 23.3 / 22.5 / 20.1.
+    const uint32_t left = a.m % WG_TOK;
+    const bool short_last = tile_short_body<MT, WM, DUMP>() && m_tiles > 2 && left >= 1 && left <= 32 &&
+                            (size_t)m_tiles * n_tiles > 2 * (size_t)device_cus();
+    const TileGrid tg = short_last ? tile_order_grid3_short_last(m_tiles, n_tiles) : tile_order_grid3(m_tiles, n_tiles);
     const dim3 grid = a.offsets ? dim3(n_tiles * m_tiles) : dim3(tg.x, tg.y, tg.z);
     const size_t lds = (size_t)tile_padded_sub_blocks(a.k) * WG_TOK * 2;
     auto kern = &gemm_tile_kernel<F, MT, NT, WM, DIST, DUMP, ADIST>;

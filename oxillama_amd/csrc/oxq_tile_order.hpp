@@ -56,6 +56,21 @@ OXQ_HOST_DEVICE bool tile_order_at3(uint32_t x, uint32_t set, uint32_t m_tiles, 
     return n_tile < n_tiles;
 }
 
+// The same with the tiles of the last, shorter token tile behind all others (of several token tiles): a grid of more work groups
+// than the chip holds at a time ends on the shorter ones.  Its width tells it from the other grid.
+OXQ_HOST_DEVICE TileGrid tile_order_grid3_short_last(uint32_t m_tiles, uint32_t n_tiles) {
+    const uint32_t full = m_tiles - 1, sets = (n_tiles + 7) / 8, all = sets + (sets + full - 1) / full;
+    const uint32_t y = all < 32768 ? all : 32768;
+    return TileGrid{8 * full, y, (all + y - 1) / y};
+}
+OXQ_HOST_DEVICE bool tile_order_at3_short_last(uint32_t x, uint32_t set, uint32_t m_tiles, uint32_t n_tiles, uint32_t &m_tile, uint32_t &n_tile) {
+    const uint32_t full = m_tiles - 1, sets = (n_tiles + 7) / 8;
+    if (set < sets) return tile_order_at3(x, set, full, n_tiles, m_tile, n_tile);
+    m_tile = full;
+    n_tile = ((set - sets) * full + (x >> 3)) * 8 + 7 - (x & 7);  // (from the XCDs to which the last full ones go least)
+    return n_tile < n_tiles;
+}
+
 // An even deal of units (a unit: one super-block of one tile, the tiles one after another) over as many work groups as there
 // are compute units: a work group takes a run of units, so that at most two of the tiles it meets are not all its own, the
 // first and the last of its run, and their sums go to its two slots.  Neighbouring runs sit on one XCD.

@@ -38,6 +38,24 @@ int main() {
                 }
             for (int t : taken) ok = ok && t == 2;
             for (uint32_t x : on3) ok = ok && x <= most;
+            if (m > 1) {  // the last token tile's behind all others; an XCD at most one of them above its share
+                const oxq::TileGrid l = oxq::tile_order_grid3_short_last(m, n);
+                uint32_t on_last[8] = {0};
+                bool last = false;
+                ok = ok && l.x == 8 * (m - 1);
+                for (uint32_t s = 0; ok && s < l.y * l.z; s++)
+                    for (uint32_t x = 0; x < l.x; x++) {
+                        uint32_t mt, nt;
+                        if (!oxq::tile_order_at3_short_last(x, s, m, n, mt, nt)) continue;
+                        last = last || mt == m - 1;
+                        ok = ok && mt < m && nt < n && (mt == m - 1) == last;
+                        if (!ok) break;
+                        taken[nt * m + mt]++;
+                        on_last[x & 7]++;
+                    }
+                for (int t : taken) ok = ok && t == 3;
+                for (uint32_t x : on_last) ok = ok && x <= most + 1;
+            }
             grids++;
             if (!ok) {
                 std::printf("%u x %u tiles\n", m, n);

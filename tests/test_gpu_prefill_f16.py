@@ -424,3 +424,31 @@ def test_tiles_of_at_most_32_rows(hip, ref, tuning, t, k, variant):
     rows = [0, 31, 32, m - 1]
     want = oracle_rows(ref, t, w, acts, n, k, rows)
     assert np.abs(full.cpu().numpy()[rows] - want).max() <= FP32_REL_TOL * np.abs(want).max()
+
+
+@pytest.mark.parametrize("variant,n", [(23, 5600), (16, 22400)])
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q8_0], ids=lambda t: O.NAMES[t])
+def test_short_tiles_behind_the_others(hip, ref, tuning, t, variant, n):
+    """Grids of more tiles than the chip holds at a time (175 sets of weight rows, which the XCDs do not share evenly) launch a
+    third, short token tile last: the bits of full tiles, every tile once, nothing past the rows, 1e-5 of the oracle."""
+    k = 256
+    say("short tiles last", O.NAMES[t], n, variant)
+    tuning("gemm_variant", variant)
+    w = O.random_blocks(t, 75, n, k).reshape(-1)
+    acts = ref.quantize_q8_0(synth.normal_f32(76, 192 * k)).reshape(-1)
+    kern = hip.HipKernel(t)
+    dw, da = torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda()
+    full = torch.empty((192, n), dtype=torch.float32, device="cuda")
+    ws = torch.empty(kern.gemm_workspace_bytes(192, n, k), dtype=torch.uint8, device="cuda")
+    kern.gemm_q8_dev(dw, da, full, 192, n, k, accumulate=False, workspace=ws)
+    grids = {last_launch()}
+    for rows in (129, 142, 160, 161):
+        y = torch.full((rows + 1, n), 7.0, dtype=torch.float32, device="cuda")
+        kern.gemm_q8_dev(dw, da, y, rows, n, k, accumulate=False, workspace=ws)
+        grids.add(last_launch())
+        assert torch.equal(y[:rows], full[:rows]) and bool((y[rows] == 7.0).all()), rows
+    if hip.device_info()["compute_units"] < 260:
+        assert len(grids) == 2, grids  # (161 and 192 rows: three whole tiles)
+    rows = [0, 63, 128, 191]
+    want = oracle_rows(ref, t, w, acts, n, k, rows)
+    assert np.abs(full.cpu().numpy()[rows] - want).max() <= FP32_REL_TOL * np.abs(want).max()
