@@ -275,7 +275,7 @@ __global__ __launch_bounds__(64 * RW * KS) __attribute__((amdgpu_waves_per_eu(2,
         tile = rank * rounds, whole = rounds, unit = r.begin, unit_end = r.end, slot = 2 * rank;
         if (whole == 0 && unit == unit_end) return;
     } else {
-        if (!tile_order_at(blockIdx.x, gridDim.x, m_tiles, n_tiles, m_tile, n_tile)) return;  // the whole work group
+        if (!tile_run_at(blockIdx.x, gridDim.x, m_tiles, n_tiles, m_tile, n_tile)) return;  // the whole work group
     }
     do {  // (DEAL: the work group's run of a tile, then its run of the next one)
     if constexpr (DEAL) {

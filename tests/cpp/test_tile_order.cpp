@@ -11,11 +11,16 @@ int main() {
     for (uint32_t m = 1; m <= 40; m++)
         for (uint32_t n = 1; n <= 260; n += n < 40 ? 1 : 7) {
             const uint32_t grid = oxq::tile_order_grid(m, n), most = (m * n + 7) / 8;
-            std::vector<int> taken(m * n, 0);
+            std::vector<int> taken(m * n, 0), in_run(m * n, 0);
             uint32_t on_xcd[8] = {0};
             bool ok = grid == 8 * most;
             for (uint32_t b = 0; b < grid; b++) {
                 uint32_t mt, nt;
+                if (oxq::tile_run_at(b, grid, m, n, mt, nt)) {  // (an XCD's work groups: `most` at most)
+                    ok = ok && mt < m && nt < n;
+                    if (!ok) break;
+                    in_run[nt * m + mt]++;
+                }
                 if (!oxq::tile_order_at(b, grid, m, n, mt, nt)) continue;
                 ok = ok && mt < m && nt < n;
                 if (!ok) break;
@@ -23,6 +28,7 @@ int main() {
                 on_xcd[b & 7]++;
             }
             for (int t : taken) ok = ok && t == 1;
+            for (int t : in_run) ok = ok && t == 1;
             for (uint32_t x : on_xcd) ok = ok && x <= most;
             const oxq::TileGrid g = oxq::tile_order_grid3(m, n);  // (x fastest, a multiple of 8: the XCD is x % 8)
             uint32_t on3[8] = {0};
