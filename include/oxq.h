@@ -278,20 +278,26 @@ int oxq_activation_route(void);
  * with the 6-bit sub-block scale inside the weight operand (exact) and d / dmin applied per
  * super-block: the same integers, fp32 inside the same 1e-5 bar; the workspace size covers both.  Many token rows of
  * Q6_K, and of Q5_K and Q4_K on other shapes that fill the chip, take the same arithmetic from the Q8_0 rows
- * themselves, without workspace; where their tiles would leave much of the chip idle, parts of k go to several work groups,
- * whose sums take 64 MiB of workspace (part of the size; a smaller workspace that holds what the other kernels need is
- * taken too, by those). */
+ * themselves, without workspace.
+ * oxq_gemm_q8_workspace_bytes() is what a call must have: a smaller workspace is refused (OXQ_ERR_BUFFER_TOO_SMALL: needed,
+ * given).  oxq_gemm_q8_best_workspace_bytes() is never less, and more for Q4_K, Q5_K and Q6_K prompts whose tiles would leave
+ * much of the chip idle: there parts of k go to several work groups, whose sums take 64 MiB (two of 128 KiB per compute
+ * unit) whatever the shape, in place of the rest.  A call takes that kernel if its workspace has the room (as the library's
+ * own scratch and oxq_gemm_q8_static_dev have), the others' sums are added in another order: two calls that are to agree to
+ * the last bit need workspaces on the same side of the best size.  One workspace for the best kernel at any number
+ * of rows up to m: the larger of oxq_gemm_q8_workspace_bytes() at m rows and 64 MiB. */
 size_t oxq_gemm_q8_workspace_bytes(uint32_t type, size_t m, size_t n, size_t k);
+size_t oxq_gemm_q8_best_workspace_bytes(uint32_t type, size_t m, size_t n, size_t k);
 int oxq_gemm_q8_dev(uint32_t type, const uint8_t *d_weights, const uint8_t *d_acts_q8,
                     float *d_out, size_t m, size_t n, size_t k, int accumulate,
                     void *d_workspace, size_t workspace_bytes, void *stream);
 /* oxq_gemm_q8_dev for callers that cannot allocate device memory and have no workspace to pass
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  No
- * counterpart in the reference.  The tile kernel's workspace is a static array in device
- * memory that the library holds on each GPU it was initialised on (16 MiB:
- * oxq_gemm_q8_static_max_workspace_bytes()); the call allocates nothing, synchronises nothing and
- * gives the bits of oxq_gemm_q8_dev (the sums of parts of k have room beside the 16 MiB and do not count).  Other shapes whose
- * oxq_gemm_q8_workspace_bytes exceeds the array return OXQ_ERR_BUFFER_TOO_SMALL (needed, available); oxq_init must have run (the call
+ * counterpart in the reference.  The workspace is a static array of 64 MiB in device
+ * memory that the library holds on each GPU it was initialised on; the call allocates nothing, synchronises nothing and
+ * gives the bits of oxq_gemm_q8_dev with a workspace of the best size.  Shapes whose oxq_gemm_q8_workspace_bytes()
+ * exceeds oxq_gemm_q8_static_max_workspace_bytes() (16 MiB; the rest of the array is for the sums that the best size
+ * counts) return OXQ_ERR_BUFFER_TOO_SMALL (needed, available); oxq_init must have run (the call
  * does not initialise lazily: OXQ_ERR_NO_DEVICE) for the device the calling thread has current,
  * whose copy of the array the call uses.  All calls on one GPU share the array: issue them on
  * ONE stream per GPU (or order the streams with events yourself) -- calls that overlap in time

@@ -21,8 +21,8 @@ hipError_t launch_dequant(uint32_t type, const uint8_t *blocks, size_t n_blocks,
 // its own copy at its own address until the process ends; host code reaches it only through the address that
 // hipGetSymbolAddress returned for that device (static_scratch_ptr), never through this name.
 constexpr size_t STATIC_SCRATCH_BYTES = (size_t)16 << 20;
-// ... and room for the sums that the f16 kernel's even deal exchanges (128 KB twice for each of 256 compute units), which a
-// call's size for that limit leaves out: what ran with 16 MiB runs, and in the kernels of the workspace form
+// The array itself holds what the f16 kernel's even deal exchanges (128 KB twice for each of 256 compute units), in place of
+// those planes: a shape within the limit runs on the kernels that a workspace of its best size would get.
 constexpr size_t STATIC_DEAL_BYTES = (size_t)64 << 20;
 static __device__ __align__(256) uint8_t scratch[STATIC_DEAL_BYTES];
 
@@ -770,7 +770,7 @@ static int gemm_host(uint32_t type, const uint8_t *data, size_t data_len, const 
     ga.workspace = nullptr;
     if (oxq::gemm_uses_tiles(type, (uint32_t)m, (uint32_t)n_rows, (uint32_t)n_cols) ||
         oxq::gemm_few_rows_pay(type, (uint32_t)m, (uint32_t)n_rows, (uint32_t)n_cols)) {
-        const size_t wbytes = oxq::gemm_workspace_bytes((uint32_t)m, (uint32_t)n_cols, (uint32_t)n_rows, type);
+        const size_t wbytes = oxq::gemm_best_workspace_bytes((uint32_t)m, (uint32_t)n_cols, (uint32_t)n_rows, type);
         if ((st = g.s_work.reserve(wbytes)) != OXQ_OK) return st;
         ga.workspace = (uint8_t *)g.s_work.ptr;
         ga.workspace_bytes = wbytes;
@@ -978,6 +978,11 @@ size_t oxq_gemm_q8_workspace_bytes(uint32_t type, size_t m, size_t n, size_t k) 
     return oxq::gemm_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type);
 }
 
+size_t oxq_gemm_q8_best_workspace_bytes(uint32_t type, size_t m, size_t n, size_t k) {
+    if (oxq_gemm_q8_workspace_bytes(type, m, n, k) == 0) return 0;
+    return oxq::gemm_best_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type);
+}
+
 static int gemm_dev(uint32_t type, const uint8_t *d_weights, const uint8_t *d_acts_q8, float *d_out, int32_t *d_sums,
                     size_t m, size_t n, size_t k, int accumulate, const float *d_bias, void *d_workspace,
                     size_t workspace_bytes, void *stream) {
@@ -1002,14 +1007,13 @@ static int gemm_dev(uint32_t type, const uint8_t *d_weights, const uint8_t *d_ac
     // a few rows fewer still pay on the few-token kernel, if the caller's workspace has the room (without one the
     // call would have to take the library's scratch and wait for the stream: the GEMV launches stay)
     if (!tiles && d_workspace && !d_sums && oxq::gemm_few_rows_pay(type, (uint32_t)m, (uint32_t)n, (uint32_t)k) &&
-        workspace_bytes >= oxq::gemm_workspace_least_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) &&
+        workspace_bytes >= oxq::gemm_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) &&
         (reinterpret_cast<uintptr_t>(d_workspace) & 255) == 0)
         tiles = true;
     ga.by_rows = !tiles;
     const size_t need = tiles ? oxq::gemm_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) : 0;
     if (need && d_workspace) {
-        if (workspace_bytes < oxq::gemm_workspace_least_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type))
-            return fail(OXQ_ERR_BUFFER_TOO_SMALL, need, workspace_bytes, "workspace too small");
+        if (workspace_bytes < need) return fail(OXQ_ERR_BUFFER_TOO_SMALL, need, workspace_bytes, "workspace too small");
         if (reinterpret_cast<uintptr_t>(d_workspace) & 255)
             return fail(OXQ_ERR_KERNEL, 256, reinterpret_cast<uintptr_t>(d_workspace) & 255, "workspace must be 256-byte aligned");
         ga.workspace = (uint8_t *)d_workspace;
@@ -1020,10 +1024,11 @@ static int gemm_dev(uint32_t type, const uint8_t *d_weights, const uint8_t *d_ac
     if (need) {
         // Library-owned scratch: calls serialise on the lock and wait for the stream, because
         // the scratch is shared.
+        const size_t best = d_sums ? need : oxq::gemm_best_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type);
         std::lock_guard<std::mutex> lock(g.mu);
-        if ((st = g.s_work.reserve(need)) != OXQ_OK) return st;
+        if ((st = g.s_work.reserve(best)) != OXQ_OK) return st;
         ga.workspace = (uint8_t *)g.s_work.ptr;
-        ga.workspace_bytes = need;
+        ga.workspace_bytes = best;
         OXQ_HIP(oxq::launch_gemm_q8(type, ga, (hipStream_t)stream));
         OXQ_HIP(hipStreamSynchronize((hipStream_t)stream));
         return OXQ_OK;
@@ -1056,8 +1061,8 @@ int oxq_gemm_q8_static_dev(uint32_t type, const uint8_t *d_weights, const uint8_
     if (m == 0 || n == 0 || k == 0) return OXQ_OK;
     const bool tiles = oxq::gemm_uses_tiles(type, (uint32_t)m, (uint32_t)n, (uint32_t)k) ||
                        (oxq::gemm_few_rows_pay(type, (uint32_t)m, (uint32_t)n, (uint32_t)k) &&
-                        oxq::gemm_workspace_least_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) <= STATIC_SCRATCH_BYTES);
-    const size_t need = tiles ? oxq::gemm_workspace_least_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) : 0;
+                        oxq::gemm_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) <= STATIC_SCRATCH_BYTES);
+    const size_t need = tiles ? oxq::gemm_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) : 0;
     if (need > STATIC_SCRATCH_BYTES)
         return fail(OXQ_ERR_BUFFER_TOO_SMALL, need, STATIC_SCRATCH_BYTES,
                     "shape needs more workspace than the static scratch holds: use oxq_gemm_q8_dev with a workspace");

@@ -84,12 +84,12 @@ size_t gemm_grouped_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t
     const size_t planes = (gemm_planes_bytes(m, k) + 255) & ~(size_t)255;
     return planes + gemm_grouped_partial_bytes(type, m, n, k);
 }
-size_t gemm_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t type) {
-    const size_t least = gemm_workspace_least_bytes(m, k, n, type);
+size_t gemm_best_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t type) {
+    const size_t needed = gemm_workspace_bytes(m, k, n, type);
     const size_t deal = gemm_f16_deal_pays(type, m, n, k) ? gemm_f16_deal_bytes() : 0;
-    return least > deal ? least : deal;
+    return needed > deal ? needed : deal;
 }
-size_t gemm_workspace_least_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t type) {
+size_t gemm_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t type) {
     const size_t planes = (gemm_planes_bytes(m, k) + 255) & ~(size_t)255;
     const size_t tiles = planes + gemm_partial_bytes(type, m, n, k);
     // the prefill kernel lays its own planes (f16 token operands) over the head of the same workspace; the size is
@@ -236,7 +236,7 @@ hipError_t launch_gemm_q8(uint32_t type, const GemmArgs &a, hipStream_t stream) 
     const int perm = act_perm(type);
     TilePlan plan = {q8t, P, da16, mpad};
     if (!a.offsets && gemm_partial_bytes(type, a.m, a.n, a.k) &&
-        a.workspace_bytes >= gemm_workspace_least_bytes(a.m, a.k, a.n, type))
+        a.workspace_bytes >= gemm_workspace_bytes(a.m, a.k, a.n, type))
         plan.partial = reinterpret_cast<float *>(a.workspace + ((gemm_planes_bytes(a.m, a.k) + 255) & ~(size_t)255));
     if (a.offsets && gemm_grouped_partial_bytes(type, a.m, a.n, a.k) &&
         a.workspace_bytes >= gemm_grouped_workspace_bytes(a.m, a.k, a.n, type))

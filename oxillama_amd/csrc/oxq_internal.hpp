@@ -221,10 +221,10 @@ hipError_t launch_gemm_q8(uint32_t type, const GemmArgs &a, hipStream_t stream);
 // Device scratch the tile kernel needs for m tokens of k columns (activation re-layout).
 // With n and the format: plus, for a matmul of at most 32 token rows that the few-token kernel would split over k,
 // the room for its per-split sums (behind the re-tiled activations, 256-byte aligned).
-// And for the f16 kernel's even deal the sums of shared tiles, at the head.  The least size is the one without them: a
-// call with a workspace in between takes the kernels that need no more.
+// The best size has room for the f16 kernel's even deal too (the sums of shared tiles, at the head): a call with a
+// workspace in between takes the kernels that need no more.
 size_t gemm_workspace_bytes(uint32_t m, uint32_t k, uint32_t n = 0, uint32_t type = 0);
-size_t gemm_workspace_least_bytes(uint32_t m, uint32_t k, uint32_t n = 0, uint32_t type = 0);
+size_t gemm_best_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t type);
 // ... of the grouped form: the planes, plus room for two per-split sums of [m x n] where the few-token kernel may
 // split an expert's k in two (Q4_K / IQ4_XS, k a multiple of 1024, at most 8192 rows per expert).
 size_t gemm_grouped_workspace_bytes(uint32_t m, uint32_t k, uint32_t n, uint32_t type);

@@ -288,6 +288,11 @@ class HipKernel:
                                             int(accumulate), raw_stream()))
 
     def gemm_workspace_bytes(self, m, n, k):
+        """With room for the fastest kernel of this shape; gemm_q8_dev takes gemm_least_workspace_bytes too."""
+        return self._lib.oxq_gemm_q8_best_workspace_bytes(self.tensor_type, m, n, k)
+
+    def gemm_least_workspace_bytes(self, m, n, k):
+        """What gemm_q8_dev must have, and what the limit of gemm_q8_static_dev counts."""
         return self._lib.oxq_gemm_q8_workspace_bytes(self.tensor_type, m, n, k)
 
     def gemm_q8_dev(self, d_weights, d_acts, d_out, m, n, k, accumulate=False, workspace=None):
@@ -295,7 +300,8 @@ class HipKernel:
         _check(capi.bind().gemm_q8(self.tensor_type, d_weights, d_acts, d_out, m, n, k, int(accumulate), workspace))
 
     def gemm_q8_static_dev(self, d_weights, d_acts, d_out, m, n, k, accumulate=False):
-        """gemm_q8_dev on the library's static device scratch: allocates nothing (shapes up to the scratch size)."""
+        """gemm_q8_dev on the library's static device scratch: allocates nothing (shapes whose gemm_least_workspace_bytes is at most
+        oxq_gemm_q8_static_max_workspace_bytes, 16 MiB)."""
         _check(self._lib.oxq_gemm_q8_static_dev(self.tensor_type, d_weights.data_ptr(), d_acts.data_ptr(),
                                                 d_out.data_ptr(), m, n, k, int(accumulate), raw_stream()))
 

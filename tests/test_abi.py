@@ -208,6 +208,25 @@ def test_gemm_workspace_size_is_a_function_of_the_shape():
     assert w(q6k, 64, 4864, 288) == 0
 
 
+def test_gemm_workspace_sizes_needed_and_best():
+    """The size that a call must have does not count the sums of parts of k that several work groups share (it decides what
+    oxq_gemm_q8_static_dev takes, and grows with the rows); the best size does, 64 MiB where a shape takes that kernel."""
+    lib = capi.load()
+    need, best, most = lib.oxq_gemm_q8_workspace_bytes, lib.oxq_gemm_q8_best_workspace_bytes, lib.oxq_gemm_q8_static_max_workspace_bytes()
+    q4k, q5k, q6k = 12, 13, 14
+    for t, m, n, k in ((q4k, 333, 11008, 4096), (q4k, 333, 4096, 14336), (q5k, 65, 28672, 4096), (q6k, 200, 4096, 11008)):
+        rows = (m + 127) // 128 * 128
+        per_block = max((rows + 128) * 46, rows * 74 if t == q4k else 0)
+        assert need(t, m, n, k) == (k // 32 * per_block + 255) // 256 * 256 <= most
+        assert best(t, m, n, k) == 64 << 20
+    assert need(q4k, 1100, 4096, 14336) > most and best(q4k, 1100, 4096, 14336) == 64 << 20
+    for t, m, n, k in ((q4k, 333, 4096, 4096), (q5k, 64, 28672, 4096), (8, 333, 11008, 4096), (q4k, 16, 14336, 4000)):
+        assert best(t, m, n, k) == need(t, m, n, k)
+    for t in (q4k, q5k, q6k):  # (beyond the few-token kernel's rows)
+        sizes = [need(t, m, 11008, 4096) for m in range(33, 2100)]
+        assert sizes == sorted(sizes)
+
+
 def test_quant_linear_hands_over_the_weight_as_it_is_at_the_call(monkeypatch):
     """The address, length and shape that a call passes are the weight's of that moment: its array resized or replaced,
     its bytes in another array type, its shape changed."""
