@@ -100,6 +100,16 @@ int main() {
                     const bool shared = oxq::deal_owner(begin, groups, units) != oxq::deal_owner(begin + per_tile - 1, groups, units);
                     ok = owner == rank_of[u] && slot_of[u] == (shared ? oxq::deal_slot(owner, begin, groups, units) : 2 * groups);
                 }
+                // whole rounds of tiles before the runs: every tile once, as a work group's own or by units of its runs
+                const uint32_t own = tiles / groups, tile0 = own * groups, rest = (tiles - tile0) * per_tile;
+                std::vector<uint32_t> had(tiles, 0);
+                for (uint32_t b = 0; ok && b < groups; b++) {
+                    const uint32_t rank = oxq::deal_rank(b, groups);
+                    const oxq::DealRange r = oxq::deal_range(rank, groups, rest);
+                    for (uint32_t i = 0; i < own; i++) had[rank * own + i] += per_tile;
+                    for (uint32_t u = r.begin; u < r.end; u++) had[tile0 + u / per_tile]++;
+                }
+                for (uint32_t h : had) ok = ok && h == per_tile;
                 deals++;
                 if (!ok) {
                     std::printf("%u tiles of %u units to %u work groups\n", tiles, per_tile, groups);

@@ -355,6 +355,77 @@ def test_f16_kernel_on_an_even_deal(hip, ref, tuning, t, shape):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("shape", [(258, 256 * 96 - 3, 2048), (130, 256 * 170 - 3, 1024), (130, 256 * 128, 512)],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q5_K, O.Q6_K], ids=lambda t: O.NAMES[t])
+def test_f16_even_deal_behind_whole_tiles(hip, ref, tuning, t, shape):
+    """A whole tile to each work group before its run, of two and three token tiles: runs of a unit, runs that cross tiles, and no
+    run at all (256 tiles, no second launch).  The large shape's bits where a tile is one work group's, nothing past the rows, 1e-5 of the
+    oracle for tokens of every token tile."""
+    if hip.device_info()["compute_units"] != 256:
+        pytest.skip("the whole tiles are those of 256 compute units")
+    m, n, k = shape
+    say("f16 even deal behind whole tiles", O.NAMES[t], shape)
+    w = O.random_blocks(t, 50 + m, n, k)
+    acts = ref.quantize_q8_0(synth.normal_f32(51, m * k))
+    kern = hip.HipKernel(t)
+    ws = torch.full((64 << 20,), 255, dtype=torch.uint8, device="cuda")  # (NaNs wherever nothing is stored)
+    dw, da = torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda()
+    dy, whole = (torch.full((m + 1, n), 7.0, dtype=torch.float32, device="cuda") for _ in range(2))
+    for y, variant, name in ((dy, 303, "gemm_f16_deal_kernel"), (whole, 301, "gemm_f16_kernel")):
+        tuning("gemm_variant", variant)
+        kern.gemm_q8_dev(dw, da, y, m, n, k, accumulate=False, workspace=ws)
+        assert last_launch().startswith(name), last_launch()
+    torch.cuda.synchronize()
+    assert bool((dy[m] == 7.0).all())
+    m_tiles = (m + 127) // 128
+    own = torch.zeros((m, n), dtype=torch.bool)  # the tiles before the runs: 256, the token tiles of a set of weight rows together
+    for tile in range(256):
+        own[tile % m_tiles * 128:(tile % m_tiles + 1) * 128, tile // m_tiles * 256:(tile // m_tiles + 1) * 256] = True
+    own = own.cuda()
+    assert torch.equal(dy[:m][own], whole[:m][own])
+    rows = sorted({0, 127, 128, 129, m // 2, m - 1})
+    y, want = dy[rows].cpu().numpy(), oracle_rows(ref, t, w, acts, n, k, rows)
+    assert (np.abs(y - want).max(axis=1) <= FP32_REL_TOL * np.abs(want).max(axis=1)).all()
+
+
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q5_K, O.Q6_K], ids=lambda t: O.NAMES[t])
+def test_f16_even_deal_on_infinite_block_scales(hip, ref, tuning, t):
+    """Infinite and NaN block scales in runs that several work groups share: infinities and NaNs where whole tiles have them,
+    every other token as without them."""
+    if hip.device_info()["compute_units"] != 256:
+        pytest.skip("the runs are those of 256 compute units")
+    m, n, k = 130, 300, 16384
+    say("f16 even deal, infinite scales", O.NAMES[t])
+    w = O.random_blocks(t, 73, n, k)
+    acts = ref.quantize_q8_0(synth.normal_f32(74, m * k)).reshape(m, k // 32, 34)
+    clean = acts.copy()
+    acts[3, 5, :2] = [0x00, 0x7C]    # +inf in one block of token 3
+    acts[7, 300, :2] = [0x00, 0xFC]  # -inf in another run of token 7
+    acts[129, :, :2] = [0x00, 0x7C]  # in all of token 129
+    acts[40, 511, :2] = [0x00, 0x7E]  # a NaN
+    kern = hip.HipKernel(t)
+    ws = torch.empty(64 << 20, dtype=torch.uint8, device="cuda")
+    dw = torch.from_numpy(w).cuda()
+
+    def product(a, v, name):
+        tuning("gemm_variant", v)
+        dy = torch.empty((m, n), dtype=torch.float32, device="cuda")
+        kern.gemm_q8_dev(dw, torch.from_numpy(a.reshape(-1)).cuda(), dy, m, n, k, accumulate=False, workspace=ws)
+        torch.cuda.synchronize()
+        assert last_launch().startswith(name), last_launch()
+        return dy.cpu().numpy()
+
+    deal, whole = product(acts, 303, "gemm_f16_deal_kernel"), product(acts, 301, "gemm_f16_kernel")
+    y_clean = product(clean, 303, "gemm_f16_deal_kernel")
+    for r in (3, 7, 40, 129):
+        assert not np.isfinite(whole[r]).any(), r
+        assert np.array_equal(np.isnan(deal[r]), np.isnan(whole[r])), r
+        assert np.array_equal(np.sign(deal[r][np.isinf(deal[r])]), np.sign(whole[r][np.isinf(whole[r])])), r
+    rest = [r for r in range(m) if r not in (3, 7, 40, 129)]
+    assert np.array_equal(deal[rest], y_clean[rest]) and np.isfinite(y_clean).all()
+
+
 @pytest.mark.parametrize("t,m,n,k,deal", [
     (O.Q4_K, 333, 4096, 14336, True), (O.Q4_K, 333, 4096, 4096, False), (O.Q5_K, 65, 28672, 4096, True),
     (O.Q5_K, 64, 28672, 4096, False), (O.Q6_K, 200, 4096, 4096, False), (O.Q6_K, 200, 4096, 11008, True),
