@@ -40,6 +40,7 @@
 // 42 / 51; Q5_K 2048 x 4096 x 14336 388 / 454, 512 x 4096 x 4096 48 / 54.
 #include "oxq_gemm_f16_util.hpp"
 #include "oxq_tile_order.hpp"
+#include "oxq_tile_rule.hpp"
 
 namespace oxq {
 namespace {
@@ -702,8 +703,7 @@ bool gemm_f16_deal_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
     if (!gemm_f16_supported(type, m, n, k) || m <= 64 || n < 256) return false;
     const int f = type == OXQ_TYPE_Q4_K ? 0 : type == OXQ_TYPE_Q5_K ? 1 : 2;
     const uint64_t groups = f16_deal_groups(), cus = device_cus(), n_super = k / 256;
-    auto tiles_of = [&](uint32_t t, uint32_t r) { return (uint64_t)((m + t - 1) / t) * ((n + r - 1) / r); };
-    const uint64_t tiles = tiles_of(128, 256), whole = tiles / groups, rest = tiles % groups;
+    const uint64_t tiles = tile_count(m, n, 128, 256), whole = tiles / groups, rest = tiles % groups;
     if (rest * n_super < groups) return false;
     // tenths of a microsecond
     static constexpr uint32_t RAMP[3] = {175, 203, 209}, RUN[3] = {69, 74, 95};
@@ -714,15 +714,13 @@ bool gemm_f16_deal_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
     if (gemm_prefill_supported(type, m, n, k) && gemm_prefill_pays(m, n)) {
         per_round = PREFILL, wgs = tiles;
     } else if (const int shape = gemm_f16_shape(type, m, n, k)) {
-        per_round = shape == 1 ? LARGE[f] : SMALL[f], wgs = shape == 1 ? tiles : tiles_of(64, 128);
-    } else if (m > 384 && k <= 16384 && tiles_of(128, 64) >= cus) {  // (the tile kernel's shapes: launch_tiles)
-        wgs = tiles_of(128, 128);
-        const bool square = 2 * wgs >= 3 * cus || (2 * wgs > cus && wgs <= cus && (f != 0 || k >= 8192));
-        per_round = square ? T128X128[f] : T128X64[f];
-        if (!square) wgs = tiles_of(128, 64);
-    } else if (k <= 32768) {
-        const bool wide = !(m > 384 && k <= 16384) && 4 * tiles_of(64, 128) >= 7 * cus;
-        per_round = wide ? T64X128[f] : T64X32[f], wgs = wide ? tiles_of(64, 128) : tiles_of(64, 32);
+        per_round = shape == 1 ? LARGE[f] : SMALL[f], wgs = shape == 1 ? tiles : tile_count(m, n, 64, 128);
+    } else if (tile_big(m, n, k, 1, cus)) {
+        const bool square = tile_square(type, tile_count(m, n, 128, 128), k, cus);
+        per_round = square ? T128X128[f] : T128X64[f], wgs = tile_count(m, n, 128, square ? 128 : 64);
+    } else if (tile_scales_fit(k, 64)) {
+        const bool wide = !tile_narrow(m, n, k, 1, cus) && tile_mid_wide(32 * tile_count(m, n, 64, 128), cus);
+        per_round = wide ? T64X128[f] : T64X32[f], wgs = tile_count(m, n, 64, wide ? 128 : 32);
     } else {
         return false;
     }

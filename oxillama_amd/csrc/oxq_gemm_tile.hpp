@@ -31,6 +31,7 @@
 #include "oxq_gemv_kernel.hpp"
 #include "oxq_internal.hpp"
 #include "oxq_tile_order.hpp"
+#include "oxq_tile_rule.hpp"
 
 namespace oxq {
 
@@ -917,15 +918,13 @@ static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t
     (void)variant;  // (read by the fixed-shape knobs, which the second translation unit leaves out)
     // The f16 token scales of a work group's tokens for the whole k sit in LDS (k / 32 * 2 bytes per token): 128-token
     // tiles up to k = 16384, 64-token tiles up to 32768, 32-token tiles beyond (up to 65536).
-    const uint32_t nsb_pad = tile_padded_sub_blocks(a.k);
-    const bool fits128 = (size_t)nsb_pad * 256 <= 128 * 1024, fits64 = (size_t)nsb_pad * 128 <= 128 * 1024;
+    const bool fits64 = tile_scales_fit(a.k, 64);
+    const size_t cus = device_cus(), groups = a.offsets ? a.n_experts : 1;
     // more than 384 tokens on a matrix so narrow that even 128 x 64 tiles leave compute units without one (the key /
     // value projections of grouped-query attention): the 64 x 32 split-k tiles of the mid range -- 1024 x 4096 at
     // 512 / 1024 tokens 20.7 / 30.7 us against 45.7 / 49.0, 1024 x 8192 Q8_0 35.7 against 98.9, 3072 x 3072 30.7
     // against 38.5; from one tile per compute unit on (1024 x 4096, 2048 tokens) a tie
-    const bool narrow = rows > 384 && fits128 &&
-                        (size_t)((rows + 127) / 128) * ((a.n + 63) / 64) * (a.offsets ? a.n_experts : 1) < (size_t)device_cus();
-    const bool big = rows > 384 && fits128 && !narrow;
+    const bool narrow = tile_narrow(rows, a.n, a.k, groups, cus), big = tile_big(rows, a.n, a.k, groups, cus);
     const bool mid = !big && rows > 64 && fits64;
     // 65..384 tokens (more where k is too long for the 128-token tiles): 64 x 128 tiles (a wave per 32 weight rows)
     // where they give the chip 1.75 work groups per compute
@@ -934,8 +933,8 @@ static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t
     // 196 / 198 / 206 against 66 / 125 / 183; 4096 x 4096 Q4_K 44 / 45 / 48 against 19 / 27 / 37, Q8_0 51 / 51 / 54
     // against 21 / 33 / 46; 14336 x 4096 Q4_K 128 / 192 tokens 49 / 70 against 45 / 63, 256 a tie, 384 108 against 113.
     const size_t row_tiles = (a.n + 127) / 128, group_32 = tiles64 ? tiles64 : 32 * ((rows + 63) / 64);
-    const uint32_t line_32 = !tiles64 ? 56 : F::BLOCK_BYTES >= 210 ? 112 : 90;  // 32nds of a tile, per compute unit
-    bool wide_grid = group_32 * row_tiles * (a.offsets ? a.n_experts : 1) >= line_32 * (size_t)device_cus();
+    const uint32_t line_32 = !tiles64 ? TILE_MID_WIDE_LINE : F::BLOCK_BYTES >= 210 ? 112 : 90;
+    bool wide_grid = tile_mid_wide(group_32 * row_tiles * groups, cus, line_32);
     // Expert groups, whose tiles are part empty, follow the same line (a full chip, 64 x 128 against 64 x 32 split, Q4_K: 8 of
     // 4096 x 14336 at a mean of 80 / 96 rows 230 against 295 / 228 against 299, of 6144 x 2048 59 against 69, 128 of 1536 x 3072
     // at 96 349 against 379; Q6_K 8 of 4096 x 14336 at 96 366 against 428).  But:
@@ -998,7 +997,7 @@ static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t
             // 128 x 128 tiles (two waves per SIMD, weight bytes fetched two steps ahead) where they still give the
             // chip one and a half work groups per compute unit: 14336 x 4096, 512 tokens 123 us against 125 us,
             // 2048 tokens 383 us against 422 us; 4096 x 14336 has too few such tiles (214 us against 140 us)
-            const size_t wgs = (size_t)((rows + 127) / 128) * ((a.n + 127) / 128) * (a.offsets ? a.n_experts : 1);
+            const size_t wgs = tile_count(rows, a.n, 128, 128) * groups;
             // Within the 128 x 128 tile a wave takes 128 tokens x 32 rows (four token tiles against ONE weight-row
             // tile) rather than 64 x 64: half the weight loads per MFMA, and those are the loads in which every lane
             // reads its own row.  Same bits.  512 x 14336 x 4096: Q8_0 122 us against 158, Q4_0 122 against 141,
@@ -1009,13 +1008,12 @@ static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t
             // with two of them takes twice as long as one with one, so 129..256 of the larger tiles, one per compute
             // unit, finish first (4096 x 14336, 768 tokens: Q8_0 248 us against 348, Q6_K 339 against 397, Q4_K 228
             // against 266; 1024 tokens Q6_K 368 against 421)
-            const size_t cus = device_cus();
             // (Q4_K on rows of 4096 columns is the exception: 4096 x 4096, 768 / 1024 tokens 72 / 77 us against 76 / 82)
-            if (2 * wgs >= 3 * cus || (2 * wgs > cus && wgs <= cus && (wide || a.k >= 8192)))
+            if (tile_square(F::TYPE, wgs, a.k, cus))
                 return wide ? launch_tile<F, 4, 1, 1, 1, false>(a, p, stream) : launch_tile<F, 2, 2, 2, 2, false>(a, p, stream);
             // one to one and a half work groups per compute unit: still the better shape for the formats of a
             // byte and more per weight (512 x 8192 x 8192 Q8_0: 149 us against 180)
-            if (wide && F::BLOCK_BYTES >= 256 && wgs >= (size_t)device_cus()) return launch_tile<F, 4, 1, 1, 1, false>(a, p, stream);
+            if (wide && F::BLOCK_BYTES >= 256 && wgs >= cus) return launch_tile<F, 4, 1, 1, 1, false>(a, p, stream);
             return launch_tile<F, 2, 1, 2, 1, false, 3>(a, p, stream);
         }
         if (mid)
@@ -1023,12 +1021,11 @@ static hipError_t launch_tiles(const GemmArgs &a, const TilePlan &p, hipStream_t
         if (short_groups) return launch_tile<F, 2, 1, 1, 2, false>(a, p, stream);
         // split k; 64 weight rows (or 64 tokens) per work group only where that still leaves every
         // compute unit at least one work group, else 32 x 32
-        const size_t groups = a.offsets ? a.n_experts : 1;
         // 33..64 tokens: one 64-token tile where 32-row tiles still give every compute unit a work group
         // (14336 x 4096, 64 rows: 26.6 us against 31.1 with 32 x 32 tiles; 4096 rows: 61 against 50)
-        if (rows > 32 && fits64 && (size_t)((a.n + 31) / 32) * groups >= device_cus())
+        if (rows > 32 && fits64 && (size_t)((a.n + 31) / 32) * groups >= cus)
             return launch_tile<F, 2, 1, 0, 2, false, 2, 2>(a, p, stream);
-        if ((size_t)((a.n + 63) / 64) * groups < device_cus())
+        if ((size_t)((a.n + 63) / 64) * groups < cus)
             return launch_tile<F, 1, 1, 0, 2, false, 2, 2>(a, p, stream);
         if (rows > 32 && fits64) return launch_tile<F, 2, 1, 0, 2, false, 2, 2>(a, p, stream);
         // (also: any number of tokens on rows of more than 32768 columns)
