@@ -11,6 +11,7 @@
 
 #include "oxq_internal.hpp"
 #include "oxq_lds_opt_in.hpp"
+#include "oxq_scratch.hpp"
 
 namespace oxq {
 hipError_t launch_dequant(uint32_t type, const uint8_t *blocks, size_t n_blocks, float *out, hipStream_t stream);
@@ -58,25 +59,25 @@ int fail_hip(hipError_t e, const char *what) {
         if (e_ != hipSuccess) return fail_hip(e_, #call); \
     } while (0)
 
-// A growable device buffer.
-struct Scratch {
-    void *ptr = nullptr;
-    size_t cap = 0;
+struct Scratch : oxq::ScratchBuffer {
     int reserve(size_t n) {
-        if (n <= cap) return OXQ_OK;
-        if (ptr) (void)hipFree(ptr);
-        ptr = nullptr;
-        cap = 0;
-        size_t want = n + n / 4 + 256;
-        hipError_t e = hipMalloc(&ptr, want);
-        if (e != hipSuccess) return fail_hip(e, "hipMalloc(scratch)");
-        cap = want;
-        return OXQ_OK;
+        size_t got;
+        return reserve(n, n, &got);
+    }
+    // *got: `best` bytes, or `need` where the device has no more
+    int reserve(size_t best, size_t need, size_t *got) {
+        int e = 0;
+        *got = grow(best, need, e,
+                    [](void **p, size_t n) {
+                        const hipError_t st = hipMalloc(p, n);
+                        if (st != hipSuccess) (void)hipGetLastError();  // (else the next launch would report it)
+                        return (int)st;
+                    },
+                    [](void *p) { (void)hipFree(p); });
+        return e == 0 ? OXQ_OK : fail_hip((hipError_t)e, "hipMalloc(scratch)");
     }
     void release() {
-        if (ptr) (void)hipFree(ptr);
-        ptr = nullptr;
-        cap = 0;
+        ScratchBuffer::release([](void *p) { (void)hipFree(p); });
     }
 };
 
@@ -770,10 +771,11 @@ static int gemm_host(uint32_t type, const uint8_t *data, size_t data_len, const 
     ga.workspace = nullptr;
     if (oxq::gemm_uses_tiles(type, (uint32_t)m, (uint32_t)n_rows, (uint32_t)n_cols) ||
         oxq::gemm_few_rows_pay(type, (uint32_t)m, (uint32_t)n_rows, (uint32_t)n_cols)) {
-        const size_t wbytes = oxq::gemm_best_workspace_bytes((uint32_t)m, (uint32_t)n_cols, (uint32_t)n_rows, type);
-        if ((st = g.s_work.reserve(wbytes)) != OXQ_OK) return st;
+        const uint32_t mm = (uint32_t)m, nn = (uint32_t)n_rows, kk = (uint32_t)n_cols;
+        if ((st = g.s_work.reserve(oxq::gemm_best_workspace_bytes(mm, kk, nn, type), oxq::gemm_workspace_bytes(mm, kk, nn, type),
+                                   &ga.workspace_bytes)) != OXQ_OK)
+            return st;
         ga.workspace = (uint8_t *)g.s_work.ptr;
-        ga.workspace_bytes = wbytes;
     }
     ga.m = (uint32_t)m;
     ga.n = (uint32_t)n_rows;
@@ -1026,9 +1028,8 @@ static int gemm_dev(uint32_t type, const uint8_t *d_weights, const uint8_t *d_ac
         // the scratch is shared.
         const size_t best = d_sums ? need : oxq::gemm_best_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type);
         std::lock_guard<std::mutex> lock(g.mu);
-        if ((st = g.s_work.reserve(best)) != OXQ_OK) return st;
+        if ((st = g.s_work.reserve(best, need, &ga.workspace_bytes)) != OXQ_OK) return st;
         ga.workspace = (uint8_t *)g.s_work.ptr;
-        ga.workspace_bytes = best;
         OXQ_HIP(oxq::launch_gemm_q8(type, ga, (hipStream_t)stream));
         OXQ_HIP(hipStreamSynchronize((hipStream_t)stream));
         return OXQ_OK;

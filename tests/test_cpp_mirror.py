@@ -1,7 +1,7 @@
 """Runs tests/cpp/test_quant_kernel.bin: the reference crate's own unit tests replayed
 through the C++ mirror of its interface (include/oxq/quant_kernel.hpp -> C ABI), and the
-host tests beside it: the kernels' LDS limits asked for by several threads, and the order
-in which work groups take tiles."""
+host tests beside it: the kernels' LDS limits asked for by several threads, the order
+in which work groups take tiles, and the library's scratch on a full device."""
 import os
 import subprocess
 
@@ -27,6 +27,10 @@ def test_lds_limits_are_only_raised():
 
 def test_tiles_are_dealt_evenly_to_the_xcds():
     _run(binary=os.path.join(CPP, "test_tile_order.bin"))
+
+
+def test_scratch_falls_back_to_what_a_call_needs():
+    _run(binary=os.path.join(CPP, "test_scratch.bin"))
 
 
 def test_cpp_mirror_host_cases():
