@@ -876,10 +876,22 @@ static hipError_t launch_tile(const GemmArgs &a, const TilePlan &p, hipStream_t 
     // (333 x 4096 x 4096, 768 work groups for 512 places, us without short tiles / with them in their set's place / at the end: Q5_K
     // 39.2 / 43.5 / 38.6, Q4_K 34.4 / 37.7 / 33.9; 145 x 8192 x 2048 Q4_0 26.0 / 29.4 / 24.3; ten matrices at 145 to 345 rows, twelve
     // formats, in the mean 0.98 / 0.94 of the first, at worst 1.14 / 1.04).  Two token tiles stay in their sets, where they share the weights'
-    // reads: 77 x 11008 x 4096 Q4_0 41.4 / 38.8 / 43.6, 8960 x 1536 23.3 / 22.5 / 20.1.
+    // reads: 77 x 11008 x 4096 Q4_0 41.4 / 38.8 / 43.6, 8960 x 1536 23.3 / 22.5 / 20.1.  So do (at the end against in place; fifteen
+    // matrices at 129 to 350 rows, of which the rest are 0.95 in the mean)
+    //   - formats of a byte and more per weight, whose second reading of the weights is the dearest: Q8_0 1.01 in the mean, 129 x
+    //     13824 x 5120 89 against 82
+    //   - 64 x 128 tiles of which the full ones alone are more than a round: 333 x 13824 x 5120 Q4_0 147 against 137, IQ4_NL 138 / 133
+    //     (up to a round, 260 x 13824 x 5120, 0.94)
+    //   - grids of a few tiles more than whole rounds, which end with those rounds as their short ones are in place: 129 x 11008 x
+    //     4096, 1032 tiles, Q4_1 57 against 53, Q5_K 45.6 / 43
+    //   - the formats of 32-weight blocks on rows of more than 12288 columns: 333 x 5120 x 13824 Q4_0 174 against 164, IQ4_NL 171 / 161, x
+    //     4096 x 14336 Q5_0 149 / 145 (the others there, Q3_K, Q2_K, IQ4_XS, 0.9)
     const uint32_t left = a.m % WG_TOK;
-    const bool short_last = tile_short_body<MT, WM, DUMP>() && m_tiles > 2 && left >= 1 && left <= 32 &&
-                            (size_t)m_tiles * n_tiles > 2 * (size_t)device_cus();
+    const size_t round = 2 * (size_t)device_cus(), tiles = (size_t)m_tiles * n_tiles, full = tiles - n_tiles;
+    const bool long_rows = tile_ragged_k<F>::value && a.k > 12288;
+    const bool one_round = full <= round, just_over = tiles % round >= 1 && tiles % round <= round / 16;
+    const bool short_last = tile_short_body<MT, WM, DUMP>() && m_tiles > 2 && left >= 1 && left <= 32 && tiles > round &&
+                            F::BLOCK_BYTES < 256 && !long_rows && (one_round || (WM == 0 && !just_over));
     const TileGrid tg = short_last ? tile_order_grid3_short_last(m_tiles, n_tiles) : tile_order_grid3(m_tiles, n_tiles);
     const dim3 grid = a.offsets ? dim3(n_tiles * m_tiles) : dim3(tg.x, tg.y, tg.z);
     const size_t lds = (size_t)tile_padded_sub_blocks(a.k) * WG_TOK * 2;

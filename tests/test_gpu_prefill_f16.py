@@ -498,7 +498,7 @@ def test_tiles_of_at_most_32_rows(hip, ref, tuning, t, k, variant):
 
 
 @pytest.mark.parametrize("variant,n", [(23, 5600), (16, 22400)])
-@pytest.mark.parametrize("t", [O.Q4_K, O.Q8_0], ids=lambda t: O.NAMES[t])
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q4_0], ids=lambda t: O.NAMES[t])
 def test_short_tiles_behind_the_others(hip, ref, tuning, t, variant, n):
     """Grids of more tiles than the chip holds at a time (175 sets of weight rows, which the XCDs do not share evenly) launch a
     third, short token tile last: the bits of full tiles, every tile once, nothing past the rows, 1e-5 of the oracle."""
