@@ -32,7 +32,8 @@ int oxq_set_gemm_tile_min_rows(unsigned rows);
  * per shape).  1..23: a fixed tile shape / prefetch depth of the int8-MFMA tile kernel; 99: the tile kernel's own
  * choice, never the few-token kernel nor the prefill kernel; 300: the prefill kernel (f16 matrix cores, Q4_K) for any
  * number of token rows; 301, 302: the f16 matrix-core kernel without a preparation launch (Q4_K, Q5_K, Q6_K) in its large
- * and its small shape; 200..205: the
+ * and its small shape, 303: the large one on an even deal of the parts of k (a workspace of 64 MiB, which the size queries
+ * count only for shapes that take it by default, and a part of k for every compute unit, else the default choice); 200..205: the
  * few-token kernel (16 x 16 x 32 MFMA, groups of at most 32 token rows) in a fixed shape; 206: its form that holds the
  * whole k of up to 16 token rows in LDS.  A value a format or
  * shape cannot take falls back to the default tile choice. */

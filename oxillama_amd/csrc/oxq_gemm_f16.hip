@@ -21,9 +21,12 @@
 // prompts' grids lie between rounds (333 rows on 11008 weight rows: 129 tiles for 256 compute units).  Here a work group per
 // compute unit takes the same number of whole tiles and then a run of (tile, super-block) units of the rest; a tile that
 // several have runs of is added up by a second launch, in the order of k.  What it costs: a ramp of the pipeline per run and 128 KB
-// of sums, 32 to 64 MB written together at the end and read by the second launch (8 to 11 us): 128 x 4096 x 14336, Q4_K,
-// runs of four super-blocks, 36 us + 8, where whole tiles take 5.8 per super-block.  Storing the sums past the caches: no gain
-// (333 x 11008 x 4096 77 us against 75).
+// of sums, 32 to 64 MB written together at the end and read by the second launch (9 to 14 us: 10 of 96 tiles of 333 x 4096 x
+// 11008, 14 of 129 of 333 x 11008 x 4096): 128 x 4096 x 14336, Q4_K, runs of four super-blocks, 36 us + 8, where whole tiles take 5.8
+// per super-block.  And registers: what a work group keeps from run to run takes Q5_K and Q6_K over the 256 there are (ten and
+// eighteen spilled, 44 and 76 bytes of scratch a lane; without the deal one and none), part of why a super-block of a run is
+// 7.4 / 9.5 us where it is 6.2 / 7.6 of a whole tile.  Storing the sums past the caches: no gain (333 x 11008 x 4096 77 us
+// against 75).
 //
 // Shapes: MT token tiles of 32 against RW waves of 32 rows, KS parts of k; eight waves, one work group per compute unit.
 //   (4, 8, 1)  128 tokens x 256 rows: the least unpacking and staging per result
@@ -688,18 +691,21 @@ int gemm_f16_shape(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
 // Whether a call takes the even deal: where its time, estimated, is less than that of the kernel that the call would take
 // otherwise.  Both are lines through measured times (294 calls with 40 to 2048 rows, 768 to 28672 weight rows and columns):
 //   the deal     17 / 20 / 21 us (Q4_K / Q5_K / Q6_K) for the ramp, the exchange of up to 64 MB of sums and the second launch,
-//                6.9 / 7.4 / 9.5 per super-block of the longest run, 8 where whole tiles go before the runs; nine calls in ten within 10 %
+//                6.9 / 7.4 / 9.5 per super-block of the longest run, 8 where whole tiles go before the runs
 //   the others   a time per round of the chip and 4096 columns, the least that was measured for the shape (the calls with
 //                short rows and partly used tiles take up to a third more): the prefill kernel 90, this kernel's whole
 //                tiles 100 / 122 (Q5_K / Q6_K) and 38 / 43 / 45.6 (small), the tile kernel 57 / 57 / 88 (128 x 128 tiles), 30 / 33
 //                / 53 (128 x 64), 33 / 37.5 / 50 (64 x 128), 9.7 / 11.3 / 14.7 (64 x 32, k split)
-// so that the line errs towards the kernels with whole tiles.  On those 294 calls the mean is 8 % less, the best choice of
-// each 10 % less, and the worst of the calls that change loses 3 %.  us, before and now: Q4_K 333 x 11008 x 4096 93 and 75, 1100 x
-// 4096 x 14336 384 and 225, 512 x 4096 x 14336 126 and 104; Q5_K 333 x 11008 x 4096 105 and 82; Q6_K 333 x 4096 x 11008 135 and 97, 768
-// x 4096 x 14336 307 and 209, 1100 x 4096 x 4096 143 and 104.  Q4_K 333 x 4096 x 4096, where runs are three super-blocks, stays (33, 38).
+// so that the line errs towards the kernels with whole tiles.  On 529 other calls (profiles/even_deal_against_other_kernels.txt) four
+// estimates of the deal in five are within 10 %, the mean over the calls is 8 % less than without the deal, the best choice of
+// each 9 % less, and the worst of the 208 calls that take it loses 5 % (Q4_K 200 x 14336 x 4096 64 us, 61).  us, without and with it: Q4_K
+// 333 x 11008 x 4096 77 and 75, 1100 x 4096 x 14336 390 and 221, 512 x 4096 x 14336 121 and 102; Q5_K 333 x 11008 x 4096 92 and 81; Q6_K
+// 333 x 4096 x 11008 127 and 96, 768 x 4096 x 14336 324 and 206, 1100 x 4096 x 4096 143 and 102.  Q4_K 333 x 4096 x 4096, where runs are three
+// super-blocks, stays (33, 40).
 bool gemm_f16_deal_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
-    // (a token tile half empty, against 32-token tiles; matrices narrower than a tile keep the kernel whose fp32 sums the
-    // dump of the integer sums repeats bit for bit)
+    // (a token tile half empty, against 32-token tiles.  Matrices narrower than a tile: not for the time, which the deal would
+    // more than halve on long rows -- 333 x 128 x 28672 Q4_K 74 us against 32, 1024 x 192 x 14336 Q6_K 59 against 34 -- but because
+    // there a call's fp32 sums are those of the integer sums' dump, bit for bit, and are held to it)
     if (!gemm_f16_supported(type, m, n, k) || m <= 64 || n < 256) return false;
     const int f = type == OXQ_TYPE_Q4_K ? 0 : type == OXQ_TYPE_Q5_K ? 1 : 2;
     const uint64_t groups = f16_deal_groups(), cus = device_cus(), n_super = k / 256;

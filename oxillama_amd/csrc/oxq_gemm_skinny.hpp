@@ -1136,14 +1136,16 @@ static int skinny_shape(const GemmArgs &a, bool has_partial, uint32_t rows, int 
     return SK_NONE;
 }
 
-// <NT, WAVES, TT, PER>; LDS = PER * 8 * TT * 640 + WAVES * NT * 7 KB
+// <NT, WAVES, TT, PER>; LDS = PER * 8 * TT * (672, two factors to a block 736, with a zero-point term 864) + WAVES * NT * 5.3 to 8.5 KB.
+// The shapes that calls take by default are made for two work groups on a compute unit.
 template <class F>
 static hipError_t launch_skinny(const GemmArgs &a, const TilePlan &p, hipStream_t stream, int shape) {
     if constexpr (Skinny<F>::OK)
         if (shape == SK_WHOLE) return launch_skinny_whole<F>(a, stream);
     if constexpr (Skinny<F>::OK && Skinny<F>::ONE_TILE) {
         // Q6_K, Q8_0: 8 KB of LDS and more per wave; with chunks of two super-blocks of one token tile two work
-        // groups still share a compute unit (75 and 78 KB each)
+        // groups still share a compute unit (74 and 79 KB each)
+        static_assert(skinny_waves_per_simd<F, 1, 8, 1, 2>() == 4, "two work groups in a compute unit's LDS");
         switch (shape) {
         case SK_1_4:
         case SK_1_8: return a.sums ? launch_skinny_shape<F, 1, 8, 1, 2, true>(a, p, stream) : launch_skinny_shape<F, 1, 8, 1, 2>(a, p, stream);
@@ -1152,6 +1154,8 @@ static hipError_t launch_skinny(const GemmArgs &a, const TilePlan &p, hipStream_
         default: break;
         }
     } else if constexpr (Skinny<F>::OK) {
+        static_assert(skinny_waves_per_simd<F, 1, 8, 1, 4>() == 4 && skinny_waves_per_simd<F, 1, 8, 2, 2>() == 4,
+                      "two work groups in a compute unit's LDS");
         switch (shape) {
         case SK_1_4: return a.sums ? launch_skinny_shape<F, 1, 8, 1, 4, true>(a, p, stream) : launch_skinny_shape<F, 1, 8, 1, 4>(a, p, stream);
         case SK_2_2: return a.sums ? launch_skinny_shape<F, 1, 8, 2, 2, true>(a, p, stream) : launch_skinny_shape<F, 1, 8, 2, 2>(a, p, stream);
