@@ -460,6 +460,46 @@ def test_f16_even_deal_by_default(hip, ref, t, m, n, k, deal):
         assert np.abs(got.cpu().numpy()[rows] - y_ref).max() <= FP32_REL_TOL * np.abs(y_ref).max()
 
 
+def test_workspaces_of_a_shape_on_the_even_deal(hip, ref):
+    """What a call must have and what it runs best with: refused below the first with that size, on the other kernels below the
+    second, on the deal from there on, without a workspace, and in a captured graph."""
+    if hip.device_info()["compute_units"] != 256:
+        pytest.skip("the lines are of 256 compute units")
+    t, m, n, k = O.Q4_K, 333, 4096, 14336
+    say("workspaces of the even deal")
+    kern = hip.HipKernel(t)
+    least, best = kern.gemm_least_workspace_bytes(m, n, k), kern.gemm_workspace_bytes(m, n, k)
+    assert least <= capi.load().oxq_gemm_q8_static_max_workspace_bytes() < best == 64 << 20
+    acts = ref.quantize_q8_0(synth.normal_f32(98, m * k))
+    dw, da = torch.from_numpy(O.random_blocks(t, 97, n, k)).cuda(), torch.from_numpy(acts).cuda()
+    ws = torch.empty(best, dtype=torch.uint8, device="cuda")
+    want, got = (torch.empty((m, n), dtype=torch.float32, device="cuda") for _ in range(2))
+    with pytest.raises(hip.BufferTooSmall) as e:
+        kern.gemm_q8_dev(dw, da, got, m, n, k, workspace=ws[:least - 256])
+    assert (e.value.needed, e.value.available) == (least, least - 256)
+    for size, deal in ((least, False), (best - 256, False), (best, True)):
+        kern.gemm_q8_dev(dw, da, want, m, n, k, workspace=ws[:size])
+        assert last_launch().startswith("gemm_f16_deal_kernel") == deal, (size, last_launch())
+    for call in (lambda: kern.gemm_q8_dev(dw, da, got, m, n, k), lambda: kern.gemm_q8_static_dev(dw, da, got, m, n, k)):
+        got.zero_()
+        call()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        kern.gemm_q8_dev(dw, da, got, m, n, k, workspace=ws)
+    for _ in range(3):
+        got.zero_()
+        ws.fill_(255)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+    big = 1100  # (more than the static form's limit, though its array would hold the sums)
+    with pytest.raises(hip.BufferTooSmall) as e:
+        kern.gemm_q8_static_dev(dw, da, got, big, n, k)
+    assert (e.value.needed, e.value.available) == (kern.gemm_least_workspace_bytes(big, n, k), 16 << 20)
+
+
 @pytest.mark.parametrize("variant", [16, 23])
 @pytest.mark.parametrize("t,k", [(O.Q4_K, 1024), (O.Q6_K, 768), (O.Q4_0, 1056), (O.IQ4_XS, 1280)], ids=lambda v: str(v))
 def test_tiles_of_at_most_32_rows(hip, ref, tuning, t, k, variant):
