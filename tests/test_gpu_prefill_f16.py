@@ -537,6 +537,32 @@ def test_tiles_of_at_most_32_rows(hip, ref, tuning, t, k, variant):
     assert np.abs(full.cpu().numpy()[rows] - want).max() <= FP32_REL_TOL * np.abs(want).max()
 
 
+@pytest.mark.parametrize("variant", [16, 23])
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q6_K, O.Q8_0], ids=lambda t: O.NAMES[t])
+def test_short_tiles_of_many_experts(hip, ref, tuning, t, variant):
+    """150 experts of 0 to 130 rows (three scans of 64), their tiles of at most 32 rows behind the others or not: every row is the
+    plain matmul's, bit for bit, and nothing is stored past the last."""
+    n, k, e = 129, 256, 150
+    say("short tiles of many experts", O.NAMES[t], variant)
+    rng = np.random.default_rng(7 + variant)
+    groups = rng.permutation(np.concatenate([rng.integers(0, 131, e - 12), [0, 1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129]]))
+    offsets = np.concatenate([[0], np.cumsum(groups)]).astype(np.int32)
+    m = int(offsets[-1])
+    tuning("gemm_variant", variant)
+    tuning("gemm_tile_min_rows", 1)
+    w = O.random_blocks(t, 79, n, k).reshape(-1)
+    acts = ref.quantize_q8_0(synth.normal_f32(80, m * k))
+    kern = hip.HipKernel(t)
+    dw, da = torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda()
+    want = torch.empty((m, n), dtype=torch.float32, device="cuda")
+    ws = torch.empty(max(kern.gemm_workspace_bytes(m, n, k), kern.moe_gemm_workspace_bytes(m, n, k)), dtype=torch.uint8, device="cuda")
+    kern.gemm_q8_dev(dw, da, want, m, n, k, accumulate=False, workspace=ws)
+    y = torch.full((m + 1, n), 7.0, dtype=torch.float32, device="cuda")
+    kern.moe_gemm_q8_dev(dw.repeat(e), w.nbytes, e, da, torch.from_numpy(offsets).cuda(), m, int(groups.max()), y, n, k, ws)
+    assert last_launch().startswith("gemm_tile_kernel"), last_launch()
+    assert torch.equal(y[:m], want) and bool((y[m] == 7.0).all())
+
+
 @pytest.mark.parametrize("variant,n", [(23, 5600), (16, 22400)])
 @pytest.mark.parametrize("t", [O.Q4_K, O.Q4_0], ids=lambda t: O.NAMES[t])
 def test_short_tiles_behind_the_others(hip, ref, tuning, t, variant, n):
