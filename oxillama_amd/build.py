@@ -31,6 +31,9 @@ HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall", "-Wno-unused-function",
+    # kernel arguments arrive in scalar registers with the launch instead of by a first load of each wave: 0.1 to 0.15 us a
+    # launch (four decode layers of an 8B model, 24 launches: 178.2 us to 175.2; vocabulary projection and sampler 103.2 / 101.8)
+    "-mllvm", "-amdgpu-kernarg-preload-count=16",
 ]
 
 
