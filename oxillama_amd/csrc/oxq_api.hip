@@ -1013,6 +1013,7 @@ static int gemm_dev(uint32_t type, const uint8_t *d_weights, const uint8_t *d_ac
         (reinterpret_cast<uintptr_t>(d_workspace) & 255) == 0)
         tiles = true;
     ga.by_rows = !tiles;
+    ga.few_rows_direct = !tiles && d_workspace && !d_sums && oxq::gemm_direct_few_rows_pay(type, (uint32_t)m, (uint32_t)n, (uint32_t)k);
     const size_t need = tiles ? oxq::gemm_workspace_bytes((uint32_t)m, (uint32_t)k, (uint32_t)n, type) : 0;
     if (need && d_workspace) {
         if (workspace_bytes < need) return fail(OXQ_ERR_BUFFER_TOO_SMALL, need, workspace_bytes, "workspace too small");
@@ -1075,6 +1076,7 @@ int oxq_gemm_q8_static_dev(uint32_t type, const uint8_t *d_weights, const uint8_
     ga.workspace_bytes = tiles ? STATIC_DEAL_BYTES : 0;
     ga.workspace = tiles ? static_scratch_ptr[device] : nullptr;    // every byte the tile kernel reads is written
     ga.by_rows = !tiles;                                            // by the preparation kernel of this same call
+    ga.few_rows_direct = !tiles && oxq::gemm_direct_few_rows_pay(type, (uint32_t)m, (uint32_t)n, (uint32_t)k);
     ga.m = (uint32_t)m;
     ga.n = (uint32_t)n;
     ga.k = (uint32_t)k;

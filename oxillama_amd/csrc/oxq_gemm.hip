@@ -187,6 +187,22 @@ static hipError_t gemm_grouped_by_gemv(uint32_t type, const GemmArgs &a, hipStre
     return launch_gemv_q8(type, g, stream);
 }
 
+// Fewer rows than the tile kernel's threshold on matrices below 2^25 weights: from the second GEMV pass on (as gemm_few_rows_pay)
+// the kernel that takes the weights straight into registers is the faster one (Q4_K 2560 x 2560, 5 to 8 rows: 15.8 us against 5.4).
+// For device calls that bring a workspace; the host route's batched results are its GEMV's.
+bool gemm_direct_few_rows_pay(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
+    return g_gemm_tile_min_rows.load(std::memory_order_relaxed) == 0 && g_gemm_variant.load(std::memory_order_relaxed) == 0 &&
+           gemm_direct_pays(type, m, n, k) && (uint64_t)n * k < (1ull << 25) && m >= (gemv_vecs_max(type, k) <= 2 ? 3u : 5u);
+}
+// Whether a call that would take the few-token or the tile kernel takes that one instead.
+static bool gemm_direct_takes(uint32_t type, const GemmArgs &a) {
+    const int variant = g_gemm_variant.load(std::memory_order_relaxed);
+    if (variant == 207) return true;
+    // (the dump of the integer sums of matrices small enough for the whole-k kernel stays on the kernels that had it)
+    return variant == 0 && !a.scaled_sums && gemm_direct_pays(type, a.m, a.n, a.k) &&
+           (!a.sums || !skinny_whole_pays(type, a.n, a.k, skinny_splits(a.n, a.k) >= 2));
+}
+
 hipError_t launch_gemm_q8(uint32_t type, const GemmArgs &a, hipStream_t stream) {
     if (a.offsets && !a.sums && !a.bias && a.m <= grouped_gemv_max_rows(a.n_experts) && a.n_experts <= 4096 &&
         g_gemm_variant.load(std::memory_order_relaxed) == 0) {
@@ -194,6 +210,10 @@ hipError_t launch_gemm_q8(uint32_t type, const GemmArgs &a, hipStream_t stream) 
         if (e != hipErrorNotSupported) return e;
     }
     const bool tiles = a.workspace != nullptr && gemm_tiles_supported(type, a.m, a.k) && (a.offsets || !a.by_rows);
+    if (!a.offsets && (a.few_rows_direct || (tiles && gemm_direct_takes(type, a)))) {
+        const hipError_t e = launch_gemm_direct(type, a, stream);
+        if (e != hipErrorNotSupported) return e;
+    }
     if (!tiles) {
         if (a.offsets) return hipErrorInvalidValue;  // grouped form exists for the tile kernel only
         return gemm_by_rows(type, a, stream);

@@ -188,6 +188,7 @@ struct GemmArgs {
                                  // bytes leave room for the few-token kernel's split-k sums
     bool by_rows = false;  // plain matmul: take the GEMV launches even though a workspace is there (the caller's
                            // snapshot of gemm_uses_tiles, so that one call reads the tuning knobs once)
+    bool few_rows_direct = false;  // with by_rows: the direct kernel instead (gemm_direct_few_rows_pay)
     uint32_t m, n, k;   // m = all token rows (of all experts in the grouped form)
     int accumulate;
     const float *bias = nullptr;  // with accumulate == 0: out[t][r] = y + bias[r] (QuantLinear::forward_batch)
@@ -218,6 +219,11 @@ struct GemmArgs {
     SplitSums *defer_reduce = nullptr;
 };
 hipError_t launch_gemm_q8(uint32_t type, const GemmArgs &a, hipStream_t stream);
+// The few-token kernel that takes weights straight into registers (oxq_gemm_direct.hpp; plain matmuls of up to 32 rows, no
+// workspace): where a call should take it, the launch.
+bool gemm_direct_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k);
+bool gemm_direct_few_rows_pay(uint32_t type, uint32_t m, uint32_t n, uint32_t k);
+hipError_t launch_gemm_direct(uint32_t type, const GemmArgs &a, hipStream_t stream);
 // Device scratch the tile kernel needs for m tokens of k columns (activation re-layout).
 // With n and the format: plus, for a matmul of at most 32 token rows that the few-token kernel would split over k,
 // the room for its per-split sums (behind the re-tiled activations, 256-byte aligned).

@@ -1,0 +1,108 @@
+"""The few-token kernel whose weights go straight from memory into the matrix core's registers (oxq_gemm_direct.hpp), on one matrix
+of up to 32 token rows, against the CPU oracle: fp32 within 1e-5 * |y_ref|_inf, the integer sums of its debug dump bit-exact."""
+import pytest
+
+import oracle as O
+from oxillama_amd import synth
+from test_gpu_gemm_skinny import last_launch, ref_sums, sum_groups, weights
+from test_gpu_parity import assert_close, canonical_ref, say
+
+pytestmark = pytest.mark.gpu
+
+FORMATS = [O.Q4_K, O.Q5_K, O.Q6_K, O.IQ4_XS, O.Q4_0, O.Q8_0]
+
+# (rows, n, k).  512..1024: four parts of k, two row tiles at a time (two, three and four super-blocks: parts without work);
+# 1280..2048: eight parts (five and eight super-blocks); 2304..4096: sixteen (nine, fifteen, sixteen), for 17 to 32 rows eight
+# of two (the last of them with one super-block or none); longer: each wave its own run (17: runs of two and three; 33; 43).
+# Row tiles with rows to spare (18 rows, not one: the bar is 1e-5 of the largest of a token's results, and a single result can be far
+# smaller than its terms), an odd number of tiles, more tiles than work groups; odd super-blocks put every second row
+# of the formats of 18, 34 and 210 bytes off a dword.
+SHAPES = [(16, 33, 512), (1, 18, 768), (7, 20, 1024), (16, 4129, 512), (13, 100, 1280), (5, 8300, 2048), (9, 4113, 2304), (16, 40, 3840),
+          (16, 17, 4096), (3, 4099, 4096), (17, 33, 768), (32, 100, 1280), (21, 4131, 2048), (18, 50, 2304), (32, 35, 3840), (25, 8210, 4096),
+          (16, 35, 4352), (2, 16, 8448), (11, 4099, 11008)]
+
+
+@pytest.mark.parametrize("t", FORMATS, ids=lambda t: O.NAMES[t])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_direct_kernel(hip, ref, tuning, t, shape):
+    import torch
+    from oxillama_amd import linear
+    m, n, k_ = shape
+    say("direct", O.NAMES[t], shape)
+    w = weights(t, 171, n, k_)
+    acts = ref.quantize_q8_0(synth.normal_f32(172 + m, m * k_)).reshape(m, k_ // 32 * 34)
+    bias = synth.normal_f32(173, n)
+    kern = hip.HipKernel(t)
+    dw, da, db = torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda(), torch.from_numpy(bias).cuda()
+    tuning("gemm_tile_min_rows", 1)
+    tuning("gemm_variant", 207)
+    ws = torch.empty(kern.gemm_workspace_bytes(m, n, k_), dtype=torch.uint8, device="cuda")
+    dy = torch.full((m + 1, n), 7.0, dtype=torch.float32, device="cuda")
+    kern.gemm_q8_dev(dw, da, dy, m, n, k_, workspace=ws)
+    torch.cuda.synchronize()
+    assert "_direct<" in last_launch(), last_launch()
+    y = dy.cpu().numpy()
+    assert (y[m:] == 7.0).all()
+    for r in sorted({0, m // 2, min(15, m - 1), m - 1}):
+        assert_close(y[r], canonical_ref(ref, t, w, acts[r], n, k_), f"{shape} row {r}")
+    dy2 = dy[:m].clone()
+    kern.gemm_q8_dev(dw, da, dy2, m, n, k_, accumulate=True, workspace=ws)
+    dy3 = torch.zeros((m, n), dtype=torch.float32, device="cuda")
+    linear.linear_forward_batch_dev(t, dw, da, dy3, m, n, k_, d_bias=db, workspace=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(dy2, dy[:m] + dy[:m]) and torch.equal(dy3, dy[:m] + db[None, :])
+    # the dump: the same bits, the oracle's integers
+    dy4 = torch.zeros((m, n), dtype=torch.float32, device="cuda")
+    dsum = torch.full((m, n, sum_groups(t, k_)), -1, dtype=torch.int32, device="cuda")
+    kern.gemm_block_sums_dev(dw, da, dy4, dsum, m, n, k_, workspace=ws)
+    torch.cuda.synchronize()
+    assert "_direct<" in last_launch(), last_launch()
+    assert torch.equal(dy4, dy[:m])
+    for r in (0, m - 1):
+        assert (dsum[r].cpu().numpy() == ref_sums(ref, t, w, acts[r], n, k_)).all(), f"integer sums of row {r}"
+
+
+@pytest.mark.parametrize("t,m,n,k_,direct", [
+    (O.Q4_K, 5, 2560, 2560, True), (O.Q4_K, 4, 2560, 2560, False), (O.IQ4_XS, 3, 2560, 4096, True), (O.Q4_K, 33, 2560, 2560, False),
+    (O.Q6_K, 16, 4096, 5120, True), (O.Q6_K, 16, 4112, 5120, False), (O.Q6_K, 17, 4096, 5120, False), (O.Q8_0, 16, 1024, 5120, False),
+    (O.Q8_0, 16, 1536, 5120, True), (O.Q4_0, 16, 48, 33024, False), (O.Q4_1, 16, 2560, 2560, False)],
+    ids=lambda v: O.NAMES.get(v, str(v)) if isinstance(v, int) and not isinstance(v, bool) else str(v))
+def test_direct_kernel_by_default(hip, ref, t, m, n, k_, direct):
+    """The library's own choice on both sides of each bound (16 x 256 compute units; 4097 to 32768 columns; the first row counts
+    at which GEMV launches end)."""
+    import torch
+    if hip.device_info()["compute_units"] != 256:
+        pytest.skip("the bounds above are those of 256 compute units")
+    w = weights(t, 181, n, k_)
+    acts = ref.quantize_q8_0(synth.normal_f32(182, m * k_)).reshape(m, k_ // 32 * 34)
+    kern = hip.HipKernel(t)
+    ws = torch.empty(kern.gemm_workspace_bytes(m, n, k_), dtype=torch.uint8, device="cuda")
+    dy = torch.zeros((m, n), dtype=torch.float32, device="cuda")
+    kern.gemm_q8_dev(torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda(), dy, m, n, k_, workspace=ws)
+    torch.cuda.synchronize()
+    assert ("_direct<" in last_launch()) == direct, last_launch()
+    assert_close(dy[m - 1].cpu().numpy(), canonical_ref(ref, t, w, acts[m - 1], n, k_, threads=16), f"m={m}")
+
+
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q8_0], ids=lambda t: O.NAMES[t])
+@pytest.mark.parametrize("which", ["weights", "tokens"])
+@pytest.mark.parametrize("m", [6, 16])
+def test_pointers_off_their_boundary_take_the_other_kernels(hip, ref, t, which, m):
+    """Weights off a dword, tokens off 16 bytes: accepted as before, by the kernels that served such calls."""
+    import torch
+    n, k_ = 200, 1024
+    w = weights(t, 191, n, k_)
+    acts = ref.quantize_q8_0(synth.normal_f32(192, m * k_)).reshape(m, k_ // 32 * 34)
+    off_w, off_a = (2, 0) if which == "weights" else (0, 4)
+    dw = torch.zeros(w.nbytes + 16, dtype=torch.uint8, device="cuda")
+    da = torch.zeros(acts.nbytes + 16, dtype=torch.uint8, device="cuda")
+    dw[off_w:off_w + w.nbytes] = torch.from_numpy(w.reshape(-1)).cuda()
+    da[off_a:off_a + acts.nbytes] = torch.from_numpy(acts.reshape(-1)).cuda()
+    kern = hip.HipKernel(t)
+    ws = torch.empty(kern.gemm_workspace_bytes(m, n, k_), dtype=torch.uint8, device="cuda")
+    dy = torch.zeros((m, n), dtype=torch.float32, device="cuda")
+    kern.gemm_q8_dev(dw[off_w:off_w + w.nbytes], da[off_a:off_a + acts.nbytes], dy, m, n, k_, workspace=ws)
+    torch.cuda.synchronize()
+    assert "_direct<" not in last_launch(), last_launch()
+    for r in (0, m - 1):
+        assert_close(dy[r].cpu().numpy(), canonical_ref(ref, t, w, acts[r], n, k_), f"row {r}")
