@@ -35,7 +35,8 @@ int oxq_set_gemm_tile_min_rows(unsigned rows);
  * and its small shape, 303: the large one on an even deal of the parts of k (a workspace of 64 MiB, which the size queries
  * count only for shapes that take it by default, and a part of k for every compute unit, else the default choice); 200..205: the
  * few-token kernel (16 x 16 x 32 MFMA, groups of at most 32 token rows) in a fixed shape; 206: its form that holds the
- * whole k of up to 16 token rows in LDS.  A value a format or
+ * whole k of up to 16 token rows in LDS; 207: the kernel that takes weights straight into registers and keeps its tokens there
+ * (Q4_K, Q5_K, Q6_K, IQ4_XS, Q4_0, Q8_0; up to 512 token rows).  A value a format or
  * shape cannot take falls back to the default tile choice. */
 int oxq_set_gemm_variant(int variant);
 /* Launch-phase probe of the decode GEMV (Q4_0, Q8_0, Q4_K, Q6_K rows of at most two 64-unit steps, and the

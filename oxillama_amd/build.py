@@ -17,7 +17,7 @@ import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
-HIP_SOURCES = ["oxq_api.hip", "oxq_gemv.hip", "oxq_gemv_more.hip", "oxq_gemv_f32.hip", "oxq_gemm.hip", "oxq_gemm_more.hip", "oxq_gemm_prefill.hip", "oxq_gemm_f16.hip", "oxq_gemm_direct.hip", "oxq_quantize.hip", "oxq_linear.hip", "oxq_gguf.hip", "oxq_topk.hip", "oxq_lm_head.hip", "oxq_moe.hip"]
+HIP_SOURCES = ["oxq_api.hip", "oxq_gemv.hip", "oxq_gemv_more.hip", "oxq_gemv_f32.hip", "oxq_gemm.hip", "oxq_gemm_more.hip", "oxq_gemm_prefill.hip", "oxq_gemm_f16.hip", "oxq_gemm_direct.hip", "oxq_gemm_direct_wide.hip", "oxq_quantize.hip", "oxq_linear.hip", "oxq_gguf.hip", "oxq_topk.hip", "oxq_lm_head.hip", "oxq_moe.hip"]
 HIP_LIB = os.path.join(HERE, "liboxq_hip.so")
 BIND_LIB = os.path.join(HERE, "_bind.so")
 SYNTH_LIB = os.path.join(HERE, "liboxq_synth.so")

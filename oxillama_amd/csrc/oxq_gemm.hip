@@ -200,7 +200,7 @@ static bool gemm_direct_takes(uint32_t type, const GemmArgs &a) {
     if (variant == 207) return true;
     // (the dump of the integer sums of matrices small enough for the whole-k kernel stays on the kernels that had it)
     return variant == 0 && !a.scaled_sums && gemm_direct_pays(type, a.m, a.n, a.k) &&
-           (!a.sums || !skinny_whole_pays(type, a.n, a.k, skinny_splits(a.n, a.k) >= 2));
+           (!a.sums || a.m > 16 || !skinny_whole_pays(type, a.n, a.k, skinny_splits(a.n, a.k) >= 2));
 }
 
 hipError_t launch_gemm_q8(uint32_t type, const GemmArgs &a, hipStream_t stream) {

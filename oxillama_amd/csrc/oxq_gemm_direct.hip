@@ -1,38 +1,21 @@
 // The few-token kernel that keeps its tokens in registers (oxq_gemm_direct.hpp), instantiated for its formats.
-#include "oxq_gemm_direct.hpp"
-#include "oxq_gemm_skinny.hpp"
+#include "oxq_gemm_direct_launch.hpp"
 
 namespace oxq {
 
-// KP == 0: the streamed form
-template <class F, int PB, int KP, int TT, int WAVES = 8>
-static hipError_t launch_direct_shape(const GemmArgs &a, hipStream_t stream) {
-    auto kern = a.sums ? &gemm_direct_kernel<F, PB, KP, TT, WAVES, true> : &gemm_direct_kernel<F, PB, KP, TT, WAVES, false>;
-    constexpr size_t lds = KP ? direct_lds<F, PB, TT, WAVES>() : direct_streamed_lds<F, TT, WAVES>();
-    static_assert(lds <= 160 * 1024, "LDS of a compute unit");
-    const hipError_t e = allow_lds(reinterpret_cast<const void *>(kern), lds);
-    if (e != hipSuccess) return e;
-    constexpr uint32_t RG = KP ? WAVES / KP : 1;
-    const uint32_t sets = ((a.n + 15) / 16 + RG - 1) / RG;
-    const dim3 grid(sets < device_cus() ? sets : device_cus());
-    // (named by what the call would take otherwise)
-    note_launch(TT == 1 && a.workspace && !a.by_rows && skinny_whole_pays(F::TYPE, a.n, a.k, skinny_splits(a.n, a.k) >= 2) ? "gemm_skinny_whole_kernel_direct"
-                                                                                            : "gemm_skinny_kernel_direct",
-                F::TYPE, PB, KP, TT, WAVES, grid.x, 1, 64 * WAVES);
-    hipLaunchKernelGGL(kern, grid, dim3(64 * WAVES), lds, stream, a.W, a.A, a.out, a.sums, a.m, a.n, a.k, a.accumulate, a.bias);
-    return hipGetLastError();
+// Token tiles a work group takes: as many as registers hold, fewer where the matrix has so few row tiles that work groups for more
+// runs of tokens still find a compute unit each (256 x 1536 of Q4_K, 77 rows: five runs of one tile, 3.5 us).
+static uint32_t direct_token_tiles(uint32_t m, uint32_t n, uint32_t k) {
+    const uint32_t tiles = (m + 15) / 16, most = k > 2048 && k <= 4096 ? 2 : 4, rows = (n + 15) / 16;
+    const uint32_t fewest = (tiles + most - 1) / most, fill = device_cus() / rows;
+    const uint32_t chunks = fill > tiles ? tiles : fill > fewest ? fill : fewest;
+    return (tiles + chunks - 1) / chunks;
 }
-template <class F, int TT>
-static hipError_t launch_direct(const GemmArgs &a, hipStream_t stream) {
-    const uint32_t nb = a.k / 256;
-    if constexpr (TT == 1) {
-        if (nb > 16) return launch_direct_shape<F, 1, 0, 1>(a, stream);
-        if (nb > 8) return launch_direct_shape<F, 1, 16, 1, 16>(a, stream);
-    } else {
-        if (nb > 8) return launch_direct_shape<F, 2, 8, 2>(a, stream);
-    }
-    if (nb > 4) return launch_direct_shape<F, 1, 8, TT>(a, stream);
-    return launch_direct_shape<F, 1, 4, TT>(a, stream);
+// Row tiles that a work group walks.
+static uint32_t direct_walk(uint32_t m, uint32_t n, uint32_t k, uint32_t tt) {
+    const uint32_t chunks = (m + 16 * tt - 1) / (16 * tt), room = device_cus() > chunks ? device_cus() / chunks : 1;
+    const uint32_t rows = (n + 15) / 16, sets = k <= 1024 ? (rows + 1) / 2 : rows;
+    return (sets + room - 1) / room;
 }
 
 static bool direct_format(uint32_t type) {
@@ -48,27 +31,42 @@ static bool direct_format(uint32_t type) {
 //    tile.  16 rows of 4096 x 14336: Q4_K 19.3 / 16.4, Q6_K 25.3 / 20.8, IQ4_XS 20 / 15.2, Q8_0 26.7 / 25.6; 28672 x 8192 of Q4_K
 //    39 / 61.  Q8_0 of 1024 x 8192 13.5 / 14.3, 1536 x 8960 16.6 / 12.3.  Beyond 32768 columns: not measured.
 //  * Q8_0 vocabularies, where the bytes are the time: 128256 x 4096 119 / 136.
+// More than 32 rows, up to 512 (3000 calls of Q4_K, IQ4_XS, Q6_K, Q8_0 against the tile kernel and its token re-layout launch): the tile
+// kernel is a serial chain of k / 4 where the work groups here meet k / 8 or k / 16, and gains on this one only by weights unpacked
+// for more tokens.  So the line is drawn at the tiles of 16 x 16 a work group goes through (`work`):
+//  * up to 2048 columns 28 (0.63 of the time in the mean, the worst 1.04: Q6_K 333 rows of 4096 x 1536 26.6 / 27.7; from 32 on 0.81 to
+//    1.14), Q8_0 56.  77 rows of Q4_0: 1536 x 1536 12.2 / 6.3, 256 x 1536 12.1 / 3.7, 8960 x 1536 22.4 / 13.3;
+//  * up to 4096 columns, two tokens tiles at most and two super-blocks a wave, a part of which is idle in shorter rows (hence the
+//    square): Q4_K 28 (64 rows of 4096 x 4096 13.7 / 11, 1024 x 4096 12.2 / 5.4, 128 of 14336 x 4096 44 / 35.5), IQ4_XS 14, Q6_K
+//    8 (64 rows of 4096 x 4096 18.9 / 15.2; 112 of 14336 x 4096, 16, 1.13 of the f16 kernel's), Q8_0 4 (16.1 / 7.9; 80 rows of 4096 x 4096, 8, 20.7 / 23.1);
+//  * longer rows (streamed): one row tile a work group, as with 16 rows.  64 rows of 2048 x 8192 Q4_K 0.66 of the time, 4096 x
+//    14336 Q6_K 48.9 / 39; two row tiles 0.9 to 1.3.  Four token tiles where they fill the chip: not for the light formats
+//    (Q4_K 64 rows of 4096 x 14336 31.3 / 32.3), nor against the f16 kernel (Q4_K 128 rows of 2048 x 14336 1.06).  17 to 32
+//    rows beyond 20480 columns: a tie in the light ones.
+// Where the f16 kernels would serve the call they are faster or level (Q6_K 112 rows of 14336 x 1536 1.17; longer rows up to three token tiles 0.86).
 bool gemm_direct_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
-    if (!direct_format(type) || m == 0 || m > 32 || k % 256 != 0 || k < 512) return false;
-    if (k > 4096) return m <= 16 && n <= 16 * device_cus() && k <= 32768 && (type != OXQ_TYPE_Q8_0 || n >= 1536);
-    return type != OXQ_TYPE_Q8_0 || n < 256 * device_cus();
+    if (!direct_format(type) || m == 0 || m > DIRECT_MAX_ROWS || k % 256 != 0 || k < 512 || k > 32768) return false;
+    const bool heavy = type == OXQ_TYPE_Q6_K || type == OXQ_TYPE_Q8_0;
+    if (m <= 16 && k > 4096) return n <= 16 * device_cus() && (type != OXQ_TYPE_Q8_0 || n >= 1536);
+    if (m <= 32 && k <= 4096) return type != OXQ_TYPE_Q8_0 || n < 256 * device_cus();
+    const uint32_t tt = direct_token_tiles(m, n, k), walk = direct_walk(m, n, k, tt), nb = k / 256;
+    const bool f16 = gemm_f16_shape(type, m, n, k) != 0 || gemm_f16_deal_pays(type, m, n, k) ||
+                     (gemm_prefill_supported(type, m, n, k) && gemm_prefill_pays(m, n));
+    if (k > 4096) return walk == 1 && (m > 32 || heavy || k <= 20480) && (tt <= 3 || (!f16 && (heavy || m > 64)));
+    if (f16) return false;
+    const uint64_t work = (uint64_t)walk * tt;
+    if (k <= 2048) return work <= (type == OXQ_TYPE_Q8_0 ? 56u : 28u);
+    return work * 256 <= (uint64_t)nb * nb * (type == OXQ_TYPE_Q8_0 ? 4u : type == OXQ_TYPE_Q6_K ? 8u : type == OXQ_TYPE_IQ4_XS ? 14u : 28u);
 }
 
 hipError_t launch_gemm_direct(uint32_t type, const GemmArgs &a, hipStream_t stream) {
-    if (a.offsets || a.m == 0 || a.m > 32 || a.k % 256 != 0 || a.k < 512 || (a.m > 16 && a.k > 4096) ||
+    if (a.offsets || a.m == 0 || a.m > DIRECT_MAX_ROWS || a.k % 256 != 0 || a.k < 512 ||
         (size_t)a.m * (a.k / 32) * Q8_BLOCK_BYTES > 0x7FFFFFFF || (reinterpret_cast<uintptr_t>(a.W) & 3) ||
         (reinterpret_cast<uintptr_t>(a.A) & 15))  // (what loads straight to LDS and the dword-wise loads were built for)
         return hipErrorNotSupported;
-#define OXQ_DIRECT(T, F) \
-    if (type == T) return a.m <= 16 ? launch_direct<F, 1>(a, stream) : launch_direct<F, 2>(a, stream);
-    OXQ_DIRECT(OXQ_TYPE_Q4_K, TileQ4K)
-    OXQ_DIRECT(OXQ_TYPE_Q5_K, DirectQ5K)
-    OXQ_DIRECT(OXQ_TYPE_Q6_K, TileQ6K)
-    OXQ_DIRECT(OXQ_TYPE_IQ4_XS, TileIQ4XS)
-    OXQ_DIRECT(OXQ_TYPE_Q4_0, TileQ4_0)
-    OXQ_DIRECT(OXQ_TYPE_Q8_0, TileQ8_0)
-#undef OXQ_DIRECT
-    return hipErrorNotSupported;
+    uint32_t tt = direct_token_tiles(a.m, a.n, a.k);
+    if (a.sums && tt > 2) tt = 2;  // (the dump: the same parts of k, so the same bits)
+    return tt > 2 ? launch_direct_wide(type, tt, a, stream) : launch_direct_of<1, 2>(type, tt, a, stream);
 }
 
 }  // namespace oxq

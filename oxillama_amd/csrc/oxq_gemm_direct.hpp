@@ -1,11 +1,13 @@
 // Few tokens per weight matrix, weights straight from memory into the matrix core's registers: the batched fused matvec
 //   out[m x n] (+)= A_q8[m rows of Q8_0 blocks] x W[n x k]^T
 // (the reference's gemm loop over matvec_q8_fused, crates/oxillama-quant/src/reference/q4_k.rs:186-201, :218-333) for a
-// decode batch of up to 16 rows on one matrix, or an expert group.
+// decode batch or a short prompt on one matrix, where its few tiles of 16 rows x 16 tokens make the launch's ramp and the
+// chain along k the time (77 rows of Q4_0: 1536 x 1536 12.2 us on the tile kernel, 6.3 here; 8960 x 1536 22.4 / 13.3).
 //
 //  * k is dealt to the waves of a work group, PB super-blocks each, and a wave keeps its part of the tokens in registers, in
 //    operand order, for as long as the work group walks tiles of 16 weight rows: nothing about the tokens is read again.
 //    The parts' sums meet in LDS, in the order of k, so there is no reduction launch.
+//  * A work group takes TT tiles of 16 tokens: the weights are unpacked once for them.  More tokens are further work groups' (grid y).
 //  * Weights: four lanes share a row; a lane loads 16 bytes of each 64 of a super-block.  Those are 16 weights of one or two
 //    sub-blocks where the operand needs 8 of every sub-block from each of the four: two or four v_permlane{32,16}_swap
 //    per 16 bytes put them there.  No LDS on the way.
@@ -336,7 +338,14 @@ constexpr bool direct_exchange_apart() {
     return direct_tables<F, WAVES>() + direct_strips<PB, TT, WAVES>() + direct_exchange<TT, direct_turn<TT, WAVES>(), WAVES>() <= 160 * 1024;
 }
 template <class F, int TT, int WAVES>
-constexpr uint32_t direct_streamed_lds() { return direct_tables<F, WAVES>() + direct_strips<1, TT, WAVES>() + direct_exchange<TT, 1, WAVES>(); }
+constexpr bool direct_streamed_apart() {
+    return direct_tables<F, WAVES>() + direct_strips<1, TT, WAVES>() + direct_exchange<TT, 1, WAVES>() <= 160 * 1024;
+}
+template <class F, int TT, int WAVES>
+constexpr uint32_t direct_streamed_lds() {
+    constexpr uint32_t s = direct_strips<1, TT, WAVES>(), e = direct_exchange<TT, 1, WAVES>();
+    return direct_tables<F, WAVES>() + (direct_streamed_apart<F, TT, WAVES>() ? s + e : s > e ? s : e);
+}
 template <class F, int PB, int TT, int WAVES>
 constexpr uint32_t direct_lds() {
     constexpr uint32_t s = direct_strips<PB, TT, WAVES>(), e = direct_exchange<TT, direct_turn<TT, WAVES>(), WAVES>();
@@ -502,7 +511,8 @@ struct DirectJob {
     const float *bias;
     uint32_t rows, n, k;
     int accumulate;
-    uint32_t first, step;  // sets of RG row tiles: first, first + step, ...
+    uint32_t first, end, step;  // sets of RG row tiles: first, first + step, ..., below end
+    uint32_t sb0, sbs;          // super-blocks of k (streamed: all of them)
 };
 
 template <int N, int TT>
@@ -535,7 +545,7 @@ struct DirectExchange {
         const uint32_t e = threadIdx.x + THREADS * i, t = (e >> 8) % TT, g = (e >> 8) / TT % RG, x = (e >> 8) / TT / RG;
         row = 16 * ((set + x * j.step) * RG + g) + (e & 15), tok = 16 * t + ((e >> 4) & 15);
         slot = (g * KP * XT + x) * TT + t;
-        return e < TILES * 256 && row < j.n && tok < j.rows;
+        return e < TILES * 256 && set + x * j.step < j.end && row < j.n && tok < j.rows;
     }
     // what the sums are added to, requested before they are formed
     __device__ __forceinline__ void request(float (&old)[NE], uint32_t set) const {
@@ -581,9 +591,9 @@ __device__ __forceinline__ void direct_resident(const DirectJob j, uint8_t *lds)
     constexpr int U = 2, XT = direct_turn<TT, WAVES>();  // row tiles whose weights are in flight; that are exchanged at once
     const uint32_t lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), part = wave % KP, rg = wave / KP;
-    const uint32_t nb = j.k / 256, blk0 = part * PB, live = nb > blk0 ? min((uint32_t)PB, nb - blk0) : 0;
-    const uint32_t tiles = (j.n + 15) / 16, sets = (tiles + RG - 1) / RG;
-    const uint32_t row_bytes = nb * D::BLOCK, arow = nb * 272;
+    const uint32_t live = j.sbs > part * PB ? min((uint32_t)PB, j.sbs - part * PB) : 0;
+    const uint32_t blk0 = j.sb0 + part * PB, sets = j.end;
+    const uint32_t row_bytes = j.k / 256 * D::BLOCK, arow = j.k / 256 * 272;
     constexpr bool APART = direct_exchange_apart<F, PB, TT, WAVES>();
     uint8_t *const tab = lds + wave * (direct_tables<F, WAVES>() / WAVES);
     uint8_t *const strips = lds + direct_tables<F, WAVES>(), *const strip = strips + wave * (direct_strips<PB, TT, WAVES>() / WAVES);
@@ -595,7 +605,9 @@ __device__ __forceinline__ void direct_resident(const DirectJob j, uint8_t *lds)
     typename D::W ring[U][PB];
     auto load = [&](int u, int b, uint32_t set) __attribute__((always_inline)) {
         // (rows past the last lie past the end of the buffer: zeros.  Super-blocks past the last: others', not used)
-        const uint32_t row0 = min(16 * (set * RG + rg), j.n - 1);
+        // (sets past the last: the matrix's last row alone, so that what is requested ahead of the end costs little.  No branch, as with the tokens)
+        const uint32_t past = (uint32_t)((int32_t)(sets - 1 - set) >> 31) & 0x7FFFFFFu;
+        const uint32_t row0 = min(16 * (set * RG + rg) + past, j.n - 1);
         const size_t left = ((size_t)(j.n - row0) * row_bytes + 3) & ~(size_t)3;  // (the dword of the last byte)
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint8_t *>(j.W + (size_t)row0 * row_bytes), 0, (int)min(left, (size_t)0x7FFFFFFF), BUFFER_FLAGS);
@@ -691,7 +703,8 @@ __device__ __forceinline__ void direct_streamed(const DirectJob j, uint8_t *lds)
     const uint32_t row_bytes = nb * D::BLOCK, arow = nb * 272, wrow = c * row_bytes;
     uint8_t *const tab = lds + wave * (direct_tables<F, WAVES>() / WAVES);
     uint8_t *const strips = lds + direct_tables<F, WAVES>(), *const strip = strips + wave * (direct_strips<1, TT, WAVES>() / WAVES);
-    uint8_t *const ex = strips + direct_strips<1, TT, WAVES>();
+    constexpr bool APART = direct_streamed_apart<F, TT, WAVES>();
+    uint8_t *const ex = APART ? strips + direct_strips<1, TT, WAVES>() : strips;
     const __amdgpu_buffer_rsrc_t rs_a = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(j.A), 0, (int)(j.rows * arow), BUFFER_FLAGS);
     v4i32 magic;
     asm volatile("v_mov_b32 %0, 0x4b400000\n\tv_mov_b32 %1, 0x4b400000\n\tv_mov_b32 %2, 0x4b400000\n\tv_mov_b32 %3, 0x4b400000"
@@ -742,18 +755,29 @@ __device__ __forceinline__ void direct_streamed(const DirectJob j, uint8_t *lds)
 #pragma clang loop unroll(disable)
         for (; i + 1 < run; i += 2) super_block(0, i), super_block(1, i + 1);
         if (i < run) super_block(0, i);
-        xc.finish(acc, old, tile);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (what was requested past the run's end: the strip is written again)
+        if constexpr (APART) {
+            xc.finish(acc, old, tile);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (what was requested past the run's end: the strip is written again)
+        } else {
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();  // nothing is on its way to a strip and none is read any more
+            xc.finish(acc, old, tile);
+            if (tile + j.step < tiles) __syncthreads();  // the sums have been read
+        }
     }
 }
 
 // The kernels.  KP == 0: k streamed.
+// blockIdx.y: a run of 16 * TT token rows
 template <class F, int PB, int KP, int TT, int WAVES, bool DUMP>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVES / 4, WAVES / 4))) void gemm_direct_kernel(
     const uint8_t *__restrict__ W, const uint8_t *__restrict__ A, float *__restrict__ out, int32_t *__restrict__ sums, uint32_t m,
     uint32_t n, uint32_t k, int accumulate, const float *__restrict__ bias) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const DirectJob j = {W, A, out, sums, bias, m, n, k, accumulate, blockIdx.x, gridDim.x};
+    const uint32_t t0 = blockIdx.y * (16 * TT), nb = k / 256, tiles = (n + 15) / 16;
+    constexpr uint32_t RG = KP ? WAVES / (KP ? KP : 1) : 1;
+    const DirectJob j = {W, A + (size_t)t0 * nb * 272, out + (size_t)t0 * n, DUMP ? sums + (size_t)t0 * n * (nb * 8 * Direct<F>::KS) : nullptr, bias,
+                         min(m - t0, (uint32_t)(16 * TT)), n, k, accumulate, blockIdx.x, (tiles + RG - 1) / RG, gridDim.x, 0, nb};
     if constexpr (KP == 0) direct_streamed<F, TT, WAVES, DUMP>(j, lds);
     else direct_resident<F, PB, KP, TT, WAVES, DUMP>(j, lds);
 }

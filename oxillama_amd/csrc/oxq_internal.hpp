@@ -219,7 +219,7 @@ struct GemmArgs {
     SplitSums *defer_reduce = nullptr;
 };
 hipError_t launch_gemm_q8(uint32_t type, const GemmArgs &a, hipStream_t stream);
-// The few-token kernel that takes weights straight into registers (oxq_gemm_direct.hpp; plain matmuls of up to 32 rows, no
+// The few-token kernel that takes weights straight into registers (oxq_gemm_direct.hpp; plain matmuls of up to 512 rows, no
 // workspace): where a call should take it, the launch.
 bool gemm_direct_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k);
 bool gemm_direct_few_rows_pay(uint32_t type, uint32_t m, uint32_t n, uint32_t k);

@@ -20,6 +20,10 @@ FORMATS = [O.Q4_K, O.Q5_K, O.Q6_K, O.IQ4_XS, O.Q4_0, O.Q8_0]
 SHAPES = [(16, 33, 512), (1, 18, 768), (7, 20, 1024), (16, 4129, 512), (13, 100, 1280), (5, 8300, 2048), (9, 4113, 2304), (16, 40, 3840),
           (16, 17, 4096), (3, 4099, 4096), (17, 33, 768), (32, 100, 1280), (21, 4131, 2048), (18, 50, 2304), (32, 35, 3840), (25, 8210, 4096),
           (16, 35, 4352), (2, 16, 8448), (11, 4099, 11008)]
+# More than 32 rows: token tiles in one run and several, full and not; three and four of them to a work group (33 rows of 4128 weight rows and more: few
+# enough row tiles are dealt to more work groups with fewer tokens), resident and streamed; row tiles more than work groups.
+WIDE = [(33, 4130, 512), (64, 4128, 1024), (77, 8200, 1280), (130, 4118, 2048), (49, 18, 768), (512, 50, 512), (333, 100, 2048),
+        (35, 4100, 2304), (65, 2100, 4096), (40, 2080, 4352), (64, 4113, 5120), (100, 33, 8448), (115, 2050, 11008), (17, 4099, 4352)]
 
 
 @pytest.mark.parametrize("t", FORMATS, ids=lambda t: O.NAMES[t])
@@ -63,9 +67,10 @@ def test_direct_kernel(hip, ref, tuning, t, shape):
 
 
 @pytest.mark.parametrize("t,m,n,k_,direct", [
-    (O.Q4_K, 5, 2560, 2560, True), (O.Q4_K, 4, 2560, 2560, False), (O.IQ4_XS, 3, 2560, 4096, True), (O.Q4_K, 33, 2560, 2560, False),
-    (O.Q6_K, 16, 4096, 5120, True), (O.Q6_K, 16, 4112, 5120, False), (O.Q6_K, 17, 4096, 5120, False), (O.Q8_0, 16, 1024, 5120, False),
-    (O.Q8_0, 16, 1536, 5120, True), (O.Q4_0, 16, 48, 33024, False), (O.Q4_1, 16, 2560, 2560, False)],
+    (O.Q4_K, 5, 2560, 2560, True), (O.Q4_K, 4, 2560, 2560, False), (O.IQ4_XS, 3, 2560, 4096, True), (O.Q4_K, 33, 2560, 2560, True),
+    (O.Q6_K, 16, 4096, 5120, True), (O.Q6_K, 16, 4112, 5120, False), (O.Q6_K, 17, 4096, 5120, True), (O.Q6_K, 17, 4112, 5120, False), (O.Q8_0, 16, 1024, 5120, False),
+    (O.Q8_0, 16, 1536, 5120, True), (O.Q4_0, 16, 48, 33024, False), (O.Q4_0, 77, 8960, 1536, True), (O.Q4_K, 64, 4096, 14336, False), (O.Q6_K, 64, 4096, 14336, True),
+    (O.Q4_K, 128, 14336, 4096, True), (O.Q6_K, 80, 14336, 4096, False), (O.Q8_0, 512, 1024, 2048, True), (O.Q4_K, 513, 256, 2048, False), (O.Q4_1, 16, 2560, 2560, False)],
     ids=lambda v: O.NAMES.get(v, str(v)) if isinstance(v, int) and not isinstance(v, bool) else str(v))
 def test_direct_kernel_by_default(hip, ref, t, m, n, k_, direct):
     """The library's own choice on both sides of each bound (16 x 256 compute units; 4097 to 32768 columns; the first row counts
@@ -106,3 +111,48 @@ def test_pointers_off_their_boundary_take_the_other_kernels(hip, ref, t, which, 
     assert "_direct<" not in last_launch(), last_launch()
     for r in (0, m - 1):
         assert_close(dy[r].cpu().numpy(), canonical_ref(ref, t, w, acts[r], n, k_), f"row {r}")
+
+
+@pytest.mark.parametrize("t", FORMATS, ids=lambda t: O.NAMES[t])
+@pytest.mark.parametrize("shape", WIDE, ids=lambda s: "x".join(map(str, s)))
+def test_direct_kernel_on_more_token_tiles(hip, ref, tuning, t, shape):
+    import torch
+    from oxillama_amd import linear
+    m, n, k_ = shape
+    say("direct wide", O.NAMES[t], shape)
+    w = weights(t, 271, n, k_)
+    acts = ref.quantize_q8_0(synth.normal_f32(272 + m, m * k_)).reshape(m, k_ // 32 * 34)
+    bias = synth.normal_f32(273, n)
+    kern = hip.HipKernel(t)
+    dw, da, db = torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda(), torch.from_numpy(bias).cuda()
+    tuning("gemm_tile_min_rows", 1)
+    tuning("gemm_variant", 207)
+    ws = torch.empty(kern.gemm_workspace_bytes(m, n, k_), dtype=torch.uint8, device="cuda")
+    dy = torch.full((m + 1, n), 7.0, dtype=torch.float32, device="cuda")
+    kern.gemm_q8_dev(dw, da, dy, m, n, k_, workspace=ws)
+    torch.cuda.synchronize()
+    assert "_direct<" in last_launch(), last_launch()
+    assert (dy[m:] == 7.0).all()
+    rows = [r for r in (0, 15, 16, 31, 32, 47, 48, 63, 64, m // 2, m - 1) if r < m]
+    for r in sorted(set(rows)):
+        assert_close(dy[r].cpu().numpy(), canonical_ref(ref, t, w, acts[r], n, k_, threads=16), f"{shape} row {r}")
+    # every row: the same bits as in a call of its tile alone, which takes one token tile, where k is dealt to the waves alike
+    if k_ <= 2048:
+        for r0 in range(0, m, 16):
+            part = min(16, m - r0)
+            one = torch.zeros((part, n), dtype=torch.float32, device="cuda")
+            kern.gemm_q8_dev(dw, da[r0:r0 + part].contiguous(), one, part, n, k_, workspace=ws)
+            assert torch.equal(one, dy[r0:r0 + part]), f"rows from {r0}"
+    dy2 = dy[:m].clone()
+    kern.gemm_q8_dev(dw, da, dy2, m, n, k_, accumulate=True, workspace=ws)
+    dy3 = torch.zeros((m, n), dtype=torch.float32, device="cuda")
+    linear.linear_forward_batch_dev(t, dw, da, dy3, m, n, k_, d_bias=db, workspace=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(dy2, dy[:m] + dy[:m]) and torch.equal(dy3, dy[:m] + db[None, :])
+    # the dump (two token tiles at most): the same bits, the oracle's integers
+    dy4 = torch.zeros((m, n), dtype=torch.float32, device="cuda")
+    dsum = torch.full((m, n, sum_groups(t, k_)), -1, dtype=torch.int32, device="cuda")
+    kern.gemm_block_sums_dev(dw, da, dy4, dsum, m, n, k_, workspace=ws)
+    torch.cuda.synchronize()
+    assert "_direct<" in last_launch() and torch.equal(dy4, dy[:m]), last_launch()
+    assert (dsum[m - 1].cpu().numpy() == ref_sums(ref, t, w, acts[m - 1], n, k_)).all()
