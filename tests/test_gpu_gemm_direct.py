@@ -91,7 +91,7 @@ def test_direct_kernel_by_default(hip, ref, t, m, n, k_, direct):
 
 @pytest.mark.parametrize("t", [O.Q4_K, O.Q8_0], ids=lambda t: O.NAMES[t])
 @pytest.mark.parametrize("which", ["weights", "tokens"])
-@pytest.mark.parametrize("m", [6, 16])
+@pytest.mark.parametrize("m", [6, 16, 77])
 def test_pointers_off_their_boundary_take_the_other_kernels(hip, ref, t, which, m):
     """Weights off a dword, tokens off 16 bytes: accepted as before, by the kernels that served such calls."""
     import torch
