@@ -36,13 +36,14 @@ static bool direct_format(uint32_t type) {
 // for more tokens.  So the line is drawn at the tiles of 16 x 16 a work group goes through (`work`):
 //  * up to 2048 columns 28 (0.63 of the time in the mean, the worst 1.04: Q6_K 333 rows of 4096 x 1536 26.6 / 27.7; from 32 on 0.81 to
 //    1.14), Q8_0 56.  77 rows of Q4_0: 1536 x 1536 12.2 / 6.3, 256 x 1536 12.1 / 3.7, 8960 x 1536 22.4 / 13.3;
-//  * up to 4096 columns, two tokens tiles at most and two super-blocks a wave, a part of which is idle in shorter rows (hence the
+//  * up to 4096 columns, two token tiles at most and two super-blocks a wave, a part of which is idle in shorter rows (hence the
 //    square): Q4_K 28 (64 rows of 4096 x 4096 13.7 / 11, 1024 x 4096 12.2 / 5.4, 128 of 14336 x 4096 44 / 35.5), IQ4_XS 14, Q6_K
 //    8 (64 rows of 4096 x 4096 18.9 / 15.2; 112 of 14336 x 4096, 16, 1.13 of the f16 kernel's), Q8_0 4 (16.1 / 7.9; 80 rows of 4096 x 4096, 8, 20.7 / 23.1);
 //  * longer rows (streamed): one row tile a work group, as with 16 rows.  64 rows of 2048 x 8192 Q4_K 0.66 of the time, 4096 x
 //    14336 Q6_K 48.9 / 39; two row tiles 0.9 to 1.3.  Four token tiles where they fill the chip: not for the light formats
 //    (Q4_K 64 rows of 4096 x 14336 31.3 / 32.3), nor against the f16 kernel (Q4_K 128 rows of 2048 x 14336 1.06).  17 to 32
 //    rows beyond 20480 columns: a tie in the light ones.
+// Q4_0 and Q5_K at Q4_K's lines: 320 calls of 21 matrices 0.68 of the tile kernel's time in the mean, none above 1.04.
 // Where the f16 kernels would serve the call they are faster or level (Q6_K 112 rows of 14336 x 1536 1.17; longer rows up to three token tiles 0.86).
 bool gemm_direct_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
     if (!direct_format(type) || m == 0 || m > DIRECT_MAX_ROWS || k % 256 != 0 || k < 512 || k > 32768) return false;
