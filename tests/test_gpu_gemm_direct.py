@@ -1,5 +1,6 @@
 """The few-token kernel whose weights go straight from memory into the matrix core's registers (oxq_gemm_direct.hpp), on one matrix
 of up to 32 token rows, against the CPU oracle: fp32 within 1e-5 * |y_ref|_inf, the integer sums of its debug dump bit-exact."""
+import numpy as np
 import pytest
 
 import oracle as O
@@ -156,3 +157,53 @@ def test_direct_kernel_on_more_token_tiles(hip, ref, tuning, t, shape):
     torch.cuda.synchronize()
     assert "_direct<" in last_launch() and torch.equal(dy4, dy[:m]), last_launch()
     assert (dsum[m - 1].cpu().numpy() == ref_sums(ref, t, w, acts[m - 1], n, k_)).all()
+
+
+@pytest.mark.parametrize("t", FORMATS, ids=lambda t: O.NAMES[t])
+@pytest.mark.parametrize("shape", [(13, 100, 1024), (16, 50, 4096), (21, 60, 2304), (77, 4130, 512), (16, 40, 5120), (40, 2080, 4352)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_direct_kernel_on_infinite_block_scales(hip, ref, tuning, t, shape):
+    """Tokens with infinite block scales (activations beyond f16's range) and a NaN among them: infinities of the same sign and NaNs
+    where the tile kernel has them (and the oracle, where a sub-block is one term), and every other token as without them.  Four,
+    sixteen and eight parts of k in registers, streamed, one to four token tiles."""
+    import torch
+    m, n, k_ = shape
+    say("direct, infinite scales", O.NAMES[t], shape)
+    w = weights(t, 371, n, k_)
+    clean = ref.quantize_q8_0(synth.normal_f32(372, m * k_)).reshape(m, k_ // 32, 34)
+    acts = clean.copy()
+    acts[3, 5, :2] = [0x00, 0x7C]                 # +inf in one block
+    acts[6, k_ // 32 - 1, :2] = [0x00, 0xFC]      # -inf in the last one
+    acts[9, :, :2] = [0x00, 0x7C]                 # in all of a token
+    acts[m - 1, k_ // 64, :2] = [0x00, 0x7E]      # a NaN
+    kern = hip.HipKernel(t)
+    dw = torch.from_numpy(w).cuda()
+    ws = torch.empty(kern.gemm_workspace_bytes(m, n, k_), dtype=torch.uint8, device="cuda")
+    tuning("gemm_tile_min_rows", 1)
+
+    def product(a, variant):
+        tuning("gemm_variant", variant)
+        dy = torch.zeros((m, n), dtype=torch.float32, device="cuda")
+        kern.gemm_q8_dev(dw, torch.from_numpy(a.reshape(-1)).cuda(), dy, m, n, k_, workspace=ws)
+        torch.cuda.synchronize()
+        assert ("_direct<" in last_launch()) == (variant == 207), last_launch()
+        return dy.cpu().numpy()
+
+    y, tile, y_clean = product(acts, 207), product(acts, 99), product(clean, 207)
+    odd = (3, 6, 9, m - 1)
+    assert np.isfinite(y_clean).all() and not np.isfinite(tile[3]).any() and np.isnan(tile[m - 1]).all()
+    # (where there is a zero-point term, it and the block's product are mostly infinities of opposite signs)
+    assert t in (O.Q4_K, O.Q5_K, O.Q4_0) or np.isinf(tile[3]).any()
+    expected = [(tile, odd)]
+    if t in (O.IQ4_XS, O.Q8_0):  # (the zero-point terms of the others, and the halves of Q6_K, are infinities of their own)
+        want = np.zeros_like(y)
+        for r in odd:
+            want[r] = canonical_ref(ref, t, w, acts[r].reshape(-1), n, k_)
+        expected.append((want, odd))
+    for want, rows in expected:
+        for r in rows:
+            assert np.array_equal(np.isnan(y[r]), np.isnan(want[r])), r
+            assert np.array_equal(np.isinf(y[r]), np.isinf(want[r])), r
+            assert np.array_equal(y[r][np.isinf(y[r])], want[r][np.isinf(want[r])]), r
+    rest = [r for r in range(m) if r not in odd]
+    assert np.array_equal(y[rest], y_clean[rest])
