@@ -6,7 +6,7 @@
   * oxillama_amd/liboxq_synth.so -- host-side synthetic weight generator
   * oxillama_amd/liboxq_benchkit.so -- copy / streaming-read kernels for measurement calibration
   * tests/cpp/test_quant_kernel.bin -- C++ mirror of the reference interface + its replayed unit tests
-  * tests/cpp/test_lds_opt_in.bin, test_tile_order.bin, test_scratch.bin -- host tests of the kernels' LDS limits, of their
+  * tests/cpp/test_lds_opt_in.bin, test_tile_order.bin, test_direct_window.bin, test_scratch.bin -- host tests of the kernels' LDS limits, of their
     tile order and of the library's scratch
 hipcc cross-compiles gfx950 code objects without a GPU present.
 """
@@ -23,7 +23,7 @@ BIND_LIB = os.path.join(HERE, "_bind.so")
 SYNTH_LIB = os.path.join(HERE, "liboxq_synth.so")
 BENCHKIT_LIB = os.path.join(HERE, "liboxq_benchkit.so")
 CPP_TEST_BIN = os.path.join(os.path.dirname(HERE), "tests", "cpp", "test_quant_kernel.bin")
-HOST_TESTS = [os.path.join(os.path.dirname(HERE), "tests", "cpp", name) for name in ("test_lds_opt_in", "test_tile_order", "test_scratch")]
+HOST_TESTS = [os.path.join(os.path.dirname(HERE), "tests", "cpp", name) for name in ("test_lds_opt_in", "test_tile_order", "test_direct_window", "test_scratch")]
 
 # -ffp-contract=off: the fp32 epilogues follow the reference's operation order (Rust
 # never fuses a*b+c).  Packed fp32 instructions are switched off.

@@ -20,6 +20,7 @@
 // the zero-point term as a 16 x 16 x 4 fp32 MFMA per four sub-blocks.
 #pragma once
 #include "oxq_gemm_tile.hpp"
+#include "oxq_direct_window.hpp"
 
 namespace oxq {
 
@@ -607,12 +608,9 @@ __device__ __forceinline__ void direct_resident(const DirectJob j, uint8_t *lds)
     typename D::W ring[U][PB];
     auto load = [&](int u, int b, uint32_t set) __attribute__((always_inline)) {
         // (rows past the last lie past the end of the buffer: zeros.  Super-blocks past the last: others', not used)
-        // (sets past the last: the matrix's last row alone, so that what is requested ahead of the end costs little.  No branch, as with the tokens)
-        const uint32_t past = (uint32_t)((int32_t)(sets - 1 - set) >> 31) & 0x7FFFFFFu;
-        const uint32_t row0 = min(16 * (set * RG + rg) + past, j.n - 1);
-        const size_t left = ((size_t)(j.n - row0) * row_bytes + 3) & ~(size_t)3;  // (the dword of the last byte)
+        const DirectWindow win = direct_window(set, sets, rg, RG, j.n, row_bytes);
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint8_t *>(j.W + (size_t)row0 * row_bytes), 0, (int)min(left, (size_t)0x7FFFFFFF), BUFFER_FLAGS);
+            const_cast<uint8_t *>(j.W + (size_t)win.row0 * row_bytes), 0, (int)win.records, BUFFER_FLAGS);
         D::load(ring[u][b], rs, wrow, q, (blk0 + b) * D::BLOCK);
     };
     __builtin_amdgcn_sched_barrier(0);
@@ -714,9 +712,9 @@ __device__ __forceinline__ void direct_streamed(const DirectJob j, uint8_t *lds)
     DirectExchange<WAVES, TT, XT, WAVES> xc{j, ex, 0};
 #pragma clang loop unroll(disable)
     for (uint32_t tile = j.first; tile < tiles; tile += j.step) {
-        const size_t left = ((size_t)(j.n - 16 * tile) * row_bytes + 3) & ~(size_t)3;  // (the dword of the last byte)
+        const DirectWindow win = direct_window(tile, tiles, 0, 1, j.n, row_bytes);
         const __amdgpu_buffer_rsrc_t rs_w = __builtin_amdgcn_make_buffer_rsrc(
-            const_cast<uint8_t *>(j.W + (size_t)(16 * tile) * row_bytes), 0, (int)min(left, (size_t)0x7FFFFFFF), BUFFER_FLAGS);
+            const_cast<uint8_t *>(j.W + (size_t)win.row0 * row_bytes), 0, (int)win.records, BUFFER_FLAGS);
         typename D::W ring[2];
         // super-block i of the run (past its end: the last one again, not used)
         auto request_tokens = [&](uint32_t i) __attribute__((always_inline)) {

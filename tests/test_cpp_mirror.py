@@ -1,7 +1,7 @@
 """Runs tests/cpp/test_quant_kernel.bin: the reference crate's own unit tests replayed
 through the C++ mirror of its interface (include/oxq/quant_kernel.hpp -> C ABI), and the
 host tests beside it: the kernels' LDS limits asked for by several threads, the order
-in which work groups take tiles, and the library's scratch on a full device."""
+in which work groups take tiles, where weight requests ahead of the end reach, and the library's scratch on a full device."""
 import os
 import subprocess
 
@@ -27,6 +27,10 @@ def test_lds_limits_are_only_raised():
 
 def test_tiles_are_dealt_evenly_to_the_xcds():
     _run(binary=os.path.join(CPP, "test_tile_order.bin"))
+
+
+def test_requests_ahead_of_the_end_stay_in_the_matrix():
+    _run(binary=os.path.join(CPP, "test_direct_window.bin"))
 
 
 def test_scratch_falls_back_to_what_a_call_needs():
