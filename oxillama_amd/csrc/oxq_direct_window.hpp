@@ -22,5 +22,9 @@ OXQ_HOST_DEVICE DirectWindow direct_window(uint32_t set, uint32_t sets, uint32_t
     const size_t left = ((size_t)(n - row0) * row_bytes + 3) & ~(size_t)3;
     return DirectWindow{row0, left < 0x7FFFFFFF ? (uint32_t)left : 0x7FFFFFFFu};
 }
+// Super-block `at` of a row of nb; for a part of k (or the end of one) past the last, whose values are not used, the last one: the offset
+// in a row goes to the request's scalar offset, and what the range check makes of one beyond the descriptor's size is
+// nowhere written down.
+OXQ_HOST_DEVICE uint32_t direct_super_block(uint32_t at, uint32_t nb) { return at < nb ? at : nb - 1; }
 
 }  // namespace oxq

@@ -607,11 +607,11 @@ __device__ __forceinline__ void direct_resident(const DirectJob j, uint8_t *lds)
     const uint32_t wrow = c * row_bytes;
     typename D::W ring[U][PB];
     auto load = [&](int u, int b, uint32_t set) __attribute__((always_inline)) {
-        // (rows past the last lie past the end of the buffer: zeros.  Super-blocks past the last: others', not used)
+        // (rows past the last lie past the end of the buffer: zeros)
         const DirectWindow win = direct_window(set, sets, rg, RG, j.n, row_bytes);
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint8_t *>(j.W + (size_t)win.row0 * row_bytes), 0, (int)win.records, BUFFER_FLAGS);
-        D::load(ring[u][b], rs, wrow, q, (blk0 + b) * D::BLOCK);
+        D::load(ring[u][b], rs, wrow, q, direct_super_block(blk0 + b, j.k / 256) * D::BLOCK);
     };
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll

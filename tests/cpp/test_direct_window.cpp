@@ -1,5 +1,5 @@
 // The descriptors of the direct kernel's weight requests, those past the last row tile among them: on a dword, with the tile's rows in
-// them, and not a byte behind the dword in which the matrix ends.
+// them, and not a byte behind the dword in which the matrix ends; every scalar offset, also of parts of k past the last super-block, in them.
 #include <cstdio>
 #include <initializer_list>
 
@@ -24,6 +24,10 @@ int main() {
                                     const size_t tile_end = (size_t)(row + 16 < n ? row + 16 : n) * row_bytes;
                                     ok = ok && w.row0 == row && base + w.records >= tile_end;
                                 }
+                                for (uint32_t parts : {4u, 8u, 16u})  // of one super-block, eight also of two
+                                    for (uint32_t at = 0; at < (parts == 8 ? 16 : parts); at++)
+                                        ok = ok && (oxq::direct_super_block(at, nb) + 1) * block <= w.records &&
+                                             (at >= nb || oxq::direct_super_block(at, nb) == at);
                                 windows++;
                                 if (!ok && failed++ < 10)
                                     std::printf("block %u x %u, n %u, set %u of %u, tile %u of %u: row %u, %u bytes\n", block, nb, n, set,
