@@ -23,10 +23,7 @@ hipError_t launch_direct_shape(const GemmArgs &a, hipStream_t stream) {
     const uint32_t sets = ((a.n + 15) / 16 + RG - 1) / RG, chunks = (a.m + 16 * TT - 1) / (16 * TT);
     const uint32_t room = device_cus() > chunks ? device_cus() / chunks : 1, walk = (sets + room - 1) / room;
     const dim3 grid(chunks == 1 ? (sets < room ? sets : room) : (sets + walk - 1) / walk, chunks);
-    // (named by what the call would take otherwise)
-    note_launch(a.m > 32 ? "gemm_tile_kernel_direct" : TT == 1 && a.workspace && !a.by_rows && skinny_whole_pays(F::TYPE, a.n, a.k, skinny_splits(a.n, a.k) >= 2) ? "gemm_skinny_whole_kernel_direct"
-                                                                                            : "gemm_skinny_kernel_direct",
-                F::TYPE, PB, KP, TT, WAVES, grid.x, grid.y, 64 * WAVES);
+    note_launch("gemm_direct_kernel", F::TYPE, PB, KP, TT, WAVES, grid.x, grid.y, 64 * WAVES);
     hipLaunchKernelGGL(kern, grid, dim3(64 * WAVES), lds, stream, a.W, a.A, a.out, a.sums, a.m, a.n, a.k, a.accumulate, a.bias);
     return hipGetLastError();
 }

@@ -45,7 +45,7 @@ def test_direct_kernel(hip, ref, tuning, t, shape):
     dy = torch.full((m + 1, n), 7.0, dtype=torch.float32, device="cuda")
     kern.gemm_q8_dev(dw, da, dy, m, n, k_, workspace=ws)
     torch.cuda.synchronize()
-    assert "_direct<" in last_launch(), last_launch()
+    assert last_launch().startswith("gemm_direct_kernel<"), last_launch()
     y = dy.cpu().numpy()
     assert (y[m:] == 7.0).all()
     for r in sorted({0, m // 2, min(15, m - 1), m - 1}):
@@ -61,7 +61,7 @@ def test_direct_kernel(hip, ref, tuning, t, shape):
     dsum = torch.full((m, n, sum_groups(t, k_)), -1, dtype=torch.int32, device="cuda")
     kern.gemm_block_sums_dev(dw, da, dy4, dsum, m, n, k_, workspace=ws)
     torch.cuda.synchronize()
-    assert "_direct<" in last_launch(), last_launch()
+    assert last_launch().startswith("gemm_direct_kernel<"), last_launch()
     assert torch.equal(dy4, dy[:m])
     for r in (0, m - 1):
         assert (dsum[r].cpu().numpy() == ref_sums(ref, t, w, acts[r], n, k_)).all(), f"integer sums of row {r}"
@@ -86,7 +86,7 @@ def test_direct_kernel_by_default(hip, ref, t, m, n, k_, direct):
     dy = torch.zeros((m, n), dtype=torch.float32, device="cuda")
     kern.gemm_q8_dev(torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda(), dy, m, n, k_, workspace=ws)
     torch.cuda.synchronize()
-    assert ("_direct<" in last_launch()) == direct, last_launch()
+    assert last_launch().startswith("gemm_direct_kernel<") == direct, last_launch()
     assert_close(dy[m - 1].cpu().numpy(), canonical_ref(ref, t, w, acts[m - 1], n, k_, threads=16), f"m={m}")
 
 
@@ -109,7 +109,7 @@ def test_pointers_off_their_boundary_take_the_other_kernels(hip, ref, t, which, 
     dy = torch.zeros((m, n), dtype=torch.float32, device="cuda")
     kern.gemm_q8_dev(dw[off_w:off_w + w.nbytes], da[off_a:off_a + acts.nbytes], dy, m, n, k_, workspace=ws)
     torch.cuda.synchronize()
-    assert "_direct<" not in last_launch(), last_launch()
+    assert not last_launch().startswith("gemm_direct_kernel<"), last_launch()
     for r in (0, m - 1):
         assert_close(dy[r].cpu().numpy(), canonical_ref(ref, t, w, acts[r], n, k_), f"row {r}")
 
@@ -132,7 +132,7 @@ def test_direct_kernel_on_more_token_tiles(hip, ref, tuning, t, shape):
     dy = torch.full((m + 1, n), 7.0, dtype=torch.float32, device="cuda")
     kern.gemm_q8_dev(dw, da, dy, m, n, k_, workspace=ws)
     torch.cuda.synchronize()
-    assert "_direct<" in last_launch(), last_launch()
+    assert last_launch().startswith("gemm_direct_kernel<"), last_launch()
     assert (dy[m:] == 7.0).all()
     rows = [r for r in (0, 15, 16, 31, 32, 47, 48, 63, 64, m // 2, m - 1) if r < m]
     for r in sorted(set(rows)):
@@ -155,7 +155,7 @@ def test_direct_kernel_on_more_token_tiles(hip, ref, tuning, t, shape):
     dsum = torch.full((m, n, sum_groups(t, k_)), -1, dtype=torch.int32, device="cuda")
     kern.gemm_block_sums_dev(dw, da, dy4, dsum, m, n, k_, workspace=ws)
     torch.cuda.synchronize()
-    assert "_direct<" in last_launch() and torch.equal(dy4, dy[:m]), last_launch()
+    assert last_launch().startswith("gemm_direct_kernel<") and torch.equal(dy4, dy[:m]), last_launch()
     assert (dsum[m - 1].cpu().numpy() == ref_sums(ref, t, w, acts[m - 1], n, k_)).all()
 
 
@@ -186,7 +186,7 @@ def test_direct_kernel_on_infinite_block_scales(hip, ref, tuning, t, shape):
         dy = torch.zeros((m, n), dtype=torch.float32, device="cuda")
         kern.gemm_q8_dev(dw, torch.from_numpy(a.reshape(-1)).cuda(), dy, m, n, k_, workspace=ws)
         torch.cuda.synchronize()
-        assert ("_direct<" in last_launch()) == (variant == 207), last_launch()
+        assert last_launch().startswith("gemm_direct_kernel<" if variant == 207 else "gemm_tile_kernel<"), last_launch()
         return dy.cpu().numpy()
 
     y, tile, y_clean = product(acts, 207), product(acts, 99), product(clean, 207)

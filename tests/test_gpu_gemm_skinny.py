@@ -50,6 +50,28 @@ def shaped_rows(counts, max_rows):
     return min(2 * ((total + len(counts) - 1) // len(counts)), total)
 
 
+# The formats of the kernel that keeps its tokens in registers (oxq_gemm_direct.hpp), which serves plain matmuls of theirs where
+# it is the faster one: for whole 256-weight blocks, up to 32 rows, as below.  Tokens off 16 bytes take the kernels tested here.
+DIRECT = [O.Q4_K, O.Q5_K, O.Q6_K, O.IQ4_XS, O.Q4_0, O.Q8_0]
+
+
+def takes_direct(t, m, n, k_):
+    """(on 256 compute units)"""
+    if t not in DIRECT:
+        return False
+    if k_ <= 4096:
+        return t != O.Q8_0 or n < 65536
+    return n <= 4096 and (t != O.Q8_0 or n >= 1536 if m <= 16 else t in (O.Q6_K, O.Q8_0) or k_ <= 20480)
+
+
+def off_16_bytes(acts):
+    """The tokens on the device, four bytes off a boundary of 16."""
+    import torch
+    buf = torch.zeros(acts.nbytes + 16, dtype=torch.uint8, device="cuda")
+    buf[4:4 + acts.nbytes] = torch.from_numpy(acts.reshape(-1)).cuda()
+    return buf[4:4 + acts.nbytes]
+
+
 def last_launch():
     from oxillama_amd import capi
     buf = C.create_string_buffer(256)
@@ -230,12 +252,14 @@ def test_skinny_full_size_c5_gate(hip, ref):
                                    # 17..32 rows on fewer than 8192 weight rows: two token tiles (Q6_K, Q8_0: two passes)
                                    (21, 4096, 8192), (32, 2100, 16384), (17, 4100, 8192),
                                    # an odd number of super-blocks (43, 17): the last split ends on half a step
-                                   (16, 4096, 11008), (9, 8200, 4352), (21, 4096, 11008)],
+                                   (16, 4096, 11008), (9, 8200, 4352), (21, 4096, 11008),
+                                   # long rows on more than 4096 weight rows: this kernel in every format by default
+                                   (16, 4112, 8192), (32, 4100, 11008)],
                          ids=lambda s: "x".join(map(str, s)))
 def test_skinny_one_matrix_split_k(hip, ref, t, shape):
     """One matrix, up to 16 token rows (32 on fewer than 8192 weight rows), at least 2^25 weights: k is split over work groups, each writes its sums for its
     part of k, a second launch adds the parts in index order.  Integer sums ==, fp32 1e-5, bias, accumulate, ragged n,
-    splits of unequal length."""
+    splits of unequal length.  Where the kernel that keeps its tokens in registers is the default choice, tokens off 16 bytes."""
     import torch
     from oxillama_amd import linear
     m, n, k_ = shape
@@ -246,6 +270,14 @@ def test_skinny_one_matrix_split_k(hip, ref, t, shape):
     kern = hip.HipKernel(t)
     dw, da, db = torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda(), torch.from_numpy(bias).cuda()
     ws = torch.empty(kern.gemm_workspace_bytes(m, n, k_), dtype=torch.uint8, device="cuda")
+    if hip.device_info()["compute_units"] == 256:
+        direct = takes_direct(t, m, n, k_)
+        kern.gemm_q8_dev(dw, da, torch.zeros((m, n), dtype=torch.float32, device="cuda"), m, n, k_, workspace=ws)
+        assert last_launch().startswith("gemm_direct_kernel" if direct else "gemm_skinny_kernel"), last_launch()
+    else:
+        direct = t in DIRECT
+    if direct:
+        da = off_16_bytes(acts)
     dy = torch.full((m + 1, n), 7.0, dtype=torch.float32, device="cuda")
     dsum = torch.full((m, n, sum_groups(t, k_)), -1, dtype=torch.int32, device="cuda")
     kern.gemm_block_sums_dev(dw, da, dy, dsum, m, n, k_, workspace=ws)
@@ -280,65 +312,72 @@ def test_skinny_one_matrix_split_k(hip, ref, t, shape):
     assert st == capi.ERR_BUFFER_TOO_SMALL
 
 
-def test_skinny_one_matrix_with_many_row_groups(hip, ref):
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q4_1], ids=lambda t: O.NAMES[t])
+def test_skinny_one_matrix_with_many_row_groups(hip, ref, t):
     """One matrix with at least two groups of 128 rows per compute unit (a vocabulary projection) and up to 16 token
     rows: the few-token kernel without a split of k."""
     import torch
-    t, m, n, k_ = O.Q4_K, 9, 65600, 512
-    w = synth.weights(t, 85, n, k_)
+    m, n, k_ = 9, 65600, 512
+    w = weights(t, 85, n, k_)
     acts = ref.quantize_q8_0(synth.normal_f32(86, m * k_)).reshape(m, k_ // 32 * 34)
     kern = hip.HipKernel(t)
     ws = torch.empty(kern.gemm_workspace_bytes(m, n, k_), dtype=torch.uint8, device="cuda")
     dy = torch.full((m + 1, n), 7.0, dtype=torch.float32, device="cuda")
     dsum = torch.full((m, n, k_ // 32), -1, dtype=torch.int32, device="cuda")
-    kern.gemm_block_sums_dev(torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda(), dy, dsum, m, n, k_, workspace=ws)
+    da = off_16_bytes(acts) if t in DIRECT else torch.from_numpy(acts).cuda()
+    kern.gemm_block_sums_dev(torch.from_numpy(w).cuda(), da, dy, dsum, m, n, k_, workspace=ws)
     torch.cuda.synchronize()
     assert last_launch().startswith("gemm_skinny_kernel"), last_launch()
     y, s = dy.cpu().numpy(), dsum.cpu().numpy()
     assert np.all(y[m:] == 7.0)
     for r in (0, 4, m - 1):
         assert_close(y[r], canonical_ref(ref, t, w, acts[r], n, k_, threads=16), f"many row groups, row {r}")
-        assert np.array_equal(s[r], ref.block_sums(t, w, acts[r], n, k_))
+        assert np.array_equal(s[r], ref_sums(ref, t, w, acts[r], n, k_))
 
 
-def test_skinny_split_k_on_the_host_routes(hip, ref):
+@pytest.mark.parametrize("t,n,k_,kernel", [(O.Q4_1, 8192, 4096, "gemm_skinny_kernel"), (O.Q4_K, 8192, 8192, "gemm_skinny_kernel"),
+                                           (O.Q4_K, 8192, 4096, "gemm_direct_kernel")], ids=["Q4_1", "Q4_K_8192", "Q4_K_4096"])
+def test_skinny_split_k_on_the_host_routes(hip, ref, t, n, k_, kernel):
     """The routes that size their own scratch -- QuantKernel::gemm on host slices, oxq_gemm_q8_dev without a
     workspace -- leave room for the per-split sums and take the same kernel."""
     import torch
-    t, m, n, k_ = O.Q4_K, 8, 8192, 4096
+    m = 8
     w = weights(t, 81, n, k_)
     x = synth.normal_f32(82, m * k_)
     acts = ref.quantize_q8_0(x).reshape(m, k_ // 32 * 34)
     kern = hip.HipKernel(t)
     y = np.zeros(m * n, dtype=np.float32)
     kern.gemm(hip.QuantTensor(w, [n, k_], t), x, y, m, n, k_)
-    assert last_launch().startswith("gemm_skinny_kernel"), last_launch()
+    assert last_launch().startswith(kernel), last_launch()
     y = y.reshape(m, n)
     for r in (0, 3, m - 1):
         assert_close(y[r], canonical_ref(ref, t, w, acts[r], n, k_, threads=16), f"host gemm row {r}")
     dy = torch.zeros((m, n), dtype=torch.float32, device="cuda")
     kern.gemm_q8_dev(torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda(), dy, m, n, k_)  # library-owned scratch
     torch.cuda.synchronize()
-    assert last_launch().startswith("gemm_skinny_kernel"), last_launch()
+    assert last_launch().startswith(kernel), last_launch()
     assert np.array_equal(dy.cpu().numpy(), y)
 
 
 @pytest.mark.parametrize("case", [(O.IQ4_XS, 3, 8192, 4096), (O.Q4_K, 5, 4096, 8192), (O.Q4_K, 4, 8192, 4096),
-                                  (O.Q6_K, 5, 4096, 8192), (O.Q6_K, 4, 4096, 8192)],
+                                  (O.Q6_K, 5, 4096, 8192), (O.Q6_K, 4, 4096, 8192), (O.Q6_K, 5, 4112, 8192), (O.IQ4_XS, 3, 4112, 8192),
+                                  (O.Q4_1, 3, 8192, 4096)],
                          ids=lambda c: "%s_m%d_%dx%d" % (O.NAMES[c[0]], c[1], c[2], c[3]))
 def test_few_rows_take_the_few_token_kernel_when_a_workspace_has_room(hip, ref, case):
     """Below the tile kernel's row threshold the GEMV launches serve a matmul, four rows per pass -- except where the
     few-token kernel is faster still (from 3 rows where a GEMV launch takes two vectors at most, else from 5, on shapes it splits over k) and the caller's
-    workspace has room for its sums.  Without a workspace, or with a small one, the GEMV launches stay."""
+    workspace has room for its sums (or the kernel that keeps its tokens in registers, which stands in for it).  Without a workspace, or
+    with a small one, the GEMV launches stay."""
     import torch
     t, m, n, k_ = case
-    w = synth.weights(t, 91, n, k_)
+    w = weights(t, 91, n, k_)
     acts = ref.quantize_q8_0(synth.normal_f32(92, m * k_)).reshape(m, k_ // 32 * 34)
     kern = hip.HipKernel(t)
+    kernel = "gemm_direct_kernel" if takes_direct(t, m, n, k_) else "gemm_skinny_kernel"
     dw, da = torch.from_numpy(w).cuda(), torch.from_numpy(acts).cuda()
     ws = torch.empty(kern.gemm_workspace_bytes(m, n, k_), dtype=torch.uint8, device="cuda")
     # from 3 rows where a GEMV launch takes at most two vectors (rows of 2 or 5..8 steps of 64 lanes), else from 5
-    steps = -(-(k_ // (32 if t == O.IQ4_XS else 64)) // 64)
+    steps = -(-(k_ // (32 if t in (O.IQ4_XS, O.Q4_1) else 64)) // 64)
     expect_skinny = m >= (5 if steps in (1, 3, 4) else 3)
     outs = []
     for workspace in (ws, ws[:4096], None):
@@ -347,7 +386,7 @@ def test_few_rows_take_the_few_token_kernel_when_a_workspace_has_room(hip, ref, 
         torch.cuda.synchronize()
         took = last_launch()
         say(" ", O.NAMES[t], m, "workspace", None if workspace is None else workspace.numel(), "->", took)
-        assert took.startswith("gemm_skinny_kernel") == (expect_skinny and workspace is ws), took
+        assert took.startswith(kernel if expect_skinny and workspace is ws else "gemv_"), took
         outs.append(dy.cpu().numpy())
     for r in range(m):
         y_ref = canonical_ref(ref, t, w, acts[r], n, k_, threads=16)
@@ -443,15 +482,18 @@ def test_whole_k_in_lds(hip, ref, tuning, t, shape):
     assert torch.equal(dy2, dy[:m] + dy[:m]) and torch.equal(dy3, dy[:m] + db[None, :])
 
 
-def test_whole_k_in_lds_by_default(hip, ref):
-    """The default choice for matrices below 2^25 weights: from the rows on at which the GEMV launches end, up to 16."""
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q4_1], ids=lambda t: O.NAMES[t])
+def test_whole_k_in_lds_by_default(hip, ref, t):
+    """The default choice for matrices below 2^25 weights: from the rows on at which the GEMV launches end, up to 16.  (Q4_K: of
+    tokens off 16 bytes; the others' is the kernel that keeps its tokens in registers.)"""
     import torch
-    t, n, k_ = O.Q4_K, 2560, 2560
-    w, kern = weights(t, 95, n, k_), hip.HipKernel(O.Q4_K)
+    n, k_ = 2560, 2560
+    w, kern = weights(t, 95, n, k_), hip.HipKernel(t)
     dw = torch.from_numpy(w).cuda()
     for m, whole in ((8, False), (9, True), (16, True), (17, False)):
         acts = ref.quantize_q8_0(synth.normal_f32(96, m * k_)).reshape(m, k_ // 32 * 34)
-        da, dy = torch.from_numpy(acts).cuda(), torch.zeros((m, n), dtype=torch.float32, device="cuda")
+        da = off_16_bytes(acts) if t in DIRECT else torch.from_numpy(acts).cuda()
+        dy = torch.zeros((m, n), dtype=torch.float32, device="cuda")
         ws = torch.empty(kern.gemm_workspace_bytes(m, n, k_), dtype=torch.uint8, device="cuda")
         kern.gemm_q8_dev(dw, da, dy, m, n, k_, workspace=ws)
         torch.cuda.synchronize()
@@ -459,16 +501,16 @@ def test_whole_k_in_lds_by_default(hip, ref):
         assert_close(dy[m - 1].cpu().numpy(), canonical_ref(ref, t, w, acts[m - 1], n, k_), f"m={m}")
 
 
-@pytest.mark.parametrize("t", [O.Q4_K, O.Q6_K], ids=lambda t: O.NAMES[t])
+@pytest.mark.parametrize("t", [O.Q4_K, O.Q6_K, O.Q4_1], ids=lambda t: O.NAMES[t])
 def test_whole_k_in_lds_up_to_a_row_tile_per_compute_unit(hip, ref, t):
     """Rows of 4096 columns, whose k can be split over work groups instead: the whole k at once as long as no work group
-    walks a second row tile."""
+    walks a second row tile.  (Q4_K, Q6_K: of tokens off 16 bytes.)"""
     import torch
     m, k_ = 16, 4096
     one_each = 16 * hip.device_info()["compute_units"]
     kern = hip.HipKernel(t)
     acts = ref.quantize_q8_0(synth.normal_f32(97, m * k_)).reshape(m, k_ // 32 * 34)
-    da = torch.from_numpy(acts).cuda()
+    da = off_16_bytes(acts) if t in DIRECT else torch.from_numpy(acts).cuda()
     for n, whole in ((one_each, True), (one_each + 1, False)):
         say("whole k, a tile each", O.NAMES[t], n)
         w = weights(t, 98, n, k_)

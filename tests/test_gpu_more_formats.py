@@ -280,6 +280,7 @@ def test_prefill_tile_kernel(hip, ref, tuning, shape, t):
     the reference's fused kernel, every tile shape (split k, 64 x 128, 128 x 64), ragged edges, accumulate."""
     say("prefill", O.NAMES[t], shape)
     tuning("gemm_tile_min_rows", 1)
+    tuning("gemm_variant", 99)
     _prefill_tile_case(hip, ref, shape, t)
 
 

@@ -558,6 +558,7 @@ def test_prefill_tile_kernel(hip, ref, tuning, shape, t):
     m, n, k_ = shape
     say("prefill", O.NAMES[t], shape)
     tuning("gemm_tile_min_rows", 1)  # small shapes would otherwise take the GEMV route
+    tuning("gemm_variant", 99)       # and others the kernel that keeps its tokens in registers
     _prefill_tile_case(hip, ref, shape, t)
 
 
@@ -607,6 +608,7 @@ def test_prefill_tile_kernel_long_rows(hip, ref, tuning, shape, t):
     from test_gpu_prefill_f16 import last_launch
     say("prefill, long rows", O.NAMES[t], shape)
     tuning("gemm_tile_min_rows", 1)
+    tuning("gemm_variant", 99)
     _prefill_tile_case(hip, ref, shape, t)
     assert last_launch().startswith("gemm_tile_kernel"), last_launch()  # (the last call there is the sums' dump)
 
