@@ -475,15 +475,16 @@ __device__ __forceinline__ void direct_block(const typename Direct<F>::W &w, con
     using D = Direct<F>;
     constexpr float MAGIC = 12582912.0f;  // 1.5 * 2^23
     constexpr int KS = D::KS;
-    if constexpr (D::HAS_MIN) {
-#pragma unroll
-        for (int g = 0; g < 2; g++)
-#pragma unroll
-            for (int t = 0; t < TT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(z[g], tp[t][g], acc[t], 0, 0, 0);
-    }
     const uint64_t half = (q & 1) ? 0ull : ~0ull;
 #pragma unroll
     for (int s = 0; s < 8; s++) {
+        if constexpr (D::HAS_MIN) {
+            // Between the products of its four sub-blocks, which it mostly takes back: partial sums stay small.  (All of them first:
+            // 1.3 to 1.6 times the error against 64 bits on 1024 columns of Q4_K, Q5_K, Q4_0.)
+            if (s % 4 == 2)
+#pragma unroll
+                for (int t = 0; t < TT; t++) acc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(z[s / 4], tp[t][s / 4], acc[t], 0, 0, 0);
+        }
         const long op = D::operand(w, s);
 #pragma unroll
         for (int is = 0; is < KS; is++) {
