@@ -728,8 +728,11 @@ __device__ __forceinline__ void direct_streamed(const DirectJob j, uint8_t *lds)
             D::load(ring[u], rs_w, wrow, q, (blk0 + min(i, run - 1)) * D::BLOCK);
             __builtin_amdgcn_sched_barrier(0);
         };
-        v4f32 acc[XT][TT];
-        zero_sums<XT, TT>(acc);
+        // One token tile: the run's even and odd super-blocks apart, which halves the length of the chain (one chain: 1.2 times the
+        // error against 64 bits of the few-token kernel's split of k, Q6_K 4096 x 14336).  More: no registers left, nor is their error larger than the tile kernel's.
+        constexpr int CHAINS = TT == 1 ? 2 : 1;
+        v4f32 acc[CHAINS][TT];
+        zero_sums<CHAINS, TT>(acc);
         float old[xc.NE];
         xc.request(old, tile);
         request_tokens(0), request_weights(0, 0), request_weights(1, 1);
@@ -748,7 +751,7 @@ __device__ __forceinline__ void direct_streamed(const DirectJob j, uint8_t *lds)
             auto sink = [&](int t, int v, int s, int is, int ri) __attribute__((always_inline)) {
                 if (DUMP) direct_dump<F>(j, ri, 16 * tile + 4 * q + v, 16 * t + c, blk0 + i, s, is, true);
             };
-            direct_block<F, TT>(ring[u], tab, z, tk.a[0], tk.d[0], tk.p[0], q, magic, acc[0], sink);
+            direct_block<F, TT>(ring[u], tab, z, tk.a[0], tk.d[0], tk.p[0], q, magic, acc[u % CHAINS], sink);
             wave_lds_fence();
             request_weights(u, i + 2);
         };
@@ -756,13 +759,14 @@ __device__ __forceinline__ void direct_streamed(const DirectJob j, uint8_t *lds)
 #pragma clang loop unroll(disable)
         for (; i + 1 < run; i += 2) super_block(0, i), super_block(1, i + 1);
         if (i < run) super_block(0, i);
+        if constexpr (CHAINS == 2) acc[0][0] += acc[1][0];
         if constexpr (APART) {
-            xc.finish(acc, old, tile);
+            xc.finish(reinterpret_cast<v4f32(&)[1][TT]>(acc[0]), old, tile);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (what was requested past the run's end: the strip is written again)
         } else {
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();  // nothing is on its way to a strip and none is read any more
-            xc.finish(acc, old, tile);
+            xc.finish(reinterpret_cast<v4f32(&)[1][TT]>(acc[0]), old, tile);
             if (tile + j.step < tiles) __syncthreads();  // the sums have been read
         }
     }
