@@ -192,7 +192,8 @@ static hipError_t gemm_grouped_by_gemv(uint32_t type, const GemmArgs &a, hipStre
 // For device calls that bring a workspace; the host route's batched results are its GEMV's.
 bool gemm_direct_few_rows_pay(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
     return g_gemm_tile_min_rows.load(std::memory_order_relaxed) == 0 && g_gemm_variant.load(std::memory_order_relaxed) == 0 &&
-           gemm_direct_pays(type, m, n, k) && (uint64_t)n * k < (1ull << 25) && m >= (gemv_vecs_max(type, k) <= 2 ? 3u : 5u);
+           gemm_direct_pays(type, m, n, k) && (uint64_t)n * k < (1ull << 25) && m >= (gemv_vecs_max(type, k) <= 2 ? 3u : 5u) &&
+           (type != OXQ_TYPE_Q4_0 || k <= 4096);  // (256 x 6144, 5 / 8 rows: 5.9 / 6.7 us against 7.2 / 7.3)
 }
 // Whether a call that would take the few-token or the tile kernel takes that one instead.
 static bool gemm_direct_takes(uint32_t type, const GemmArgs &a) {

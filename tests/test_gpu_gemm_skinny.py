@@ -56,12 +56,14 @@ DIRECT = [O.Q4_K, O.Q5_K, O.Q6_K, O.IQ4_XS, O.Q4_0, O.Q8_0]
 
 
 def takes_direct(t, m, n, k_):
-    """(on 256 compute units)"""
+    """(the shapes below, on 256 compute units)"""
     if t not in DIRECT:
         return False
     if k_ <= 4096:
         return t != O.Q8_0 or n < 65536
-    return n <= 4096 and (t != O.Q8_0 or n >= 1536 if m <= 16 else t in (O.Q6_K, O.Q8_0) or k_ <= 20480)
+    if t == O.Q8_0 and k_ % 8192 == 0:  # (there the split of k is the faster one for up to 16 rows, and on few row tiles)
+        return n == 4096 and m > 16
+    return n <= 4096
 
 
 def off_16_bytes(acts):
