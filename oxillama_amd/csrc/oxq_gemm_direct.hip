@@ -24,9 +24,9 @@ static bool direct_format(uint32_t type) {
 }
 // Up to 32 rows of more than 4096 columns, of which a wave goes through nb / 8 super-blocks, against the few-token kernel's split of k: a
 // chain of `per` of them in every work group and a reduction launch, which this kernel does not have.  So the line is what its
-// chain may be longer by, in super-blocks of the matrix (8 a wave), fitted to 2400 calls of 3 to 16 rows: 20, 28 up to
-// eight rows (Q4_K 16 rows of 2048 x 13312, 20 above: 0.85 of the split's time, 2048 x 16384, 32: 0.95, 2048 x 20480, 32: 1.14); the light
-// Q4_0 8 and 16, Q8_0, whose split reads as fast as memory gives, -4 and 4 (2048 x 7680, -18, 0.80; 2048 x 14336, 24, 1.24).
+// chain may be longer by, in super-blocks of the matrix (8 a wave), fitted to 2400 calls of 3 to 16 rows: Q5_K, Q6_K 20,
+// Q4_K 24, IQ4_XS 28, and 8 more up to eight rows (Q4_K 16 rows of 2048 x 13312, 20 above: 0.85 of the split's time, x 16384, 32: 0.95 to 1.03,
+// x 20480, 32: 1.14); the light Q4_0 8 and 16, Q8_0, whose split reads as fast as memory gives, -4 and 4 (2048 x 7680, -18, 0.80; 2048 x 14336, 24, 1.24).
 // Where the split makes more work groups than there are compute units, two of them share some: 48 (Q5_K 40, Q4_0 32, Q8_0 28; 4096 x
 // 14336, 16 rows, Q4_K 0.83, Q6_K 0.83, Q8_0 0.98).  17 to 32 rows are split from 2^25 weights on, and take two passes
 // in Q6_K and Q8_0.
@@ -38,7 +38,8 @@ static bool direct_chain_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k,
     if (m <= 16) {
         const int most = type == OXQ_TYPE_Q8_0   ? (shared ? 28 : -4)
                          : type == OXQ_TYPE_Q4_0 ? (shared ? 32 : 8)
-                                                 : (shared ? (type == OXQ_TYPE_Q5_K ? 40 : 48) : 20);
+                         : shared                ? (type == OXQ_TYPE_Q5_K ? 40 : 48)
+                                                 : (type == OXQ_TYPE_IQ4_XS ? 28 : type == OXQ_TYPE_Q4_K ? 24 : 20);
         return above <= most + (m <= 8 ? 8 : 0);
     }
     if (type == OXQ_TYPE_Q8_0 || type == OXQ_TYPE_Q6_K) {
@@ -54,14 +55,14 @@ static bool direct_chain_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k,
 // 14336 x 4096 16.5 / 12.5, 8960 x 1536 7.9 / 5.9, 128256 x 4096 71 / 67; Q6_K 4096 x 4096 10.3 / 7.2, 14336 x 4096 23.1 / 19.7; Q8_0 10.1 / 8.7,
 // 24.2 / 22.8; 32 rows of Q4_K 4096 x 4096 13.3 / 8.7, 14336 x 4096 21.5 / 16.4.
 //  * Longer rows (streamed: a wave's tokens pass through its registers once per row tile): while no work group walks a second row
-//    tile, and by direct_chain_pays (867 calls of up to 32 rows on 29 matrices, 0.70 of the time in the mean, the worst 1.07).  16 rows of 4096 x 14336: Q4_K 19.3 / 15.8, Q6_K 25.4 / 21.2, IQ4_XS 19.9 / 15.2, Q8_0 26.5 / 26;
+//    tile, and by direct_chain_pays (887 calls of up to 32 rows on 29 matrices, 0.70 of the time in the mean, the worst 1.07).  16 rows of 4096 x 14336: Q4_K 19.3 / 15.8, Q6_K 25.4 / 21.2, IQ4_XS 19.9 / 15.2, Q8_0 26.5 / 26;
 //    28672 x 8192 of Q4_K 42 / 63.  Beyond 32768 columns: not measured.  Q8_0 of 1024 x 8192 14.3 / 15.9.
 //  * Q8_0 vocabularies, where the bytes are the time: 128256 x 4096, 16 rows, 117 / 134.
-// More than 32 rows, up to 512, against the tile kernel and its token re-layout launch: 2478 calls of six formats on 57
+// More than 32 rows, up to 512, against the tile kernel and its token re-layout launch: 2480 calls of six formats on 57
 // matrices, 0.62 of the time in the mean.  The tile kernel is a serial chain
 // of k / 4 where the work groups here meet k / 8 or k / 16, and gains on this one only by weights unpacked
 // for more tokens.  So the line is drawn at the tiles of 16 x 16 a work group goes through (`work`):
-//  * up to 2048 columns 28, Q6_K 24 (1114 calls, 0.65 of the time in the mean, the worst 1.06; beyond 0.81 to 1.14, Q6_K 333 rows of 4096 x
+//  * up to 2048 columns 28, Q6_K beyond 1024 24 (1116 calls, 0.65 of the time in the mean, the worst 1.05; beyond 0.81 to 1.14, Q6_K 333 rows of 4096 x
 //    1536, 28, 27.8 / 29.3), Q8_0 56.  77 rows of Q4_0: 1536 x 1536 12.1 / 6.1, 256 x 1536 11.6 / 3.7, 8960 x 1536 22.1 / 13;
 //  * up to 4096 columns, two token tiles at most and two super-blocks a wave, a part of which is idle in shorter rows (hence the
 //    square): Q4_K 28 (64 rows of 4096 x 4096 13.5 / 11.1, 1024 x 4096 12.2 / 5.4, 128 of 14336 x 4096 42.8 / 36.9), IQ4_XS 14, Q6_K
@@ -88,7 +89,7 @@ bool gemm_direct_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k) {
     }
     if (f16) return false;
     const uint64_t work = (uint64_t)walk * tt;
-    if (k <= 2048) return work <= (type == OXQ_TYPE_Q8_0 ? 56u : type == OXQ_TYPE_Q6_K ? 24u : 28u);
+    if (k <= 2048) return work <= (type == OXQ_TYPE_Q8_0 ? 56u : type == OXQ_TYPE_Q6_K && k > 1024 ? 24u : 28u);
     return work * 256 <= (uint64_t)nb * nb * (type == OXQ_TYPE_Q8_0 ? 4u : type == OXQ_TYPE_Q6_K ? 8u : type == OXQ_TYPE_IQ4_XS ? 14u : 28u);
 }
 

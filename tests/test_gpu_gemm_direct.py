@@ -73,7 +73,7 @@ def test_direct_kernel(hip, ref, tuning, t, shape):
     (O.Q8_0, 16, 1536, 5120, True), (O.Q4_0, 16, 48, 33024, False), (O.Q4_0, 77, 8960, 1536, True), (O.Q4_K, 64, 4096, 14336, False), (O.Q6_K, 64, 4096, 14336, True),
     (O.Q4_K, 128, 14336, 4096, True), (O.Q6_K, 80, 14336, 4096, False), (O.Q8_0, 512, 1024, 2048, True), (O.Q4_K, 513, 256, 2048, False), (O.Q4_1, 16, 2560, 2560, False),
     # long rows: the chain against the few-token kernel's split of k, alone on its compute units and not, up to eight rows and up to 32
-    (O.Q4_K, 16, 2048, 13312, True), (O.Q4_K, 16, 2048, 14336, False), (O.Q4_K, 8, 2048, 14336, True), (O.Q4_K, 8, 2048, 20480, False), (O.Q4_K, 16, 4096, 26624, True),
+    (O.Q4_K, 16, 2048, 13312, True), (O.Q4_K, 16, 2048, 14336, True), (O.Q4_K, 16, 2048, 15360, False), (O.Q4_K, 8, 2048, 15360, True), (O.IQ4_XS, 16, 2048, 15360, True), (O.Q5_K, 16, 2048, 14336, False), (O.Q4_K, 8, 2048, 20480, True), (O.Q4_K, 8, 2048, 22528, False), (O.Q4_K, 16, 4096, 26624, True),
     (O.Q5_K, 16, 4096, 26624, True), (O.Q5_K, 16, 4096, 27648, False), (O.Q4_0, 16, 2048, 11264, False), (O.Q8_0, 16, 2048, 7168, True), (O.Q8_0, 16, 2048, 8192, False),
     (O.Q8_0, 16, 4096, 14336, True), (O.Q8_0, 32, 2048, 14336, True), (O.Q8_0, 32, 2048, 16384, False), (O.Q6_K, 32, 1024, 32512, True),
     (O.Q6_K, 32, 1024, 32768, False), (O.Q4_K, 32, 2560, 16384, True), (O.Q4_K, 32, 2560, 17408, False), (O.Q4_0, 5, 256, 6144, False),
