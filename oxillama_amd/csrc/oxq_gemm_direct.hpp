@@ -426,7 +426,7 @@ __device__ __forceinline__ void direct_tokens(DirectTokens<F, PB, TT> &tk, const
 #pragma unroll
             for (int g = 0; g < 2; g++) {
                 // lane q reads the scale of sub-block 4g + q; every lane needs all four
-                // (a super-block past the last: nothing was staged, zeros)
+                // (a super-block past the last: the next token's bytes were staged, or zeros; neither counts)
                 const float d = (uint32_t)b < live ? h2f(reinterpret_cast<const lds_h1 *>(scale + 272 * b + 136 * g)->v) : 0.0f;
                 uint32_t d0 = __builtin_bit_cast(uint32_t, d), d1 = d0;
                 swap16(d0, d1);
@@ -507,7 +507,7 @@ __device__ __forceinline__ void direct_block(const typename Direct<F>::W &w, con
     }
 }
 
-// What a work group of eight waves works on: one matrix (or expert), at most 16 * TT token rows.
+// What a work group works on: row tiles of the matrix, at most 16 * TT token rows.
 struct DirectJob {
     const uint8_t *W, *A;  // the matrix; the first token's blocks
     float *out;            // the first token's row
@@ -515,8 +515,7 @@ struct DirectJob {
     const float *bias;
     uint32_t rows, n, k;
     int accumulate;
-    uint32_t first, end, step;  // sets of RG row tiles: first, first + step, ..., below end
-    uint32_t sb0, sbs;          // super-blocks of k (streamed: all of them)
+    uint32_t first, end, step;  // sets of RG row tiles (streamed: one): first, first + step, ..., below end
 };
 
 template <int N, int TT>
@@ -595,9 +594,9 @@ __device__ __forceinline__ void direct_resident(const DirectJob j, uint8_t *lds)
     constexpr int U = 2, XT = direct_turn<TT, WAVES>();  // row tiles whose weights are in flight; that are exchanged at once
     const uint32_t lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), part = wave % KP, rg = wave / KP;
-    const uint32_t live = j.sbs > part * PB ? min((uint32_t)PB, j.sbs - part * PB) : 0;
-    const uint32_t blk0 = j.sb0 + part * PB, sets = j.end;
-    const uint32_t row_bytes = j.k / 256 * D::BLOCK, arow = j.k / 256 * 272;
+    const uint32_t nb = j.k / 256, blk0 = part * PB, sets = j.end;
+    const uint32_t live = nb > blk0 ? min((uint32_t)PB, nb - blk0) : 0;  // super-blocks of this part
+    const uint32_t row_bytes = nb * D::BLOCK, arow = nb * 272;
     constexpr bool APART = direct_exchange_apart<F, PB, TT, WAVES>();
     uint8_t *const tab = lds + wave * (direct_tables<F, WAVES>() / WAVES);
     uint8_t *const strips = lds + direct_tables<F, WAVES>(), *const strip = strips + wave * (direct_strips<PB, TT, WAVES>() / WAVES);
@@ -612,7 +611,7 @@ __device__ __forceinline__ void direct_resident(const DirectJob j, uint8_t *lds)
         const DirectWindow win = direct_window(set, sets, rg, RG, j.n, row_bytes);
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint8_t *>(j.W + (size_t)win.row0 * row_bytes), 0, (int)win.records, BUFFER_FLAGS);
-        D::load(ring[u][b], rs, wrow, q, direct_super_block(blk0 + b, j.k / 256) * D::BLOCK);
+        D::load(ring[u][b], rs, wrow, q, direct_super_block(blk0 + b, nb) * D::BLOCK);
     };
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -696,10 +695,9 @@ __device__ __forceinline__ void direct_resident(const DirectJob j, uint8_t *lds)
 template <class F, int TT, int WAVES, bool DUMP>
 __device__ __forceinline__ void direct_streamed(const DirectJob j, uint8_t *lds) {
     using D = Direct<F>;
-    constexpr int XT = 1;
     const uint32_t lane = threadIdx.x & 63, c = lane & 15, q = lane >> 4;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint32_t nb = j.k / 256, tiles = (j.n + 15) / 16;
+    const uint32_t nb = j.k / 256, tiles = j.end;
     const uint32_t blk0 = wave * (nb / WAVES) + min(wave, nb % WAVES), run = nb / WAVES + (wave < nb % WAVES ? 1 : 0);  // (nb >= WAVES: no empty run)
     const uint32_t row_bytes = nb * D::BLOCK, arow = nb * 272, wrow = c * row_bytes;
     uint8_t *const tab = lds + wave * (direct_tables<F, WAVES>() / WAVES);
@@ -710,7 +708,7 @@ __device__ __forceinline__ void direct_streamed(const DirectJob j, uint8_t *lds)
     v4i32 magic;
     asm volatile("v_mov_b32 %0, 0x4b400000\n\tv_mov_b32 %1, 0x4b400000\n\tv_mov_b32 %2, 0x4b400000\n\tv_mov_b32 %3, 0x4b400000"
                  : "=v"(magic[0]), "=v"(magic[1]), "=v"(magic[2]), "=v"(magic[3]));
-    DirectExchange<WAVES, TT, XT, WAVES> xc{j, ex, 0};
+    DirectExchange<WAVES, TT, 1, WAVES> xc{j, ex, 0};
 #pragma clang loop unroll(disable)
     for (uint32_t tile = j.first; tile < tiles; tile += j.step) {
         const DirectWindow win = direct_window(tile, tiles, 0, 1, j.n, row_bytes);
@@ -782,7 +780,7 @@ __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(WAVE
     const uint32_t t0 = blockIdx.y * (16 * TT), nb = k / 256, tiles = (n + 15) / 16;
     constexpr uint32_t RG = KP ? WAVES / (KP ? KP : 1) : 1;
     const DirectJob j = {W, A + (size_t)t0 * nb * 272, out + (size_t)t0 * n, DUMP ? sums + (size_t)t0 * n * (nb * 8 * Direct<F>::KS) : nullptr, bias,
-                         min(m - t0, (uint32_t)(16 * TT)), n, k, accumulate, blockIdx.x, (tiles + RG - 1) / RG, gridDim.x, 0, nb};
+                         min(m - t0, (uint32_t)(16 * TT)), n, k, accumulate, blockIdx.x, (tiles + RG - 1) / RG, gridDim.x};
     if constexpr (KP == 0) direct_streamed<F, TT, WAVES, DUMP>(j, lds);
     else direct_resident<F, PB, KP, TT, WAVES, DUMP>(j, lds);
 }

@@ -1,5 +1,5 @@
-"""The few-token kernel whose weights go straight from memory into the matrix core's registers (oxq_gemm_direct.hpp), on one matrix
-of up to 32 token rows, against the CPU oracle: fp32 within 1e-5 * |y_ref|_inf, the integer sums of its debug dump bit-exact."""
+"""The kernel whose weights go straight from memory into the matrix core's registers and whose tokens stay there (oxq_gemm_direct.hpp), on
+one matrix and up to 512 token rows, against the CPU oracle: fp32 within 1e-5 * |y_ref|_inf, the integer sums of its debug dump bit-exact."""
 import numpy as np
 import pytest
 
@@ -17,7 +17,7 @@ FORMATS = [O.Q4_K, O.Q5_K, O.Q6_K, O.IQ4_XS, O.Q4_0, O.Q8_0]
 # of two (the last of them with one super-block or none); longer: each wave its own run (17: runs of two and three; 33; 43).
 # Row tiles with rows to spare (18 rows, not one: the bar is 1e-5 of the largest of a token's results, and a single result can be far
 # smaller than its terms), an odd number of tiles, more tiles than work groups; odd super-blocks put every second row
-# of the formats of 18, 34 and 210 bytes off a dword.
+# of Q6_K off a dword.
 SHAPES = [(16, 33, 512), (1, 18, 768), (7, 20, 1024), (16, 4129, 512), (13, 100, 1280), (5, 8300, 2048), (9, 4113, 2304), (16, 40, 3840),
           (16, 17, 4096), (3, 4099, 4096), (17, 33, 768), (32, 100, 1280), (21, 4131, 2048), (18, 50, 2304), (32, 35, 3840), (25, 8210, 4096),
           (16, 35, 4352), (2, 16, 8448), (11, 4099, 11008)]
