@@ -58,6 +58,8 @@ __device__ __forceinline__ long i8x8(uint32_t lo, uint32_t hi) { return (long)((
 //   BLOCK      bytes of 256 weights
 //   KS         scale factors per sub-block (two: of 16 weights each)
 //   HAS_MIN    a zero-point term
+//   TIMES      what the operand is a multiple of (a power of two that the factors take out again)
+//   OFFSET     what the dump of the integer sums has added to every weight
 //   ORDER      which of a block's token bytes the k-slots of lane q hold: 0 the eight from 8 * {0, 2, 1, 3}[q] on; 1 the eight
 //              from 8 q on, even ones first
 //   W, load    the lane's bytes of a super-block (at byte `so` of the row that starts at `row`): lane q's share, LOADS
@@ -75,7 +77,7 @@ template <>
 struct Direct<TileQ4K> {  // reference/q4_k.rs:27-99
     static constexpr bool OK = true, HAS_MIN = true;
     static constexpr uint32_t BLOCK = 144, LOADS = 3;
-    static constexpr int KS = 1, ORDER = 0;
+    static constexpr int KS = 1, ORDER = 0, TIMES = 1, OFFSET = 0;
     struct W {
         u32x4 hdr, qs[2];
     };
@@ -126,7 +128,7 @@ template <>
 struct Direct<TileQ6K> {
     static constexpr bool OK = true, HAS_MIN = false;
     static constexpr uint32_t BLOCK = 210, LOADS = 5;
-    static constexpr int KS = 2, ORDER = 0;
+    static constexpr int KS = 2, ORDER = 0, TIMES = 4, OFFSET = 0;
     struct W {
         u32x4 ql[2], qh;
         uint32_t sc, d, shift;
@@ -172,7 +174,7 @@ template <>
 struct Direct<TileIQ4XS> {
     static constexpr bool OK = true, HAS_MIN = false;
     static constexpr uint32_t BLOCK = 136, LOADS = 3;
-    static constexpr int KS = 1, ORDER = 1;
+    static constexpr int KS = 1, ORDER = 1, TIMES = 1, OFFSET = 0;
     struct W {
         u32x4 qs[2];
         u32x2 hdr;
@@ -207,7 +209,7 @@ template <>
 struct Direct<DirectQ5K> {
     static constexpr bool OK = true, HAS_MIN = true;
     static constexpr uint32_t BLOCK = 176, LOADS = 4;
-    static constexpr int KS = 1, ORDER = 0;
+    static constexpr int KS = 1, ORDER = 0, TIMES = 1, OFFSET = 0;
     struct W {
         u32x4 hdr, qs[2];
         u32x2 qh;
@@ -240,12 +242,14 @@ struct Direct<DirectQ5K> {
 // payload starts on one, the dword in which the even block ends also holds the odd one's scale.)
 
 // Q4_0 (reference/q4_0.rs:22-49): eight blocks of 18 bytes stand for a super-block; a lane takes the nibbles of blocks q and
-// q + 4.  The operand is the unsigned nibble, the "- 8" goes through the zero-point term.
+// q + 4.  The operand is 16 (n - 8), the nibble at bits 4 .. 7 with the topmost inverted: no zero-point term, which would cost an
+// infinite token its infinities (the GEMV that serves fewer rows has them) and sums as exact as integers are.  The dump is
+// the other kernels', of the unsigned nibbles.
 template <>
 struct Direct<TileQ4_0> {
-    static constexpr bool OK = true, HAS_MIN = true;
+    static constexpr bool OK = true, HAS_MIN = false;
     static constexpr uint32_t BLOCK = 144, LOADS = 4;
-    static constexpr int KS = 1, ORDER = 1;
+    static constexpr int KS = 1, ORDER = 1, TIMES = 16, OFFSET = 8;
     struct W {
         u32x4 qs[2];
         uint32_t x[2];
@@ -265,15 +269,16 @@ struct Direct<TileQ4_0> {
             w.d[i] = q & 1 ? w.x[i] >> 16 : w.qs[i][0] & 0xFFFF;
             w.qs[i] = from_dword(w.qs[i], w.x[i], q & 1 ? 0 : 16);
             transpose_pieces(w.qs[i]);
+            for (int j = 0; j < 4; j++) w.qs[i][j] ^= 0x88888888u;
         }
     }
     static __device__ __forceinline__ long operand(const W &w, int s) {
         const uint32_t v = w.qs[s >> 2][s & 3];
-        return i8x8(v & 0x0F0F0F0Fu, (v >> 4) & 0x0F0F0F0Fu);
+        return i8x8((v << 4) & 0xF0F0F0F0u, v & 0xF0F0F0F0u);
     }
-    static __device__ __forceinline__ void factors(const W &w, uint32_t, float (&f)[2], float (&z)[2]) {
+    static __device__ __forceinline__ void factors(const W &w, uint32_t, float (&f)[2], float (&)[2]) {
 #pragma unroll
-        for (int i = 0; i < 2; i++) f[i] = h2f(w.d[i]), z[i] = -(8.0f * f[i]);
+        for (int i = 0; i < 2; i++) f[i] = 0.0625f * h2f(w.d[i]);
     }
 };
 
@@ -282,7 +287,7 @@ template <>
 struct Direct<TileQ8_0> {
     static constexpr bool OK = true, HAS_MIN = false;
     static constexpr uint32_t BLOCK = 272, LOADS = 8;
-    static constexpr int KS = 1, ORDER = 0;
+    static constexpr int KS = 1, ORDER = 0, TIMES = 1, OFFSET = 0;
     struct W {
         u32x4 qs[4];
         uint32_t x[4];
@@ -467,8 +472,8 @@ __device__ __forceinline__ void direct_factors(const typename Direct<F>::W &w, u
 }
 
 // One super-block of the wave's rows (arranged; factors in the table) against its tokens.
-// sink(t, v, s, is, sum): every integer sum, as the MFMA left it.
-template <class F, int TT, class Sink>
+// sink(t, v, s, is, sum): every integer sum, as the MFMA left it (for the dump, with OFFSET times the token's).
+template <class F, int TT, bool DUMP, class Sink>
 __device__ __forceinline__ void direct_block(const typename Direct<F>::W &w, const uint8_t *tab, const float (&z)[2],
                                              const u32x2 (&ta)[TT][8], const float (&td)[TT][8], const float (&tp)[TT][2], uint32_t q,
                                              const v4i32 magic, v4f32 (&acc)[TT], const Sink &sink) {
@@ -495,11 +500,14 @@ __device__ __forceinline__ void direct_block(const typename Direct<F>::W &w, con
                 const u32x2 a = ta[t][s];
                 const float da = td[t][s];
                 const v4i32 r = __builtin_amdgcn_mfma_i32_16x16x32_i8(o, i8x8(a[0], a[1]), magic, 0, 0, 0);
+                v4i32 token = {0, 0, 0, 0};
+                if constexpr (DUMP && D::OFFSET) token = __builtin_amdgcn_mfma_i32_16x16x32_i8(0x0101010101010101l, i8x8(a[0], a[1]), token, 0, 0, 0);
 #pragma unroll
                 for (int v = 0; v < 4; v++) {
-                    const int ri = r[v];
+                    int ri = r[v];
                     const float x = fmaf(__builtin_bit_cast(float, ri), dsc[v], corr[v]);  // fl(dsc * isum)
                     acc[t][v] = fmaf(x, da, acc[t][v]);
+                    if constexpr (DUMP) ri += D::TIMES * D::OFFSET * token[v];
                     sink(t, v, s, is, ri);
                 }
             }
@@ -531,7 +539,7 @@ template <class F>
 __device__ __forceinline__ void direct_dump(const DirectJob &j, int ri, uint32_t row, uint32_t tok, uint32_t blk, int s, int is, bool live) {
     using D = Direct<F>;
     if (row < j.n && tok < j.rows && live)
-        j.sums[((size_t)tok * j.n + row) * (j.k / 32 * D::KS) + (blk * 8 + s) * D::KS + is] = (ri - 0x4B400000) / (D::KS == 2 ? 4 : 1);
+        j.sums[((size_t)tok * j.n + row) * (j.k / 32 * D::KS) + (blk * 8 + s) * D::KS + is] = (ri - 0x4B400000) / D::TIMES;
 }
 
 // Where the parts' sums of XT sets of WAVES / KP row tiles meet, [turn][wave][set][token tile] in LDS: thread e of each 256 takes row
@@ -654,7 +662,7 @@ __device__ __forceinline__ void direct_resident(const DirectJob j, uint8_t *lds)
             auto sink = [&](int t, int v, int s, int is, int ri) __attribute__((always_inline)) {
                 if (DUMP) direct_dump<F>(j, ri, 16 * (set * RG + rg) + 4 * q + v, 16 * t + c, blk0 + b, s, is, (uint32_t)b < live);
             };
-            direct_block<F, TT>(ring[u][b], tb, z, tk.a[b], tk.d[b], tk.p[b], q, magic, acc, sink);
+            direct_block<F, TT, DUMP>(ring[u][b], tb, z, tk.a[b], tk.d[b], tk.p[b], q, magic, acc, sink);
             wave_lds_fence();
             // (only now: a load while the slot is still in use would go to other registers and be copied when it arrives)
             load(u, b, set + U * j.step);
@@ -749,7 +757,7 @@ __device__ __forceinline__ void direct_streamed(const DirectJob j, uint8_t *lds)
             auto sink = [&](int t, int v, int s, int is, int ri) __attribute__((always_inline)) {
                 if (DUMP) direct_dump<F>(j, ri, 16 * tile + 4 * q + v, 16 * t + c, blk0 + i, s, is, true);
             };
-            direct_block<F, TT>(ring[u], tab, z, tk.a[0], tk.d[0], tk.p[0], q, magic, acc[u % CHAINS], sink);
+            direct_block<F, TT, DUMP>(ring[u], tab, z, tk.a[0], tk.d[0], tk.p[0], q, magic, acc[u % CHAINS], sink);
             wave_lds_fence();
             request_weights(u, i + 2);
         };
