@@ -4,7 +4,7 @@
 namespace oxq {
 
 // Token tiles a work group takes: as many as registers hold, fewer where the matrix has so few row tiles that work groups for more
-// runs of tokens still find a compute unit each (256 x 1536 of Q4_K, 77 rows: five runs of one tile, 3.7 us).
+// runs of tokens still find a compute unit each (256 x 1536 of Q4_K, 77 rows: five runs of one tile, 3.6 us).
 static uint32_t direct_token_tiles(uint32_t m, uint32_t n, uint32_t k) {
     const uint32_t tiles = (m + 15) / 16, most = k > 2048 && k <= 4096 ? 2 : 4, rows = (n + 15) / 16;
     const uint32_t fewest = (tiles + most - 1) / most, fill = device_cus() / rows;
@@ -59,11 +59,11 @@ static bool direct_chain_pays(uint32_t type, uint32_t m, uint32_t n, uint32_t k,
 //    28672 x 8192 of Q4_K 42 / 63.  Beyond 32768 columns: not measured.  Q8_0 of 1024 x 8192 14.3 / 15.9.
 //  * Q8_0 vocabularies, where the bytes are the time: 128256 x 4096, 16 rows, 117 / 134.
 // More than 32 rows, up to 512, against the tile kernel and its token re-layout launch: 2480 calls of six formats on 57
-// matrices, 0.62 of the time in the mean.  The tile kernel is a serial chain
+// matrices, 0.61 of the time in the mean.  The tile kernel is a serial chain
 // of k / 4 where the work groups here meet k / 8 or k / 16, and gains on this one only by weights unpacked
 // for more tokens.  So the line is drawn at the tiles of 16 x 16 a work group goes through (`work`):
-//  * up to 2048 columns 28, Q6_K beyond 1024 24 (1116 calls, 0.65 of the time in the mean, the worst 1.05; beyond 0.81 to 1.14, Q6_K 333 rows of 4096 x
-//    1536, 28, 27.8 / 29.3), Q8_0 56.  77 rows of Q4_0: 1536 x 1536 12.1 / 6.1, 256 x 1536 11.6 / 3.7, 8960 x 1536 22.1 / 13;
+//  * up to 2048 columns 28, Q6_K beyond 1024 24 (1116 calls, 0.64 of the time in the mean, the worst 1.05; beyond 0.81 to 1.14, Q6_K 333 rows of 4096 x
+//    1536, 28, 27.8 / 29.3), Q8_0 56.  77 rows of Q4_0: 1536 x 1536 12.2 / 5.6, 256 x 1536 11.6 / 3.6, 8960 x 1536 22.3 / 12.2;
 //  * up to 4096 columns, two token tiles at most and two super-blocks a wave, a part of which is idle in shorter rows (hence the
 //    square): Q4_K 28 (64 rows of 4096 x 4096 13.5 / 11.1, 1024 x 4096 12.2 / 5.4, 128 of 14336 x 4096 42.8 / 36.9), IQ4_XS 14, Q6_K
 //    8 (64 rows of 4096 x 4096 18.8 / 15.2; 112 of 14336 x 4096, 16, 1.12 of the f16 kernel's), Q8_0 4 (64 rows of 4096 x 4096 19.4 / 14.9; 80, 8, 21.2 / 21.9);

@@ -2,7 +2,7 @@
 //   out[m x n] (+)= A_q8[m rows of Q8_0 blocks] x W[n x k]^T
 // (the reference's gemm loop over matvec_q8_fused, crates/oxillama-quant/src/reference/q4_k.rs:186-201, :218-333) for a
 // decode batch or a short prompt on one matrix, where its few tiles of 16 rows x 16 tokens make the launch's ramp and the
-// chain along k the time (77 rows of Q4_0: 1536 x 1536 12.1 us on the tile kernel, 6.1 here; 8960 x 1536 22.1 / 13).
+// chain along k the time (77 rows of Q4_0: 1536 x 1536 12.2 us on the tile kernel, 5.6 here; 8960 x 1536 22.3 / 12.2).
 //
 //  * k is dealt to the waves of a work group, PB super-blocks each, and a wave keeps its part of the tokens in registers, in
 //    operand order, for as long as the work group walks tiles of 16 weight rows: nothing about the tokens is read again.
